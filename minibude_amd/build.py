@@ -40,6 +40,7 @@ LIB_SOURCES = [
     "prep.cpp",
     "deck_synth.cpp",
     "deck_io.cpp",
+    "items.hip",
     "fasten_plain.hip",
     "capi_plain.hip",
     "capi_noalloc.hip",

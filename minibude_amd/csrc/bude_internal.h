@@ -64,7 +64,7 @@ PairCoef pair_coef(const BudeFFParams &p, const BudeFFParams &l);
 // constant over a group, so the kernels load them once per (ligand atom,
 // group) and stream only coordinates inside a group.
 struct ProteinGroups {
-  std::vector<float> xyzw;        // 4 floats per atom (x, y, z, 0), grouped
+  std::vector<float> xyzw;        // 4 floats per atom (x, y, z, group index bits), grouped
   std::vector<int32_t> begin;     // ngroups + 1 offsets into the atoms
   std::vector<int32_t> type;      // forcefield type of each group
   size_t ngroups() const { return type.size(); }

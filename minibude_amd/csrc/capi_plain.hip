@@ -12,6 +12,7 @@
 #include "bude_internal.h"
 #include "fasten_plain.h"
 #include "hip_util.h"
+#include "items.h"
 
 namespace {
 
@@ -30,6 +31,7 @@ struct bude_ctx {
   int device = 0;
   size_t natpro = 0, natlig = 0, ntypes = 0, nposes = 0, ngroups = 0;
   bude::DeviceBuffer protein, group_begin, coef, ligand, poses, energies;
+  bude::items::Deck sorted;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double context_ms = 0.0;
@@ -140,6 +142,9 @@ extern "C" int bude_mi355x_create(int device, const BudeAtom *protein, size_t na
                                    hipMemcpyHostToDevice),
                          "hipMemcpy poses");
   if (!st) st = c->energies.alloc(nposes * sizeof(float));
+  if (!st)
+    st = c->sorted.prepare(groups, forcefield, std::vector<BudeAtom>(ligand, ligand + natlig), {0, int32_t(natlig)},
+                           {bude::items::Segment{0, 0, int64_t(nposes)}});
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev0), "hipEventCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev1), "hipEventCreate");
@@ -182,7 +187,10 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   for (size_t i = 0; i < warmup + iterations; i++) {
     const auto t0 = std::chrono::steady_clock::now();
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
-    if (int st = bude::hip_check(bude::launch_plain(a, int(wgsize), ctx->stream), "fasten_plain launch")) return st;
+    const hipError_t le = ctx->sorted.usable()
+                              ? ctx->sorted.launch(a.protein, a.poses, a.stride, a.energies, ctx->stream)
+                              : bude::launch_plain(a, int(wgsize), ctx->stream);
+    if (int st = bude::hip_check(le, "fasten_plain launch")) return st;
     if (int st = bude::hip_check(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord")) return st;
     if (int st = bude::hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return st;
     if (host_ms) host_ms[i] = ms_since(t0);

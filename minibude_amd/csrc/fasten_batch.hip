@@ -61,17 +61,20 @@ __global__ __launch_bounds__(WG) void fasten_batch_kernel(
     }
     for (int il = 0; il < m.natlig; ++il) {
       const float4 la = ligands[m.lig_off + il];
-      float lx[RB], ly[RB], lz[RB];
+      float lx[RB], ly[RB], lz[RB], ea[RB];
 #pragma unroll
       for (int k = 0; k < RB; ++k) {
         const float *mm = tr[k].m;
-        lx[k] = mm[3] + la.x * mm[0] + la.y * mm[1] + la.z * mm[2];
-        ly[k] = mm[7] + la.x * mm[4] + la.y * mm[5] + la.z * mm[6];
-        lz[k] = mm[11] + la.x * mm[8] + la.y * mm[9] + la.z * mm[10];
+        lx[k] = place(mm[0], mm[1], mm[2], mm[3], la);
+        ly[k] = place(mm[4], mm[5], mm[6], mm[7], la);
+        lz[k] = place(mm[8], mm[9], mm[10], mm[11], la);
+        ea[k] = 0.f;
       }
       const PairCoef *cl = coef + size_t(m.coef_off) + size_t(il) * ngroups;
       for (int g = 0; g < ngroups; ++g)
-        group_dispatch<RB, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, e);
+        group_dispatch<RB, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, ea);
+#pragma unroll
+      for (int k = 0; k < RB; ++k) e[k] += ea[k];
     }
 #pragma unroll
     for (int k = 0; k < RB; ++k) {

@@ -40,6 +40,12 @@ __device__ __forceinline__ Xform make_xform(const float *__restrict__ poses, siz
   return t;
 }
 
+// One coordinate of a ligand atom under a transform's row (r0, r1, r2, t):
+// written out, so that every kernel rounds it the same way.
+__device__ __forceinline__ float place(float r0, float r1, float r2, float t, const float4 la) {
+  return __builtin_fmaf(la.z, r2, __builtin_fmaf(la.y, r1, __builtin_fmaf(la.x, r0, t)));
+}
+
 // Hinge forms of the charge / desolvation terms (see PairCoef):
 //   kFormB  sat(1 + b * neg_e1) with b = d - radij (one extra subtraction,
 //           matches the reference's rounding of 1 - b*elcdst1 exactly)
@@ -143,9 +149,11 @@ __device__ __forceinline__ void group_pairs(const float4 *__restrict__ prot, int
 }
 
 // One protein group: its pairs are summed into a fresh partial sum that is
-// then added to the pose total, so the running FP32 total takes one rounding
-// per (ligand atom, group) instead of three per pair (a shorter, smaller-
-// magnitude accumulation than the reference's single running sum).
+// then added to the ligand atom's total e, which every kernel in turn adds to
+// its pose's, so the running FP32 totals take one rounding per group and per
+// ligand atom instead of three per pair (shorter, smaller-magnitude
+// accumulations than the reference's single running sum), and a ligand
+// atom's energy does not depend on which kernel or wave computed it.
 template <int RB, int FORM>
 __device__ __forceinline__ void group_dispatch(const float4 *__restrict__ prot, int i0, int i1, const PairCoef c,
                                                const float (&lx)[RB], const float (&ly)[RB],

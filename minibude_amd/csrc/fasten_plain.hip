@@ -52,17 +52,20 @@ __global__ __launch_bounds__(WG) void fasten_plain_kernel(
 
     for (int il = 0; il < natlig; ++il) {
       const float4 la = ligand[il];
-      float lx[RB], ly[RB], lz[RB];
+      float lx[RB], ly[RB], lz[RB], ea[RB];
 #pragma unroll
       for (int k = 0; k < RB; ++k) {
         const float *m = t[k].m;
-        lx[k] = m[3] + la.x * m[0] + la.y * m[1] + la.z * m[2];
-        ly[k] = m[7] + la.x * m[4] + la.y * m[5] + la.z * m[6];
-        lz[k] = m[11] + la.x * m[8] + la.y * m[9] + la.z * m[10];
+        lx[k] = place(m[0], m[1], m[2], m[3], la);
+        ly[k] = place(m[4], m[5], m[6], m[7], la);
+        lz[k] = place(m[8], m[9], m[10], m[11], la);
+        ea[k] = 0.f;
       }
       const PairCoef *cl = coef + size_t(il) * ngroups;
       for (int g = 0; g < ngroups; ++g)
-        group_dispatch<RB, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, e);
+        group_dispatch<RB, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, ea);
+#pragma unroll
+      for (int k = 0; k < RB; ++k) e[k] += ea[k];
     }
 
 #pragma unroll

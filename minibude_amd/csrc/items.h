@@ -1,0 +1,109 @@
+// items.h -- exact pose energies from sorted (pose, ligand atom) items.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <vector>
+
+#include "bude_internal.h"
+#include "hip_util.h"
+
+namespace bude {
+namespace items {
+
+// What the items are scored against: the grouped protein (a group index in
+// the w bits of every atom), and per ligand-atom slot (a forcefield type of
+// the ligand set) and group the pair coefficients and the squared distance
+// beyond which every hinge of the pair is exactly zero.
+struct Scene {
+  const float4 *protein = nullptr;
+  const PairCoef *coef = nullptr;   // [nslots][ngroups]
+  const float *reach2 = nullptr;    // [nslots][ngroups]
+  int natpro = 0, ngroups = 0;
+  int form = 1;                     // hinge form (plain_form())
+  float lo[3] = {}, hi[3] = {};     // the protein's box, widened by the largest reach
+};
+
+// n poses of one ligand, rows pose_off .. pose_off + n - 1 of the pose
+// arrays (or of the index into them); their energies go to the same rows.
+struct Segment {
+  int32_t lig;
+  int64_t pose_off;
+  int64_t n;
+};
+
+// Distance beyond which all three hinges of a pair are exactly zero in
+// either hinge form: the largest zero crossing of the terms present, widened
+// far above the rounding of the distances compared with it.  Negative when
+// the pair has no such distance (a radius sum that is not positive, or a
+// coefficient that is not finite), so that no pair may be left out.
+float pair_reach(const PairCoef &c);
+
+// The squared reaches of a coefficient table and their largest; false when
+// some pair has none.
+bool reach_table(const std::vector<PairCoef> &coef, std::vector<float> &reach2, float *largest);
+
+// The box of the grouped protein's finite atoms widened by `reach`.
+void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]);
+
+// Whether sorting pays for scoring segs against natpro atoms.
+bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
+
+// Device scratch of a pass; one stream at a time may use it.
+struct Workspace {
+  DeviceBuffer items, partial, xform, hist, base, bounds;
+  void release() {
+    for (DeviceBuffer *b : {&items, &partial, &xform, &hist, &base, &bounds}) b->reset();
+  }
+};
+
+// The work of one pass, split into chunks of at most kChunkItems items.
+class Plan {
+ public:
+  // atoms: every ligand's atoms (w bits: slot), ligand l's at lig_off[l] ..
+  // lig_off[l + 1] - 1.  The tables are uploaded synchronously.
+  int build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
+            const std::vector<Segment> &segs);
+  int reserve(Workspace &w) const;
+  // Queues the pass: energies[row] of every row of every segment.  index:
+  // the pose row of row i of a segment is pose_off + index[pose_off + i].
+  hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
+                    float *energies, hipStream_t s) const;
+  bool empty() const { return chunks_.empty(); }
+  double items() const { return items_; }
+
+ private:
+  struct Chunk {
+    int nblocks, ntasks, nslots_rows, ppt, rb, cell_bits;
+    size_t blocks, tasks, refs, rows, slot_rows, slot_items, slot_units;  // offsets into tables_
+    uint32_t nitems, npartial, nxform, nrows;
+    int nunits;
+  };
+  std::vector<Chunk> chunks_;
+  DeviceBuffer tables_, atoms_;
+  int nslots_ = 0;
+  float radius_ = 0.f;  // of the ligand atoms about their frame's origin
+  double items_ = 0;
+};
+
+// Everything one deck's passes need on the sorted path, from the host deck:
+// scene, plan and workspace.  usable() is false where the path does not
+// apply (see worth_sorting, pair_reach) or its memory cannot be had; the
+// caller then scores with the tiled kernels.
+class Deck {
+ public:
+  int prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
+              const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
+  bool usable() const { return usable_; }
+  hipError_t launch(const float4 *protein, const float *poses, size_t stride, float *energies, hipStream_t s) const;
+
+ private:
+  bool usable_ = false;
+  Scene scene_;
+  Plan plan_;
+  Workspace work_;
+  DeviceBuffer coef_, reach2_;
+};
+
+}  // namespace items
+}  // namespace bude

@@ -1,0 +1,775 @@
+// items.hip -- exact pose energies from sorted items.
+//
+// An item is one ligand atom under one pose.  Its energy is a sum over the
+// protein atoms of three hinges that are exactly zero beyond a few Angstrom
+// (pair_reach), about 2 % of the pairs in a protein of 4,096 atoms.  A
+// wave can leave a protein atom out only when it is out of reach of all its
+// items, and 64 poses of one ligand atom lie all over the protein; so the
+// items are first sorted by (forcefield type of the ligand atom, cell of
+// space), and a wave then scores 64 x RB neighbouring items of one type
+// against the protein atoms within reach of their box.  The pairs left out
+// add fma(w, 0, e) == e; the others are summed in the same order by the
+// same code as the tiled kernels' (fasten_core.h), and the energies of a
+// pose's atoms are added in the ligand's order, so an energy is the tiled
+// kernels' bit for bit however the items fell.
+//
+// One pass, per chunk of the plan:
+//   prep_kernel    pose transforms, and the box of the translations
+//   bin_kernel<0>  per (type, block of poses): items per cell, from LDS counts
+//   column_kernel  those counts summed over the blocks, per (type, cell)
+//   scan_kernel    the first item of every (type, cell)
+//   bin_kernel<1>  items (x, y, z, where its energy goes) into their places
+//   score_kernel   the items' energies
+//   reduce_kernel  pose energies, the atoms' energies in order
+// An item's place within its cell is whichever atomic came first; nothing an
+// item's energy is made of depends on it.
+//
+// Measured against the tiled kernel on the same deck (whole pass, energies
+// copied out): 4,096 x 64 atoms x 1,048,576 poses 79.4 -> 5.4 ms (score
+// 3.7, items into place 0.8, counts 0.12, reduction 0.12); 2,672 x 2,672 x
+// 65,536 289 -> 10.0 ms; 938 x 26 x 65,536 1,079 -> 208 us.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
+#include <cstring>
+
+#include "fasten_core.h"
+#include "items.h"
+
+namespace bude {
+namespace items {
+
+namespace {
+
+using namespace core;
+
+constexpr int kThreads = 1024;      // of the prep and bin kernels
+constexpr int kCells = 4096;        // 16 per axis, in Morton order
+constexpr int kMaxBounds = 256;     // work-groups of the prep kernel
+
+struct Block {
+  int64_t pose_off;      // row of the block's first pose
+  uint32_t part_off;     // partial of (atom 0, first pose)
+  uint32_t part_stride;  // from one atom to the next
+  int32_t npose, natlig;
+  uint32_t xf_off;       // first transform
+  int32_t seg_pose;      // the first pose's place in its segment
+};
+static_assert(sizeof(Block) == 32, "Block is 32 bytes");
+
+// The atoms of one type in one block: one row of the counts.
+struct Row {
+  int32_t block, atom0, natoms, slot;
+};
+
+// Rows ref[ref0 .. ref0 + nref) of one block, for one work-group.
+struct Task {
+  int32_t block, ref0, nref, pad;
+};
+
+struct Space {
+  float lo[3], hi[3];  // where an item can have an energy
+  float radius;        // of the ligand atoms about their frame's origin
+};
+
+__device__ __forceinline__ float wave_min(float v) {
+  for (int d = 32; d; d >>= 1) v = fminf(v, __shfl_xor(v, d));
+  return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+  for (int d = 32; d; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
+  return v;
+}
+
+// Transforms of every pose of the chunk, and per work-group the box of its
+// poses' translations (bounds[group]: three minima, three maxima).
+__global__ __launch_bounds__(kThreads) void prep_kernel(const Block *__restrict__ blocks, int nblocks,
+                                                        const float *__restrict__ poses, size_t stride,
+                                                        const uint32_t *__restrict__ index, float4 *__restrict__ xf,
+                                                        size_t nxf, float *__restrict__ bounds) {
+  __shared__ float part[kThreads / 64][6];
+  float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+  for (int b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const Block bk = blocks[b];
+    for (int j = threadIdx.x; j < bk.npose; j += kThreads) {
+      const size_t row = size_t(bk.pose_off) + size_t(j);
+      size_t q = row;
+      if (index) q = size_t(bk.pose_off - bk.seg_pose) + index[row];
+      const Xform t = make_xform(poses, stride, q);
+      const size_t i = size_t(bk.xf_off) + size_t(j);
+      xf[i] = make_float4(t.m[0], t.m[1], t.m[2], t.m[3]);
+      xf[nxf + i] = make_float4(t.m[4], t.m[5], t.m[6], t.m[7]);
+      xf[2 * nxf + i] = make_float4(t.m[8], t.m[9], t.m[10], t.m[11]);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        lo[k] = fminf(lo[k], t.m[4 * k + 3]);
+        hi[k] = fmaxf(hi[k], t.m[4 * k + 3]);
+      }
+    }
+  }
+  const int wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float a = wave_min(lo[k]), b = wave_max(hi[k]);
+    if ((threadIdx.x & 63) == 0) {
+      part[wave][k] = a;
+      part[wave][3 + k] = b;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    float v = part[0][threadIdx.x];
+    for (int w = 1; w < kThreads / 64; w++)
+      v = threadIdx.x < 3 ? fminf(v, part[w][threadIdx.x]) : fmaxf(v, part[w][threadIdx.x]);
+    bounds[size_t(blockIdx.x) * 6 + threadIdx.x] = v;
+  }
+}
+
+// 16 cells per axis over the box of the chunk's items (the translations'
+// box widened by the ligands' radius) where it meets the scene's.
+struct CellGrid {
+  float lo[3], inv[3];
+};
+
+__device__ __forceinline__ CellGrid cell_grid(const float *__restrict__ bounds, int nbounds, const Space &sp,
+                                              float *red /* LDS, 96 */) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // waves 0-2 the minima, 3-5 the maxima
+  if (wave < 6) {
+    float v = wave < 3 ? FLT_MAX : -FLT_MAX;
+    for (int i = lane; i < nbounds; i += 64) {
+      const float x = bounds[size_t(i) * 6 + wave];
+      v = wave < 3 ? fminf(v, x) : fmaxf(v, x);
+    }
+    v = wave < 3 ? wave_min(v) : wave_max(v);
+    if (lane == 0) red[wave] = v;
+  }
+  __syncthreads();
+  CellGrid g;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float a = fmaxf(red[k] - sp.radius, sp.lo[k]), b = fminf(red[3 + k] + sp.radius, sp.hi[k]);
+    g.lo[k] = a;
+    g.inv[k] = b > a ? 16.0f / (b - a) : 0.0f;
+  }
+  return g;
+}
+
+__device__ __forceinline__ uint32_t spread(uint32_t v) {  // bits 0-3 to 0, 3, 6, 9
+  v = (v | (v << 4)) & 0x0c3u;
+  return (v | (v << 2)) & 0x249u;
+}
+
+// (clamped to the grid; NaN falls into cell 0 of its axis)
+__device__ __forceinline__ uint32_t axis_cell(float x, float lo, float inv) {
+  return uint32_t(__builtin_amdgcn_fmed3f((x - lo) * inv, 0.0f, 15.0f));
+}
+
+__device__ __forceinline__ uint32_t cell_of(const CellGrid &g, float x, float y, float z) {
+  return spread(axis_cell(x, g.lo[0], g.inv[0])) | (spread(axis_cell(y, g.lo[1], g.inv[1])) << 1) |
+         (spread(axis_cell(z, g.lo[2], g.inv[2])) << 2);
+}
+
+// SCATTER 0: counts of each row's items per cell.  SCATTER 1: each item into
+// its place.  One work-group per task, PPT poses per work-item.  Both read
+// the same transforms and place items by the same explicit operations, so an
+// item's cell is the same in both.
+template <int PPT, int SCATTER>
+__global__ __launch_bounds__(kThreads) void bin_kernel(const Task *__restrict__ tasks, const Block *__restrict__ blocks,
+                                                       const int32_t *__restrict__ refs, const Row *__restrict__ rows,
+                                                       const float4 *__restrict__ atoms,
+                                                       const float4 *__restrict__ xf, size_t nxf,
+                                                       const float *__restrict__ bounds, int nbounds, const Space sp,
+                                                       int bits, uint32_t *__restrict__ hist,
+                                                       const uint32_t *__restrict__ base, float4 *__restrict__ items) {
+  __shared__ uint32_t h[kCells];
+  __shared__ float red[6];
+  const CellGrid g = cell_grid(bounds, nbounds, sp, red);
+  const Task t = tasks[blockIdx.x];
+  const Block bk = blocks[t.block];
+  const int ncells = 1 << bits, shift = 12 - bits;
+  float4 m0[PPT], m1[PPT], m2[PPT];
+#pragma unroll
+  for (int k = 0; k < PPT; k++) {
+    const int j = int(threadIdx.x) + k * kThreads;
+    const size_t i = size_t(bk.xf_off) + size_t(j < bk.npose ? j : 0);
+    m0[k] = xf[i];
+    m1[k] = xf[nxf + i];
+    m2[k] = xf[2 * nxf + i];
+  }
+  for (int r = 0; r < t.nref; r++) {
+    const int id = refs[t.ref0 + r];
+    const Row row = rows[id];
+    uint32_t *hr = hist + size_t(id) * size_t(ncells);
+    const uint32_t *br = base + size_t(row.slot) * size_t(ncells);
+    for (int c = threadIdx.x; c < ncells; c += kThreads) h[c] = SCATTER ? br[c] + hr[c] : 0u;
+    __syncthreads();
+    for (int a = 0; a < row.natoms; a++) {
+      const float4 la = atoms[row.atom0 + a];  // w bits: the atom's place in its ligand
+      const uint32_t out = bk.part_off + uint32_t(__float_as_int(la.w)) * bk.part_stride;
+#pragma unroll
+      for (int k = 0; k < PPT; k++) {
+        const int j = int(threadIdx.x) + k * kThreads;
+        const float x = place(m0[k].x, m0[k].y, m0[k].z, m0[k].w, la);
+        const float y = place(m1[k].x, m1[k].y, m1[k].z, m1[k].w, la);
+        const float z = place(m2[k].x, m2[k].y, m2[k].z, m2[k].w, la);
+        if (j < bk.npose) {
+          const uint32_t c = cell_of(g, x, y, z) >> shift;
+          const uint32_t at = atomicAdd(&h[c], 1u);
+          if constexpr (SCATTER) items[at] = make_float4(x, y, z, __uint_as_float(out + uint32_t(j)));
+        }
+      }
+    }
+    __syncthreads();
+    if constexpr (!SCATTER) {
+      for (int c = threadIdx.x; c < ncells; c += kThreads) hr[c] = h[c];
+      __syncthreads();
+    }
+  }
+}
+
+// hist[row][cell] of each type's rows to the counts of the rows before it;
+// base[type][cell] = the type's count.
+__global__ __launch_bounds__(256) void column_kernel(const int32_t *__restrict__ slot_rows, int bits,
+                                                     uint32_t *__restrict__ hist, uint32_t *__restrict__ base) {
+  const int slot = blockIdx.y, ncells = 1 << bits;
+  const int c = int(blockIdx.x) * 256 + int(threadIdx.x);
+  const int r1 = slot_rows[slot + 1];
+  uint32_t run = 0;
+  int r = slot_rows[slot];
+  for (; r + 8 <= r1; r += 8) {  // eight loads in flight
+    uint32_t v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = hist[size_t(r + k) * size_t(ncells) + size_t(c)];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      hist[size_t(r + k) * size_t(ncells) + size_t(c)] = run;
+      run += v[k];
+    }
+  }
+  for (; r < r1; r++) {
+    const uint32_t v = hist[size_t(r) * size_t(ncells) + size_t(c)];
+    hist[size_t(r) * size_t(ncells) + size_t(c)] = run;
+    run += v;
+  }
+  base[size_t(slot) * size_t(ncells) + size_t(c)] = run;
+}
+
+// base[type][cell] from counts to the first item of the cell; one
+// work-group per type.
+__global__ __launch_bounds__(kThreads) void scan_kernel(const int32_t *__restrict__ slot_items, int bits,
+                                                        uint32_t *__restrict__ base) {
+  __shared__ uint32_t wsum[kThreads / 64];
+  const int per = (1 << bits) >> 10 ? (1 << bits) >> 10 : 1;  // cells per work-item: 4 (12 bits) or 1
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c0 = int(threadIdx.x) * per;
+  const bool on = c0 < (1 << bits);
+  uint32_t *b = base + (size_t(blockIdx.x) << bits);
+  uint32_t v[4], sum = 0;
+  for (int i = 0; i < per; i++) {
+    v[i] = on ? b[c0 + i] : 0u;
+    sum += v[i];
+  }
+  uint32_t x = sum;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) wsum[wave] = x;
+  __syncthreads();
+  uint32_t run = uint32_t(slot_items[blockIdx.x]) + x - sum;
+  for (int w = 0; w < wave; w++) run += wsum[w];
+  if (on)
+    for (int i = 0; i < per; i++) {
+      b[c0 + i] = run;
+      run += v[i];
+    }
+}
+
+// The protein atoms of `mask` (lanes of the wave's 64 atoms x, y, z), all of
+// one group, in order.
+template <int RB, int FORM, bool CHG, bool DSLV>
+__device__ __forceinline__ void mask_pairs(uint64_t mask, float x, float y, float z, const PairCoef &c,
+                                           const float (&lx)[RB], const float (&ly)[RB], const float (&lz)[RB],
+                                           float (&e)[RB]) {
+  float c0 = 0.f, e0 = 0.f;
+  if constexpr (FORM == kFormD) {
+    if constexpr (CHG) c0 = vgpr_copy(c.c0);
+    if constexpr (DSLV) e0 = vgpr_copy(c.e0);
+  }
+  do {
+    const int j = __builtin_ctzll(mask);
+    mask &= mask - 1;
+    float4 p;
+    p.x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j));
+    p.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(y), j));
+    p.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), j));
+    p.w = 0.f;
+    atom_pairs<RB, FORM, CHG, DSLV>(p, c, c0, e0, lx, ly, lz, e);
+  } while (mask);
+}
+
+// One wave per 64 x RB consecutive items of one type: the protein 64 atoms at
+// a time (lane = atom) against the items' box, then every atom in reach out
+// of its lane (three readlanes) to all lanes' RB items.  RB > 1 shares the
+// 64-atom steps and the readlanes between items at the price of a larger
+// box; VALU issue bounds it (about 12 VALU per pair in reach of the box and
+// 3 / RB for its atom).
+template <int RB, int FORM>
+__global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ protein, int natpro,
+                                                    const PairCoef *__restrict__ coef,
+                                                    const float *__restrict__ reach2, int ngroups,
+                                                    const float4 *__restrict__ items,
+                                                    const int32_t *__restrict__ slot_items,
+                                                    const int32_t *__restrict__ slot_units, int nslots, int nunits,
+                                                    float *__restrict__ partial) {
+  const int lane = threadIdx.x & 63;
+  const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * 4 + int(threadIdx.x >> 6));
+  if (u >= nunits) return;
+  int slot = 0;  // the last type whose first unit is at or before u
+  for (int s0 = 0; s0 < nslots; s0 += 64)
+    slot += __popcll(__ballot(s0 + lane < nslots && slot_units[s0 + lane + 1] <= u));
+  const int i1 = slot_items[slot + 1];
+  const int i0 = slot_items[slot] + (u - slot_units[slot]) * 64 * RB;
+
+  float lx[RB], ly[RB], lz[RB], e[RB], part[RB];
+  uint32_t out[RB];
+  float bl[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, bh[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+#pragma unroll
+  for (int k = 0; k < RB; k++) {
+    const float4 it = items[min(i0 + k * 64 + lane, i1 - 1)];  // (past the end: the last item again, not written)
+    lx[k] = it.x;
+    ly[k] = it.y;
+    lz[k] = it.z;
+    out[k] = __float_as_uint(it.w);
+    e[k] = part[k] = 0.f;
+    bl[0] = fminf(bl[0], it.x), bh[0] = fmaxf(bh[0], it.x);
+    bl[1] = fminf(bl[1], it.y), bh[1] = fmaxf(bh[1], it.y);
+    bl[2] = fminf(bl[2], it.z), bh[2] = fmaxf(bh[2], it.z);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    bl[k] = wave_min(bl[k]);
+    bh[k] = wave_max(bh[k]);
+  }
+  const float *r2 = reach2 + size_t(slot) * size_t(ngroups);
+  const PairCoef *cs = coef + size_t(slot) * size_t(ngroups);
+  PairCoef c{};
+  int cur = -1;
+  // two steps ahead: the atoms; one step ahead: their reach
+  float4 p = protein[min(lane, natpro - 1)], p1 = protein[min(64 + lane, natpro - 1)];
+  float reach = r2[__float_as_int(p.w)];
+  for (int base = 0; base < natpro; base += 64) {
+    const float reach1 = r2[__float_as_int(p1.w)];
+    const float4 p2 = protein[min(base + 128 + lane, natpro - 1)];
+    const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, bl[0], bh[0]);
+    const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, bl[1], bh[1]);
+    const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, bl[2], bh[2]);
+    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+    uint64_t mask = __ballot(base + lane < natpro && d2 < reach);
+    const int pg = __float_as_int(p.w);
+    while (mask) {
+      const int g = __builtin_amdgcn_readlane(pg, __builtin_ctzll(mask));
+      if (g != cur) {
+#pragma unroll
+        for (int k = 0; k < RB; k++) {
+          e[k] += part[k];
+          part[k] = 0.f;
+        }
+        cur = g;
+        c = cs[g];
+      }
+      const uint64_t sub = mask & __ballot(pg == g);
+      mask &= ~sub;
+      const bool chg = c.wq != 0.f, dslv = c.wd != 0.f;
+      if (chg && dslv) mask_pairs<RB, FORM, true, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+      else if (chg) mask_pairs<RB, FORM, true, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+      else if (dslv) mask_pairs<RB, FORM, false, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+      else mask_pairs<RB, FORM, false, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+    }
+    p = p1;
+    p1 = p2;
+    reach = reach1;
+  }
+#pragma unroll
+  for (int k = 0; k < RB; k++)
+    if (i0 + k * 64 + lane < i1) partial[out[k]] = e[k] + part[k];
+}
+
+// energies[row] = half the sum of the pose's atoms' energies, in the
+// ligand's order.  `per` work-groups of 256 per block.
+__global__ __launch_bounds__(256) void reduce_kernel(const Block *__restrict__ blocks, int per,
+                                                     const float *__restrict__ partial, float *__restrict__ energies) {
+  const Block bk = blocks[blockIdx.x / unsigned(per)];
+  const int j = int(blockIdx.x % unsigned(per)) * 256 + int(threadIdx.x);
+  if (j >= bk.npose) return;
+  const float *p = partial + size_t(bk.part_off) + size_t(j);
+  float e = 0.f;
+  int a = 0;
+  for (; a + 8 <= bk.natlig; a += 8) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = p[size_t(a + k) * bk.part_stride];
+#pragma unroll
+    for (int k = 0; k < 8; k++) e += v[k];
+  }
+  for (; a < bk.natlig; a++) e += p[size_t(a) * bk.part_stride];
+  energies[size_t(bk.pose_off) + size_t(j)] = e * 0.5f;
+}
+
+template <int PPT, int SCATTER, class... A> void launch_bin(int ntasks, hipStream_t s, A... args) {
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(bin_kernel<PPT, SCATTER>), dim3(unsigned(ntasks)), dim3(kThreads), 0, s, args...);
+}
+
+template <int SCATTER, class... A> void launch_bin_ppt(int ppt, int ntasks, hipStream_t s, A... args) {
+  if (ppt >= 8) launch_bin<8, SCATTER>(ntasks, s, args...);
+  else if (ppt >= 4) launch_bin<4, SCATTER>(ntasks, s, args...);
+  else if (ppt >= 2) launch_bin<2, SCATTER>(ntasks, s, args...);
+  else launch_bin<1, SCATTER>(ntasks, s, args...);
+}
+
+template <int RB, class... A> void launch_score(int form, int nunits, hipStream_t s, A... args) {
+  const dim3 grid(unsigned((nunits + 3) / 4));
+  if (form == kFormD) hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormD>), grid, dim3(256), 0, s, args...);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormB>), grid, dim3(256), 0, s, args...);
+}
+
+// Items of one chunk: 20 bytes each in the workspace.
+constexpr int64_t kChunkItems = int64_t(1) << 26;
+
+int slot_of(const float4 &a) {
+  int s;
+  std::memcpy(&s, &a.w, sizeof s);
+  return s;
+}
+
+}  // namespace
+
+float pair_reach(const PairCoef &c) {
+  const float all[] = {c.radij, c.neg_rr, c.neg_e1, c.wq, c.neg_rd, c.wd, c.c0, c.e0};
+  for (float v : all)
+    if (!std::isfinite(v)) return -1.f;
+  if (!(c.radij > 0.f) || !(c.neg_rr < 0.f) || !(c.neg_e1 < 0.f) || (c.wd != 0.f && !(c.neg_rd < 0.f))) return -1.f;
+  float r = std::max(c.radij, -1.0f / c.neg_rr);
+  if (c.wq != 0.f) r = std::max({r, c.c0 / -c.neg_e1, c.radij - 1.0f / c.neg_e1});
+  if (c.wd != 0.f) r = std::max({r, c.e0 / -c.neg_rd, c.radij - 1.0f / c.neg_rd});
+  r = r * 1.0001f + 1e-3f;
+  return std::isfinite(r * r) ? r : -1.f;
+}
+
+bool reach_table(const std::vector<PairCoef> &coef, std::vector<float> &reach2, float *largest) {
+  reach2.resize(coef.size());
+  *largest = 0.f;
+  for (size_t i = 0; i < coef.size(); i++) {
+    const float r = pair_reach(coef[i]);
+    if (r < 0.f) return false;
+    reach2[i] = r * r;
+    *largest = std::max(*largest, r);
+  }
+  return true;
+}
+
+void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]) {
+  for (int k = 0; k < 3; k++) {
+    float a = FLT_MAX, b = -FLT_MAX;
+    for (size_t i = size_t(k); i < xyzw.size(); i += 4)
+      if (std::isfinite(xyzw[i])) {
+        a = std::min(a, xyzw[i]);
+        b = std::max(b, xyzw[i]);
+      }
+    lo[k] = a - reach;
+    hi[k] = b + reach;
+  }
+}
+
+bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs) {
+  double items = 0;
+  for (const Segment &s : segs) {
+    const int64_t L = lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)];
+    if (L > kChunkItems / 64) return false;
+    items += double(L) * double(s.n);
+  }
+  // seven launches and the sort cost about 60 us whatever the size, which the
+  // tiled kernels score some 2e8 pairs in; a segment is to fill the
+  // work-groups that sort it
+  return items * double(natpro) >= 1.5e8 && items >= 65536 * 1.0 && items >= 4096.0 * double(segs.size());
+}
+
+int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
+                const std::vector<Segment> &segs) {
+  chunks_.clear();
+  nslots_ = nslots;
+  items_ = 0;
+  radius_ = 0.f;
+  // every ligand's atoms grouped by type (stable), w bits: place in the ligand
+  const size_t nlig = lig_off.size() - 1;
+  std::vector<float4> grouped;
+  std::vector<std::vector<Row>> lig_rows(nlig);
+  for (size_t l = 0; l < nlig; l++) {
+    const int32_t a0 = lig_off[l], n = lig_off[l + 1] - a0;
+    std::vector<int32_t> order(static_cast<size_t>(n), 0);
+    for (int32_t i = 0; i < n; i++) order[size_t(i)] = i;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int32_t x, int32_t y) { return slot_of(atoms[size_t(a0 + x)]) < slot_of(atoms[size_t(a0 + y)]); });
+    for (int32_t i : order) {
+      float4 a = atoms[size_t(a0 + i)];
+      const int s = slot_of(a);
+      const float r = std::sqrt(a.x * a.x + a.y * a.y + a.z * a.z);
+      if (std::isfinite(r)) radius_ = std::max(radius_, r);
+      if (lig_rows[l].empty() || lig_rows[l].back().slot != s)
+        lig_rows[l].push_back(Row{0, int32_t(grouped.size()), 0, s});
+      lig_rows[l].back().natoms++;
+      std::memcpy(&a.w, &i, sizeof i);
+      grouped.push_back(a);
+    }
+  }
+  radius_ = radius_ * 1.0001f;
+
+  // pieces of segments, in chunks of at most kChunkItems items
+  struct Piece {
+    int32_t lig;
+    int64_t seg_off, first, n;
+  };
+  std::vector<std::vector<Piece>> parts(1);
+  int64_t room = kChunkItems;
+  for (const Segment &s : segs) {
+    const int64_t L = lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)];
+    if (L <= 0 || L > kChunkItems / 64) return fail(BUDE_ERR_RUNTIME, "items: ligand too large for a chunk");
+    items_ += double(L) * double(s.n);
+    for (int64_t j = 0; j < s.n;) {
+      int64_t take = std::min(s.n - j, room / L);
+      if (take < s.n - j) take = take / 64 * 64;
+      if (take <= 0) {
+        parts.emplace_back();
+        room = kChunkItems;
+        continue;
+      }
+      parts.back().push_back(Piece{s.lig, s.pose_off, j, take});
+      room -= take * L;
+      j += take;
+    }
+  }
+  if (parts.back().empty()) parts.pop_back();
+
+  std::vector<char> bytes;
+  auto put = [&](const void *p, size_t n) {
+    bytes.resize((bytes.size() + 63) / 64 * 64);
+    const size_t at = bytes.size();
+    bytes.insert(bytes.end(), static_cast<const char *>(p), static_cast<const char *>(p) + n);
+    return at;
+  };
+  for (const std::vector<Piece> &pieces : parts) {
+    Chunk ch{};
+    // poses per work-item: as many as leave enough (type, block) rows to fill the device
+    int64_t nrows = 0, nitems = 0, longest = 0;
+    for (const Piece &p : pieces) longest = std::max(longest, p.n);
+    for (ch.ppt = 8;; ch.ppt /= 2) {
+      if (ch.ppt > 1 && kThreads * ch.ppt / 2 >= longest) continue;
+      nrows = 0;
+      for (const Piece &p : pieces)
+        nrows += (p.n + kThreads * ch.ppt - 1) / (kThreads * ch.ppt) * int64_t(lig_rows[size_t(p.lig)].size());
+      if (ch.ppt == 1 || nrows >= 512) break;
+    }
+    std::vector<Block> blocks;
+    std::vector<std::vector<Row>> by_slot(static_cast<size_t>(nslots));
+    std::vector<int32_t> slot_rows(size_t(nslots) + 1, 0), slot_items(size_t(nslots) + 1, 0),
+        slot_units(size_t(nslots) + 1, 0);
+    std::vector<int64_t> count(static_cast<size_t>(nslots), 0);
+    int64_t part = 0, xf = 0;
+    for (const Piece &p : pieces) {
+      const int64_t L = lig_off[size_t(p.lig) + 1] - lig_off[size_t(p.lig)];
+      for (int64_t j = 0; j < p.n; j += kThreads * ch.ppt) {
+        const int64_t n = std::min<int64_t>(kThreads * ch.ppt, p.n - j);
+        for (Row r : lig_rows[size_t(p.lig)]) {
+          r.block = int32_t(blocks.size());
+          by_slot[size_t(r.slot)].push_back(r);
+          count[size_t(r.slot)] += n * r.natoms;
+        }
+        blocks.push_back(Block{p.seg_off + p.first + j, uint32_t(part + j), uint32_t(p.n), int32_t(n), int32_t(L),
+                               uint32_t(xf + j), int32_t(p.first + j)});
+      }
+      part += p.n * L;
+      xf += p.n;
+    }
+    int64_t used = 0;
+    for (int t = 0; t < nslots; t++) {
+      nitems += count[size_t(t)];
+      used += count[size_t(t)] > 0;
+    }
+    const int64_t mean = nitems / std::max<int64_t>(1, used);
+    ch.rb = mean >= 131072 ? 4 : mean >= 32768 ? 2 : 1;
+    ch.cell_bits = mean >= 16384 ? 12 : 9;
+    std::vector<Row> rows;
+    std::vector<std::vector<int32_t>> refs_of(blocks.size());
+    for (int t = 0; t < nslots; t++) {
+      for (const Row &r : by_slot[size_t(t)]) {
+        refs_of[size_t(r.block)].push_back(int32_t(rows.size()));
+        rows.push_back(r);
+      }
+      slot_rows[size_t(t) + 1] = int32_t(rows.size());
+      slot_items[size_t(t) + 1] = slot_items[size_t(t)] + int32_t(count[size_t(t)]);
+      slot_units[size_t(t) + 1] =
+          slot_units[size_t(t)] + int32_t((count[size_t(t)] + 64 * ch.rb - 1) / (64 * ch.rb));
+    }
+    const size_t per_task = std::max<size_t>(1, rows.size() / 768);
+    std::vector<int32_t> refs;
+    std::vector<Task> tasks;
+    for (size_t b = 0; b < blocks.size(); b++)
+      for (size_t i = 0; i < refs_of[b].size(); i += per_task) {
+        const size_t n = std::min(per_task, refs_of[b].size() - i);
+        tasks.push_back(Task{int32_t(b), int32_t(refs.size()), int32_t(n), 0});
+        refs.insert(refs.end(), refs_of[b].begin() + long(i), refs_of[b].begin() + long(i + n));
+      }
+    ch.nblocks = int(blocks.size());
+    ch.ntasks = int(tasks.size());
+    ch.nrows = uint32_t(rows.size());
+    ch.nitems = uint32_t(nitems);
+    ch.npartial = uint32_t(part);
+    ch.nxform = uint32_t(xf);
+    ch.nunits = slot_units.back();
+    ch.blocks = put(blocks.data(), blocks.size() * sizeof(Block));
+    ch.tasks = put(tasks.data(), tasks.size() * sizeof(Task));
+    ch.refs = put(refs.data(), refs.size() * 4);
+    ch.rows = put(rows.data(), rows.size() * sizeof(Row));
+    ch.slot_rows = put(slot_rows.data(), slot_rows.size() * 4);
+    ch.slot_items = put(slot_items.data(), slot_items.size() * 4);
+    ch.slot_units = put(slot_units.data(), slot_units.size() * 4);
+    chunks_.push_back(ch);
+  }
+  if (int st = atoms_.assign(grouped.data(), grouped.size() * sizeof(float4))) return st;
+  return tables_.assign(bytes.data(), bytes.size());
+}
+
+int Plan::reserve(Workspace &w) const {
+  size_t items = 0, partial = 0, xf = 0, hist = 0, base = 0;
+  for (const Chunk &c : chunks_) {
+    items = std::max(items, size_t(c.nitems) * sizeof(float4));
+    partial = std::max(partial, size_t(c.npartial) * 4);
+    xf = std::max(xf, size_t(c.nxform) * 3 * sizeof(float4));
+    hist = std::max(hist, (size_t(c.nrows) << c.cell_bits) * 4);
+    base = std::max(base, (size_t(nslots_) << c.cell_bits) * 4);
+  }
+  int st = w.items.reserve(items);
+  if (!st) st = w.partial.reserve(partial);
+  if (!st) st = w.xform.reserve(xf);
+  if (!st) st = w.hist.reserve(hist);
+  if (!st) st = w.base.reserve(base);
+  if (!st) st = w.bounds.reserve(kMaxBounds * 6 * 4);
+  return st;
+}
+
+hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
+                        float *energies, hipStream_t s) const {
+  Space sp{};
+  for (int k = 0; k < 3; k++) {
+    sp.lo[k] = sc.lo[k];
+    sp.hi[k] = sc.hi[k];
+  }
+  sp.radius = radius_;
+  const auto *tables = static_cast<const char *>(tables_.ptr);
+  const auto *atoms = static_cast<const float4 *>(atoms_.ptr);
+  auto *items = static_cast<float4 *>(w.items.ptr);
+  auto *partial = static_cast<float *>(w.partial.ptr);
+  auto *xf = static_cast<float4 *>(w.xform.ptr);
+  auto *hist = static_cast<uint32_t *>(w.hist.ptr);
+  auto *base = static_cast<uint32_t *>(w.base.ptr);
+  auto *bounds = static_cast<float *>(w.bounds.ptr);
+  for (const Chunk &c : chunks_) {
+    if (size_t(c.nitems) * sizeof(float4) > w.items.bytes || size_t(c.npartial) * 4 > w.partial.bytes ||
+        size_t(c.nxform) * 48 > w.xform.bytes || (size_t(c.nrows) << c.cell_bits) * 4 > w.hist.bytes ||
+        (size_t(nslots_) << c.cell_bits) * 4 > w.base.bytes || w.bounds.bytes < kMaxBounds * 24)
+      return hipErrorInvalidValue;
+    const auto *blocks = reinterpret_cast<const Block *>(tables + c.blocks);
+    const auto *tasks = reinterpret_cast<const Task *>(tables + c.tasks);
+    const auto *refs = reinterpret_cast<const int32_t *>(tables + c.refs);
+    const auto *rows = reinterpret_cast<const Row *>(tables + c.rows);
+    const auto *slot_rows = reinterpret_cast<const int32_t *>(tables + c.slot_rows);
+    const auto *slot_items = reinterpret_cast<const int32_t *>(tables + c.slot_items);
+    const auto *slot_units = reinterpret_cast<const int32_t *>(tables + c.slot_units);
+    const int nb = std::min(c.nblocks, kMaxBounds);
+    hipLaunchKernelGGL(prep_kernel, dim3(unsigned(nb)), dim3(kThreads), 0, s, blocks, c.nblocks, poses, stride, index,
+                       xf, size_t(c.nxform), bounds);
+    launch_bin_ppt<0>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),
+                      size_t(c.nxform), static_cast<const float *>(bounds), nb, sp, c.cell_bits, hist,
+                      static_cast<const uint32_t *>(base), items);
+    hipLaunchKernelGGL(column_kernel, dim3((1u << c.cell_bits) / 256u, unsigned(nslots_)), dim3(256), 0, s, slot_rows,
+                       c.cell_bits, hist, base);
+    hipLaunchKernelGGL(scan_kernel, dim3(unsigned(nslots_)), dim3(kThreads), 0, s, slot_items, c.cell_bits, base);
+    launch_bin_ppt<1>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),
+                      size_t(c.nxform), static_cast<const float *>(bounds), nb, sp, c.cell_bits, hist,
+                      static_cast<const uint32_t *>(base), items);
+    switch (c.rb) {
+      case 1:
+        launch_score<1>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
+                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
+        break;
+      case 2:
+        launch_score<2>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
+                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
+        break;
+      default:
+        launch_score<4>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
+                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
+        break;
+    }
+    const int per = 4 * c.ppt;  // work-groups of 256 per block of 1024 ppt poses
+    hipLaunchKernelGGL(reduce_kernel, dim3(unsigned(c.nblocks) * unsigned(per)), dim3(256), 0, s, blocks, per,
+                       static_cast<const float *>(partial), energies);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
+                  const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs) {
+  usable_ = false;
+  const size_t natpro = size_t(groups.begin.back());
+  if (!worth_sorting(natpro, lig_off, segs)) return BUDE_OK;
+  // slots: the forcefield types the ligands use, ascending
+  std::vector<int32_t> types;
+  for (const BudeAtom &a : atoms) types.push_back(a.type);
+  std::sort(types.begin(), types.end());
+  types.erase(std::unique(types.begin(), types.end()), types.end());
+  std::vector<BudeAtom> probe;
+  for (int32_t t : types) probe.push_back(BudeAtom{0.f, 0.f, 0.f, t});
+  const std::vector<PairCoef> coef = coef_table(probe.data(), probe.size(), groups, ff);
+  std::vector<float> reach2;
+  float largest = 0.f;
+  if (!reach_table(coef, reach2, &largest)) return BUDE_OK;
+  std::vector<float4> slotted;
+  for (const BudeAtom &a : atoms) {
+    const int32_t s = int32_t(std::lower_bound(types.begin(), types.end(), a.type) - types.begin());
+    float4 v = make_float4(a.x, a.y, a.z, 0.f);
+    std::memcpy(&v.w, &s, sizeof s);
+    slotted.push_back(v);
+  }
+  if (int st = coef_.upload(coef.data(), coef.size() * sizeof(PairCoef))) return st;
+  if (int st = reach2_.upload(reach2.data(), reach2.size() * 4)) return st;
+  if (int st = plan_.build(slotted, lig_off, int(types.size()), segs)) return st;
+  scene_.coef = static_cast<const PairCoef *>(coef_.ptr);
+  scene_.reach2 = static_cast<const float *>(reach2_.ptr);
+  scene_.natpro = int(natpro);
+  scene_.ngroups = int(groups.ngroups());
+  scene_.form = plain_form();
+  protein_box(groups.xyzw, largest, scene_.lo, scene_.hi);
+  const int st = plan_.reserve(work_);
+  if (st == BUDE_ERR_OUT_OF_MEMORY) {  // (the tiled kernels need none of it)
+    work_.release();
+    return BUDE_OK;
+  }
+  usable_ = st == BUDE_OK;
+  return st;
+}
+
+hipError_t Deck::launch(const float4 *protein, const float *poses, size_t stride, float *energies,
+                        hipStream_t s) const {
+  if (!usable_) return hipErrorInvalidValue;
+  Scene sc = scene_;
+  sc.protein = protein;
+  return plan_.launch(sc, work_, poses, stride, nullptr, energies, s);
+}
+
+}  // namespace items
+}  // namespace bude

@@ -6,6 +6,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <numeric>
 
 namespace bude {
@@ -73,11 +74,12 @@ ProteinGroups group_protein(const BudeAtom *protein, size_t natpro) {
     g.xyzw[4 * i + 0] = a.x;
     g.xyzw[4 * i + 1] = a.y;
     g.xyzw[4 * i + 2] = a.z;
-    g.xyzw[4 * i + 3] = 0.f;
     if (i == 0 || a.type != protein[order[i - 1]].type) {
       g.begin.push_back(int32_t(i));
       g.type.push_back(a.type);
     }
+    const int32_t group = int32_t(g.type.size()) - 1;
+    std::memcpy(&g.xyzw[4 * i + 3], &group, sizeof group);
   }
   g.begin.push_back(int32_t(natpro));
   return g;

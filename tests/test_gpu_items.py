@@ -1,0 +1,61 @@
+"""The sorted-item pass behind Context.fasten against the tiled kernel
+(Batch.run_separate: one tiled launch per ligand): the pairs the sorted pass
+leaves out are exactly zero and the rest are summed in the same order, so
+every energy is equal bit for bit."""
+import numpy as np
+import pytest
+
+from minibude_amd import deck as D
+from minibude_amd.batch import Batch, LigandSet
+from minibude_amd.model import Context
+
+pytestmark = pytest.mark.gpu
+
+
+def tiled(d: D.Deck, device: int) -> np.ndarray:
+    with Batch(LigandSet(d.protein, d.forcefield, [d.ligand], [d.poses]), device) as b:
+        b.clear()
+        b.run_separate(1, 256)
+        return b.energies(0)
+
+
+def same(d: D.Deck, device: int, label: str) -> np.ndarray:
+    with Context(d, device) as c:
+        got = c.fasten(1, 256).energies
+    want = tiled(d, device)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"{label}: {np.count_nonzero(got != want)} differ"
+    return got
+
+
+@pytest.mark.parametrize("natpro, natlig, nposes, ntypes", [
+    (938, 26, 65536, 34),    # the small deck
+    (4096, 64, 1025, 34),    # just past one block of 1,024 poses
+    (2000, 12, 8193, 34),    # a block of one pose
+    (4095, 9, 131073, 3),    # few types: long rows, whole units of 4 x 64 items and a remainder
+    (63, 1, 2500000, 1),     # one atom, one type, fewer protein atoms than lanes
+    (65, 1030, 65537, 34),   # more than one chunk of items
+])
+def test_sorted_equals_tiled(gpu_device, natpro, natlig, nposes, ntypes):
+    same(D.synth_deck(natpro, natlig, nposes, seed=71, ntypes=ntypes), gpu_device, f"{natpro}x{natlig}x{nposes}")
+
+
+def test_poses_out_of_reach_and_not_finite(gpu_device):
+    d = D.synth_deck(938, 26, 65536, seed=72)
+    d.poses[3, ::7] += 1000.0     # far from the protein
+    d.poses[4, ::11] = np.nan
+    d.poses[5, 5::13] = np.inf
+    d.poses[3, 6::13] = -np.inf
+    d.poses[0, 3::17] = np.nan    # no rotation
+    e = same(d, gpu_device, "scattered")
+    assert np.all(e[::11] == 0.0) and np.all(e[::7] == 0.0)
+    d.poses[3:] = d.poses[3:, :1]  # every pose at one place
+    d.poses[:3] = 0.1
+    same(d, gpu_device, "one place")
+
+
+@pytest.mark.parametrize("field, value", [("radius", -3.0), ("radius", 0.0), ("elsc", 1e30), ("hphb", -np.inf)])
+def test_forcefields_without_a_reach(gpu_device, field, value):
+    # a radius sum that is not positive or a weight that is not finite: no pair may be left out
+    d = D.synth_deck(600, 20, 65536, seed=73)
+    d.forcefield[field][3] = value
+    same(d, gpu_device, f"{field}={value}")
