@@ -6,16 +6,18 @@
 // (energies) in device memory.  What bude_mi355x_create derives from the deck
 // and keeps in its own allocations -- protein atoms regrouped by forcefield
 // type, group offsets, the per-(ligand atom, group) pair coefficients and the
-// ligand coordinates -- is written here by two small kernels into `scratch`,
-// one fixed array per device that lives as long as the process.  The energy
-// kernel is the plain kernel itself (launch_plain), so the energies equal
-// bude_mi355x_fasten's bit for bit on the same deck.
+// ligand coordinates -- is written here by one small kernel into `scratch`,
+// one fixed array per device that lives as long as the process; what is left
+// of it holds the direct pass's sums (launch_direct), as many poses at a
+// time as fit, so the energies equal bude_mi355x_fasten's bit for bit on the
+// same deck.
 //
 // Every call on a device reuses that device's array and overwrites what it
 // reads: concurrent calls on one device (from several threads or streams)
 // race on it and must be serialised by the caller.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -23,6 +25,7 @@
 #include "bude_internal.h"
 #include "fasten_plain.h"
 #include "hip_util.h"
+#include "items.h"
 
 namespace {
 
@@ -108,7 +111,11 @@ __device__ bude::PairCoef pair_coef_dev(const BudeFFParams p, const BudeFFParams
   return c;
 }
 
-// One work-group: a stable counting sort of the protein atoms by forcefield
+// Work-groups 1 and up: coef[il * ntypes + g] = pair_coef(forcefield[g],
+// forcefield[type(il)]), one entry per work-item (none for a ligand atom
+// whose type is outside the forcefield; the call is rejected then).
+//
+// Work-group 0: a stable counting sort of the protein atoms by forcefield
 // type (atoms of one type keep their deck order, as bude::group_protein's
 // stable sort), writing the grouped coordinates and ntypes + 1 group offsets
 // (a type with no atom is an empty group; an empty group adds an exact 0 to a
@@ -117,9 +124,18 @@ __device__ bude::PairCoef pair_coef_dev(const BudeFFParams p, const BudeFFParams
 // [0, ntypes) sets *status to 1 and nothing reads past the forcefield.
 __global__ __launch_bounds__(kPrepThreads) void group_kernel(const BudeAtom *__restrict__ protein, int natpro,
                                                              const BudeAtom *__restrict__ ligand, int natlig,
-                                                             int ntypes, float4 *__restrict__ grouped,
+                                                             const BudeFFParams *__restrict__ ff, int ntypes,
+                                                             float4 *__restrict__ grouped,
                                                              int32_t *__restrict__ group_begin,
+                                                             bude::PairCoef *__restrict__ coef,
                                                              float4 *__restrict__ lig4, int32_t *__restrict__ status) {
+  if (blockIdx.x > 0) {
+    const int i = (int(blockIdx.x) - 1) * kPrepThreads + int(threadIdx.x);
+    if (i >= natlig * ntypes) return;
+    const int il = i / ntypes, g = i % ntypes, t = ligand[il].type;
+    if (t >= 0 && t < ntypes) coef[i] = pair_coef_dev(ff[g], ff[t]);
+    return;
+  }
   __shared__ int32_t count[kMaxTypes];           // atoms per type, then running write offset per type
   __shared__ int32_t wave_count[kPrepWaves][kMaxTypes];
   __shared__ int32_t bad;
@@ -191,15 +207,6 @@ __global__ __launch_bounds__(kPrepThreads) void group_kernel(const BudeAtom *__r
   }
 }
 
-// coef[il * ntypes + g] = pair_coef(forcefield[g], forcefield[type(il)]).
-__global__ void coef_kernel(const BudeAtom *__restrict__ ligand, int natlig, const BudeFFParams *__restrict__ ff,
-                            int ntypes, const int32_t *__restrict__ status, bude::PairCoef *__restrict__ coef) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= natlig * ntypes || *status) return;
-  const int il = i / ntypes, g = i % ntypes;
-  coef[i] = pair_coef_dev(ff[g], ff[ligand[il].type]);
-}
-
 }  // namespace
 
 extern "C" int bude_mi355x_fasten_noalloc(int device, const BudeAtom *protein, size_t natpro,
@@ -246,25 +253,43 @@ extern "C" int bude_mi355x_fasten_noalloc(int device, const BudeAtom *protein, s
   auto *status = reinterpret_cast<int32_t *>(base + l.status);
   const auto s = static_cast<hipStream_t>(stream);
 
-  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kPrepThreads), 0, s, protein, int(natpro), ligand, int(natlig),
-                     int(ntypes), grouped, group_begin, lig4, status);
-  if (int st = bude::hip_check(hipGetLastError(), "group_kernel launch")) return st;
   const int pairs = int(natlig * ntypes);
-  hipLaunchKernelGGL(coef_kernel, dim3((pairs + 255) / 256), dim3(256), 0, s, ligand, int(natlig), forcefield,
-                     int(ntypes), status, coef);
-  if (int st = bude::hip_check(hipGetLastError(), "coef_kernel launch")) return st;
-  // the deck check comes back before the energy kernel runs, so a rejected
-  // deck leaves the energies untouched
+  hipLaunchKernelGGL(group_kernel, dim3(unsigned(1 + (pairs + kPrepThreads - 1) / kPrepThreads)), dim3(kPrepThreads), 0,
+                     s, protein, int(natpro), ligand, int(natlig), forcefield, int(ntypes), grouped, group_begin, coef,
+                     lig4, status);
+  if (int st = bude::hip_check(hipGetLastError(), "group_kernel launch")) return st;
+  // 1 when the deck was rejected; every energy kernel below leaves the
+  // energies untouched then
   int32_t bad = 0;
-  if (int st = bude::hip_check(hipMemcpyAsync(&bad, status, sizeof(bad), hipMemcpyDeviceToHost, s),
-                               "hipMemcpyAsync status"))
-    return st;
-  if (int st = bude::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;
-  if (bad)
-    return bude::fail(BUDE_ERR_INVALID_ARGUMENT,
-                      std::string(who) + ": an atom type is outside the forcefield (" + std::to_string(ntypes) +
-                          " rows); the energies were not written");
+  auto read_status = [&]() -> int {
+    if (int st = bude::hip_check(hipMemcpyAsync(&bad, status, sizeof(bad), hipMemcpyDeviceToHost, s),
+                                 "hipMemcpyAsync status"))
+      return st;
+    if (int st = bude::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;
+    if (bad)
+      return bude::fail(BUDE_ERR_INVALID_ARGUMENT,
+                        std::string(who) + ": an atom type is outside the forcefield (" + std::to_string(ntypes) +
+                            " rows); the energies were not written");
+    return BUDE_OK;
+  };
 
+  const size_t room = kScratchBytes - l.end;
+  // poses at a time: all of them, or the whole tiles whose atom sums fit
+  const size_t fit = room / (natlig * sizeof(float)) / 64 * 64;
+  const size_t at_once = std::min(fit, nposes);
+  if (at_once) {
+    for (size_t j = 0; j < nposes; j += at_once) {
+      const bude::items::DirectArgs a{grouped,       group_begin, coef,        lig4,        poses + j,
+                                      energies + j,  pose_stride, std::min(at_once, nposes - j), int(natlig),
+                                      int(ntypes),   bude::plain_form(),       status,
+                                      reinterpret_cast<float *>(base + l.end)};
+      if (int st = bude::hip_check(bude::items::launch_direct(a, s), "direct pass launch")) return st;
+    }
+    return read_status();
+  }
+
+  // a ligand whose sums do not fit for 64 poses: the tiled kernel, after the check
+  if (int st = read_status()) return st;
   bude::PlainArgs a{};
   a.protein = grouped;
   a.group_begin = group_begin;

@@ -32,6 +32,7 @@ struct bude_ctx {
   size_t natpro = 0, natlig = 0, ntypes = 0, nposes = 0, ngroups = 0;
   bude::DeviceBuffer protein, group_begin, coef, ligand, poses, energies;
   bude::items::Deck sorted;
+  float *direct = nullptr;  // scratch of the direct pass, behind the energies (null: not used)
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double context_ms = 0.0;
@@ -141,10 +142,13 @@ extern "C" int bude_mi355x_create(int device, const BudeAtom *protein, size_t na
     st = bude::hip_check(hipMemcpy(static_cast<float *>(c->poses.ptr) + k * nposes, poses[k], nposes * sizeof(float),
                                    hipMemcpyHostToDevice),
                          "hipMemcpy poses");
-  if (!st) st = c->energies.alloc(nposes * sizeof(float));
   if (!st)
     st = c->sorted.prepare(groups, forcefield, std::vector<BudeAtom>(ligand, ligand + natlig), {0, int32_t(natlig)},
                            {bude::items::Segment{0, 0, int64_t(nposes)}});
+  const size_t direct = bude::items::direct_bytes(nposes, natlig), padded = (nposes + 63) / 64 * 64;
+  const bool use_direct = !c->sorted.usable() && direct <= bude::items::kDirectBytes;
+  if (!st) st = c->energies.alloc(padded * sizeof(float) + (use_direct ? direct : 0));
+  if (!st && use_direct) c->direct = static_cast<float *>(c->energies.ptr) + padded;
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev0), "hipEventCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev1), "hipEventCreate");
@@ -183,13 +187,17 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   a.ngroups = int(ctx->ngroups);
   a.ppwi = int(ppwi);
   a.form = bude::plain_form();
+  const bude::items::DirectArgs direct{a.protein, a.group_begin, a.coef,   a.ligand, a.poses, a.energies, a.stride,
+                                       a.nposes,  a.natlig,      a.ngroups, a.form,   nullptr,
+                                       ctx->direct};
 
   for (size_t i = 0; i < warmup + iterations; i++) {
     const auto t0 = std::chrono::steady_clock::now();
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
     const hipError_t le = ctx->sorted.usable()
                               ? ctx->sorted.launch(a.protein, a.poses, a.stride, a.energies, ctx->stream)
-                              : bude::launch_plain(a, int(wgsize), ctx->stream);
+                          : ctx->direct ? bude::items::launch_direct(direct, ctx->stream)
+                                            : bude::launch_plain(a, int(wgsize), ctx->stream);
     if (int st = bude::hip_check(le, "fasten_plain launch")) return st;
     if (int st = bude::hip_check(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord")) return st;
     if (int st = bude::hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return st;

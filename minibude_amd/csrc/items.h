@@ -86,6 +86,28 @@ class Plan {
   double items_ = 0;
 };
 
+// The pass over every pair, for decks too small to sort (and those whose
+// pairs have no reach): one wave per 64 poses and ligand atom or, while those
+// are too few for the device, several that share the protein's groups; then the sums in
+// the tiled kernels' order, so the energies are theirs bit for bit.
+struct DirectArgs {
+  const float4 *protein;
+  const int32_t *group_begin;  // ngroups + 1
+  const PairCoef *coef;        // [natlig][ngroups]
+  const float4 *ligand;
+  const float *poses;          // 6 rows of `stride` floats
+  float *energies;             // nposes
+  size_t stride, nposes;
+  int natlig, ngroups, form;
+  const int32_t *skip;         // device flag: nothing is scored when set (may be null)
+  float *scratch;              // direct_bytes(nposes, natlig)
+};
+// Scratch of a direct pass over n poses.  Above kDirectBytes the tiled kernel
+// scores as fast without it.
+constexpr size_t kDirectBytes = size_t(64) << 20;
+size_t direct_bytes(size_t n, size_t natlig);
+hipError_t launch_direct(const DirectArgs &a, hipStream_t s);
+
 // Everything one deck's passes need on the sorted path, from the host deck:
 // scene, plan and workspace.  usable() is false where the path does not
 // apply (see worth_sorting, pair_reach) or its memory cannot be had; the

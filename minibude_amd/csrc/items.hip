@@ -398,6 +398,21 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
     if (i0 + k * 64 + lane < i1) partial[out[k]] = e[k] + part[k];
 }
 
+// p[0] + p[stride] + ... in order, eight loads in flight.
+__device__ __forceinline__ float sum_column(const float *__restrict__ p, int n, size_t stride) {
+  float e = 0.f;
+  int a = 0;
+  for (; a + 8 <= n; a += 8) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = p[size_t(a + k) * stride];
+#pragma unroll
+    for (int k = 0; k < 8; k++) e += v[k];
+  }
+  for (; a < n; a++) e += p[size_t(a) * stride];
+  return e;
+}
+
 // energies[row] = half the sum of the pose's atoms' energies, in the
 // ligand's order.  `per` work-groups of 256 per block.
 __global__ __launch_bounds__(256) void reduce_kernel(const Block *__restrict__ blocks, int per,
@@ -405,18 +420,62 @@ __global__ __launch_bounds__(256) void reduce_kernel(const Block *__restrict__ b
   const Block bk = blocks[blockIdx.x / unsigned(per)];
   const int j = int(blockIdx.x % unsigned(per)) * 256 + int(threadIdx.x);
   if (j >= bk.npose) return;
-  const float *p = partial + size_t(bk.part_off) + size_t(j);
-  float e = 0.f;
-  int a = 0;
-  for (; a + 8 <= bk.natlig; a += 8) {
-    float v[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) v[k] = p[size_t(a + k) * bk.part_stride];
-#pragma unroll
-    for (int k = 0; k < 8; k++) e += v[k];
+  energies[size_t(bk.pose_off) + size_t(j)] =
+      0.5f * sum_column(partial + size_t(bk.part_off) + size_t(j), bk.natlig, bk.part_stride);
+}
+
+// Few poses leave a wave per 64 of them alone with every pair: a serial chain
+// on a nearly idle device (938 x 26 atoms x 64 poses took 980 us, and takes
+// 14; 700 x 19 x 4,096, 574 and 31; latency and the last waves bound it).  One work-group of `blockDim.x / 64` waves per (64 poses, ligand
+// atom): its waves share the groups, their parts meet in LDS and wave 0 adds
+// them in order (SPLIT); or, where those waves are enough already, one wave
+// per (64 poses, ligand atom).  out[atom][pose], rows of 64 poses per tile.
+template <int FORM, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 1024 : 256) void direct_kernel(
+    const float4 *__restrict__ protein, const int32_t *__restrict__ group_begin, const PairCoef *__restrict__ coef,
+    const float4 *__restrict__ ligand, const float *__restrict__ poses, size_t stride, size_t n, int ntiles,
+    int natlig, int ngroups, const int32_t *__restrict__ skip, float *__restrict__ out) {
+  extern __shared__ float parts[];  // SPLIT: [ngroups][64]
+  if (skip && *skip) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int nwaves = int(blockDim.x >> 6);
+  const int64_t w = SPLIT ? int64_t(blockIdx.x) : int64_t(blockIdx.x) * nwaves + wave;
+  const int il = int(w / ntiles), tile = int(w - int64_t(il) * ntiles);
+  if (il >= natlig) return;  // (whole waves; with SPLIT none)
+  const size_t j = size_t(tile) * 64 + size_t(lane);
+  const Xform t = make_xform(poses, stride, j < n ? j : n - 1);
+  const float4 la = ligand[il];
+  const float lx[1] = {place(t.m[0], t.m[1], t.m[2], t.m[3], la)};
+  const float ly[1] = {place(t.m[4], t.m[5], t.m[6], t.m[7], la)};
+  const float lz[1] = {place(t.m[8], t.m[9], t.m[10], t.m[11], la)};
+  const PairCoef *cl = coef + size_t(il) * size_t(ngroups);
+  float e[1] = {0.f};
+  if constexpr (SPLIT) {
+    for (int g = wave; g < ngroups; g += nwaves) {
+      e[0] = 0.f;
+      group_dispatch<1, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, e);
+      parts[g * 64 + lane] = e[0];
+    }
+    __syncthreads();
+    if (wave) return;
+    e[0] = 0.f;
+#pragma unroll 8
+    for (int g = 0; g < ngroups; g++) e[0] += parts[g * 64 + lane];
+  } else {
+    for (int g = 0; g < ngroups; ++g)
+      group_dispatch<1, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, e);
   }
-  for (; a < bk.natlig; a++) e += p[size_t(a) * bk.part_stride];
-  energies[size_t(bk.pose_off) + size_t(j)] = e * 0.5f;
+  out[size_t(il) * size_t(ntiles) * 64 + j] = e[0];
+}
+
+// Pose energies from the atoms' (partial[atom][pose]), one work-item per pose.
+__global__ __launch_bounds__(256) void atom_sum_kernel(const float *__restrict__ partial, size_t npad, size_t n,
+                                                       int natlig, const int32_t *__restrict__ skip,
+                                                       float *__restrict__ energies) {
+  if (skip && *skip) return;
+  const size_t j = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (j >= n) return;
+  energies[j] = 0.5f * sum_column(partial + j, natlig, npad);
 }
 
 template <int PPT, int SCATTER, class... A> void launch_bin(int ntasks, hipStream_t s, A... args) {
@@ -435,6 +494,8 @@ template <int RB, class... A> void launch_score(int form, int nunits, hipStream_
   if (form == kFormD) hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormD>), grid, dim3(256), 0, s, args...);
   else hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormB>), grid, dim3(256), 0, s, args...);
 }
+
+constexpr size_t kDirectWaves = 16384;
 
 // Items of one chunk: 20 bytes each in the workspace.
 constexpr int64_t kChunkItems = int64_t(1) << 26;
@@ -491,10 +552,14 @@ bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std
     if (L > kChunkItems / 64) return false;
     items += double(L) * double(s.n);
   }
-  // seven launches and the sort cost about 60 us whatever the size, which the
-  // tiled kernels score some 2e8 pairs in; a segment is to fill the
-  // work-groups that sort it
-  return items * double(natpro) >= 1.5e8 && items >= 65536 * 1.0 && items >= 4096.0 * double(segs.size());
+  // The direct pass scores some 1.8e9 pairs a millisecond; the sort's seven
+  // launches cost 40-50 us whatever the size, and with few items (large
+  // boxes) scoring them grows with the protein.  Both measured, direct and
+  // sorted, over 64 .. 131,072 poses: 300 x 8 atoms cross at 1.5e8 pairs
+  // (67 and 65 us), 700 x 19 at 1e8, 938 x 26 at 1.4e8, 938 x 64 at 2e8,
+  // 4,096 x 26 at 4.4e8 (189 and 192 us), 4,096 x 96 at 6e8.  A segment is to
+  // fill the work-groups that sort it.
+  return items * double(natpro) >= 6e7 + 8e4 * double(natpro) && items >= 4096.0 * double(segs.size());
 }
 
 int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
@@ -720,6 +785,36 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+size_t direct_bytes(size_t n, size_t natlig) { return (n + 63) / 64 * 64 * natlig * sizeof(float); }
+
+hipError_t launch_direct(const DirectArgs &a, hipStream_t s) {
+  const size_t ntiles = (a.nposes + 63) / 64, npad = ntiles * 64, natlig = size_t(a.natlig);
+  if (a.nposes == 0 || ntiles * natlig > 0x7fffffffu || !a.scratch) return hipErrorInvalidValue;
+  // waves per (tile, ligand atom): until they number some sixteen per SIMD
+  // (256 CUs of 4), so that the last ones end together (4,096 x 26 atoms,
+  // 4,096 poses: 198 us with four per SIMD, 152 with sixteen; 938 x 26: 64
+  // and 52 us); as far as the parts fit 64 KB of LDS
+  size_t split = std::min({size_t(16), size_t(a.ngroups), kDirectWaves / (ntiles * natlig)});
+  const size_t lds = size_t(a.ngroups) * 64 * sizeof(float);
+  if (lds > 65536) split = 1;
+  auto run = [&](auto kernel, size_t blocks, size_t threads, size_t bytes) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(unsigned(threads)), unsigned(bytes), s, a.protein,
+                       a.group_begin, a.coef, a.ligand, a.poses, a.stride, a.nposes, int(ntiles), a.natlig, a.ngroups,
+                       a.skip, a.scratch);
+  };
+  if (split > 1) {
+    if (a.form == kFormD) run(direct_kernel<kFormD, true>, ntiles * natlig, 64 * split, lds);
+    else run(direct_kernel<kFormB, true>, ntiles * natlig, 64 * split, lds);
+  } else {
+    if (a.form == kFormD) run(direct_kernel<kFormD, false>, (ntiles * natlig + 3) / 4, 256, 0);
+    else run(direct_kernel<kFormB, false>, (ntiles * natlig + 3) / 4, 256, 0);
+  }
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  hipLaunchKernelGGL(atom_sum_kernel, dim3(unsigned((a.nposes + 255) / 256)), dim3(256), 0, s, a.scratch, npad,
+                     a.nposes, a.natlig, a.skip, a.energies);
+  return hipGetLastError();
 }
 
 int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,

@@ -1,10 +1,15 @@
-"""The sorted-item pass behind Context.fasten against the tiled kernel
+"""The sorted-item pass and the direct pass (small decks) behind
+Context.fasten and the no-allocation entry point against the tiled kernel
 (Batch.run_separate: one tiled launch per ligand): the pairs the sorted pass
 leaves out are exactly zero and the rest are summed in the same order, so
 every energy is equal bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
+from minibude_amd import capi
 from minibude_amd import deck as D
 from minibude_amd.batch import Batch, LigandSet
 from minibude_amd.model import Context
@@ -37,6 +42,30 @@ def same(d: D.Deck, device: int, label: str) -> np.ndarray:
 ])
 def test_sorted_equals_tiled(gpu_device, natpro, natlig, nposes, ntypes):
     same(D.synth_deck(natpro, natlig, nposes, seed=71, ntypes=ntypes), gpu_device, f"{natpro}x{natlig}x{nposes}")
+
+
+@pytest.mark.parametrize("natpro, natlig, nposes, ntypes", [
+    (5, 1, 1, 2),          # one pose, fewer groups than waves
+    (938, 26, 65, 34),     # 16 waves per tile, a tile of one pose
+    (300, 200, 4097, 34),  # two waves per tile
+    (40, 300, 8191, 300),  # more groups than fit in LDS
+    (40, 300, 4096, 34),   # one wave per tile, four tiles per work-group
+])
+def test_direct_equals_tiled(gpu_device, natpro, natlig, nposes, ntypes):
+    same(D.synth_deck(natpro, natlig, nposes, seed=74, ntypes=ntypes), gpu_device, f"{natpro}x{natlig}x{nposes}")
+
+
+def test_noalloc_in_several_passes(gpu_device):
+    # the sums of 1,000 ligand atoms fit the fixed scratch for some 700 poses at a time
+    d = D.synth_deck(400, 1000, 5001, seed=75)
+    up = [torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).cuda()
+          for a in (d.protein, d.ligand, d.forcefield, d.poses)]
+    e = torch.full((d.nposes,), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    p = [ctypes.c_void_p(t.data_ptr()) for t in up]
+    capi.check(capi.lib().bude_mi355x_fasten_noalloc(gpu_device, p[0], d.natpro, p[1], d.natlig, p[2], d.ntypes, p[3],
+                                                     d.nposes, d.nposes, 1, 64, ctypes.c_void_p(e.data_ptr()), None))
+    assert np.array_equal(e.cpu().numpy().view(np.uint32), tiled(d, gpu_device).view(np.uint32))
 
 
 def test_poses_out_of_reach_and_not_finite(gpu_device):
