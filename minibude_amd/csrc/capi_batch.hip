@@ -17,6 +17,7 @@
 #include "fasten_batch.h"
 #include "fasten_plain.h"
 #include "hip_util.h"
+#include "items.h"
 
 namespace {
 
@@ -39,6 +40,7 @@ struct bude_batch {
   std::vector<size_t> nposes, pose_off;
   std::vector<bude::LigandMeta> meta_host;
   bude::DeviceBuffer protein, group_begin, coef, ligands, meta, poses, energies, counter;
+  bude::items::Deck sorted;
   // tile lists per (ppwi, order)
   std::map<std::pair<int, int>, std::unique_ptr<bude::DeviceBuffer>> tiles;
   std::map<std::pair<int, int>, int> ntiles;
@@ -92,7 +94,14 @@ int tiles_for(bude_batch *b, int ppwi, int order, const bude::DeviceBuffer **buf
   return BUDE_OK;
 }
 
+// One pass over the batch: the sorted-item pass where it applies (the
+// configuration shapes the tiled kernel only), else the tiled kernel.
 int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
+  if (b->sorted.usable())
+    return bude::hip_check(b->sorted.launch(static_cast<const float4 *>(b->protein.ptr),
+                                            static_cast<const float *>(b->poses.ptr), b->total_poses,
+                                            static_cast<float *>(b->energies.ptr), b->stream),
+                           "sorted batch launch");
   const bude::DeviceBuffer *tb = nullptr;
   int nt = 0;
   if (int st = tiles_for(b, cfg->ppwi, cfg->order, &tb, &nt)) return st;
@@ -116,13 +125,15 @@ int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
 }
 
 int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
-  const auto key = std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
+  const auto key = b->sorted.usable() ? std::make_tuple(0, 0, 0, 0)
+                                      : std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
   auto it = b->graphs.find(key);
   if (it == b->graphs.end()) {
     // build tiles before capture (the upload is not capturable)
     const bude::DeviceBuffer *tb = nullptr;
     int nt = 0;
-    if (int st = tiles_for(b, cfg->ppwi, cfg->order, &tb, &nt)) return st;
+    if (!b->sorted.usable())
+      if (int st = tiles_for(b, cfg->ppwi, cfg->order, &tb, &nt)) return st;
     auto g = std::make_unique<GraphExec>();
     if (int st = bude::hip_check(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
                                  "hipStreamBeginCapture"))
@@ -189,6 +200,9 @@ extern "C" int bude_mi355x_batch_create(int device, const BudeAtom *protein, siz
 
   std::vector<float> lig4;
   std::vector<bude::PairCoef> coef;
+  std::vector<BudeAtom> atoms;
+  std::vector<int32_t> lig_off(1, 0);
+  std::vector<bude::items::Segment> segs;
   size_t total = 0;
   for (size_t i = 0; i < nligands; i++) {
     bude::LigandMeta m{};
@@ -205,6 +219,9 @@ extern "C" int bude_mi355x_batch_create(int device, const BudeAtom *protein, siz
     coef.insert(coef.end(), c.begin(), c.end());
     if (coef.size() > 0x7fffffffu || lig4.size() / 4 > 0x7fffffffu)
       return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_batch_create: batch too large");
+    atoms.insert(atoms.end(), ligands[i], ligands[i] + natlig[i]);
+    lig_off.push_back(int32_t(atoms.size()));
+    segs.push_back(bude::items::Segment{int32_t(i), int64_t(total), int64_t(nposes[i])});
     b->meta_host.push_back(m);
     b->natlig.push_back(int32_t(natlig[i]));
     b->nposes.push_back(nposes[i]);
@@ -228,6 +245,7 @@ extern "C" int bude_mi355x_batch_create(int device, const BudeAtom *protein, siz
                            "hipMemcpy poses");
   if (!st) st = b->energies.alloc(total * sizeof(float));
   if (!st) st = b->counter.alloc(256);
+  if (!st) st = b->sorted.prepare(groups, forcefield, atoms, lig_off, segs);
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&b->ev0), "hipEventCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&b->ev1), "hipEventCreate");
