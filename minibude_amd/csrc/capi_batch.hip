@@ -94,17 +94,28 @@ int tiles_for(bude_batch *b, int ppwi, int order, const bude::DeviceBuffer **buf
   return BUDE_OK;
 }
 
-// One pass over the batch: the sorted-item pass where it applies (the
-// configuration shapes the tiled kernel only), else the tiled kernel.
+// Whether a batch that is not sorted is so small that a wave of the
+// persistent kernel would score one tile or a few nearly alone on its SIMD:
+// fewer than four 64-pose tiles per SIMD of 256 CUs.
+bool few_tiles(const bude_batch *b) {
+  size_t t = 0;
+  for (size_t n : b->nposes) t += (n + 63) / 64;
+  return t <= 4096;
+}
+
+// One pass over the batch: the sorted-item pass where it applies, else
+// work-groups per tile where the tiles are few (the configuration shapes
+// the persistent kernel only), else the persistent kernel.
 int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
   if (b->sorted.usable())
     return bude::hip_check(b->sorted.launch(static_cast<const float4 *>(b->protein.ptr),
-                                            static_cast<const float *>(b->poses.ptr), b->total_poses,
+                                            static_cast<const float *>(b->poses.ptr), b->total_poses, nullptr,
                                             static_cast<float *>(b->energies.ptr), b->stream),
                            "sorted batch launch");
   const bude::DeviceBuffer *tb = nullptr;
   int nt = 0;
-  if (int st = tiles_for(b, cfg->ppwi, cfg->order, &tb, &nt)) return st;
+  const bool few = few_tiles(b);
+  if (int st = tiles_for(b, few ? 1 : cfg->ppwi, cfg->order, &tb, &nt)) return st;
   bude::BatchArgs a{};
   a.protein = static_cast<const float4 *>(b->protein.ptr);
   a.group_begin = static_cast<const int32_t *>(b->group_begin.ptr);
@@ -119,6 +130,7 @@ int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
   a.ngroups = int(b->ngroups);
   a.ntiles = nt;
   a.form = bude::plain_form();
+  if (few) return bude::hip_check(bude::launch_tiles(a, std::min(nt, 2 * b->cus), b->stream), "fasten_tile launch");
   const int waves = b->cus * 4 * cfg->waves_per_simd;
   const int blocks = std::max(1, waves / (cfg->wgsize / 64));
   return bude::hip_check(bude::launch_batch(a, cfg->ppwi, cfg->wgsize, blocks, b->stream), "fasten_batch launch");
@@ -133,7 +145,7 @@ int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
     const bude::DeviceBuffer *tb = nullptr;
     int nt = 0;
     if (!b->sorted.usable())
-      if (int st = tiles_for(b, cfg->ppwi, cfg->order, &tb, &nt)) return st;
+      if (int st = tiles_for(b, few_tiles(b) ? 1 : cfg->ppwi, cfg->order, &tb, &nt)) return st;
     auto g = std::make_unique<GraphExec>();
     if (int st = bude::hip_check(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
                                  "hipStreamBeginCapture"))

@@ -27,6 +27,7 @@
 #include "fasten_batch.h"
 #include "field.h"
 #include "hip_util.h"
+#include "items.h"
 #include "mlp.h"
 #include "select.h"
 #include "surrogate.h"
@@ -150,7 +151,11 @@ Norm norm_of(std::vector<float> e, float clip_q, float tail_q) {
 struct ProteinSlot {
   size_t ngroups = 0;
   std::vector<int32_t> coef_off;
-  DeviceBuffer protein, group_begin, coef, slot_coef;
+  DeviceBuffer protein, group_begin, coef, slot_coef, reach2;
+  // what the sorted passes score against (its tables are slot_coef and
+  // reach2); reachable: every pair of the protein's has a reach
+  bude::items::Scene scene;
+  bool reachable = false;
   // exact_sel[pose_off[l] + j] is the exact energy of pose
   // sel_idx[pose_off[l] + j] of pair l (j < nsel[l]); meta_rs / tiles_rs /
   // rs_ntiles the rescoring tables (tiles of each chunk, counts per chunk
@@ -226,13 +231,22 @@ struct bude_combined {
   // [chunk_lig[k], chunk_lig[k + 1]): the second stream scores, selects and
   // builds the rescoring tables of chunk k while the first rescores chunk
   // k - 1.  Per chunk: its selection plan, the first slot of its rescoring
-  // tiles (of Σ ceil(n / 64) over its pairs), the tiles its selection is
-  // expected to give, and two events (scores done, tables done).
+  // tiles (of Σ ceil(n / 64) over its pairs), and two events (scores done,
+  // tables done).
   std::vector<size_t> chunk_lig;
   std::vector<std::unique_ptr<bude::sel::Plan>> chunk_plan;
   std::vector<int64_t> chunk_tile;
-  std::vector<int64_t> chunk_expect;
-  std::vector<int64_t> lig_expect;    // expected rescoring tiles of each pair: ceil(k / 64)
+  // Sorted passes (items.h), each on one stream with that stream's scratch:
+  // the rescoring of every chunk and of the whole set over the first
+  // ceil(keep n) selected rows of each pair (sorted_rows; the tiled kernel
+  // scores rows past them: ties, and what widening adds), every pose of every
+  // pair (planned when first wanted) and of a protein's fallback pairs, on
+  // the first stream; the sampled poses on the third.  sorted_ok: their memory could be had.
+  std::vector<std::unique_ptr<bude::items::Plan>> chunk_sorted;
+  bude::items::Plan whole_sorted, all_sorted, fb_sorted, label_sorted;
+  bude::items::Workspace work, label_work;
+  DeviceBuffer sorted_rows;
+  bool sorted_ok = false, label_sorted_ok = false, all_planned = false;
   bool plan_ok = false;               // the selection tables above are complete
   bude::field::Grid grid{};
   // the screen's proteins: the one screened last is slots[cur]; a batch
@@ -285,7 +299,7 @@ struct Span {
 // the sampled poses' tables), with room for the 256-byte alignment.
 size_t stage_bound(const bude_combined *c, size_t natpro) {
   const size_t L = c->nlig, lpp = std::min<size_t>(c->cfg.labels_per_pair, c->total);
-  return natpro * 16 + (natpro + 2) * 4 + c->slot_type.size() * c->ff.size() * sizeof(bude::PairCoef) +
+  return natpro * 16 + (natpro + 2) * 4 + c->slot_type.size() * c->ff.size() * (sizeof(bude::PairCoef) + sizeof(float)) +
          3 * L * sizeof(bude::LigandMeta) + 2 * L * lpp * 4 + L * (lpp / bude::kSplitTile + 1) * 8 + (L + 1) * 8 +
          L * sizeof(bude::sel::Segment) + 16 * 256;
 }
@@ -323,6 +337,35 @@ int stage_upload(ProteinSlot &ps, DeviceBuffer &dst, const void *src, size_t n, 
 // Synchronous upload, or staged on stream s when s is not null.
 int put(bude_combined *c, DeviceBuffer &dst, const void *src, size_t n, hipStream_t s) {
   return s ? stage_upload(c->s(), dst, src, n, s) : dst.assign(src, n);
+}
+
+// A sorted pass is planned over the ligands' atoms with their map slots.
+int plan_sorted(const bude_combined *c, bude::items::Plan &plan, const std::vector<bude::items::Segment> &segs) {
+  std::vector<float4> atoms;
+  std::vector<int32_t> off;
+  for (const std::vector<BudeAtom> &l : c->lig) {
+    off.push_back(int32_t(atoms.size()));
+    for (const BudeAtom &a : l) {
+      float4 v = make_float4(a.x, a.y, a.z, 0.f);
+      std::memcpy(&v.w, &c->slot_of_type[size_t(a.type)], 4);
+      atoms.push_back(v);
+    }
+  }
+  off.push_back(int32_t(atoms.size()));
+  return plan.build(atoms, off, int(c->slot_type.size()), segs);
+}
+
+// Room for a planned pass; *ok is false when the device has none (the tiled
+// kernels then score instead).
+int reserve_sorted(const bude::items::Plan &plan, bude::items::Workspace &w, bool *ok) {
+  const int st = plan.reserve(w);
+  *ok = st == BUDE_OK;
+  return st == BUDE_ERR_OUT_OF_MEMORY ? BUDE_OK : st;
+}
+
+// Whether protein slot ps is scored by this sorted pass.
+bool use_sorted(const ProteinSlot &ps, const bude::items::Plan &plan, bool ok) {
+  return ok && ps.reachable && plan.worth(size_t(ps.scene.natpro));
 }
 
 // Work tables of one persistent batched launch scoring spans[i].n poses of
@@ -383,13 +426,16 @@ int launch_exact(bude_combined *c, const float *poses, size_t stride, float *ene
   return bude::hip_check(bude::launch_batch(a, kBatchPpwi, g.wgsize, g.blocks, c->stream), "combined batch launch");
 }
 
-// The sampled-pose pass (about a thousand poses per pair): the split form,
-// 16-pose tiles, four lanes per pose, so the short pass fills the SIMDs
-// instead of leaving one latency-bound wave on each.  Its energies only
-// train or validate the surrogate; every energy the screen returns comes
-// from the tiled kernel.
+// The sampled-pose pass (about a thousand poses per pair): sorted, or, where
+// that does not apply, the split form: 16-pose tiles, four lanes per pose, so
+// the short pass fills the SIMDs instead of leaving one latency-bound wave on
+// each.  Its energies only train or validate the surrogate; every energy the
+// screen returns comes from the sorted or the tiled kernels.
 int launch_sampled(bude_combined *c, const float *poses, size_t stride, float *energies, const DeviceBuffer &meta,
                    const DeviceBuffer &tiles, int ntiles, hipStream_t stream) {
+  if (use_sorted(c->s(), c->label_sorted, c->label_sorted_ok))
+    return bude::hip_check(c->label_sorted.launch(c->s().scene, c->label_work, poses, stride, nullptr, energies, stream),
+                           "combined sampled-pose pass");
   if (ntiles == 0) return BUDE_OK;
   bude::BatchArgs a{};
   a.protein = static_cast<const float4 *>(c->s().protein.ptr);
@@ -407,8 +453,20 @@ int launch_sampled(bude_combined *c, const float *poses, size_t stride, float *e
   return bude::hip_check(bude::launch_split(a, stream), "combined sampled-pose launch");
 }
 
+// Exact energies of whole pairs on the first stream, through `plan` (planned
+// over the spans by the caller, null: not planned) where it applies.
 int exact_ragged(bude_combined *c, const std::vector<Span> &spans, const float *poses, size_t stride,
-                 float *energies, DeviceBuffer &meta, DeviceBuffer &tiles) {
+                 float *energies, DeviceBuffer &meta, DeviceBuffer &tiles, const bude::items::Plan *plan = nullptr) {
+  if (plan && !spans.empty()) {
+    bool ok = plan->fits(c->work);
+    if (!ok && use_sorted(c->s(), *plan, true)) {  // (growing the scratch frees what queued passes use)
+      if (int st = bude::hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return st;
+      if (int st = reserve_sorted(*plan, c->work, &ok)) return st;
+    }
+    if (use_sorted(c->s(), *plan, ok))
+      return bude::hip_check(plan->launch(c->s().scene, c->work, poses, stride, nullptr, energies, c->stream),
+                             "combined sorted pass");
+  }
   int nt = 0;
   if (int st = prepare_exact(c, spans, meta, tiles, &nt)) return st;
   return launch_exact(c, poses, stride, energies, meta, tiles, nt);
@@ -629,8 +687,9 @@ int train_atom(bude_combined *c, uint64_t pseed) {
 // Per-pair top-k of pred over the pairs of `plan` (pairs first .. first +
 // n - 1) and their rescoring tables from the ligand list `order` (n
 // entries) into tiles / *ntiles, on stream s.
+// `sorted`: a sorted pass scores each pair's first sorted_rows rows.
 int select_and_tables(bude_combined *c, const bude::sel::Plan &plan, size_t first, const int32_t *order, int n,
-                      int2 *tiles, int32_t *ntiles, hipStream_t s) {
+                      int2 *tiles, int32_t *ntiles, bool sorted, hipStream_t s) {
   uint32_t *sel_n = static_cast<uint32_t *>(c->s().sel_n.ptr);
   if (int st = bude::hip_check(bude::sel::select_lowest_segments(plan, static_cast<const float *>(c->pred.ptr),
                                                                  static_cast<uint32_t *>(c->s().sel_idx.ptr),
@@ -638,14 +697,21 @@ int select_and_tables(bude_combined *c, const bude::sel::Plan &plan, size_t firs
                                "select"))
     return st;
   return bude::hip_check(
-      bude::build_rescore_tables(order, n, sel_n, static_cast<bude::LigandMeta *>(c->s().meta_rs.ptr), tiles, ntiles, s),
+      bude::build_rescore_tables(order, n, sel_n, sorted ? static_cast<const uint32_t *>(c->sorted_rows.ptr) : nullptr,
+                                 static_cast<bude::LigandMeta *>(c->s().meta_rs.ptr), tiles, ntiles, s),
       "rescoring tables");
 }
 
-// Exact energies of the selected poses listed by tiles / *ntiles (written
-// on the device by select_and_tables) into exact_sel, on the first stream;
-// `expect` tiles set the grid depth.
-int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, int64_t expect) {
+// Exact energies of the selected poses into exact_sel, on the first stream:
+// with `plan`, its rows by the sorted pass; those listed by tiles / *ntiles
+// (written on the device by select_and_tables) by work-groups per tile.
+int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, const bude::items::Plan *plan) {
+  if (plan)
+    if (int st = bude::hip_check(plan->launch(c->s().scene, c->work, static_cast<const float *>(c->poses.ptr), c->total,
+                                              static_cast<const uint32_t *>(c->s().sel_idx.ptr),
+                                              static_cast<float *>(c->s().exact_sel.ptr), c->stream),
+                                 "combined sorted rescoring"))
+      return st;
   bude::BatchArgs a{};
   a.protein = static_cast<const float4 *>(c->s().protein.ptr);
   a.group_begin = static_cast<const int32_t *>(c->s().group_begin.ptr);
@@ -655,15 +721,12 @@ int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, i
   a.tiles = tiles;
   a.poses = static_cast<const float *>(c->poses.ptr);
   a.energies = static_cast<float *>(c->s().exact_sel.ptr);
-  a.counter = static_cast<unsigned int *>(c->counter.ptr);
   a.stride = c->total;
   a.ngroups = int(c->s().ngroups);
   a.form = bude::plain_form();
   a.pose_index = static_cast<const uint32_t *>(c->s().sel_idx.ptr);
   a.ntiles_dev = ntiles;
-  const bude::PinnedGrid g = bude::pinned_grid(c->cus, c->lds_per_cu, batch_waves_per_simd(expect, c->cus));
-  a.lds_bytes = g.lds_bytes;
-  return bude::hip_check(bude::launch_batch_indexed(a, g.blocks, c->stream), "combined rescoring launch");
+  return bude::hip_check(bude::launch_tiles(a, 2 * c->cus, c->stream), "combined rescoring launch");
 }
 
 // The ligands [a, b) heaviest first (ties in index order).
@@ -683,17 +746,15 @@ int plan_selection(bude_combined *c, float keep) {
   c->plan_ok = false;
   const size_t L = c->nlig;
   std::vector<bude::sel::Segment> segs(L);
-  std::vector<int64_t> &kt = c->lig_expect, cap(L);
-  kt.assign(L, 0);
+  std::vector<int64_t> cap(L);
   int64_t expect_all = 0;
   double cost = 0;
   for (size_t i = 0; i < L; i++) {
     const double kf = std::ceil(double(keep) * double(c->nposes[i]));
     const uint32_t k = uint32_t(std::min<double>(double(c->nposes[i]), std::max(1.0, kf)));
     segs[i] = bude::sel::Segment{int64_t(c->pose_off[i]), uint32_t(c->nposes[i]), k};
-    kt[i] = int64_t((k + 63) / 64);
     cap[i] = int64_t((c->nposes[i] + 63) / 64);
-    expect_all += kt[i];
+    expect_all += int64_t((k + 63) / 64);
     cost += double(c->nposes[i]) * double(c->lig[i].size());
   }
   if (int st = c->plan.prepare(segs)) return st;
@@ -715,7 +776,6 @@ int plan_selection(bude_combined *c, float keep) {
   K = c->chunk_lig.size() - 1;
   c->chunk_plan.clear();
   c->chunk_tile.assign(K + 1, 0);
-  c->chunk_expect.assign(K, 0);
   std::vector<int32_t> order;
   for (size_t k = 0; k < K; k++) {
     const size_t a = c->chunk_lig[k], b = c->chunk_lig[k + 1];
@@ -723,10 +783,7 @@ int plan_selection(bude_combined *c, float keep) {
     const std::vector<bude::sel::Segment> cs(segs.begin() + long(a), segs.begin() + long(b));
     if (int st = c->chunk_plan[k]->prepare(cs)) return st;
     int64_t t = 0;
-    for (size_t l = a; l < b; l++) {
-      t += cap[l];
-      c->chunk_expect[k] += kt[l];
-    }
+    for (size_t l = a; l < b; l++) t += cap[l];
     c->chunk_tile[k + 1] = c->chunk_tile[k] + t;
     const std::vector<int32_t> o = heaviest_first(c, a, b, nullptr);
     order.insert(order.end(), o.begin(), o.end());
@@ -741,6 +798,23 @@ int plan_selection(bude_combined *c, float keep) {
       if (int st = bude::hip_check(hipEventCreate(&e), "hipEventCreate")) return st;
       ps.chunk_ev.push_back(e);
     }
+  }
+  // the sorted rescoring passes, over the rows that are always selected
+  std::vector<uint32_t> sorted_rows(L);
+  std::vector<bude::items::Segment> rows(L);
+  for (size_t i = 0; i < L; i++) {
+    sorted_rows[i] = segs[i].k;
+    rows[i] = bude::items::Segment{int32_t(i), int64_t(c->pose_off[i]), int64_t(segs[i].k)};
+  }
+  if (int st = c->sorted_rows.assign(sorted_rows.data(), L * 4)) return st;
+  c->chunk_sorted.clear();
+  c->sorted_ok = true;
+  for (size_t k = 0; k <= K && c->sorted_ok; k++) {  // (the last: the whole set)
+    bude::items::Plan *plan = &c->whole_sorted;
+    if (k < K) plan = (c->chunk_sorted.push_back(std::make_unique<bude::items::Plan>()), c->chunk_sorted.back().get());
+    const long a = k < K ? long(c->chunk_lig[k]) : 0, b = k < K ? long(c->chunk_lig[k + 1]) : long(L);
+    if (int st = plan_sorted(c, *plan, std::vector<bude::items::Segment>(rows.begin() + a, rows.begin() + b))) return st;
+    if (int st = reserve_sorted(*plan, c->work, &c->sorted_ok)) return st;
   }
   c->plan_ok = true;
   return BUDE_OK;
@@ -959,9 +1033,21 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     if (!st) st = ps.protein.reserve(pro_max * 16);
     if (!st) st = ps.group_begin.reserve((ntypes_ + 1) * 4);
     if (!st) st = ps.slot_coef.reserve(c->slot_type.size() * ntypes_ * sizeof(bude::PairCoef));
+    if (!st) st = ps.reach2.reserve(c->slot_type.size() * ntypes_ * sizeof(float));
     if (!st) st = ps.meta_rs.reserve(nligands * sizeof(bude::LigandMeta));
     if (!st) st = ps.coef.reserve(natoms * ntypes_ * sizeof(bude::PairCoef));
     if (!st) st = stage_reserve(ps, stage_bound(c.get(), pro_max));
+  }
+  if (!st) {  // the sampled poses: as many of every pair for every protein, gathered pair after pair
+    std::vector<bude::items::Segment> segs(nligands);
+    int64_t at = 0;
+    for (size_t i = 0; i < nligands; i++) {
+      const int64_t n = int64_t(std::min<size_t>(cfg->labels_per_pair, nposes[i]));
+      segs[i] = bude::items::Segment{int32_t(i), at, n};
+      at += n;
+    }
+    st = plan_sorted(c.get(), c->label_sorted, segs);
+    if (!st) st = reserve_sorted(c->label_sorted, c->label_work, &c->label_sorted_ok);
   }
   if (!st) st = c->counter.alloc(256);
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
@@ -1026,6 +1112,20 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     const std::vector<bude::PairCoef> sc = bude::coef_table(probe.data(), probe.size(), groups, c->ff.data());
     if (int st = stage_upload(c->s(), c->s().slot_coef, sc.data(), sc.size() * sizeof(bude::PairCoef), c->stream3))
       return st;
+    std::vector<float> reach2;
+    float largest = 0.f;
+    c->s().reachable = bude::items::reach_table(sc, reach2, &largest);
+    if (c->s().reachable) {
+      if (int st = stage_upload(c->s(), c->s().reach2, reach2.data(), reach2.size() * sizeof(float), c->stream3))
+        return st;
+      bude::items::Scene &scene = c->s().scene;
+      scene.coef = static_cast<const bude::PairCoef *>(c->s().slot_coef.ptr);
+      scene.reach2 = static_cast<const float *>(c->s().reach2.ptr);
+      scene.natpro = int(natpro);
+      scene.ngroups = int(groups.ngroups());
+      scene.form = bude::plain_form();
+      bude::items::protein_box(groups.xyzw, largest, scene.lo, scene.hi);
+    }
     std::vector<bude::LigandMeta> m(L);  // everything but the pose counts, which the selection writes
     for (size_t l = 0; l < L; l++)
       m[l] = bude::LigandMeta{c->lig_off[l], int32_t(c->lig[l].size()), c->s().coef_off[l], 0, int64_t(c->pose_off[l]), 0};
@@ -1033,6 +1133,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
       return st;
   }
   if (int st = stage_upload(c->s(), c->s().protein, groups.xyzw.data(), groups.xyzw.size() * 4, c->stream3)) return st;
+  c->s().scene.protein = static_cast<const float4 *>(c->s().protein.ptr);  // (the upload may have grown the buffer)
   if (int st = stage_upload(c->s(), c->s().group_begin, groups.begin.data(), groups.begin.size() * 4, c->stream3))
     return st;
   if (int st = record(c, 9, c->stream3)) return st;
@@ -1100,8 +1201,9 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   int nt_label = 0;
   int64_t ft_all = 0, ft_label = 0;
   const std::vector<int64_t> &tb_all = c->tb_all_host;
-  if (int st = prepare_exact(c, lab_spans, c->meta_label, c->tiles_label, &nt_label, bude::kSplitTile, c->stream3))
-    return st;
+  if (!use_sorted(c->s(), c->label_sorted, c->label_sorted_ok))
+    if (int st = prepare_exact(c, lab_spans, c->meta_label, c->tiles_label, &nt_label, bude::kSplitTile, c->stream3))
+      return st;
   if (!mlp) {
     const size_t np = c->grid.points(), nslots = c->slot_type.size();
     if (!atom) {
@@ -1123,6 +1225,9 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     }
   }
   const size_t K = c->chunk_lig.size() - 1;
+  auto chunk_sorted = [&](size_t k) {
+    return c->sorted_ok && use_sorted(c->s(), *c->chunk_sorted[k], true);
+  };
   int2 *rs_tiles = static_cast<int2 *>(c->s().tiles_rs.ptr);
   int32_t *rs_ntiles = static_cast<int32_t *>(c->s().rs_ntiles.ptr);
 
@@ -1177,7 +1282,8 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
         return st;
       if (int st = bude::hip_check(hipEventRecord(c->s().chunk_ev[2 * k], c->stream2), "hipEventRecord")) return st;
       if (int st = select_and_tables(c, *c->chunk_plan[k], a, static_cast<const int32_t *>(c->rs_order.ptr) + a,
-                                     int(b - a), rs_tiles + c->chunk_tile[k], rs_ntiles + k, c->stream2))
+                                     int(b - a), rs_tiles + c->chunk_tile[k], rs_ntiles + k, chunk_sorted(k),
+                                     c->stream2))
         return st;
       if (int st = bude::hip_check(hipEventRecord(c->s().chunk_ev[2 * k + 1], c->stream2), "hipEventRecord")) return st;
     }
@@ -1335,24 +1441,20 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     if (c->s().fallback[l]) fb.push_back(all[l]);
   const bool widened = res->widened_pairs > 0;
   const bool pipelined = !mlp && fb.empty() && !widened;
-  int64_t expect = 0;
   int nrs = 0;
   if (!pipelined) {
     std::vector<int32_t> o = heaviest_first(c, 0, L, &c->s().fallback);
-    for (int32_t l : o) expect += c->lig_expect[size_t(l)];
     nrs = int(o.size());
     if (o.empty()) o.push_back(0);  // every pair fell back: nothing to rescore
     if (int st = c->s().rs_sel.assign(o.data(), o.size() * 4)) return st;
   }
   if (widened) {  // this protein's per-pair k, into the slot's own segment table
     std::vector<bude::sel::Segment> segs(L);
-    expect = 0;
     for (size_t l = 0; l < L; l++) {  // (a fallback pair selects its lowest keep_fraction of exact energies)
       const double f = c->s().fallback[l] ? double(cfg.keep_fraction) : double(c->s().keep[l]);
       const double kf = std::ceil(f * double(c->nposes[l]));
       const uint32_t k = uint32_t(std::min<double>(double(c->nposes[l]), std::max(1.0, kf)));
       segs[l] = bude::sel::Segment{int64_t(c->pose_off[l]), uint32_t(c->nposes[l]), k};
-      if (!c->s().fallback[l]) expect += int64_t((k + 63) / 64);
     }
     if (int st = stage_upload(c->s(), c->s().wplan.segs, segs.data(), L * sizeof(segs[0]), c->stream)) return st;
   }
@@ -1368,7 +1470,12 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     if (int st = bude::hip_check(hipStreamWaitEvent(c->stream, c->s().ev[4], 0), "hipStreamWaitEvent")) return st;
   }
   if (int st = record(c, 5)) return st;
-  if (int st = exact_ragged(c, fb, poses, c->total, pred, c->meta_fb, c->tiles_fb)) return st;
+  if (!fb.empty()) {  // (nothing is in flight on the last protein's plan: one with fallback pairs ends first)
+    std::vector<bude::items::Segment> segs;
+    for (const Span &sp : fb) segs.push_back(bude::items::Segment{int32_t(sp.lig), int64_t(sp.off), int64_t(sp.n)});
+    if (int st = plan_sorted(c, c->fb_sorted, segs)) return st;
+  }
+  if (int st = exact_ragged(c, fb, poses, c->total, pred, c->meta_fb, c->tiles_fb, &c->fb_sorted)) return st;
   if (int st = record(c, 6)) return st;
 
   // 8-9. per-pair top-k of the scores and exact rescoring of every
@@ -1380,17 +1487,19 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
         return st;
       if (k == 0)
         if (int st = record(c, 7)) return st;
-      if (int st = launch_rescore(c, rs_tiles + c->chunk_tile[k], rs_ntiles + k, c->chunk_expect[k])) return st;
+      if (int st = launch_rescore(c, rs_tiles + c->chunk_tile[k], rs_ntiles + k,
+                                  chunk_sorted(k) ? c->chunk_sorted[k].get() : nullptr)) return st;
     }
   } else {
+    const bool sorted = nrs > 0 && use_sorted(c->s(), c->whole_sorted, c->sorted_ok);
     if (int st = select_and_tables(c, widened ? c->s().wplan : c->plan, 0,
                                    static_cast<const int32_t *>(c->s().rs_sel.ptr), nrs, rs_tiles, rs_ntiles + K,
-                                   c->stream))
+                                   sorted, c->stream))
       return st;
     if (int st = record(c, 10)) return st;  // the scores are read
     if (int st = record(c, 7)) return st;
     if (nrs)
-      if (int st = launch_rescore(c, rs_tiles, rs_ntiles + K, expect)) return st;
+      if (int st = launch_rescore(c, rs_tiles, rs_ntiles + K, sorted ? &c->whole_sorted : nullptr)) return st;
   }
   // the counts land in pinned memory: the host does not wait here
   if (int st = bude::hip_check(hipMemcpyAsync(c->s().nsel_host, c->s().sel_n.ptr, L * 4, hipMemcpyDeviceToHost,
@@ -1617,9 +1726,15 @@ extern "C" int bude_mi355x_combined_exhaustive(bude_combined *c, double *device_
   if (int st = c->exact_all.reserve(c->total * 4)) return st;
   std::vector<Span> all(c->nlig);
   for (size_t l = 0; l < c->nlig; l++) all[l] = Span{l, c->pose_off[l], c->nposes[l]};
+  if (!c->all_planned) {
+    std::vector<bude::items::Segment> segs;
+    for (const Span &sp : all) segs.push_back(bude::items::Segment{int32_t(sp.lig), int64_t(sp.off), int64_t(sp.n)});
+    if (int st = plan_sorted(c, c->all_sorted, segs)) return st;
+    c->all_planned = true;
+  }
   if (int st = record(c, 0)) return st;
   if (int st = exact_ragged(c, all, static_cast<const float *>(c->poses.ptr), c->total,
-                            static_cast<float *>(c->exact_all.ptr), c->meta_ex, c->tiles_all))
+                            static_cast<float *>(c->exact_all.ptr), c->meta_ex, c->tiles_all, &c->all_sorted))
     return st;
   if (int st = record(c, 1)) return st;
   if (int st = sync(c)) return st;

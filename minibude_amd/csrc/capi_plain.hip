@@ -195,7 +195,7 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
     const auto t0 = std::chrono::steady_clock::now();
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
     const hipError_t le = ctx->sorted.usable()
-                              ? ctx->sorted.launch(a.protein, a.poses, a.stride, a.energies, ctx->stream)
+                              ? ctx->sorted.launch(a.protein, a.poses, a.stride, nullptr, a.energies, ctx->stream)
                           : ctx->direct ? bude::items::launch_direct(direct, ctx->stream)
                                             : bude::launch_plain(a, int(wgsize), ctx->stream);
     if (int st = bude::hip_check(le, "fasten_plain launch")) return st;

@@ -20,6 +20,7 @@
 #include "fasten_batch.h"
 #include "fasten_plain.h"
 #include "hip_util.h"
+#include "items.h"
 #include "mlp.h"
 #include "select.h"
 #include "surrogate.h"
@@ -42,11 +43,13 @@ double ms_since(std::chrono::steady_clock::time_point t0) {
 struct bude_screen {
   int device = 0;
   int cus = 0;
-  size_t lds_per_cu = 0;
   BudeScreenConfig cfg{};
   // plain-kernel deck (labels, rescoring, fallback)
   size_t natlig = 0, ngroups = 0;
   DeviceBuffer protein, group_begin, coef, ligand;
+  bude::ProteinGroups groups;
+  std::vector<BudeAtom> atoms;
+  std::vector<BudeFFParams> ff;
   // surrogate
   Net net;
   bool trained = false, fallback = false;
@@ -54,12 +57,16 @@ struct bude_screen {
   // candidate poses
   size_t ncand = 0;
   DeviceBuffer cand, pred, sel_idx, sel_n, exact;
-  // rescoring: the persistent batched kernel over the selection (its rows
-  // through sel_idx), one ligand whose pose count and tiles (0, 64 j) the
-  // device writes from the selection's size
-  DeviceBuffer rs_tiles, rs_meta, rs_counter, rs_order, rs_ntiles;
+  // rescoring: rows through sel_idx, one ligand whose pose count and tiles
+  // (first pose of 64) the device writes from the selection's size
+  DeviceBuffer rs_tiles, rs_meta, rs_order, rs_ntiles;
   bude::sel::Plan plan;  // one segment: the loaded poses, k = ceil(keep_fraction * n)
   size_t plan_n = 0, plan_k = 0;
+  // the sorted passes over the selection's first plan_k rows (the tiled
+  // kernel scores rows past them: ties) and, in fallback, over every pose
+  bude::items::Deck sel_deck, all_deck;
+  DeviceBuffer rs_done;
+  bool all_planned = false;
   size_t nsel = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev[5] = {};
@@ -90,6 +97,20 @@ struct bude_screen {
 
 namespace {
 
+// The sorted pass over rows [0, n) of a pose set (or of an index into one).
+int plan_deck(const bude_screen *s, size_t n, bude::items::Deck &d) {
+  return d.prepare(s->groups, s->ff.data(), s->atoms, {0, int32_t(s->natlig)},
+                   {bude::items::Segment{0, 0, int64_t(n)}});
+}
+
+// Exact energies of n poses on the library's stream, through the planned
+// pass where it applies.
+hipError_t score_all(const bude_screen *s, const bude::items::Deck &d, const float *poses, size_t n, float *energies) {
+  if (d.usable())
+    return d.launch(static_cast<const float4 *>(s->protein.ptr), poses, n, nullptr, energies, s->stream);
+  return bude::launch_plain(s->plain(poses, n, n, energies), 256, s->stream);
+}
+
 int upload_poses(DeviceBuffer &d, const float *const poses[6], size_t n) {
   if (int st = d.alloc(6 * n * sizeof(float))) return st;
   for (int k = 0; k < 6; k++)
@@ -101,14 +122,23 @@ int upload_poses(DeviceBuffer &d, const float *const poses[6], size_t n) {
 }
 
 // Exact energies of the selected poses (rows sel_idx[0, nsel) of the
-// candidates) into exact[0, nsel): the persistent batched kernel
-// (bit-identical to the plain kernel) on tiles of 64 poses pulled from a
-// queue by a grid pinned to 3 waves on every SIMD, so the SIMDs finish
-// together on a pass of a few thousand tiles.  The tables come from the
-// selection's count on the device; the host does not wait for it.
+// candidates) into exact[0, nsel): the sorted pass over the plan_k rows that
+// are always there, where it applies, and work-groups per 64 poses
+// (bit-identical) over the rest.  The tables come from the selection's count
+// on the device; the host does not wait for it.
 int rescore(bude_screen *s) {
+  const bool sorted = s->sel_deck.usable();
+  if (sorted)
+    if (int st = bude::hip_check(s->sel_deck.launch(static_cast<const float4 *>(s->protein.ptr),
+                                                    static_cast<const float *>(s->cand.ptr), s->ncand,
+                                                    static_cast<const uint32_t *>(s->sel_idx.ptr),
+                                                    static_cast<float *>(s->exact.ptr), s->stream),
+                                 "sorted rescoring"))
+      return st;
   if (int st = bude::hip_check(bude::build_rescore_tables(static_cast<const int32_t *>(s->rs_order.ptr), 1,
                                                           static_cast<const uint32_t *>(s->sel_n.ptr),
+                                                          sorted ? static_cast<const uint32_t *>(s->rs_done.ptr)
+                                                                 : nullptr,
                                                           static_cast<bude::LigandMeta *>(s->rs_meta.ptr),
                                                           static_cast<int2 *>(s->rs_tiles.ptr),
                                                           static_cast<int32_t *>(s->rs_ntiles.ptr), s->stream),
@@ -123,15 +153,12 @@ int rescore(bude_screen *s) {
   a.tiles = static_cast<const int2 *>(s->rs_tiles.ptr);
   a.poses = static_cast<const float *>(s->cand.ptr);
   a.energies = static_cast<float *>(s->exact.ptr);
-  a.counter = static_cast<unsigned int *>(s->rs_counter.ptr);
   a.stride = s->ncand;
   a.ngroups = int(s->ngroups);
   a.form = bude::plain_form();
   a.pose_index = static_cast<const uint32_t *>(s->sel_idx.ptr);
   a.ntiles_dev = static_cast<const int32_t *>(s->rs_ntiles.ptr);
-  const bude::PinnedGrid g = bude::pinned_grid(s->cus, s->lds_per_cu, 3);
-  a.lds_bytes = g.lds_bytes;
-  return bude::hip_check(bude::launch_batch_indexed(a, g.blocks, s->stream), "rescore launch");
+  return bude::hip_check(bude::launch_tiles(a, 2 * s->cus, s->stream), "rescore launch");
 }
 
 // Surrogate predictions (normalised target units) for n poses whose 6 rows
@@ -169,9 +196,11 @@ extern "C" int bude_mi355x_screen_create(int device, const BudeAtom *protein, si
   hipDeviceProp_t props{};
   if (int st = bude::hip_check(hipGetDeviceProperties(&props, device), "hipGetDeviceProperties")) return st;
   s->cus = props.multiProcessorCount;
-  s->lds_per_cu = props.maxSharedMemoryPerMultiProcessor;
   s->natlig = natlig;
-  const bude::ProteinGroups groups = bude::group_protein(protein, natpro);
+  s->atoms.assign(ligand, ligand + natlig);
+  s->ff.assign(forcefield, forcefield + ntypes);
+  s->groups = bude::group_protein(protein, natpro);
+  const bude::ProteinGroups &groups = s->groups;
   s->ngroups = groups.ngroups();
   const std::vector<bude::PairCoef> coef = bude::coef_table(ligand, natlig, groups, forcefield);
   std::vector<float> lig4(natlig * 4);
@@ -215,9 +244,14 @@ extern "C" int bude_mi355x_screen_train(bude_screen *s, const float *const poses
   if (int st = upload_poses(tp, poses, n)) return st;
   if (int st = te.alloc(n * 4)) return st;
   auto t0 = std::chrono::steady_clock::now();
-  const bude::PlainArgs pa = s->plain(static_cast<const float *>(tp.ptr), n, n, static_cast<float *>(te.ptr));
-  if (int st = bude::hip_check(bude::launch_plain(pa, 256, st_), "label launch")) return st;
-  if (int st = bude::hip_check(hipStreamSynchronize(st_), "hipStreamSynchronize")) return st;
+  {
+    bude::items::Deck d;
+    if (int st = plan_deck(s, n, d)) return st;
+    if (int st = bude::hip_check(
+            score_all(s, d, static_cast<const float *>(tp.ptr), n, static_cast<float *>(te.ptr)), "label launch"))
+      return st;
+    if (int st = bude::hip_check(hipStreamSynchronize(st_), "hipStreamSynchronize")) return st;
+  }
   stats->label_ms = ms_since(t0);
 
   // 2. target transform from the training split: clip at a quantile (the
@@ -299,12 +333,13 @@ extern "C" int bude_mi355x_screen_load(bude_screen *s, const float *const poses[
   if (int st = bude::hip_check(hipSetDevice(s->device), "hipSetDevice")) return st;
   s->ncand = n;
   s->nsel = 0;
+  s->plan_n = 0;  // (the next run plans for these poses)
+  s->all_planned = false;
   int st = upload_poses(s->cand, poses, n);
   if (!st) st = s->pred.alloc(n * 4);
   if (!st) st = s->sel_idx.alloc(n * 4);
   if (!st) st = s->exact.alloc(n * 4);
   if (!st) st = s->rs_tiles.alloc((n + 63) / 64 * sizeof(int2));
-  if (!st) st = s->rs_counter.alloc(sizeof(unsigned int));
   if (!st) st = s->rs_ntiles.alloc(sizeof(int32_t));
   if (!st) {  // the one ligand's row of the rescoring meta (its pose count comes from the selection)
     const bude::LigandMeta m{0, int32_t(s->natlig), 0, 0, 0, 0};
@@ -329,15 +364,24 @@ extern "C" int bude_mi355x_screen_run(bude_screen *s, BudeScreenResult *res) {
   const auto t0 = std::chrono::steady_clock::now();
   if (s->plan_n != n || s->plan_k != k) {  // (uploads before any launch of this run)
     if (int st = s->plan.prepare({bude::sel::Segment{0, uint32_t(n), uint32_t(k)}})) return st;
+    if (int st = plan_deck(s, k, s->sel_deck)) return st;
+    const uint32_t done = uint32_t(k);
+    if (int st = s->rs_done.assign(&done, sizeof(done))) return st;
     s->plan_n = n;
     s->plan_k = k;
+  }
+  if (s->fallback && !s->all_planned) {
+    if (int st = plan_deck(s, n, s->all_deck)) return st;
+    s->all_planned = true;
   }
   float ms01 = 0, ms12 = 0, ms23 = 0;
   if (s->fallback) {
     // plain kernel on every pose, then the same selection on exact energies
     if (int st = bude::hip_check(hipEventRecord(s->ev[0], st_), "hipEventRecord")) return st;
-    const bude::PlainArgs pa = s->plain(static_cast<const float *>(s->cand.ptr), n, n, static_cast<float *>(s->pred.ptr));
-    if (int st = bude::hip_check(bude::launch_plain(pa, 256, st_), "fallback launch")) return st;
+    if (int st = bude::hip_check(score_all(s, s->all_deck, static_cast<const float *>(s->cand.ptr), n,
+                                           static_cast<float *>(s->pred.ptr)),
+                                 "fallback launch"))
+      return st;
     if (int st = bude::hip_check(hipEventRecord(s->ev[1], st_), "hipEventRecord")) return st;
   } else {
     if (int st = bude::hip_check(hipEventRecord(s->ev[0], st_), "hipEventRecord")) return st;
@@ -431,10 +475,13 @@ extern "C" int bude_mi355x_screen_exhaustive(bude_screen *s, float *energies, do
   if (int st = bude::hip_check(hipSetDevice(s->device), "hipSetDevice")) return st;
   DeviceBuffer out;
   if (int st = out.alloc(s->ncand * 4)) return st;
-  const bude::PlainArgs pa = s->plain(static_cast<const float *>(s->cand.ptr), s->ncand, s->ncand,
-                                      static_cast<float *>(out.ptr));
+  bude::items::Deck d;
+  if (int st = plan_deck(s, s->ncand, d)) return st;
   if (int st = bude::hip_check(hipEventRecord(s->ev[0], s->stream), "hipEventRecord")) return st;
-  if (int st = bude::hip_check(bude::launch_plain(pa, 256, s->stream), "exhaustive launch")) return st;
+  if (int st = bude::hip_check(
+          score_all(s, d, static_cast<const float *>(s->cand.ptr), s->ncand, static_cast<float *>(out.ptr)),
+          "exhaustive launch"))
+    return st;
   if (int st = bude::hip_check(hipEventRecord(s->ev[1], s->stream), "hipEventRecord")) return st;
   if (int st = bude::hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize")) return st;
   float t = 0.f;

@@ -34,7 +34,7 @@ struct BatchArgs {
   int form;                     // hinge form (plain_form())
   unsigned lds_bytes;           // dynamic LDS per work-group, unused by the kernel: sized so that exactly
                                 // n work-groups fit on a CU, it pins the waves per SIMD (0: no pinning)
-  // launch_batch_indexed only: row j of ligand l is pose meta[l].pose_off + pose_index[meta[l].pose_off + j]
+  // launch_tiles only (null: not used): row j of ligand l is pose meta[l].pose_off + pose_index[meta[l].pose_off + j]
   // (energies still at meta[l].pose_off + j), and the tile count is read from device memory
   const uint32_t *pose_index;
   const int32_t *ntiles_dev;
@@ -62,17 +62,18 @@ hipError_t launch_batch(const BatchArgs &a, int rb, int wgsize, int blocks, hipS
 // Work tables of a rescoring pass over per-segment selections, built on the
 // device from the selection counts: for the ligands order[0..n) (list
 // order, e.g. heaviest first) meta[l].nposes = sel_n[l] (every other field
-// of meta[l] set beforehand), tiles (l, 64 i) for i < ceil(sel_n[l] / 64)
+// of meta[l] set beforehand), tiles (l, d + 64 i) for d + 64 i < sel_n[l]
 // from tiles[0] (room for the worst case is the caller's), and the tile
-// count in *ntiles; one work-group, on stream s after the selection.
-hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel_n, LigandMeta *meta, int2 *tiles,
-                                int32_t *ntiles, hipStream_t s);
+// count in *ntiles; one work-group, on stream s after the selection.  d is
+// done[l], the rows another pass scores (0 when done is null).
+hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel_n, const uint32_t *done,
+                                LigandMeta *meta, int2 *tiles, int32_t *ntiles, hipStream_t s);
 
-// launch_batch over rows that are a per-segment selection (pose_index) with
-// tiles and tile count written by an earlier kernel (ntiles_dev): one pose
-// per work-item (rb 1), work-groups of 256.  Energies are bit-equal to
-// launch_batch's for the same poses.
-hipError_t launch_batch_indexed(const BatchArgs &a, int blocks, hipStream_t s);
+// The pass over few tiles of 64 poses: `blocks` work-groups of 16 waves, each
+// sharing a tile at a time.  Rows may be a per-segment selection
+// (pose_index) and the tile count an earlier kernel's (ntiles_dev).
+// Energies are bit-equal to launch_batch's for the same poses.
+hipError_t launch_tiles(const BatchArgs &a, int blocks, hipStream_t s);
 
 // The split form for short passes: a.tiles are (ligand, first pose) pairs of
 // 16 poses, one wave each, four lanes per pose; a.counter and a.lds_bytes

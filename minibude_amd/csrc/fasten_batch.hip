@@ -30,16 +30,13 @@ __global__ void reset_counter_kernel(unsigned int *__restrict__ counter) {
   if (threadIdx.x == 0) counter[0] = 0u;
 }
 
-// INDEXED: pose rows through pose_index, tile count from ntiles_dev (both
-// written by earlier kernels on the device).
-template <int RB, int WG, int FORM, bool INDEXED = false>
+template <int RB, int WG, int FORM>
 __global__ __launch_bounds__(WG) void fasten_batch_kernel(
     const float4 *__restrict__ protein, const int32_t *__restrict__ group_begin, const PairCoef *__restrict__ coef,
     const float4 *__restrict__ ligands, const LigandMeta *__restrict__ meta, const int2 *__restrict__ tiles,
     const float *__restrict__ poses, float *__restrict__ energies, unsigned int *__restrict__ counter, size_t stride,
-    int ngroups, int ntiles, const uint32_t *__restrict__ pose_index, const int32_t *__restrict__ ntiles_dev) {
+    int ngroups, int ntiles) {
   const int lane = threadIdx.x & 63;
-  if constexpr (INDEXED) ntiles = *ntiles_dev;
   for (;;) {
     // One atomic per wave; every wave leaves once the list is exhausted.
     unsigned int t = 0;
@@ -54,9 +51,7 @@ __global__ __launch_bounds__(WG) void fasten_batch_kernel(
 #pragma unroll
     for (int k = 0; k < RB; ++k) {
       const int j = tile.y + lane + k * 64;
-      size_t q = size_t(m.pose_off) + size_t(j < m.nposes ? j : m.nposes - 1);
-      if constexpr (INDEXED) q = size_t(m.pose_off) + pose_index[q];
-      tr[k] = make_xform(poses, stride, q);
+      tr[k] = make_xform(poses, stride, size_t(m.pose_off) + size_t(j < m.nposes ? j : m.nposes - 1));
       e[k] = 0.f;
     }
     for (int il = 0; il < m.natlig; ++il) {
@@ -81,6 +76,52 @@ __global__ __launch_bounds__(WG) void fasten_batch_kernel(
       const int j = tile.y + lane + k * 64;
       if (j < m.nposes) energies[size_t(m.pose_off) + size_t(j)] = e[k] * 0.5f;
     }
+  }
+}
+
+// The form for few tiles: one work-group of 16 waves per tile of 64 poses,
+// its waves sharing the ligand's atoms, whose energies meet in LDS and are
+// added in order by wave 0.  A wave that scores a tile alone is a chain over
+// every pair (56 x 2,046 atoms: 4-6 ms, however few the tiles; the rows that
+// widening adds to a combined screen's rescoring took 6.1 ms); shared by 16
+// waves a tile takes 0.5 ms.
+// Rows through pose_index when it is not null, the tile count from
+// ntiles_dev (both written by earlier kernels) when that is not null.
+template <int FORM>
+__global__ __launch_bounds__(1024) void fasten_tile_kernel(
+    const float4 *__restrict__ protein, const int32_t *__restrict__ group_begin, const PairCoef *__restrict__ coef,
+    const float4 *__restrict__ ligands, const LigandMeta *__restrict__ meta, const int2 *__restrict__ tiles,
+    const float *__restrict__ poses, float *__restrict__ energies, size_t stride, int ngroups, int ntiles,
+    const uint32_t *__restrict__ pose_index, const int32_t *__restrict__ ntiles_dev) {
+  __shared__ float atom[16][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  if (ntiles_dev) ntiles = *ntiles_dev;
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int2 tile = tiles[t];
+    const LigandMeta m = meta[tile.x];
+    const int j = tile.y + lane;
+    size_t q = size_t(m.pose_off) + size_t(j < m.nposes ? j : m.nposes - 1);
+    if (pose_index) q = size_t(m.pose_off) + pose_index[q];
+    const Xform tr = make_xform(poses, stride, q);
+    float e = 0.f;
+    for (int a0 = 0; a0 < m.natlig; a0 += 16) {
+      if (a0 + wave < m.natlig) {
+        const float4 la = ligands[m.lig_off + a0 + wave];
+        const float lx[1] = {place(tr.m[0], tr.m[1], tr.m[2], tr.m[3], la)};
+        const float ly[1] = {place(tr.m[4], tr.m[5], tr.m[6], tr.m[7], la)};
+        const float lz[1] = {place(tr.m[8], tr.m[9], tr.m[10], tr.m[11], la)};
+        const PairCoef *cl = coef + size_t(m.coef_off) + size_t(a0 + wave) * ngroups;
+        float ea[1] = {0.f};
+        for (int g = 0; g < ngroups; ++g)
+          group_dispatch<1, FORM>(protein, group_begin[g], group_begin[g + 1], cl[g], lx, ly, lz, ea);
+        atom[wave][lane] = ea[0];
+      }
+      __syncthreads();
+      if (wave == 0)
+        for (int a = 0; a < min(16, m.natlig - a0); a++) e += atom[a][lane];
+      __syncthreads();
+    }
+    if (wave == 0 && j < m.nposes) energies[size_t(m.pose_off) + size_t(j)] = e * 0.5f;
   }
 }
 
@@ -152,24 +193,27 @@ __global__ __launch_bounds__(256) void fasten_split_kernel(
 
 // Rescoring work tables of the ligands order[0..n) from their selection
 // counts, on the device right after the selection:
-// meta[l].nposes = sel_n[l], tiles (l, 64 i) for i < ceil(sel_n[l] / 64) in
-// list order from tiles[0], and the tile count in *ntiles.  One work-group
+// meta[l].nposes = sel_n[l], tiles (l, done[l] + 64 i) for the rows past
+// done[l] in list order from tiles[0], and the tile count in *ntiles.  One work-group
 // of 256; the host never waits for the counts.
 __global__ __launch_bounds__(256) void rescore_tables_kernel(const int32_t *__restrict__ order, int n,
                                                              const uint32_t *__restrict__ sel_n,
+                                                             const uint32_t *__restrict__ done,
                                                              LigandMeta *__restrict__ meta,
                                                              int2 *__restrict__ tiles, int32_t *__restrict__ ntiles) {
-  __shared__ int32_t lig[256], cnt[256], off[256], wsum[4];
+  __shared__ int32_t lig[256], first[256], cnt[256], off[256], wsum[4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int32_t base = 0;
   for (int b = 0; b < n; b += 256) {
     const int i = b + int(threadIdx.x);
-    int32_t c = 0, l = 0;
+    int32_t c = 0, l = 0, d0 = 0;
     if (i < n) {
       l = order[i];
       const uint32_t k = sel_n[l];
       meta[l].nposes = int32_t(k);
-      c = int32_t((k + 63) / 64);
+      const uint32_t d = done ? min(done[l], k) : 0u;
+      d0 = int32_t(d);
+      c = int32_t((k - d + 63) / 64);
     }
     int32_t x = c;  // inclusive scan over the wave, then over the four waves
     for (int d = 1; d < 64; d <<= 1) {
@@ -181,13 +225,14 @@ __global__ __launch_bounds__(256) void rescore_tables_kernel(const int32_t *__re
     int32_t wb = 0;
     for (int q = 0; q < w; q++) wb += wsum[q];
     lig[threadIdx.x] = l;
+    first[threadIdx.x] = d0;
     cnt[threadIdx.x] = c;
     off[threadIdx.x] = base + wb + x - c;
     const int32_t sum = wsum[0] + wsum[1] + wsum[2] + wsum[3];
     __syncthreads();
     const int m = min(256, n - b);
     for (int q = 0; q < m; q++)
-      for (int t = int(threadIdx.x); t < cnt[q]; t += 256) tiles[off[q] + t] = make_int2(lig[q], 64 * t);
+      for (int t = int(threadIdx.x); t < cnt[q]; t += 256) tiles[off[q] + t] = make_int2(lig[q], first[q] + 64 * t);
     base += sum;
     __syncthreads();  // lig/cnt/off/wsum are rewritten by the next batch
   }
@@ -199,11 +244,11 @@ hipError_t launch_rb_wg(const BatchArgs &a, int blocks, hipStream_t s) {
   if (a.form == kFormD)
     hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<RB, WG, kFormD>), dim3(unsigned(blocks)), dim3(WG),
                        a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles, nullptr, nullptr);
+                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles);
   else
     hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<RB, WG, kFormB>), dim3(unsigned(blocks)), dim3(WG),
                        a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles, nullptr, nullptr);
+                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles);
   return hipGetLastError();
 }
 
@@ -252,25 +297,22 @@ hipError_t launch_split(const BatchArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel_n, LigandMeta *meta, int2 *tiles,
-                                int32_t *ntiles, hipStream_t s) {
+hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel_n, const uint32_t *done,
+                                LigandMeta *meta, int2 *tiles, int32_t *ntiles, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rescore_tables_kernel, dim3(1), dim3(256), 0, s, order, n, sel_n, meta, tiles, ntiles);
+  hipLaunchKernelGGL(rescore_tables_kernel, dim3(1), dim3(256), 0, s, order, n, sel_n, done, meta, tiles, ntiles);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_indexed(const BatchArgs &a, int blocks, hipStream_t s) {
-  if (!a.pose_index || !a.ntiles_dev || blocks < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, s, a.counter);
-  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (a.form == kFormD)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<1, 256, kFormD, true>), dim3(unsigned(blocks)), dim3(256),
-                       a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, 0, a.pose_index, a.ntiles_dev);
-  else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<1, 256, kFormB, true>), dim3(unsigned(blocks)), dim3(256),
-                       a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, 0, a.pose_index, a.ntiles_dev);
+hipError_t launch_tiles(const BatchArgs &a, int blocks, hipStream_t s) {
+  if (blocks < 1) return hipErrorInvalidValue;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(1024), 0, s, a.protein, a.group_begin, a.coef, a.ligands,
+                       a.meta, a.tiles, a.poses, a.energies, a.stride, a.ngroups, a.ntiles, a.pose_index,
+                       a.ntiles_dev);
+  };
+  if (a.form == kFormD) run(fasten_tile_kernel<kFormD>);
+  else run(fasten_tile_kernel<kFormB>);
   return hipGetLastError();
 }
 

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <vector>
 
 #include "bude_internal.h"
@@ -46,8 +47,8 @@ bool reach_table(const std::vector<PairCoef> &coef, std::vector<float> &reach2, 
 // The box of the grouped protein's finite atoms widened by `reach`.
 void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]);
 
-// Whether sorting pays for scoring segs against natpro atoms.
-bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
+// Whether sorting pays for `items` items of `nsegs` segments against natpro atoms.
+bool worth_sorting(size_t natpro, double items, size_t nsegs);
 
 // Device scratch of a pass; one stream at a time may use it.
 struct Workspace {
@@ -61,16 +62,18 @@ struct Workspace {
 class Plan {
  public:
   // atoms: every ligand's atoms (w bits: slot), ligand l's at lig_off[l] ..
-  // lig_off[l + 1] - 1.  The tables are uploaded synchronously.
+  // lig_off[l + 1] - 1.  The tables are uploaded synchronously; no pass over
+  // an earlier plan may be in flight.  A ligand too large for a chunk leaves
+  // the plan empty.
   int build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
             const std::vector<Segment> &segs);
   int reserve(Workspace &w) const;
+  bool fits(const Workspace &w) const;
   // Queues the pass: energies[row] of every row of every segment.  index:
   // the pose row of row i of a segment is pose_off + index[pose_off + i].
   hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                     float *energies, hipStream_t s) const;
-  bool empty() const { return chunks_.empty(); }
-  double items() const { return items_; }
+  bool worth(size_t natpro) const { return !chunks_.empty() && worth_sorting(natpro, items_, nsegs_); }
 
  private:
   struct Chunk {
@@ -79,9 +82,12 @@ class Plan {
     uint32_t nitems, npartial, nxform, nrows;
     int nunits;
   };
+  // bytes of items, partial, xform, hist and base
+  std::array<size_t, 5> need() const;
   std::vector<Chunk> chunks_;
   DeviceBuffer tables_, atoms_;
   int nslots_ = 0;
+  size_t nsegs_ = 0;
   float radius_ = 0.f;  // of the ligand atoms about their frame's origin
   double items_ = 0;
 };
@@ -117,7 +123,8 @@ class Deck {
   int prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
               const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
   bool usable() const { return usable_; }
-  hipError_t launch(const float4 *protein, const float *poses, size_t stride, float *energies, hipStream_t s) const;
+  hipError_t launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index, float *energies,
+                    hipStream_t s) const;
 
  private:
   bool usable_ = false;

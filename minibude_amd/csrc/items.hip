@@ -545,13 +545,7 @@ void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float
   }
 }
 
-bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs) {
-  double items = 0;
-  for (const Segment &s : segs) {
-    const int64_t L = lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)];
-    if (L > kChunkItems / 64) return false;
-    items += double(L) * double(s.n);
-  }
+bool worth_sorting(size_t natpro, double items, size_t nsegs) {
   // The direct pass scores some 1.8e9 pairs a millisecond; the sort's seven
   // launches cost 40-50 us whatever the size, and with few items (large
   // boxes) scoring them grows with the protein.  Both measured, direct and
@@ -559,13 +553,14 @@ bool worth_sorting(size_t natpro, const std::vector<int32_t> &lig_off, const std
   // (67 and 65 us), 700 x 19 at 1e8, 938 x 26 at 1.4e8, 938 x 64 at 2e8,
   // 4,096 x 26 at 4.4e8 (189 and 192 us), 4,096 x 96 at 6e8.  A segment is to
   // fill the work-groups that sort it.
-  return items * double(natpro) >= 6e7 + 8e4 * double(natpro) && items >= 4096.0 * double(segs.size());
+  return items * double(natpro) >= 6e7 + 8e4 * double(natpro) && items >= 4096.0 * double(nsegs);
 }
 
 int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
                 const std::vector<Segment> &segs) {
   chunks_.clear();
   nslots_ = nslots;
+  nsegs_ = segs.size();
   items_ = 0;
   radius_ = 0.f;
   // every ligand's atoms grouped by type (stable), w bits: place in the ligand
@@ -601,7 +596,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
   int64_t room = kChunkItems;
   for (const Segment &s : segs) {
     const int64_t L = lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)];
-    if (L <= 0 || L > kChunkItems / 64) return fail(BUDE_ERR_RUNTIME, "items: ligand too large for a chunk");
+    if (L <= 0 || L > kChunkItems / 64) return BUDE_OK;
     items_ += double(L) * double(s.n);
     for (int64_t j = 0; j < s.n;) {
       int64_t take = std::min(s.n - j, room / L);
@@ -707,26 +702,38 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
   return tables_.assign(bytes.data(), bytes.size());
 }
 
-int Plan::reserve(Workspace &w) const {
-  size_t items = 0, partial = 0, xf = 0, hist = 0, base = 0;
+std::array<size_t, 5> Plan::need() const {
+  std::array<size_t, 5> n{};
   for (const Chunk &c : chunks_) {
-    items = std::max(items, size_t(c.nitems) * sizeof(float4));
-    partial = std::max(partial, size_t(c.npartial) * 4);
-    xf = std::max(xf, size_t(c.nxform) * 3 * sizeof(float4));
-    hist = std::max(hist, (size_t(c.nrows) << c.cell_bits) * 4);
-    base = std::max(base, (size_t(nslots_) << c.cell_bits) * 4);
+    n[0] = std::max(n[0], size_t(c.nitems) * sizeof(float4));
+    n[1] = std::max(n[1], size_t(c.npartial) * sizeof(float));
+    n[2] = std::max(n[2], size_t(c.nxform) * 3 * sizeof(float4));
+    n[3] = std::max(n[3], (size_t(c.nrows) << c.cell_bits) * sizeof(uint32_t));
+    n[4] = std::max(n[4], (size_t(nslots_) << c.cell_bits) * sizeof(uint32_t));
   }
-  int st = w.items.reserve(items);
-  if (!st) st = w.partial.reserve(partial);
-  if (!st) st = w.xform.reserve(xf);
-  if (!st) st = w.hist.reserve(hist);
-  if (!st) st = w.base.reserve(base);
-  if (!st) st = w.bounds.reserve(kMaxBounds * 6 * 4);
+  return n;
+}
+
+int Plan::reserve(Workspace &w) const {
+  const std::array<size_t, 5> n = need();
+  int st = w.items.reserve(n[0]);
+  if (!st) st = w.partial.reserve(n[1]);
+  if (!st) st = w.xform.reserve(n[2]);
+  if (!st) st = w.hist.reserve(n[3]);
+  if (!st) st = w.base.reserve(n[4]);
+  if (!st) st = w.bounds.reserve(kMaxBounds * 6 * sizeof(float));
   return st;
+}
+
+bool Plan::fits(const Workspace &w) const {
+  const std::array<size_t, 5> n = need();
+  return n[0] <= w.items.bytes && n[1] <= w.partial.bytes && n[2] <= w.xform.bytes && n[3] <= w.hist.bytes &&
+         n[4] <= w.base.bytes && w.bounds.bytes >= kMaxBounds * 6 * sizeof(float);
 }
 
 hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                         float *energies, hipStream_t s) const {
+  if (!fits(w)) return hipErrorInvalidValue;
   Space sp{};
   for (int k = 0; k < 3; k++) {
     sp.lo[k] = sc.lo[k];
@@ -742,10 +749,6 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
   auto *base = static_cast<uint32_t *>(w.base.ptr);
   auto *bounds = static_cast<float *>(w.bounds.ptr);
   for (const Chunk &c : chunks_) {
-    if (size_t(c.nitems) * sizeof(float4) > w.items.bytes || size_t(c.npartial) * 4 > w.partial.bytes ||
-        size_t(c.nxform) * 48 > w.xform.bytes || (size_t(c.nrows) << c.cell_bits) * 4 > w.hist.bytes ||
-        (size_t(nslots_) << c.cell_bits) * 4 > w.base.bytes || w.bounds.bytes < kMaxBounds * 24)
-      return hipErrorInvalidValue;
     const auto *blocks = reinterpret_cast<const Block *>(tables + c.blocks);
     const auto *tasks = reinterpret_cast<const Task *>(tables + c.tasks);
     const auto *refs = reinterpret_cast<const int32_t *>(tables + c.refs);
@@ -821,7 +824,10 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
                   const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs) {
   usable_ = false;
   const size_t natpro = size_t(groups.begin.back());
-  if (!worth_sorting(natpro, lig_off, segs)) return BUDE_OK;
+  double items = 0;
+  for (const Segment &s : segs)
+    items += double(lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)]) * double(s.n);
+  if (!worth_sorting(natpro, items, segs.size())) return BUDE_OK;
   // slots: the forcefield types the ligands use, ascending
   std::vector<int32_t> types;
   for (const BudeAtom &a : atoms) types.push_back(a.type);
@@ -843,6 +849,7 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   if (int st = coef_.upload(coef.data(), coef.size() * sizeof(PairCoef))) return st;
   if (int st = reach2_.upload(reach2.data(), reach2.size() * 4)) return st;
   if (int st = plan_.build(slotted, lig_off, int(types.size()), segs)) return st;
+  if (!plan_.worth(natpro)) return BUDE_OK;
   scene_.coef = static_cast<const PairCoef *>(coef_.ptr);
   scene_.reach2 = static_cast<const float *>(reach2_.ptr);
   scene_.natpro = int(natpro);
@@ -858,12 +865,12 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   return st;
 }
 
-hipError_t Deck::launch(const float4 *protein, const float *poses, size_t stride, float *energies,
-                        hipStream_t s) const {
+hipError_t Deck::launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index,
+                        float *energies, hipStream_t s) const {
   if (!usable_) return hipErrorInvalidValue;
   Scene sc = scene_;
   sc.protein = protein;
-  return plan_.launch(sc, work_, poses, stride, nullptr, energies, s);
+  return plan_.launch(sc, work_, poses, stride, index, energies, s);
 }
 
 }  // namespace items

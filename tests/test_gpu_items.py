@@ -12,6 +12,7 @@ import torch
 from minibude_amd import capi
 from minibude_amd import deck as D
 from minibude_amd.batch import Batch, LigandSet
+from minibude_amd.capi import BatchConfig
 from minibude_amd.model import Context
 
 pytestmark = pytest.mark.gpu
@@ -66,6 +67,27 @@ def test_noalloc_in_several_passes(gpu_device):
     capi.check(capi.lib().bude_mi355x_fasten_noalloc(gpu_device, p[0], d.natpro, p[1], d.natlig, p[2], d.ntypes, p[3],
                                                      d.nposes, d.nposes, 1, 64, ctypes.c_void_p(e.data_ptr()), None))
     assert np.array_equal(e.cpu().numpy().view(np.uint32), tiled(d, gpu_device).view(np.uint32))
+
+
+@pytest.mark.parametrize("natlig, nposes", [
+    ([1], [1]),
+    ([16, 17, 33], [64, 65, 1]),                # whole rounds of 16 atoms and remainders, masked tiles
+    ([96, 8, 40], [700, 1300, 64]),
+])
+def test_few_tiles_equal_tiled(gpu_device, natlig, nposes):
+    n = len(natlig)
+    ls = LigandSet(D.synth_protein(76, 500, 34), D.synth_forcefield(76, 34),
+                   [D.synth_ligand(77 + i, natlig[i], 34) for i in range(n)],
+                   [D.synth_poses(87 + i, nposes[i]) for i in range(n)])
+    with Batch(ls, gpu_device) as b:
+        b.clear()
+        b.run_separate(1, 64)
+        want = [b.energies(i) for i in range(n)]
+        for graph in (0, 1):
+            b.clear()
+            b.run(BatchConfig(2, 64, 4, 0, graph), warmup=0, iterations=2)
+            for i in range(n):
+                assert np.array_equal(b.energies(i).view(np.uint32), want[i].view(np.uint32)), (graph, i)
 
 
 def test_poses_out_of_reach_and_not_finite(gpu_device):
