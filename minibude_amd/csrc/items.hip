@@ -24,10 +24,10 @@
 // An item's place within its cell is whichever atomic came first; nothing an
 // item's energy is made of depends on it.
 //
-// Measured against the tiled kernel on the same deck (whole pass, energies
-// copied out): 4,096 x 64 atoms x 1,048,576 poses 79.4 -> 5.4 ms (score
-// 3.7, items into place 0.8, counts 0.12, reduction 0.12); 2,672 x 2,672 x
-// 65,536 289 -> 10.0 ms; 938 x 26 x 65,536 1,079 -> 208 us.
+// Measured against the tiled kernel on the same deck (device time): 4,096 x
+// 64 atoms x 1,048,576 poses 79.4 -> 5.0 ms (items into place 0.8, counts
+// 0.12, reduction 0.06, the rest the score kernel); 2,672 x 2,672 x 65,536
+// 289 -> 10.3 ms; 938 x 26 x 65,536 1,030 -> 134 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,7 +46,7 @@ namespace {
 using namespace core;
 
 constexpr int kThreads = 1024;      // of the prep and bin kernels
-constexpr int kCells = 4096;        // 16 per axis, in Morton order
+constexpr int kCells = 4096;        // 16 per axis
 constexpr int kMaxBounds = 256;     // work-groups of the prep kernel
 
 struct Block {
@@ -157,19 +157,54 @@ __device__ __forceinline__ CellGrid cell_grid(const float *__restrict__ bounds, 
   return g;
 }
 
-__device__ __forceinline__ uint32_t spread(uint32_t v) {  // bits 0-3 to 0, 3, 6, 9
-  v = (v | (v << 4)) & 0x0c3u;
-  return (v | (v << 2)) & 0x249u;
-}
-
 // (clamped to the grid; NaN falls into cell 0 of its axis)
 __device__ __forceinline__ uint32_t axis_cell(float x, float lo, float inv) {
   return uint32_t(__builtin_amdgcn_fmed3f((x - lo) * inv, 0.0f, 15.0f));
 }
 
-__device__ __forceinline__ uint32_t cell_of(const CellGrid &g, float x, float y, float z) {
-  return spread(axis_cell(x, g.lo[0], g.inv[0])) | (spread(axis_cell(y, g.lo[1], g.inv[1])) << 1) |
-         (spread(axis_cell(z, g.lo[2], g.inv[2])) << 2);
+// Cells are numbered along a Hilbert curve: consecutive cells share a face,
+// so items that straddle cells keep a small box (in Morton order a step can
+// cross the whole grid; scoring 4,096 x 64 atoms x 1,048,576 poses tested 165
+// atoms per item instead of 182, and 201 instead of 240 with a sixteenth of
+// the poses).  Steps of Skilling's transform ("Programming the Hilbert
+// curve", AIP Conf. Proc. 707, 2004) for a 16^3 grid.
+constexpr uint16_t hilbert_place(uint32_t x, uint32_t y, uint32_t z) {
+  uint32_t v[3] = {x, y, z};
+  for (uint32_t q = 8; q > 1; q >>= 1)
+    for (int i = 0; i < 3; i++) {
+      if (v[i] & q) {
+        v[0] ^= q - 1;
+      } else {
+        const uint32_t t = (v[0] ^ v[i]) & (q - 1);
+        v[0] ^= t;
+        v[i] ^= t;
+      }
+    }
+  v[1] ^= v[0];
+  v[2] ^= v[1];
+  uint32_t t = 0;
+  for (uint32_t q = 8; q > 1; q >>= 1)
+    if (v[2] & q) t ^= q - 1;
+  uint32_t h = 0;
+  for (int b = 3; b >= 0; b--)
+    for (int i = 0; i < 3; i++) h = h << 1 | (((v[i] ^ t) >> b) & 1);
+  return uint16_t(h);
+}
+
+struct Curve {
+  uint16_t place[kCells];
+};
+constexpr Curve make_curve() {
+  Curve c{};
+  for (uint32_t i = 0; i < uint32_t(kCells); i++) c.place[i] = hilbert_place(i & 15, (i >> 4) & 15, i >> 8);
+  return c;
+}
+__device__ const Curve kCurve = make_curve();
+
+// curve: kCurve's places, in LDS.
+__device__ __forceinline__ uint32_t cell_of(const CellGrid &g, const uint16_t *curve, float x, float y, float z) {
+  return curve[axis_cell(x, g.lo[0], g.inv[0]) | axis_cell(y, g.lo[1], g.inv[1]) << 4 |
+               axis_cell(z, g.lo[2], g.inv[2]) << 8];
 }
 
 // SCATTER 0: counts of each row's items per cell.  SCATTER 1: each item into
@@ -185,7 +220,9 @@ __global__ __launch_bounds__(kThreads) void bin_kernel(const Task *__restrict__ 
                                                        int bits, uint32_t *__restrict__ hist,
                                                        const uint32_t *__restrict__ base, float4 *__restrict__ items) {
   __shared__ uint32_t h[kCells];
+  __shared__ uint16_t curve[kCells];
   __shared__ float red[6];
+  for (int i = threadIdx.x; i < kCells; i += kThreads) curve[i] = kCurve.place[i];  // (cell_grid waits for it)
   const CellGrid g = cell_grid(bounds, nbounds, sp, red);
   const Task t = tasks[blockIdx.x];
   const Block bk = blocks[t.block];
@@ -216,7 +253,7 @@ __global__ __launch_bounds__(kThreads) void bin_kernel(const Task *__restrict__ 
         const float y = place(m1[k].x, m1[k].y, m1[k].z, m1[k].w, la);
         const float z = place(m2[k].x, m2[k].y, m2[k].z, m2[k].w, la);
         if (j < bk.npose) {
-          const uint32_t c = cell_of(g, x, y, z) >> shift;
+          const uint32_t c = cell_of(g, curve, x, y, z) >> shift;
           const uint32_t at = atomicAdd(&h[c], 1u);
           if constexpr (SCATTER) items[at] = make_float4(x, y, z, __uint_as_float(out + uint32_t(j)));
         }
@@ -659,7 +696,11 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
       used += count[size_t(t)] > 0;
     }
     const int64_t mean = nitems / std::max<int64_t>(1, used);
-    ch.rb = mean >= 131072 ? 4 : mean >= 32768 ? 2 : 1;
+    // items per lane: more share the protein's steps, fewer keep the box
+    // small where items are sparse.  Whole passes at 1, 2, 4 and 8: 24 k items
+    // of a type 73, 78, 88, 122 us; 95 k 340, 315, 326, 460; 560 k 2,050,
+    // 1,580, 1,470, 1,560; 2.2 M 7,980, 5,980, 5,140, 5,000.
+    ch.rb = mean >= 1100000 ? 8 : mean >= 230000 ? 4 : mean >= 48000 ? 2 : 1;
     ch.cell_bits = mean >= 16384 ? 12 : 9;
     std::vector<Row> rows;
     std::vector<std::vector<int32_t>> refs_of(blocks.size());
@@ -775,6 +816,10 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
         break;
       case 2:
         launch_score<2>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
+                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
+        break;
+      case 8:
+        launch_score<8>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
                         static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
         break;
       default:
