@@ -63,6 +63,25 @@ __device__ __forceinline__ float vgpr_copy(float s) {
   return v;
 }
 
+// A pair's distance.  The contraction is written out (dx^2, then fma dy, then
+// fma dz): left to the compiler it can pick another order in another kernel,
+// and every kernel sharing this code must round the same way.
+__device__ __forceinline__ float pair_distance(float dx, float dy, float dz) {
+  return __builtin_amdgcn_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
+}
+
+// The three hinges of a pair added to e; x is the distance d (kFormD) or
+// d - radij (kFormB).
+template <int FORM> __device__ __forceinline__ float steric(float x, const PairCoef &c, float e) {
+  return __builtin_fmaf(2.0f * kHardness, sat(FORM == kFormB ? x * c.neg_rr : __builtin_fmaf(x, c.neg_rr, 1.0f)), e);
+}
+template <int FORM> __device__ __forceinline__ float charge(float x, const PairCoef &c, float c0, float e) {
+  return __builtin_fmaf(c.wq, sat(__builtin_fmaf(x, c.neg_e1, FORM == kFormB ? 1.0f : c0)), e);
+}
+template <int FORM> __device__ __forceinline__ float desolvation(float x, const PairCoef &c, float e0, float e) {
+  return __builtin_fmaf(c.wd, sat(__builtin_fmaf(x, c.neg_rd, FORM == kFormB ? 1.0f : e0)), e);
+}
+
 // The pairs of one protein atom p with the RB poses of this work-item.
 template <int RB, int FORM, bool CHG, bool DSLV>
 __device__ __forceinline__ void atom_pairs(const float4 p, const PairCoef &c, float c0, float e0,
@@ -70,23 +89,11 @@ __device__ __forceinline__ void atom_pairs(const float4 p, const PairCoef &c, fl
                                            float (&e)[RB]) {
 #pragma unroll
   for (int k = 0; k < RB; ++k) {
-    const float dx = lx[k] - p.x;
-    const float dy = ly[k] - p.y;
-    const float dz = lz[k] - p.z;
-    // the contraction written out (dx^2, then fma dy, then fma dz): left to
-    // the compiler it can pick another order in another kernel, and every
-    // kernel sharing this code must round the same way
-    const float d = __builtin_amdgcn_sqrtf(__builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx)));
-    if constexpr (FORM == kFormB) {
-      const float b = d - c.radij;
-      e[k] = __builtin_fmaf(2.0f * kHardness, sat(b * c.neg_rr), e[k]);
-      if constexpr (CHG) e[k] = __builtin_fmaf(c.wq, sat(__builtin_fmaf(b, c.neg_e1, 1.0f)), e[k]);
-      if constexpr (DSLV) e[k] = __builtin_fmaf(c.wd, sat(__builtin_fmaf(b, c.neg_rd, 1.0f)), e[k]);
-    } else {
-      e[k] = __builtin_fmaf(2.0f * kHardness, sat(__builtin_fmaf(d, c.neg_rr, 1.0f)), e[k]);
-      if constexpr (CHG) e[k] = __builtin_fmaf(c.wq, sat(__builtin_fmaf(d, c.neg_e1, c0)), e[k]);
-      if constexpr (DSLV) e[k] = __builtin_fmaf(c.wd, sat(__builtin_fmaf(d, c.neg_rd, e0)), e[k]);
-    }
+    float x = pair_distance(lx[k] - p.x, ly[k] - p.y, lz[k] - p.z);
+    if constexpr (FORM == kFormB) x -= c.radij;
+    e[k] = steric<FORM>(x, c, e[k]);
+    if constexpr (CHG) e[k] = charge<FORM>(x, c, c0, e[k]);
+    if constexpr (DSLV) e[k] = desolvation<FORM>(x, c, e0, e[k]);
   }
 }
 

@@ -14,12 +14,12 @@ namespace items {
 
 // What the items are scored against: the grouped protein (a group index in
 // the w bits of every atom), and per ligand-atom slot (a forcefield type of
-// the ligand set) and group the pair coefficients and the squared distance
-// beyond which every hinge of the pair is exactly zero.
+// the ligand set) and group the pair coefficients and the squared distances
+// beyond which the pair's hinges are exactly zero.
 struct Scene {
   const float4 *protein = nullptr;
   const PairCoef *coef = nullptr;   // [nslots][ngroups]
-  const float *reach2 = nullptr;    // [nslots][ngroups]
+  const float4 *reach2 = nullptr;   // [nslots][ngroups]: steric, charge, desolvation (-1: weight 0), their largest
   int natpro = 0, ngroups = 0;
   int form = 1;                     // hinge form (plain_form())
   float lo[3] = {}, hi[3] = {};     // the protein's box, widened by the largest reach
@@ -33,16 +33,17 @@ struct Segment {
   int64_t n;
 };
 
-// Distance beyond which all three hinges of a pair are exactly zero in
-// either hinge form: the largest zero crossing of the terms present, widened
-// far above the rounding of the distances compared with it.  Negative when
-// the pair has no such distance (a radius sum that is not positive, or a
-// coefficient that is not finite), so that no pair may be left out.
-float pair_reach(const PairCoef &c);
+// Distances beyond which a pair's steric, charge and desolvation hinges are
+// exactly zero in either hinge form: their zero crossings, widened far above
+// the rounding of the distances compared with them; -1 for a hinge of weight
+// 0.  False when the pair has no such distances (a radius sum that is not
+// positive, or a coefficient that is not finite), so that no pair may be left
+// out.
+bool pair_reach(const PairCoef &c, float r[3]);
 
-// The squared reaches of a coefficient table and their largest; false when
-// some pair has none.
-bool reach_table(const std::vector<PairCoef> &coef, std::vector<float> &reach2, float *largest);
+// The squared reaches of a coefficient table and the largest reach; false
+// when some pair has none.
+bool reach_table(const std::vector<PairCoef> &coef, std::vector<float4> &reach2, float *largest);
 
 // The box of the grouped protein's finite atoms widened by `reach`.
 void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]);

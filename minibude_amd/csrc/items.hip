@@ -25,9 +25,9 @@
 // item's energy is made of depends on it.
 //
 // Measured against the tiled kernel on the same deck (device time): 4,096 x
-// 64 atoms x 1,048,576 poses 79.4 -> 5.0 ms (items into place 0.8, counts
+// 64 atoms x 1,048,576 poses 79.4 -> 4.5 ms (items into place 0.8, counts
 // 0.12, reduction 0.06, the rest the score kernel); 2,672 x 2,672 x 65,536
-// 289 -> 10.3 ms; 938 x 26 x 65,536 1,030 -> 134 us.
+// 289 -> 9.2 ms; 938 x 26 x 65,536 1,030 -> 134 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -348,6 +348,42 @@ __device__ __forceinline__ void mask_pairs(uint64_t mask, float x, float y, floa
   } while (mask);
 }
 
+// The same, each atom with the hinges whose reach it is in only (bits of ms,
+// mq, md); the others are exactly zero for all the items (of 165 atoms per
+// item of the 4,096 x 64 deck, 31 are within steric reach, 101 within the
+// charge's, 132 within the desolvation's: 9.2 VALU per pair instead of 11.1).
+// The tests are scalar branches between a pair's 6 distance VALU and the 2 of
+// each hinge: they pay with four items per lane or more (4,096 x 64 x
+// 1,048,576: 5.00 -> 4.46 ms; with one or two the branches cost as much).
+template <int RB, int FORM>
+__device__ __forceinline__ void mask_hinges(uint64_t mask, uint64_t ms, uint64_t mq, uint64_t md, float x, float y,
+                                            float z, const PairCoef &c, const float (&lx)[RB], const float (&ly)[RB],
+                                            const float (&lz)[RB], float (&e)[RB]) {
+  const float c0 = vgpr_copy(c.c0), e0 = vgpr_copy(c.e0);
+  do {
+    const int j = __builtin_ctzll(mask);
+    mask &= mask - 1;
+    const float px = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j));
+    const float py = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(y), j));
+    const float pz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), j));
+    float d[RB];
+#pragma unroll
+    for (int k = 0; k < RB; k++) {
+      d[k] = pair_distance(lx[k] - px, ly[k] - py, lz[k] - pz);
+      if constexpr (FORM == kFormB) d[k] -= c.radij;
+    }
+    if (ms >> j & 1)
+#pragma unroll
+      for (int k = 0; k < RB; k++) e[k] = steric<FORM>(d[k], c, e[k]);
+    if (mq >> j & 1)
+#pragma unroll
+      for (int k = 0; k < RB; k++) e[k] = charge<FORM>(d[k], c, c0, e[k]);
+    if (md >> j & 1)
+#pragma unroll
+      for (int k = 0; k < RB; k++) e[k] = desolvation<FORM>(d[k], c, e0, e[k]);
+  } while (mask);
+}
+
 // One wave per 64 x RB consecutive items of one type: the protein 64 atoms at
 // a time (lane = atom) against the items' box, then every atom in reach out
 // of its lane (three readlanes) to all lanes' RB items.  RB > 1 shares the
@@ -357,7 +393,7 @@ __device__ __forceinline__ void mask_pairs(uint64_t mask, float x, float y, floa
 template <int RB, int FORM>
 __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ protein, int natpro,
                                                     const PairCoef *__restrict__ coef,
-                                                    const float *__restrict__ reach2, int ngroups,
+                                                    const float4 *__restrict__ reach2, int ngroups,
                                                     const float4 *__restrict__ items,
                                                     const int32_t *__restrict__ slot_items,
                                                     const int32_t *__restrict__ slot_units, int nslots, int nunits,
@@ -391,21 +427,27 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
     bl[k] = wave_min(bl[k]);
     bh[k] = wave_max(bh[k]);
   }
-  const float *r2 = reach2 + size_t(slot) * size_t(ngroups);
+  const float4 *r2 = reach2 + size_t(slot) * size_t(ngroups);
   const PairCoef *cs = coef + size_t(slot) * size_t(ngroups);
   PairCoef c{};
   int cur = -1;
   // two steps ahead: the atoms; one step ahead: their reach
   float4 p = protein[min(lane, natpro - 1)], p1 = protein[min(64 + lane, natpro - 1)];
-  float reach = r2[__float_as_int(p.w)];
+  float4 reach = r2[__float_as_int(p.w)];
   for (int base = 0; base < natpro; base += 64) {
-    const float reach1 = r2[__float_as_int(p1.w)];
+    const float4 reach1 = r2[__float_as_int(p1.w)];
     const float4 p2 = protein[min(base + 128 + lane, natpro - 1)];
     const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, bl[0], bh[0]);
     const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, bl[1], bh[1]);
     const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, bl[2], bh[2]);
     const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-    uint64_t mask = __ballot(base + lane < natpro && d2 < reach);
+    const bool on = base + lane < natpro;
+    uint64_t mask = __ballot(on && d2 < reach.w), ms = 0, mq = 0, md = 0;
+    if constexpr (RB >= 4) {
+      ms = __ballot(on && d2 < reach.x);
+      mq = __ballot(on && d2 < reach.y);
+      md = __ballot(on && d2 < reach.z);
+    }
     const int pg = __float_as_int(p.w);
     while (mask) {
       const int g = __builtin_amdgcn_readlane(pg, __builtin_ctzll(mask));
@@ -420,11 +462,15 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
       }
       const uint64_t sub = mask & __ballot(pg == g);
       mask &= ~sub;
-      const bool chg = c.wq != 0.f, dslv = c.wd != 0.f;
-      if (chg && dslv) mask_pairs<RB, FORM, true, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-      else if (chg) mask_pairs<RB, FORM, true, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-      else if (dslv) mask_pairs<RB, FORM, false, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-      else mask_pairs<RB, FORM, false, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+      if constexpr (RB >= 4) {
+        mask_hinges<RB, FORM>(sub, ms, mq, md, p.x, p.y, p.z, c, lx, ly, lz, part);
+      } else {
+        const bool chg = c.wq != 0.f, dslv = c.wd != 0.f;
+        if (chg && dslv) mask_pairs<RB, FORM, true, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+        else if (chg) mask_pairs<RB, FORM, true, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+        else if (dslv) mask_pairs<RB, FORM, false, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+        else mask_pairs<RB, FORM, false, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+      }
     }
     p = p1;
     p1 = p2;
@@ -545,26 +591,30 @@ int slot_of(const float4 &a) {
 
 }  // namespace
 
-float pair_reach(const PairCoef &c) {
+bool pair_reach(const PairCoef &c, float r[3]) {
   const float all[] = {c.radij, c.neg_rr, c.neg_e1, c.wq, c.neg_rd, c.wd, c.c0, c.e0};
   for (float v : all)
-    if (!std::isfinite(v)) return -1.f;
-  if (!(c.radij > 0.f) || !(c.neg_rr < 0.f) || !(c.neg_e1 < 0.f) || (c.wd != 0.f && !(c.neg_rd < 0.f))) return -1.f;
-  float r = std::max(c.radij, -1.0f / c.neg_rr);
-  if (c.wq != 0.f) r = std::max({r, c.c0 / -c.neg_e1, c.radij - 1.0f / c.neg_e1});
-  if (c.wd != 0.f) r = std::max({r, c.e0 / -c.neg_rd, c.radij - 1.0f / c.neg_rd});
-  r = r * 1.0001f + 1e-3f;
-  return std::isfinite(r * r) ? r : -1.f;
+    if (!std::isfinite(v)) return false;
+  if (!(c.radij > 0.f) || !(c.neg_rr < 0.f) || !(c.neg_e1 < 0.f) || (c.wd != 0.f && !(c.neg_rd < 0.f))) return false;
+  auto wide = [](float a, float b) { return std::max(a, b) * 1.0001f + 1e-3f; };
+  r[0] = wide(c.radij, -1.0f / c.neg_rr);
+  r[1] = c.wq != 0.f ? wide(c.c0 / -c.neg_e1, c.radij - 1.0f / c.neg_e1) : -1.f;
+  r[2] = c.wd != 0.f ? wide(c.e0 / -c.neg_rd, c.radij - 1.0f / c.neg_rd) : -1.f;
+  for (int k = 0; k < 3; k++)
+    if (!std::isfinite(r[k] * r[k])) return false;
+  return true;
 }
 
-bool reach_table(const std::vector<PairCoef> &coef, std::vector<float> &reach2, float *largest) {
+bool reach_table(const std::vector<PairCoef> &coef, std::vector<float4> &reach2, float *largest) {
   reach2.resize(coef.size());
   *largest = 0.f;
   for (size_t i = 0; i < coef.size(); i++) {
-    const float r = pair_reach(coef[i]);
-    if (r < 0.f) return false;
-    reach2[i] = r * r;
-    *largest = std::max(*largest, r);
+    float r[3];
+    if (!pair_reach(coef[i], r)) return false;
+    const float most = std::max({r[0], r[1], r[2]});
+    *largest = std::max(*largest, most);
+    auto square = [](float v) { return v < 0.f ? -1.f : v * v; };
+    reach2[i] = make_float4(square(r[0]), square(r[1]), square(r[2]), square(most));
   }
   return true;
 }
@@ -699,7 +749,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
     // items per lane: more share the protein's steps, fewer keep the box
     // small where items are sparse.  Whole passes at 1, 2, 4 and 8: 24 k items
     // of a type 73, 78, 88, 122 us; 95 k 340, 315, 326, 460; 560 k 2,050,
-    // 1,580, 1,470, 1,560; 2.2 M 7,980, 5,980, 5,140, 5,000.
+    // 1,580, 1,330, 1,380; 2.2 M 7,980, 5,980, 4,720, 4,450.
     ch.rb = mean >= 1100000 ? 8 : mean >= 230000 ? 4 : mean >= 48000 ? 2 : 1;
     ch.cell_bits = mean >= 16384 ? 12 : 9;
     std::vector<Row> rows;
@@ -881,7 +931,7 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   std::vector<BudeAtom> probe;
   for (int32_t t : types) probe.push_back(BudeAtom{0.f, 0.f, 0.f, t});
   const std::vector<PairCoef> coef = coef_table(probe.data(), probe.size(), groups, ff);
-  std::vector<float> reach2;
+  std::vector<float4> reach2;
   float largest = 0.f;
   if (!reach_table(coef, reach2, &largest)) return BUDE_OK;
   std::vector<float4> slotted;
@@ -892,11 +942,11 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
     slotted.push_back(v);
   }
   if (int st = coef_.upload(coef.data(), coef.size() * sizeof(PairCoef))) return st;
-  if (int st = reach2_.upload(reach2.data(), reach2.size() * 4)) return st;
+  if (int st = reach2_.upload(reach2.data(), reach2.size() * sizeof(float4))) return st;
   if (int st = plan_.build(slotted, lig_off, int(types.size()), segs)) return st;
   if (!plan_.worth(natpro)) return BUDE_OK;
   scene_.coef = static_cast<const PairCoef *>(coef_.ptr);
-  scene_.reach2 = static_cast<const float *>(reach2_.ptr);
+  scene_.reach2 = static_cast<const float4 *>(reach2_.ptr);
   scene_.natpro = int(natpro);
   scene_.ngroups = int(groups.ngroups());
   scene_.form = plain_form();
