@@ -583,6 +583,30 @@ constexpr size_t kDirectWaves = 16384;
 // Items of one chunk: 20 bytes each in the workspace.
 constexpr int64_t kChunkItems = int64_t(1) << 26;
 
+// The device hands work-group i to XCD i mod 8, each with an L2 of its own.
+// Give an XCD a contiguous eighth of the blocks, and all of a type's rows
+// before the next type's, so that neighbouring places of a cell are written
+// by one XCD at about the same time and leave its L2 as fewer partial lines
+// (938 x 26 x 65,536: 136 -> 127 us a pass; 4,096 x 64 x 1,048,576: 4.45 ->
+// 4.34 ms).
+void spread_tasks(std::vector<Task> &tasks, const std::vector<int32_t> &refs, const std::vector<Row> &rows,
+                  size_t nblocks) {
+  constexpr size_t kXcds = 8;
+  auto slot = [&](const Task &t) { return rows[size_t(refs[size_t(t.ref0)])].slot; };
+  std::stable_sort(tasks.begin(), tasks.end(), [&](const Task &a, const Task &b) { return slot(a) < slot(b); });
+  std::vector<std::vector<Task>> of(kXcds);
+  for (const Task &t : tasks) of[size_t(t.block) * kXcds / nblocks].push_back(t);
+  tasks.clear();
+  for (size_t k = 0, more = 1; more; k++) {
+    more = 0;
+    for (const std::vector<Task> &x : of)
+      if (k < x.size()) {
+        tasks.push_back(x[k]);
+        more = 1;
+      }
+  }
+}
+
 int slot_of(const float4 &a) {
   int s;
   std::memcpy(&s, &a.w, sizeof s);
@@ -773,6 +797,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
         tasks.push_back(Task{int32_t(b), int32_t(refs.size()), int32_t(n), 0});
         refs.insert(refs.end(), refs_of[b].begin() + long(i), refs_of[b].begin() + long(i + n));
       }
+    spread_tasks(tasks, refs, rows, blocks.size());
     ch.nblocks = int(blocks.size());
     ch.ntasks = int(tasks.size());
     ch.nrows = uint32_t(rows.size());
