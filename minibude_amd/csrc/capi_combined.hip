@@ -299,7 +299,7 @@ struct Span {
 // the sampled poses' tables), with room for the 256-byte alignment.
 size_t stage_bound(const bude_combined *c, size_t natpro) {
   const size_t L = c->nlig, lpp = std::min<size_t>(c->cfg.labels_per_pair, c->total);
-  return natpro * 16 + (natpro + 2) * 4 + c->slot_type.size() * c->ff.size() * (sizeof(bude::PairCoef) + sizeof(float4)) +
+  return natpro * 16 + (natpro + 2) * 4 + (c->slot_type.size() + 1) * c->ff.size() * (sizeof(bude::PairCoef) + sizeof(float4)) +
          3 * L * sizeof(bude::LigandMeta) + 2 * L * lpp * 4 + L * (lpp / bude::kSplitTile + 1) * 8 + (L + 1) * 8 +
          L * sizeof(bude::sel::Segment) + 16 * 256;
 }
@@ -1033,7 +1033,7 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     if (!st) st = ps.protein.reserve(pro_max * 16);
     if (!st) st = ps.group_begin.reserve((ntypes_ + 1) * 4);
     if (!st) st = ps.slot_coef.reserve(c->slot_type.size() * ntypes_ * sizeof(bude::PairCoef));
-    if (!st) st = ps.reach2.reserve(c->slot_type.size() * ntypes_ * sizeof(float4));
+    if (!st) st = ps.reach2.reserve((c->slot_type.size() + 1) * ntypes_ * sizeof(float4));
     if (!st) st = ps.meta_rs.reserve(nligands * sizeof(bude::LigandMeta));
     if (!st) st = ps.coef.reserve(natoms * ntypes_ * sizeof(bude::PairCoef));
     if (!st) st = stage_reserve(ps, stage_bound(c.get(), pro_max));
@@ -1114,7 +1114,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
       return st;
     std::vector<float4> reach2;
     float largest = 0.f;
-    c->s().reachable = bude::items::reach_table(sc, reach2, &largest);
+    c->s().reachable = bude::items::reach_table(sc, groups.ngroups(), reach2, &largest);
     if (c->s().reachable) {
       if (int st = stage_upload(c->s(), c->s().reach2, reach2.data(), reach2.size() * sizeof(float4), c->stream3))
         return st;

@@ -19,7 +19,9 @@ namespace items {
 struct Scene {
   const float4 *protein = nullptr;
   const PairCoef *coef = nullptr;   // [nslots][ngroups]
-  const float4 *reach2 = nullptr;   // [nslots][ngroups]: steric, charge, desolvation (-1: weight 0), their largest
+  // [nslots + 1][ngroups]: steric, charge, desolvation (-1: weight 0), their
+  // largest; the last row the largest of every slot in w
+  const float4 *reach2 = nullptr;
   int natpro = 0, ngroups = 0;
   int form = 1;                     // hinge form (plain_form())
   float lo[3] = {}, hi[3] = {};     // the protein's box, widened by the largest reach
@@ -41,9 +43,9 @@ struct Segment {
 // out.
 bool pair_reach(const PairCoef &c, float r[3]);
 
-// The squared reaches of a coefficient table and the largest reach; false
-// when some pair has none.
-bool reach_table(const std::vector<PairCoef> &coef, std::vector<float4> &reach2, float *largest);
+// The squared reaches of a coefficient table (Scene::reach2) and the largest
+// reach; false when some pair has none.
+bool reach_table(const std::vector<PairCoef> &coef, size_t ngroups, std::vector<float4> &reach2, float *largest);
 
 // The box of the grouped protein's finite atoms widened by `reach`.
 void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]);

@@ -25,9 +25,9 @@
 // item's energy is made of depends on it.
 //
 // Measured against the tiled kernel on the same deck (device time): 4,096 x
-// 64 atoms x 1,048,576 poses 79.4 -> 4.5 ms (items into place 0.8, counts
+// 64 atoms x 1,048,576 poses 79.4 -> 4.3 ms (items into place 0.8, counts
 // 0.12, reduction 0.06, the rest the score kernel); 2,672 x 2,672 x 65,536
-// 289 -> 9.2 ms; 938 x 26 x 65,536 1,030 -> 134 us.
+// 289 -> 9.1 ms; 938 x 26 x 65,536 1,030 -> 128 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -384,13 +384,19 @@ __device__ __forceinline__ void mask_hinges(uint64_t mask, uint64_t ms, uint64_t
   } while (mask);
 }
 
-// One wave per 64 x RB consecutive items of one type: the protein 64 atoms at
-// a time (lane = atom) against the items' box, then every atom in reach out
-// of its lane (three readlanes) to all lanes' RB items.  RB > 1 shares the
-// 64-atom steps and the readlanes between items at the price of a larger
-// box; VALU issue bounds it (about 12 VALU per pair in reach of the box and
-// 3 / RB for its atom).
-template <int RB, int FORM>
+// The atoms of a work-group's share of the protein that any of its waves can
+// need: list[0 .. n) in order, of atoms base .. base + kShare - 1.
+constexpr int kShare = 4096;
+
+// One wave per 64 x RB consecutive items of one type, four waves to a
+// work-group.  With LIST (large proteins) the work-group first lists the protein atoms within reach of
+// its items' box, 4,096 at a time (each wave tests a quarter, 64 atoms to a
+// step); each wave then takes the list, or the protein, 64 atoms at a time
+// (lane = atom) against its own items' box, and every atom in reach out of its lane (three
+// readlanes) to all lanes' RB items.  RB > 1 shares the steps and the
+// readlanes between items at the price of a larger box; VALU issue bounds it
+// (about 12 VALU per pair in reach of the box and 3 / RB for its atom).
+template <int RB, int FORM, bool LIST>
 __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ protein, int natpro,
                                                     const PairCoef *__restrict__ coef,
                                                     const float4 *__restrict__ reach2, int ngroups,
@@ -398,9 +404,12 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
                                                     const int32_t *__restrict__ slot_items,
                                                     const int32_t *__restrict__ slot_units, int nslots, int nunits,
                                                     float *__restrict__ partial) {
-  const int lane = threadIdx.x & 63;
-  const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * 4 + int(threadIdx.x >> 6));
-  if (u >= nunits) return;
+  __shared__ uint16_t list[LIST ? kShare : 1];
+  __shared__ float box[4][6];
+  __shared__ int count[4], slots[4];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int unit = int(blockIdx.x) * 4 + wave, u = min(unit, nunits - 1);
+  if (!LIST && unit >= nunits) return;  // (with LIST: the last unit again, for its share of the list)
   int slot = 0;  // the last type whose first unit is at or before u
   for (int s0 = 0; s0 < nslots; s0 += 64)
     slot += __popcll(__ballot(s0 + lane < nslots && slot_units[s0 + lane + 1] <= u));
@@ -422,60 +431,116 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
     bl[1] = fminf(bl[1], it.y), bh[1] = fmaxf(bh[1], it.y);
     bl[2] = fminf(bl[2], it.z), bh[2] = fmaxf(bh[2], it.z);
   }
+  float wl[3], wh[3];  // the work-group's box
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     bl[k] = wave_min(bl[k]);
     bh[k] = wave_max(bh[k]);
+    if (LIST && lane == 0) {
+      box[wave][k] = bl[k];
+      box[wave][3 + k] = bh[k];
+    }
+  }
+  const float4 *rw = reach2;
+  if constexpr (LIST) {
+    if (lane == 0) slots[wave] = slot;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      wl[k] = fminf(fminf(box[0][k], box[1][k]), fminf(box[2][k], box[3][k]));
+      wh[k] = fmaxf(fmaxf(box[0][3 + k], box[1][3 + k]), fmaxf(box[2][3 + k], box[3][3 + k]));
+    }
+    // the reaches of the work-group's type, or of any type where it has several (the row behind the types')
+    const bool one = slots[0] == slots[1] && slots[0] == slots[2] && slots[0] == slots[3];
+    rw = reach2 + size_t(__builtin_amdgcn_readfirstlane(one ? slots[0] : nslots)) * size_t(ngroups);
   }
   const float4 *r2 = reach2 + size_t(slot) * size_t(ngroups);
   const PairCoef *cs = coef + size_t(slot) * size_t(ngroups);
+  auto at = [&](int i) { return LIST ? int(list[i]) : i; };
   PairCoef c{};
   int cur = -1;
-  // two steps ahead: the atoms; one step ahead: their reach
-  float4 p = protein[min(lane, natpro - 1)], p1 = protein[min(64 + lane, natpro - 1)];
-  float4 reach = r2[__float_as_int(p.w)];
-  for (int base = 0; base < natpro; base += 64) {
-    const float4 reach1 = r2[__float_as_int(p1.w)];
-    const float4 p2 = protein[min(base + 128 + lane, natpro - 1)];
-    const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, bl[0], bh[0]);
-    const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, bl[1], bh[1]);
-    const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, bl[2], bh[2]);
-    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-    const bool on = base + lane < natpro;
-    uint64_t mask = __ballot(on && d2 < reach.w), ms = 0, mq = 0, md = 0;
-    if constexpr (RB >= 4) {
-      ms = __ballot(on && d2 < reach.x);
-      mq = __ballot(on && d2 < reach.y);
-      md = __ballot(on && d2 < reach.z);
+  for (int base = 0; base < natpro; base += kShare) {
+    const int n = min(kShare, natpro - base), steps = (n + 63) >> 6;
+    int total = n;  // atoms of the share to score against: the listed ones, or all
+    if constexpr (LIST) {
+      const int s0 = steps * wave >> 2, s1 = steps * (wave + 1) >> 2;  // at most 16 of 64 steps
+      uint64_t mine = 0;  // lane i: the mask of step s0 + i
+      int found = 0;
+      for (int st = s0; st < s1; st++) {
+        const int i = st * 64 + lane;
+        const float4 p = protein[base + min(i, n - 1)];
+        const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, wl[0], wh[0]);
+        const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, wl[1], wh[1]);
+        const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, wl[2], wh[2]);
+        const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+        const uint64_t m = __ballot(i < n && d2 < rw[__float_as_int(p.w)].w);
+        if (lane == st - s0) mine = m;
+        found += __popcll(m);
+      }
+      if (lane == 0) count[wave] = found;
+      __syncthreads();
+      int to = 0;
+      for (int w = 0; w < wave; w++) to += count[w];
+      total = __builtin_amdgcn_readfirstlane(count[0] + count[1] + count[2] + count[3]);
+      for (int st = s0; st < s1; st++) {
+        const uint32_t mlo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(mine)), st - s0));
+        const uint32_t mhi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(mine >> 32)), st - s0));
+        const uint64_t m = uint64_t(mhi) << 32 | mlo;
+        if (m >> lane & 1) list[to + __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u))] = uint16_t(st * 64 + lane);
+        to += __popcll(m);
+      }
+      __syncthreads();
     }
-    const int pg = __float_as_int(p.w);
-    while (mask) {
-      const int g = __builtin_amdgcn_readlane(pg, __builtin_ctzll(mask));
-      if (g != cur) {
-#pragma unroll
-        for (int k = 0; k < RB; k++) {
-          e[k] += part[k];
-          part[k] = 0.f;
+    if (total) {
+      // two steps ahead: the atoms; one step ahead: their reach
+      float4 p = protein[base + at(min(lane, total - 1))], p1 = protein[base + at(min(64 + lane, total - 1))];
+      float4 reach = r2[__float_as_int(p.w)];
+      for (int k0 = 0; k0 < total; k0 += 64) {
+        const float4 reach1 = r2[__float_as_int(p1.w)];
+        const float4 p2 = protein[base + at(min(k0 + 128 + lane, total - 1))];
+        const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, bl[0], bh[0]);
+        const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, bl[1], bh[1]);
+        const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, bl[2], bh[2]);
+        const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+        const bool on = k0 + lane < total;
+        uint64_t mask = __ballot(on && d2 < reach.w), ms = 0, mq = 0, md = 0;
+        if constexpr (RB >= 4) {
+          ms = __ballot(on && d2 < reach.x);
+          mq = __ballot(on && d2 < reach.y);
+          md = __ballot(on && d2 < reach.z);
         }
-        cur = g;
-        c = cs[g];
-      }
-      const uint64_t sub = mask & __ballot(pg == g);
-      mask &= ~sub;
-      if constexpr (RB >= 4) {
-        mask_hinges<RB, FORM>(sub, ms, mq, md, p.x, p.y, p.z, c, lx, ly, lz, part);
-      } else {
-        const bool chg = c.wq != 0.f, dslv = c.wd != 0.f;
-        if (chg && dslv) mask_pairs<RB, FORM, true, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-        else if (chg) mask_pairs<RB, FORM, true, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-        else if (dslv) mask_pairs<RB, FORM, false, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
-        else mask_pairs<RB, FORM, false, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+        const int pg = __float_as_int(p.w);
+        while (mask) {
+          const int g = __builtin_amdgcn_readlane(pg, __builtin_ctzll(mask));
+          if (g != cur) {
+#pragma unroll
+            for (int k = 0; k < RB; k++) {
+              e[k] += part[k];
+              part[k] = 0.f;
+            }
+            cur = g;
+            c = cs[g];
+          }
+          const uint64_t sub = mask & __ballot(pg == g);
+          mask &= ~sub;
+          if constexpr (RB >= 4) {
+            mask_hinges<RB, FORM>(sub, ms, mq, md, p.x, p.y, p.z, c, lx, ly, lz, part);
+          } else {
+            const bool chg = c.wq != 0.f, dslv = c.wd != 0.f;
+            if (chg && dslv) mask_pairs<RB, FORM, true, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+            else if (chg) mask_pairs<RB, FORM, true, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+            else if (dslv) mask_pairs<RB, FORM, false, true>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+            else mask_pairs<RB, FORM, false, false>(sub, p.x, p.y, p.z, c, lx, ly, lz, part);
+          }
+        }
+        p = p1;
+        p1 = p2;
+        reach = reach1;
       }
     }
-    p = p1;
-    p1 = p2;
-    reach = reach1;
+    if (LIST && base + kShare < natpro) __syncthreads();  // (the list is rewritten)
   }
+  if (unit >= nunits) return;
 #pragma unroll
   for (int k = 0; k < RB; k++)
     if (i0 + k * 64 + lane < i1) partial[out[k]] = e[k] + part[k];
@@ -572,13 +637,26 @@ template <int SCATTER, class... A> void launch_bin_ppt(int ppt, int ntasks, hipS
   else launch_bin<1, SCATTER>(ntasks, s, args...);
 }
 
-template <int RB, class... A> void launch_score(int form, int nunits, hipStream_t s, A... args) {
+template <int RB, int FORM, class... A> void launch_score(bool listed, int nunits, hipStream_t s, A... args) {
   const dim3 grid(unsigned((nunits + 3) / 4));
-  if (form == kFormD) hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormD>), grid, dim3(256), 0, s, args...);
-  else hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, kFormB>), grid, dim3(256), 0, s, args...);
+  if (listed) hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, FORM, true>), grid, dim3(256), 0, s, args...);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(score_kernel<RB, FORM, false>), grid, dim3(256), 0, s, args...);
+}
+
+template <int FORM, class... A> void launch_score_rb(int rb, bool listed, int nunits, hipStream_t s, A... args) {
+  if (rb >= 8) launch_score<8, FORM>(listed, nunits, s, args...);
+  else if (rb >= 4) launch_score<4, FORM>(listed, nunits, s, args...);
+  else if (rb >= 2) launch_score<2, FORM>(listed, nunits, s, args...);
+  else launch_score<1, FORM>(listed, nunits, s, args...);
 }
 
 constexpr size_t kDirectWaves = 16384;
+
+// Proteins from which the score kernel lists a work-group's atoms first: with
+// and without, 4,096 x 64 x 262,144 1,250 and 1,340 us, 4,096 x 26 x 65,536
+// 300 and 316; 938 x 64 x 262,144 617 and 596, 300 x 64 x 131,072 249 and 234
+// (15 and 5 steps of 64 atoms per wave are no work worth sharing).
+constexpr int kListFrom = 1500;
 
 // Items of one chunk: 20 bytes each in the workspace.
 constexpr int64_t kChunkItems = int64_t(1) << 26;
@@ -629,8 +707,9 @@ bool pair_reach(const PairCoef &c, float r[3]) {
   return true;
 }
 
-bool reach_table(const std::vector<PairCoef> &coef, std::vector<float4> &reach2, float *largest) {
-  reach2.resize(coef.size());
+bool reach_table(const std::vector<PairCoef> &coef, size_t ngroups, std::vector<float4> &reach2, float *largest) {
+  reach2.resize(coef.size() + ngroups);  // (the last row: the largest reaches of any slot)
+  for (size_t g = 0; g < ngroups; g++) reach2[coef.size() + g] = make_float4(-1.f, -1.f, -1.f, 0.f);
   *largest = 0.f;
   for (size_t i = 0; i < coef.size(); i++) {
     float r[3];
@@ -639,6 +718,8 @@ bool reach_table(const std::vector<PairCoef> &coef, std::vector<float4> &reach2,
     *largest = std::max(*largest, most);
     auto square = [](float v) { return v < 0.f ? -1.f : v * v; };
     reach2[i] = make_float4(square(r[0]), square(r[1]), square(r[2]), square(most));
+    float4 &any = reach2[coef.size() + i % ngroups];
+    any.w = std::max(any.w, square(most));
   }
   return true;
 }
@@ -884,24 +965,12 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
     launch_bin_ppt<1>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),
                       size_t(c.nxform), static_cast<const float *>(bounds), nb, sp, c.cell_bits, hist,
                       static_cast<const uint32_t *>(base), items);
-    switch (c.rb) {
-      case 1:
-        launch_score<1>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
-                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
-        break;
-      case 2:
-        launch_score<2>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
-                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
-        break;
-      case 8:
-        launch_score<8>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
-                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
-        break;
-      default:
-        launch_score<4>(sc.form, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
-                        static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
-        break;
-    }
+    auto score = [&](auto run) {
+      run(c.rb, sc.natpro >= kListFrom, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
+          static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
+    };
+    if (sc.form == kFormD) score([](auto... args) { launch_score_rb<kFormD>(args...); });
+    else score([](auto... args) { launch_score_rb<kFormB>(args...); });
     const int per = 4 * c.ppt;  // work-groups of 256 per block of 1024 ppt poses
     hipLaunchKernelGGL(reduce_kernel, dim3(unsigned(c.nblocks) * unsigned(per)), dim3(256), 0, s, blocks, per,
                        static_cast<const float *>(partial), energies);
@@ -958,7 +1027,7 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   const std::vector<PairCoef> coef = coef_table(probe.data(), probe.size(), groups, ff);
   std::vector<float4> reach2;
   float largest = 0.f;
-  if (!reach_table(coef, reach2, &largest)) return BUDE_OK;
+  if (!reach_table(coef, groups.ngroups(), reach2, &largest)) return BUDE_OK;
   std::vector<float4> slotted;
   for (const BudeAtom &a : atoms) {
     const int32_t s = int32_t(std::lower_bound(types.begin(), types.end(), a.type) - types.begin());
