@@ -12,6 +12,7 @@
 #include "atomnet.h"
 #include "bude_internal.h"
 #include "hip_util.h"
+#include "items.h"
 
 namespace {
 
@@ -63,18 +64,49 @@ extern "C" int bude_mi355x_atom_energies(int device, const BudeAtom *protein, si
   if (n > (size_t(1) << 28)) return bude::fail(BUDE_ERR_INVALID_ARGUMENT, std::string(who) + ": more than 2^28 points");
   // (the protein stands in for the ligand in the deck check)
   if (int st = bude::check_deck(protein, natpro, protein, natpro, forcefield, ntypes, who)) return st;
-  for (size_t i = 0; i < n; i++)
+  std::vector<size_t> type_count(ntypes, 0);
+  for (size_t i = 0; i < n; i++) {
     if (types[i] < 0 || size_t(types[i]) >= ntypes)
       return bude::fail(BUDE_ERR_INVALID_ARGUMENT, std::string(who) + ": point " + std::to_string(i) + " has type " +
                                                        std::to_string(types[i]) + " outside the forcefield");
+    type_count[size_t(types[i])]++;
+  }
   if (int st = set_device(device, who)) return st;
   const bude::ProteinGroups groups = bude::group_protein(protein, natpro);
   const size_t ng = groups.ngroups();
   std::vector<BudeAtom> probe(ntypes);
   for (size_t t = 0; t < ntypes; t++) probe[t] = BudeAtom{0.f, 0.f, 0.f, int32_t(t)};
   const std::vector<bude::PairCoef> coef = bude::coef_table(probe.data(), ntypes, groups, forcefield);
-  // points grouped by type into whole 64-point blocks (a block's padding
-  // repeats its last point)
+  bude::DeviceBuffer dprot, dbegin, dcoef, dpts, dout;
+  int st = dprot.upload(groups.xyzw.data(), groups.xyzw.size() * 4);
+  if (!st) st = dcoef.upload(coef.data(), coef.size() * sizeof(bude::PairCoef));
+  std::vector<float4> reach2;
+  float largest = 0.f;
+  if (!st && bude::items::reach_table(coef, ng, reach2, &largest)) {  // sorted by type and place on the device
+    bude::DeviceBuffer dtypes, dreach;
+    st = dreach.upload(reach2.data(), reach2.size() * sizeof(float4));
+    if (!st) st = dpts.upload(points, n * 3 * sizeof(float));
+    if (!st) st = dtypes.upload(types, n * sizeof(int32_t));
+    if (!st) st = dout.alloc(n * sizeof(float));
+    bude::items::Points sorted;
+    if (!st)
+      st = sorted.build(nullptr, static_cast<const float *>(dpts.ptr), static_cast<const int32_t *>(dtypes.ptr), n,
+                        type_count, nullptr);
+    if (st) return st;
+    bude::items::Scene scene;
+    scene.protein = static_cast<const float4 *>(dprot.ptr);
+    scene.coef = static_cast<const bude::PairCoef *>(dcoef.ptr);
+    scene.reach2 = static_cast<const float4 *>(dreach.ptr);
+    scene.natpro = int(natpro);
+    scene.ngroups = int(ng);
+    scene.form = bude::plain_form();
+    st = bude::hip_check(sorted.launch(scene, static_cast<float *>(dout.ptr), nullptr), "atom energies");
+    if (!st) st = bude::hip_check(hipMemcpy(out, dout.ptr, n * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
+    return st ? st : bude::ok();
+  }
+  // no reach (a radius sum that is not positive, a weight that is not
+  // finite): points grouped by type into whole 64-point blocks (a block's
+  // padding repeats its last point)
   std::vector<std::vector<size_t>> by(ntypes);
   for (size_t i = 0; i < n; i++) by[size_t(types[i])].push_back(i);
   std::vector<float> pts;
@@ -92,10 +124,7 @@ extern "C" int bude_mi355x_atom_energies(int device, const BudeAtom *protein, si
     }
   }
   const size_t np = where.size();
-  bude::DeviceBuffer dprot, dbegin, dcoef, dpts, dout;
-  int st = dprot.upload(groups.xyzw.data(), groups.xyzw.size() * 4);
   if (!st) st = dbegin.upload(groups.begin.data(), groups.begin.size() * 4);
-  if (!st) st = dcoef.upload(coef.data(), coef.size() * sizeof(bude::PairCoef));
   if (!st) st = dpts.upload(pts.data(), pts.size() * 4);
   if (!st) st = dout.alloc(np * 4);
   if (!st)

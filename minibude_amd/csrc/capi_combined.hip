@@ -273,6 +273,7 @@ struct bude_combined {
   bude::atomnet::Net anet;
   bude::atomnet::Workspace aws;
   DeviceBuffer apoints, alabels, aperm, ameta;
+  bude::items::Points apoint_items;  // the points sorted for their labels
   size_t antrain = 0, anval = 0;
   // exact energies of every pair (exhaustive) and the protein they belong to
   uint64_t exact_sum = 0;
@@ -658,14 +659,14 @@ Gate gate_stats(const std::vector<double> &e, const std::vector<double> &p, doub
 int train_atom(bude_combined *c, uint64_t pseed) {
   ProteinSlot &ps = c->s();
   const size_t n = c->antrain + c->anval;
-  if (int st = bude::hip_check(bude::atomnet::label_points(static_cast<const float4 *>(ps.protein.ptr),
-                                                           static_cast<const int32_t *>(ps.group_begin.ptr),
-                                                           static_cast<const bude::PairCoef *>(ps.slot_coef.ptr),
-                                                           int(ps.ngroups), static_cast<const float4 *>(c->apoints.ptr),
-                                                           n, bude::plain_form(), static_cast<float *>(c->alabels.ptr),
-                                                           c->stream2),
-                               "label points"))
-    return st;
+  const hipError_t le =
+      ps.reachable ? c->apoint_items.launch(ps.scene, static_cast<float *>(c->alabels.ptr), c->stream2)
+                   : bude::atomnet::label_points(static_cast<const float4 *>(ps.protein.ptr),
+                                                 static_cast<const int32_t *>(ps.group_begin.ptr),
+                                                 static_cast<const bude::PairCoef *>(ps.slot_coef.ptr), int(ps.ngroups),
+                                                 static_cast<const float4 *>(c->apoints.ptr), n, bude::plain_form(),
+                                                 static_cast<float *>(c->alabels.ptr), c->stream2);
+  if (int st = bude::hip_check(le, "label points")) return st;
   if (int st = bude::atomnet::init(c->anet, c->grid, int(c->slot_type.size()), pseed, c->stream2)) return st;
   bude::atomnet::TrainParams tp;
   tp.batch = c->cfg.batch;
@@ -931,6 +932,11 @@ int prepare_atom_points(bude_combined *c) {
                                                             int(nslots), c->cfg.seed ^ 0x70017ull, n,
                                                             static_cast<float4 *>(c->apoints.ptr), nullptr),
                                "sample points"))
+    return st;
+  std::vector<size_t> slot_count(nslots, 0);  // (one slot per 64 points, in turn)
+  for (size_t b = 0; b < n / 64; b++) slot_count[b % nslots] += 64;
+  if (int st = c->apoint_items.build(static_cast<const float4 *>(c->apoints.ptr), nullptr, nullptr, n, slot_count,
+                                     nullptr))
     return st;
   std::vector<uint32_t> perm(c->antrain);
   std::iota(perm.begin(), perm.end(), 0u);

@@ -95,6 +95,25 @@ class Plan {
   double items_ = 0;
 };
 
+// Single atoms at given points, sorted once and scored against any number of
+// scenes with the same slots: out[i] is the plain kernel's energy of a
+// one-atom ligand at point i, bit for bit.
+class Points {
+ public:
+  // n points on the device, either packed (x, y, z, slot bits) or as
+  // coordinates xyz[3 i ..] and slots[i]; slot_count[s] of them have slot s.
+  // Queued on s; the inputs are read by the queued kernels only.
+  int build(const float4 *packed, const float *xyz, const int32_t *slots, size_t n,
+            const std::vector<size_t> &slot_count, hipStream_t s);
+  hipError_t launch(const Scene &sc, float *out, hipStream_t s) const;
+
+ private:
+  DeviceBuffer buf_;
+  const float4 *items_ = nullptr;
+  const int32_t *slot_items_ = nullptr, *slot_units_ = nullptr;
+  int nslots_ = 0, nunits_ = 0, rb_ = 1;
+};
+
 // The pass over every pair, for decks too small to sort (and those whose
 // pairs have no reach): one wave per 64 poses and ligand atom or, while those
 // are too few for the device, several that share the protein's groups; then the sums in

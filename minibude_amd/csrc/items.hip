@@ -325,6 +325,65 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const int32_t *__restric
     }
 }
 
+// Points as items (Points::build; 262,144 points of 34 types against 4,096
+// atoms, a whole call: 3.45 ms with the points grouped by type on the host
+// and every pair scored, 0.76 ms sorted here): the box of them and cleared
+// counts, then the counts per (slot, cell), then, the counts having become
+// first places, each into its place.
+struct PointsIn {
+  const float4 *packed;
+  const float *xyz;
+  const int32_t *slots;
+  size_t n;
+  __device__ __forceinline__ float4 get(size_t i) const {
+    if (packed) return packed[i];
+    return make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], __int_as_float(slots[i]));
+  }
+};
+
+__global__ __launch_bounds__(kThreads) void point_box_kernel(const PointsIn in, uint32_t *__restrict__ counts,
+                                                             size_t ncounts, float *__restrict__ bounds) {
+  __shared__ float part[kThreads / 64][6];
+  const size_t first = size_t(blockIdx.x) * kThreads + threadIdx.x, step = size_t(gridDim.x) * kThreads;
+  for (size_t i = first; i < ncounts; i += step) counts[i] = 0u;
+  float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+  for (size_t i = first; i < in.n; i += step) {
+    const float4 p = in.get(i);
+    v[0] = fminf(v[0], p.x), v[3] = fmaxf(v[3], p.x);
+    v[1] = fminf(v[1], p.y), v[4] = fmaxf(v[4], p.y);
+    v[2] = fminf(v[2], p.z), v[5] = fmaxf(v[5], p.z);
+  }
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    const float a = k < 3 ? wave_min(v[k]) : wave_max(v[k]);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][k] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    float a = part[0][threadIdx.x];
+    for (int w = 1; w < kThreads / 64; w++)
+      a = threadIdx.x < 3 ? fminf(a, part[w][threadIdx.x]) : fmaxf(a, part[w][threadIdx.x]);
+    bounds[size_t(blockIdx.x) * 6 + threadIdx.x] = a;
+  }
+}
+
+template <int SCATTER>
+__global__ __launch_bounds__(kThreads) void point_bin_kernel(const PointsIn in, const float *__restrict__ bounds,
+                                                             int nbounds, int bits, uint32_t *__restrict__ counts,
+                                                             float4 *__restrict__ items) {
+  __shared__ uint16_t curve[kCells];
+  __shared__ float red[6];
+  for (int i = threadIdx.x; i < kCells; i += kThreads) curve[i] = kCurve.place[i];  // (cell_grid waits for it)
+  const Space all{{-FLT_MAX, -FLT_MAX, -FLT_MAX}, {FLT_MAX, FLT_MAX, FLT_MAX}, 0.f};
+  const CellGrid g = cell_grid(bounds, nbounds, all, red);
+  for (size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x; i < in.n; i += size_t(gridDim.x) * kThreads) {
+    const float4 p = in.get(i);
+    const uint32_t c = cell_of(g, curve, p.x, p.y, p.z) >> (12 - bits);
+    const uint32_t at = atomicAdd(&counts[(size_t(__float_as_int(p.w)) << bits) + c], 1u);
+    if constexpr (SCATTER) items[at] = make_float4(p.x, p.y, p.z, __uint_as_float(uint32_t(i)));
+  }
+}
+
 // The protein atoms of `mask` (lanes of the wave's 64 atoms x, y, z), all of
 // one group, in order.
 template <int RB, int FORM, bool CHG, bool DSLV>
@@ -403,7 +462,7 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
                                                     const float4 *__restrict__ items,
                                                     const int32_t *__restrict__ slot_items,
                                                     const int32_t *__restrict__ slot_units, int nslots, int nunits,
-                                                    float *__restrict__ partial) {
+                                                    float scale, float *__restrict__ partial) {
   __shared__ uint16_t list[LIST ? kShare : 1];
   __shared__ float box[4][6];
   __shared__ int count[4], slots[4];
@@ -543,7 +602,7 @@ __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ p
   if (unit >= nunits) return;
 #pragma unroll
   for (int k = 0; k < RB; k++)
-    if (i0 + k * 64 + lane < i1) partial[out[k]] = e[k] + part[k];
+    if (i0 + k * 64 + lane < i1) partial[out[k]] = (e[k] + part[k]) * scale;
 }
 
 // p[0] + p[stride] + ... in order, eight loads in flight.
@@ -652,11 +711,30 @@ template <int FORM, class... A> void launch_score_rb(int rb, bool listed, int nu
 
 constexpr size_t kDirectWaves = 16384;
 
+// Work-groups of the point kernels, for n points.
+unsigned point_groups(size_t n) { return unsigned(std::min<size_t>(kMaxBounds, (n + kThreads - 1) / kThreads)); }
+
+// Items per lane for `mean` items of a type: more share the protein's steps,
+// fewer keep the box small where items are sparse.  Whole passes at 1, 2, 4
+// and 8: 24 k items of a type 73, 78, 98, 128 us; 95 k 340, 315, 317, 450;
+// 560 k 2,050, 1,580, 1,330, 1,380; 2.2 M 7,980, 5,980, 4,720, 4,450.
+int items_per_lane(int64_t mean) { return mean >= 1100000 ? 8 : mean >= 230000 ? 4 : mean >= 48000 ? 2 : 1; }
+
 // Proteins from which the score kernel lists a work-group's atoms first: with
 // and without, 4,096 x 64 x 262,144 1,250 and 1,340 us, 4,096 x 26 x 65,536
 // 300 and 316; 938 x 64 x 262,144 617 and 596, 300 x 64 x 131,072 249 and 234
 // (15 and 5 steps of 64 atoms per wave are no work worth sharing).
 constexpr int kListFrom = 1500;
+
+void score_items(const Scene &sc, int rb, const float4 *items, const int32_t *slot_items, const int32_t *slot_units,
+                 int nslots, int nunits, float scale, float *out, hipStream_t s) {
+  auto score = [&](auto run) {
+    run(rb, sc.natpro >= kListFrom, nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups, items,
+        slot_items, slot_units, nslots, nunits, scale, out);
+  };
+  if (sc.form == kFormD) score([](auto... args) { launch_score_rb<kFormD>(args...); });
+  else score([](auto... args) { launch_score_rb<kFormB>(args...); });
+}
 
 // Items of one chunk: 20 bytes each in the workspace.
 constexpr int64_t kChunkItems = int64_t(1) << 26;
@@ -851,11 +929,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
       used += count[size_t(t)] > 0;
     }
     const int64_t mean = nitems / std::max<int64_t>(1, used);
-    // items per lane: more share the protein's steps, fewer keep the box
-    // small where items are sparse.  Whole passes at 1, 2, 4 and 8: 24 k items
-    // of a type 73, 78, 88, 122 us; 95 k 340, 315, 326, 460; 560 k 2,050,
-    // 1,580, 1,330, 1,380; 2.2 M 7,980, 5,980, 4,720, 4,450.
-    ch.rb = mean >= 1100000 ? 8 : mean >= 230000 ? 4 : mean >= 48000 ? 2 : 1;
+    ch.rb = items_per_lane(mean);
     ch.cell_bits = mean >= 16384 ? 12 : 9;
     std::vector<Row> rows;
     std::vector<std::vector<int32_t>> refs_of(blocks.size());
@@ -965,18 +1039,63 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
     launch_bin_ppt<1>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),
                       size_t(c.nxform), static_cast<const float *>(bounds), nb, sp, c.cell_bits, hist,
                       static_cast<const uint32_t *>(base), items);
-    auto score = [&](auto run) {
-      run(c.rb, sc.natpro >= kListFrom, c.nunits, s, sc.protein, sc.natpro, sc.coef, sc.reach2, sc.ngroups,
-          static_cast<const float4 *>(items), slot_items, slot_units, nslots_, c.nunits, partial);
-    };
-    if (sc.form == kFormD) score([](auto... args) { launch_score_rb<kFormD>(args...); });
-    else score([](auto... args) { launch_score_rb<kFormB>(args...); });
+    score_items(sc, c.rb, items, slot_items, slot_units, nslots_, c.nunits, 1.0f, partial, s);
     const int per = 4 * c.ppt;  // work-groups of 256 per block of 1024 ppt poses
     hipLaunchKernelGGL(reduce_kernel, dim3(unsigned(c.nblocks) * unsigned(per)), dim3(256), 0, s, blocks, per,
                        static_cast<const float *>(partial), energies);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+int Points::build(const float4 *packed, const float *xyz, const int32_t *slots, size_t n,
+                  const std::vector<size_t> &slot_count, hipStream_t s) {
+  if (n == 0 || n > 0x7fffffffu || slot_count.empty())
+    return fail(BUDE_ERR_INVALID_ARGUMENT, "points: none, or more than 2^31");
+  nslots_ = int(slot_count.size());
+  const int64_t mean = int64_t(n / slot_count.size());
+  const int bits = mean >= 16384 ? 12 : mean >= 512 ? 9 : 6;
+  rb_ = items_per_lane(mean);
+  std::vector<int32_t> table(2 * (size_t(nslots_) + 1), 0);
+  int32_t *first = table.data(), *unit = first + nslots_ + 1;
+  for (int t = 0; t < nslots_; t++) {
+    first[t + 1] = first[t] + int32_t(slot_count[size_t(t)]);
+    unit[t + 1] = unit[t] + int32_t((int64_t(slot_count[size_t(t)]) + 64 * rb_ - 1) / (64 * rb_));
+  }
+  if (size_t(first[nslots_]) != n) return fail(BUDE_ERR_INVALID_ARGUMENT, "points: counts do not add up");
+  nunits_ = unit[nslots_];
+  // one allocation: items, counts, bounds, the table
+  auto pad = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t ncounts = size_t(nslots_) << bits;
+  const size_t at_counts = pad(n * sizeof(float4)), at_bounds = at_counts + pad(ncounts * 4),
+               at_table = at_bounds + pad(kMaxBounds * 24);
+  if (int st = buf_.reserve(at_table + table.size() * 4)) return st;
+  auto *base = static_cast<char *>(buf_.ptr);
+  auto *items = reinterpret_cast<float4 *>(base);
+  auto *counts = reinterpret_cast<uint32_t *>(base + at_counts);
+  auto *bounds = reinterpret_cast<float *>(base + at_bounds);
+  items_ = items;
+  slot_items_ = reinterpret_cast<const int32_t *>(base + at_table);
+  slot_units_ = slot_items_ + nslots_ + 1;
+  if (int st = hip_check(hipMemcpyAsync(base + at_table, table.data(), table.size() * 4, hipMemcpyHostToDevice, s),
+                         "hipMemcpyAsync"))
+    return st;
+  if (int st = hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;  // (the table is a local)
+  const PointsIn in{packed, xyz, slots, n};
+  const unsigned groups = point_groups(n);
+  hipLaunchKernelGGL(point_box_kernel, dim3(groups), dim3(kThreads), 0, s, in, counts, ncounts, bounds);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(point_bin_kernel<0>), dim3(groups), dim3(kThreads), 0, s, in,
+                     static_cast<const float *>(bounds), int(groups), bits, counts, items);
+  hipLaunchKernelGGL(scan_kernel, dim3(unsigned(nslots_)), dim3(kThreads), 0, s, slot_items_, bits, counts);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(point_bin_kernel<1>), dim3(groups), dim3(kThreads), 0, s, in,
+                     static_cast<const float *>(bounds), int(groups), bits, counts, items);
+  return hip_check(hipGetLastError(), "sort points");
+}
+
+hipError_t Points::launch(const Scene &sc, float *out, hipStream_t s) const {
+  if (!items_) return hipErrorInvalidValue;
+  score_items(sc, rb_, items_, slot_items_, slot_units_, nslots_, nunits_, 0.5f, out, s);
+  return hipGetLastError();
 }
 
 size_t direct_bytes(size_t n, size_t natlig) { return (n + 63) / 64 * 64 * natlig * sizeof(float); }

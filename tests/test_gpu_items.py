@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from minibude_amd import capi
+from minibude_amd import atomnet, capi
 from minibude_amd import deck as D
 from minibude_amd.batch import Batch, LigandSet
 from minibude_amd.capi import BatchConfig
@@ -88,6 +88,33 @@ def test_few_tiles_equal_tiled(gpu_device, natlig, nposes):
             b.run(BatchConfig(2, 64, 4, 0, graph), warmup=0, iterations=2)
             for i in range(n):
                 assert np.array_equal(b.energies(i).view(np.uint32), want[i].view(np.uint32)), (graph, i)
+
+
+@pytest.mark.parametrize("natpro, npoints, ntypes", [
+    (300, 1, 3),
+    (938, 1000, 34),        # fewer points of a type than a wave's lanes
+    (4096, 70001, 34),
+    (1500, 300000, 1),      # one type, several items per lane, a remainder
+])
+def test_atom_energies_equal_tiled(gpu_device, natpro, npoints, ntypes):
+    rng = np.random.default_rng(78)
+    pro, ff = D.synth_protein(79, natpro, ntypes), D.synth_forcefield(79, ntypes)
+    pts = rng.uniform(-25, 25, (npoints, 3)).astype(np.float32)
+    types = rng.integers(0, ntypes, npoints).astype(np.int32)
+    got = atomnet.atom_energies(pro, ff, pts, types, gpu_device)
+    used = np.unique(types)
+    ligs, poses = [], []
+    for t in used:  # a one-atom ligand at its frame's origin, translated to the points
+        lig = np.zeros(1, capi.ATOM_DTYPE)
+        lig["type"] = t
+        ligs.append(lig)
+        p = np.zeros((6, int((types == t).sum())), np.float32)
+        p[3:] = pts[types == t].T
+        poses.append(p)
+    with Batch(LigandSet(pro, ff, ligs, poses), gpu_device) as b:
+        b.run_separate(1, 64)
+        for i, t in enumerate(used):
+            assert np.array_equal(got[types == t].view(np.uint32), b.energies(i).view(np.uint32)), t
 
 
 def test_poses_out_of_reach_and_not_finite(gpu_device):
