@@ -69,6 +69,29 @@ __global__ void gather_index_kernel(const float *__restrict__ src, size_t src_st
 
 unsigned blocks_for(size_t n, unsigned t) { return unsigned((n + t - 1) / t); }
 
+// A window of pairs' selections on their way to the host: pair first + i has
+// n[i] rows from row off[i], packed from at[i]; bit i of fallback: its
+// energies are its scores.
+constexpr int kWindowPairs = 64;
+constexpr size_t kWindowRows = size_t(1) << 18;
+struct Window {
+  int64_t off[kWindowPairs];
+  uint32_t n[kWindowPairs], at[kWindowPairs];
+  uint64_t fallback;
+};
+
+__global__ __launch_bounds__(256) void window_kernel(const Window w, const uint32_t *__restrict__ idx,
+                                                     const float *__restrict__ exact, const float *__restrict__ scores,
+                                                     uint32_t *__restrict__ out_idx, float *__restrict__ out_e) {
+  const int p = blockIdx.y;
+  const int64_t off = w.off[p];
+  for (uint32_t j = blockIdx.x * 256 + threadIdx.x; j < w.n[p]; j += gridDim.x * 256) {
+    const uint32_t i = idx[off + j];
+    out_idx[w.at[p] + j] = i;
+    out_e[w.at[p] + j] = (w.fallback >> p & 1) ? scores[off + i] : exact[off + j];
+  }
+}
+
 // Pair coefficients of every ligand atom against every protein group:
 // coef[a * ngroups + g] = slot_coef[slot(a) * ngroups + g], the atom's map
 // slot in the w bits of its float4 (a coefficient depends on the ligand
@@ -176,6 +199,10 @@ struct ProteinSlot {
   std::vector<float> lab_energy;
   std::vector<size_t> lab_offs;
   uint64_t protein_sum = 0;
+  // the window of pairs [win_a, win_b) whose selections were last fetched:
+  // pair l's in the object's window buffer from row win_at[l - win_a]
+  size_t win_a = 0, win_b = 0;
+  std::vector<uint32_t> win_at;
   // begun and not yet ended; how its selection and rescoring run
   // overlap: the next protein of a batch may begin before this one ends (its
   // selection ran chunk by chunk, or as one pass over the scores that the
@@ -256,6 +283,12 @@ struct bude_combined {
   ProteinSlot &s() { return slots[cur]; }
   const ProteinSlot &s() const { return slots[cur]; }
   DeviceBuffer maps, cells, counter;
+  // selections fetched by bude_mi355x_combined_selected: indices, then
+  // energies, of the window of slot win_slot
+  DeviceBuffer win_dev;
+  bude::PinnedBuffer win_host;
+  size_t win_rows = 0;
+  int win_slot = -1;
   // per-call work tables (each its own buffer; uploaded only while no queued
   // kernel reads it)
   DeviceBuffer meta_label, tiles_label, meta_lf, meta_fb, tiles_fb, meta_all, meta_ex, tiles_all;
@@ -1055,6 +1088,9 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     st = plan_sorted(c.get(), c->label_sorted, segs);
     if (!st) st = reserve_sorted(c->label_sorted, c->label_work, &c->label_sorted_ok);
   }
+  if (!st) st = c->win_dev.alloc(kWindowRows * 8);
+  if (!st) st = c->win_host.alloc(kWindowRows * 8);
+  c->win_rows = kWindowRows;
   if (!st) st = c->counter.alloc(256);
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking), "hipStreamCreate");
@@ -1083,6 +1119,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   *res = BudeCombinedResult{};
   c->s().valid = false;
   c->s().busy = true;
+  c->s().win_a = c->s().win_b = 0;
   {  // FNV-1a of the protein: exact energies stay valid while it is unchanged
     uint64_t hsum = 1469598103934665603ull ^ uint64_t(natpro);
     const auto *bytes = reinterpret_cast<const unsigned char *>(protein);
@@ -1655,6 +1692,58 @@ extern "C" int bude_mi355x_combined_pair(bude_combined *c, size_t ligand, BudePa
   return bude::ok();
 }
 
+namespace {
+
+// The window of pairs from `ligand` on (the selections of a screen are read
+// pair after pair): one kernel packs their rows, one copy brings them.  Up to
+// kWindowPairs pairs and kWindowRows rows, or one pair of more rows.
+int fetch_window(bude_combined *c, size_t ligand) {
+  ProteinSlot &ps = c->s();
+  if (c->win_slot == c->cur && ligand >= ps.win_a && ligand < ps.win_b) return BUDE_OK;
+  Window w{};
+  size_t rows = 0, l = ligand;
+  std::vector<uint32_t> at;
+  for (; l < c->nlig && l - ligand < size_t(kWindowPairs); l++) {
+    const size_t k = ps.nsel[l], i = l - ligand;
+    if (i && rows + k > kWindowRows) break;
+    w.off[i] = int64_t(c->pose_off[l]);
+    w.n[i] = uint32_t(k);
+    w.at[i] = uint32_t(rows);
+    if (ps.fallback[l]) w.fallback |= uint64_t(1) << i;
+    at.push_back(uint32_t(rows));
+    rows += k;
+  }
+  ps.win_a = ps.win_b = 0;
+  c->win_slot = -1;
+  if (rows > c->win_rows) {
+    c->win_rows = 0;
+    if (int st = c->win_dev.alloc(rows * 8)) return st;
+    if (int st = c->win_host.alloc(rows * 8)) return st;
+    c->win_rows = rows;
+  }
+  if (rows) {
+    auto *dev = static_cast<uint32_t *>(c->win_dev.ptr);
+    auto *host = static_cast<uint32_t *>(c->win_host.ptr);
+    hipLaunchKernelGGL(window_kernel, dim3(8, unsigned(l - ligand)), dim3(256), 0, nullptr, w,
+                       static_cast<const uint32_t *>(ps.sel_idx.ptr), static_cast<const float *>(ps.exact_sel.ptr),
+                       static_cast<const float *>(c->pred.ptr), dev, reinterpret_cast<float *>(dev + c->win_rows));
+    if (int st = bude::hip_check(hipGetLastError(), "selection window")) return st;
+    for (size_t part = 0; part < 2; part++)
+      if (int st = bude::hip_check(hipMemcpyAsync(host + part * c->win_rows, dev + part * c->win_rows, rows * 4,
+                                                  hipMemcpyDeviceToHost, nullptr),
+                                   "hipMemcpyAsync"))
+        return st;
+    if (int st = bude::hip_check(hipStreamSynchronize(nullptr), "hipStreamSynchronize")) return st;
+  }
+  ps.win_a = ligand;
+  ps.win_b = l;
+  ps.win_at = std::move(at);
+  c->win_slot = c->cur;
+  return BUDE_OK;
+}
+
+}  // namespace
+
 extern "C" int bude_mi355x_combined_selected(bude_combined *c, size_t ligand, uint32_t *idx, float *energies, size_t cap,
                                              size_t *n) {
   if (!c || !n || ligand >= c->nlig)
@@ -1665,34 +1754,12 @@ extern "C" int bude_mi355x_combined_selected(bude_combined *c, size_t ligand, ui
   if (!idx && !energies) return bude::ok();
   if (cap < k) return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_combined_selected: buffer too small");
   if (int st = bude::hip_check(hipSetDevice(c->device), "hipSetDevice")) return st;
-  std::vector<uint32_t> id(k);
-  std::vector<float> ex(k);
-  const size_t po = c->pose_off[ligand];
-  if (k) {
-    if (int st = bude::hip_check(hipMemcpy(id.data(), static_cast<uint32_t *>(c->s().sel_idx.ptr) + po, k * 4,
-                                           hipMemcpyDeviceToHost),
-                                 "hipMemcpy"))
-      return st;
-    if (c->s().fallback[ligand]) {  // the scores of a fallback pair are its exact energies
-      std::vector<float> all(c->nposes[ligand]);
-      if (int st = bude::hip_check(hipMemcpy(all.data(), static_cast<float *>(c->pred.ptr) + po, all.size() * 4,
-                                             hipMemcpyDeviceToHost),
-                                   "hipMemcpy"))
-        return st;
-      for (size_t j = 0; j < k; j++) ex[j] = all[id[j]];
-    } else if (int st = bude::hip_check(hipMemcpy(ex.data(), static_cast<float *>(c->s().exact_sel.ptr) + po,
-                                                  k * 4, hipMemcpyDeviceToHost),
-                                        "hipMemcpy")) {
-      return st;
-    }
-  }
-  std::vector<size_t> ord(k);
-  std::iota(ord.begin(), ord.end(), size_t(0));
-  std::sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return id[a] < id[b]; });
-  for (size_t j = 0; j < k; j++) {
-    if (idx) idx[j] = id[ord[j]];
-    if (energies) energies[j] = ex[ord[j]];
-  }
+  if (int st = fetch_window(c, ligand)) return st;
+  const ProteinSlot &ps = c->s();
+  const auto *win = static_cast<const uint32_t *>(c->win_host.ptr);
+  const size_t at = ps.win_at[ligand - ps.win_a];
+  if (idx) std::memcpy(idx, win + at, k * sizeof(uint32_t));
+  if (energies) std::memcpy(energies, win + c->win_rows + at, k * sizeof(float));
   return bude::ok();
 }
 

@@ -443,14 +443,9 @@ extern "C" int bude_mi355x_screen_selected(bude_screen *s, uint32_t *idx, float 
     if (int st = bude::hip_check(hipMemcpy(ex.data(), s->exact.ptr, s->nsel * 4, hipMemcpyDeviceToHost), "hipMemcpy"))
       return st;
   }
-  // report in pose order
-  std::vector<size_t> ord(s->nsel);
-  std::iota(ord.begin(), ord.end(), size_t(0));
-  std::sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return id[a] < id[b]; });
-  for (size_t j = 0; j < s->nsel; j++) {
-    if (idx) idx[j] = id[ord[j]];
-    if (energies) energies[j] = ex[ord[j]];
-  }
+  // (selections are in pose order)
+  if (idx) std::copy(id.begin(), id.end(), idx);
+  if (energies) std::copy(ex.begin(), ex.end(), energies);
   return bude::ok();
 }
 

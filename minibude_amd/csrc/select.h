@@ -21,7 +21,8 @@ struct Segment {
 static_assert(sizeof(Segment) == 16, "Segment is 16 bytes");
 
 // Device state of one selection over a fixed segment list: the segments, the
-// chunk table the passes iterate over and the per-segment histograms.
+// chunk table the passes iterate over, the per-segment histograms and the
+// chunks' counts.
 struct Plan {
   size_t nseg = 0, nchunks = 0;
   DeviceBuffer segs, chunks, hist;
@@ -31,8 +32,7 @@ struct Plan {
 
 // For every segment s: out_idx[s.off + j], j < out_n[s], are the positions
 // (relative to s.off) of every value <= the k-th smallest value of the
-// segment (ties at the threshold are all kept, so out_n[s] >= k), in no
-// particular order.  x, out_idx (as long as x) and out_n (nseg) are device
+// segment (ties at the threshold are all kept, so out_n[s] >= k), ascending.  x, out_idx (as long as x) and out_n (nseg) are device
 // memory.
 hipError_t select_lowest_segments(const Plan &p, const float *x, uint32_t *out_idx, uint32_t *out_n, hipStream_t s);
 

@@ -2,8 +2,8 @@
 // over order-preserving keys.  Every pass streams each segment's values once
 // in chunks of 16,384 (one work-group per chunk, LDS histogram merged into
 // the segment's global histogram), one wave per segment then narrows the
-// key prefix; a last streaming pass writes the selected positions with one
-// atomic per wave.
+// key prefix; two last streaming passes count the selected positions of every
+// chunk and write them in ascending order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,15 +30,13 @@ __device__ __forceinline__ uint32_t order_key(float x) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-__global__ __launch_bounds__(256) void seg_init_kernel(const Segment *__restrict__ segs, uint32_t *__restrict__ hist,
-                                                       uint32_t *__restrict__ out_n) {
+__global__ __launch_bounds__(256) void seg_init_kernel(const Segment *__restrict__ segs, uint32_t *__restrict__ hist) {
   uint32_t *h = hist + size_t(blockIdx.x) * kHistStride;
   for (int i = threadIdx.x; i < kBins; i += 256) h[i] = 0;
   if (threadIdx.x == 0) {
     h[kBins] = 0;
     h[kBins + 1] = 0;
     h[kBins + 2] = segs[blockIdx.x].k;
-    out_n[blockIdx.x] = 0;
   }
 }
 
@@ -91,41 +89,66 @@ __global__ __launch_bounds__(64) void seg_pick_kernel(uint32_t *__restrict__ his
   for (int i = lane; i < kBins; i += 64) h[i] = 0;
 }
 
-// Two passes over the chunk: count (per wave, over its quarter of the
-// chunk), one atomic per chunk for the chunk's output base, then write with
-// per-wave running offsets.  (An atomic per wave and step contends on the
-// few per-segment counters.)
-__global__ __launch_bounds__(256) void seg_compact_kernel(const Segment *__restrict__ segs,
-                                                          const Chunk *__restrict__ chunks,
-                                                          const float *__restrict__ x, const uint32_t *__restrict__ hist,
-                                                          uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_n) {
-  __shared__ uint32_t wave_base[4];
+// Values at or below the threshold in each chunk.
+__global__ __launch_bounds__(256) void seg_count_kernel(const Segment *__restrict__ segs,
+                                                        const Chunk *__restrict__ chunks, const float *__restrict__ x,
+                                                        const uint32_t *__restrict__ hist,
+                                                        uint32_t *__restrict__ counts) {
+  __shared__ uint32_t wave_count[4];
   const Chunk c = chunks[blockIdx.x];
   const Segment sg = segs[c.seg];
   const uint32_t thr = hist[size_t(c.seg) * kHistStride + kBins];
   const uint32_t end = min(c.begin + kChunk, sg.n);
   const float *xs = x + sg.off;
+  uint32_t count = 0;
+  for (uint32_t j = c.begin + threadIdx.x; j < end; j += 256) count += order_key(xs[j]) <= thr;
+  for (int d = 32; d; d >>= 1) count += __shfl_xor(count, d);
+  if ((threadIdx.x & 63) == 0) wave_count[threadIdx.x >> 6] = count;
+  __syncthreads();
+  if (threadIdx.x == 0) counts[blockIdx.x] = wave_count[0] + wave_count[1] + wave_count[2] + wave_count[3];
+}
+
+// Each chunk's selected positions behind those of the segment's chunks
+// before it, so that a segment's come out ascending (the caller need not
+// sort them); every wave counts and then writes its quarter of the chunk.
+// The segment's last chunk writes its total.
+__global__ __launch_bounds__(256) void seg_compact_kernel(const Segment *__restrict__ segs,
+                                                          const Chunk *__restrict__ chunks,
+                                                          const float *__restrict__ x, const uint32_t *__restrict__ hist,
+                                                          const uint32_t *__restrict__ counts,
+                                                          uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_n) {
+  __shared__ uint32_t wave_count[4], wave_before[4];
+  const Chunk c = chunks[blockIdx.x];
+  const Segment sg = segs[c.seg];
+  const uint32_t own = counts[blockIdx.x];
+  const bool last = sg.n - c.begin <= kChunk;
+  if (own == 0 && !last) return;  // (whole work-group)
+  const uint32_t thr = hist[size_t(c.seg) * kHistStride + kBins];
+  const uint32_t end = min(c.begin + kChunk, sg.n);
+  const float *xs = x + sg.off;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t ordinal = c.begin / kChunk;  // chunks of the segment before this one
+  uint32_t before = 0;
+  for (uint32_t i = threadIdx.x; i < ordinal; i += 256) before += counts[blockIdx.x - ordinal + i];
+  for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d);
   constexpr uint32_t kQuarter = kChunk / 4;
   const uint32_t wb = c.begin + uint32_t(wave) * kQuarter, we = min(wb + kQuarter, end);
   uint32_t count = 0;
-  for (uint32_t j0 = wb; j0 < we; j0 += 64) {
-    const uint32_t j = j0 + lane;
-    count += uint32_t(__popcll(__ballot(j < we && order_key(xs[j]) <= thr)));
-  }
-  if (lane == 0) wave_base[wave] = count;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t c0 = wave_base[0], c1 = wave_base[1], c2 = wave_base[2], c3 = wave_base[3];
-    const uint32_t base = (c0 + c1 + c2 + c3) ? atomicAdd(&out_n[c.seg], c0 + c1 + c2 + c3) : 0u;
-    wave_base[0] = base;
-    wave_base[1] = base + c0;
-    wave_base[2] = base + c0 + c1;
-    wave_base[3] = base + c0 + c1 + c2;
+  if (own)
+    for (uint32_t j0 = wb; j0 < we; j0 += 64) {
+      const uint32_t j = j0 + lane;
+      count += uint32_t(__popcll(__ballot(j < we && order_key(xs[j]) <= thr)));
+    }
+  if (lane == 0) {
+    wave_count[wave] = count;
+    wave_before[wave] = before;
   }
   __syncthreads();
+  const uint32_t base = wave_before[0] + wave_before[1] + wave_before[2] + wave_before[3];
+  if (last && threadIdx.x == 0) out_n[c.seg] = base + own;
   if (count == 0) return;
-  uint32_t pos = wave_base[wave];
+  uint32_t pos = base;
+  for (int w = 0; w < wave; w++) pos += wave_count[w];
   for (uint32_t j0 = wb; j0 < we; j0 += 64) {
     const uint32_t j = j0 + lane;
     const bool take = j < we && order_key(xs[j]) <= thr;
@@ -153,7 +176,7 @@ int Plan::prepare(const std::vector<Segment> &s) {
   nchunks = c.size();
   int st = segs.upload(s.data(), s.size() * sizeof(Segment));
   if (!st) st = chunks.upload(c.data(), c.size() * sizeof(Chunk));
-  if (!st) st = hist.reserve(nseg * kHistStride * sizeof(uint32_t));
+  if (!st) st = hist.reserve((nseg * kHistStride + nchunks) * sizeof(uint32_t));
   return st;
 }
 
@@ -162,15 +185,17 @@ hipError_t select_lowest_segments(const Plan &p, const float *x, uint32_t *out_i
   const auto *segs = static_cast<const Segment *>(p.segs.ptr);
   const auto *chunks = static_cast<const Chunk *>(p.chunks.ptr);
   auto *hist = static_cast<uint32_t *>(p.hist.ptr);
-  hipLaunchKernelGGL(seg_init_kernel, dim3(unsigned(p.nseg)), dim3(256), 0, s, segs, hist, out_n);
+  hipLaunchKernelGGL(seg_init_kernel, dim3(unsigned(p.nseg)), dim3(256), 0, s, segs, hist);
   const int shifts[3] = {21, 10, 0}, bits[3] = {11, 11, 10};
   for (int q = 0; q < 3; q++) {
     hipLaunchKernelGGL(seg_hist_kernel, dim3(unsigned(p.nchunks)), dim3(256), 0, s, segs, chunks, x, shifts[q],
                        (1u << bits[q]) - 1u, hist);
     hipLaunchKernelGGL(seg_pick_kernel, dim3(unsigned(p.nseg)), dim3(64), 0, s, hist, shifts[q], bits[q]);
   }
-  hipLaunchKernelGGL(seg_compact_kernel, dim3(unsigned(p.nchunks)), dim3(256), 0, s, segs, chunks, x, hist, out_idx,
-                     out_n);
+  auto *counts = hist + p.nseg * kHistStride;
+  hipLaunchKernelGGL(seg_count_kernel, dim3(unsigned(p.nchunks)), dim3(256), 0, s, segs, chunks, x, hist, counts);
+  hipLaunchKernelGGL(seg_compact_kernel, dim3(unsigned(p.nchunks)), dim3(256), 0, s, segs, chunks, x, hist, counts,
+                     out_idx, out_n);
   return hipGetLastError();
 }
 
