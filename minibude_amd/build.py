@@ -50,6 +50,7 @@ LIB_SOURCES = [
     "surrogate.hip",
     "capi_screen.hip",
     "select.hip",
+    "gate.hip",
     "field.hip",
     "atomnet.hip",
     "capi_atomnet.hip",

@@ -26,6 +26,7 @@
 #include "bude_internal.h"
 #include "fasten_batch.h"
 #include "field.h"
+#include "gate.h"
 #include "hip_util.h"
 #include "items.h"
 #include "mlp.h"
@@ -293,6 +294,7 @@ struct bude_combined {
   // kernel reads it)
   DeviceBuffer meta_label, tiles_label, meta_lf, meta_fb, tiles_fb, meta_all, meta_ex, tiles_all;
   DeviceBuffer tb_label, tb_all, lab_src, lab_poses, lab_e, lab_lig, lab_pred, norms, bias0;
+  DeviceBuffer lab_off_dev, lab_stats;  // the sampled poses' bounds per pair; the pairs' validation statistics
   std::vector<int64_t> tb_all_host;  // field tile prefix of every pair (fixed: the poses are)
   bool field_tables = false;
   // rs_order lists each pipeline chunk's ligands heaviest first
@@ -1085,7 +1087,12 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
       segs[i] = bude::items::Segment{int32_t(i), at, n};
       at += n;
     }
-    st = plan_sorted(c.get(), c->label_sorted, segs);
+    std::vector<uint32_t> bounds;
+    for (const auto &sg : segs) bounds.push_back(uint32_t(sg.pose_off));
+    bounds.push_back(uint32_t(at));
+    st = c->lab_off_dev.upload(bounds.data(), bounds.size() * sizeof(uint32_t));
+    if (!st) st = c->lab_stats.alloc(nligands * sizeof(bude::gate::Stats));
+    if (!st) st = plan_sorted(c.get(), c->label_sorted, segs);
     if (!st) st = reserve_sorted(c->label_sorted, c->label_work, &c->label_sorted_ok);
   }
   if (!st) st = c->win_dev.alloc(kWindowRows * 8);
@@ -1332,7 +1339,11 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     }
     if (int st = record(c, 4, c->stream2)) return st;
   }
-  std::vector<float> le(nlab), lpred(nlab);
+  // the per-pair validation runs on the device where a pair's samples fit
+  // the kernel's LDS (the pose MLP validates on a part of them, after training)
+  const bool gate_on_device = !mlp && cfg.labels_per_pair <= bude::gate::kMaxSamples;
+  std::vector<bude::gate::Stats> stats(gate_on_device ? L : 0);
+  std::vector<float> le(nlab), lpred(gate_on_device ? 0 : nlab);
   if (int st = bude::hip_check(hipMemcpyAsync(le.data(), c->lab_e.ptr, nlab * 4, hipMemcpyDeviceToHost, c->stream3),
                                "hipMemcpyAsync"))
     return st;
@@ -1340,9 +1351,24 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     if (int st = bude::hip_check(hipStreamWaitEvent(c->stream3, c->s().ev[3], 0), "hipStreamWaitEvent")) return st;
     if (int st = launch_surrogate(c, lpos, nlab, lp, c->meta_lf, c->tb_label, 0, ft_label, c->stream3, c->fpart_lab))
       return st;
-    if (int st = bude::hip_check(hipMemcpyAsync(lpred.data(), lp, nlab * 4, hipMemcpyDeviceToHost, c->stream3),
-                                 "hipMemcpyAsync"))
+    if (gate_on_device) {
+      const bude::gate::Params q{double(cfg.keep_fraction), double(cfg.gate_top_fraction), double(cfg.gate_z), 0.25,
+                                 double(cfg.clip_quantile)};
+      if (int st = bude::hip_check(bude::gate::pair_stats(static_cast<const float *>(c->lab_e.ptr), lp,
+                                                          static_cast<const uint32_t *>(c->lab_off_dev.ptr), L,
+                                                          cfg.labels_per_pair, q,
+                                                          static_cast<bude::gate::Stats *>(c->lab_stats.ptr),
+                                                          c->stream3),
+                                   "pair statistics"))
+        return st;
+      if (int st = bude::hip_check(hipMemcpyAsync(stats.data(), c->lab_stats.ptr, L * sizeof(stats[0]),
+                                                  hipMemcpyDeviceToHost, c->stream3),
+                                   "hipMemcpyAsync"))
+        return st;
+    } else if (int st = bude::hip_check(hipMemcpyAsync(lpred.data(), lp, nlab * 4, hipMemcpyDeviceToHost, c->stream3),
+                                        "hipMemcpyAsync")) {
       return st;
+    }
   }
   if (int st = bude::hip_check(hipStreamSynchronize(c->stream3), "hipStreamSynchronize")) return st;
   res->label_ms = elapsed(c, 0, 1);
@@ -1355,7 +1381,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   // per-pair target transform from the training part (all samples for the field)
   std::vector<Norm> norms(L);
   std::vector<bude::mlp::TargetNorm> tn(L);
-  for (size_t l = 0; l < L; l++) {
+  for (size_t l = 0; l < L && !gate_on_device; l++) {
     const size_t b = lab_off[l], e = (mlp && lab_train[l] > 0) ? b + lab_train[l] : lab_off[l + 1];
     norms[l] = norm_of(std::vector<float>(le.begin() + long(b), le.begin() + long(e)), cfg.clip_quantile,
                        cfg.tail_quantile);
@@ -1422,21 +1448,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   c->s().keep.assign(L, cfg.keep_fraction);
   std::vector<double> need(L, 0.0);
   const double tail_q = mlp ? std::min(0.25, double(cfg.clip_quantile)) : 0.25;
-  for (size_t l = 0; l < L; l++) {
-    const size_t b = lab_off[l] + lab_train[l], e = lab_off[l + 1];
-    if (e <= b) continue;
-    {
-      std::vector<double> ev, pv;
-      for (size_t i = b; i < e; i++) {
-        ev.push_back(double(le[i]));
-        pv.push_back(mlp ? double(lpred[i]) * norms[l].sigma + norms[l].mu : double(lpred[i]));
-      }
-      const Gate g = gate_stats(ev, pv, double(cfg.keep_fraction), double(cfg.gate_top_fraction), tail_q,
-                                double(cfg.gate_z));
-      c->s().gate_z[l] = g.z;
-      c->s().sample_recall[l] = g.recall;
-      need[l] = g.need;
-    }
+  auto host_rmse = [&](size_t l, size_t b, size_t e) {
     double se = 0, sy = 0, sp = 0, syy = 0, spp = 0, syp = 0;
     for (size_t i = b; i < e; i++) {
       const double y = (double(std::min(le[i], norms[l].clip)) - norms[l].mu) / norms[l].sigma;
@@ -1457,6 +1469,29 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     // residual of the best increasing affine map of the scores onto the
     // targets: the error that matters for a ranking
     c->s().val_rmse_cal[l] = float(std::sqrt(vp > 0 && cv > 0 ? std::max(0.0, vy - cv * cv / vp) : vy));
+  };
+  for (size_t l = 0; l < L; l++) {
+    const size_t b = lab_off[l] + lab_train[l], e = lab_off[l + 1];
+    if (e <= b) continue;
+    if (gate_on_device) {
+      c->s().gate_z[l] = stats[l].z;
+      c->s().sample_recall[l] = stats[l].recall;
+      c->s().val_rmse[l] = stats[l].rmse;
+      c->s().val_rmse_cal[l] = stats[l].rmse_cal;
+      need[l] = stats[l].need;
+    } else {
+      std::vector<double> ev, pv;
+      for (size_t i = b; i < e; i++) {
+        ev.push_back(double(le[i]));
+        pv.push_back(mlp ? double(lpred[i]) * norms[l].sigma + norms[l].mu : double(lpred[i]));
+      }
+      const Gate g = gate_stats(ev, pv, double(cfg.keep_fraction), double(cfg.gate_top_fraction), tail_q,
+                                double(cfg.gate_z));
+      c->s().gate_z[l] = g.z;
+      c->s().sample_recall[l] = g.recall;
+      need[l] = g.need;
+      host_rmse(l, b, e);
+    }
     // short of the gate at keep_fraction: widened to the fraction that
     // reaches it (with a 5 % margin) if that is within widen_max
     bool fb = !(c->s().val_rmse_cal[l] <= cfg.max_val_rmse);
