@@ -123,9 +123,9 @@ struct Workspace {
   int splits[3] = {1, 1, 1};
   unsigned slices = 0;
   // per-step state in device memory (step count, learning rates, Adam bias
-  // corrections) and the step's batch indices, so that one captured step
-  // replays as every step
-  DeviceBuffer state, idx;
+  // corrections), so that one captured step replays as every step; the
+  // training points and labels in batch order
+  DeviceBuffer state, opoints, olabels;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   Workspace() = default;
@@ -142,7 +142,7 @@ struct Workspace {
 int reserve(const Net &net, Workspace &ws, size_t batch, size_t nval);
 
 // Training runs as one captured hipGraph of a whole step (the fused step
-// kernel, which reads its batch through the epoch's permutation, then one
+// kernel, which reads its batch at the step count, then one
 // Adam launch over the weights and the grid) replayed `steps` times (every per-step value is computed on the device
 // from the step count), or, with BUDE_MI355X_TRAIN_GRAPH=0 in the
 // environment, as the same kernels launched step by step; both give the

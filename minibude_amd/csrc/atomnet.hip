@@ -471,46 +471,41 @@ __global__ __launch_bounds__(256, 3) void score_kernel(const ScoreArgs a, int64_
 }
 
 // ---- fused training step ------------------------------------------------------
-// One launch does a training step's forward, loss and backward: one wave per
-// 64 points of the batch (lane = point while the point's own data are
-// formed, then the MFMA lane layout of the scorer), kStepWaves waves per
-// work-group.
-//   forward   phi from the FP32 grid (trilinear), layer 0 on MFMA over
-//             K = k0 ([phi, one-hot slot]), ReLU, layer 1 on MFMA with layer
-//             0's accumulators as its B operand (W1^T's K order permuted as
-//             in the scorer), ReLU, y = a1 . W2[:, 0] + b2 (VALU dot over the
-//             lane's neurons, summed over the four lane groups), loss
-//             gradient dz3 = bf16(2 (y - t) / batch).
+// One launch does a training step's forward, loss and backward for groups of
+// 64 points, two groups to a work-group of eight waves (a batch of 32,768
+// points is one work-group per CU).  The step is a chain of dependent stages,
+// each short: the split gives every stage all eight waves.
+//   gather    four lanes per point: two of the eight features each, phi from
+//             the FP32 grid (trilinear, corners in order)
+//   per wave, 16 points (one MFMA block), registers only:
+//   forward   layer 0 on MFMA over K = k0 ([phi, one-hot slot]), ReLU, layer
+//             1 on MFMA with layer 0's accumulators as its B operand (W1^T's
+//             K order permuted as in the scorer), ReLU, y = a1 . W2[:, 0] +
+//             b2 (VALU dot over the lane's neurons, summed over the four lane
+//             groups), loss gradient dz3 = bf16(2 (y - t) / batch).
 //   backward  dz1 = bf16(dz3 W2 * relu'(z1)) elementwise; dz0 =
 //             bf16((dz1 W1^T) * relu'(z0)) on MFMA with dz1 from registers
 //             (W1's K order permuted likewise); dL/dphi = dz0 W0[0..kF)^T on
-//             MFMA; weight and bias gradients X^T dZ as MFMAs over the
-//             wave's 64 points from LDS tiles written transposed (bias
-//             gradients against an all-ones A row); the grid gradient
-//             scattered to the 8 corners in 2^-40 fixed point by 64-bit
-//             integer atomics, one point per instruction (lane = (corner,
-//             feature)).
-// The work-group then sums its waves' gradients in wave order into its own
-// slice of gw / gb, which the Adam step sums in a fixed order: the step is
-// deterministic.  BF16 rounding sits where the layer-by-layer
+//             MFMA; activations and dz written transposed into LDS
+//   then, behind the only barrier of the backward:
+//   scatter   the grid gradient to the 8 corners in 2^-40 fixed point by
+//             64-bit integer atomics, one point per instruction (lane =
+//             (corner, feature)), 16 points per wave; nothing waits for them
+//   weights   gradients X^T dZ as MFMAs over a group's 64 points, 16 x 16
+//             tiles dealt to the waves (bias gradients against an all-ones A
+//             row); a wave adds its tile of the two groups and stores it to
+//             the work-group's slice of gw / gb, which the Adam step sums in
+//             a fixed order: the step is deterministic.
+// 32,768 points: 29.3 us with a wave of its own for each group (two waves on a
+// CU, every stage a chain over 64 points), 23.4 us; 13.6 without the atomics,
+// whose lines move between the XCDs.  BF16 rounding sits where the layer-by-layer
 // kernels put it (inputs, weights, activations, dz), so the oracle of those
 // kernels is the oracle of this one.
 constexpr int kTP = 64 + 8;  // bf16 pitch of a transposed [row][64 points] tile (padding staggers banks)
-// Waves (of 64 points) per work-group of the fused step: a batch of 32,768
-// points is then 256 work-groups, one per CU.
-constexpr int kStepWaves = 2;
+constexpr int kStepGroups = 2;                // groups of 64 points per work-group of the fused step
+constexpr int kStepWaves = 4 * kStepGroups;   // a wave per 16 points
 
-struct alignas(16) StepRow {
-  uint4 phi;  // BF16 features of the point
-  int node;   // grid node of the cell's lower corner
-  float fx, fy, fz;
-  int slot;
-  float yt;   // standardised target
-  float dz3;  // loss gradient (BF16 value)
-  int pad;
-};
-
-// The B operand of point block i from per-neuron values held as the
+// The B operand of a point block from per-neuron values held as the
 // accumulators of the two 16-neuron blocks (the permuted K order).
 __device__ __forceinline__ bf16x8 acc_operand(const floatx4 &v0, const floatx4 &v1) {
   return __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(v0[0], v0[1]), pack_bf16(v0[2], v0[3]),
@@ -520,18 +515,15 @@ __device__ __forceinline__ bf16x8 acc_operand(const floatx4 &v0, const floatx4 &
 __device__ __forceinline__ float bf16_round(float x) { return lo_bf16(pack_bf16(x, 0.f)); }
 
 struct StepArgs {
+  // rows of the launch: with state set, row r of step s (the count in state)
+  // is point (s mod per_epoch) n + r, and the launch also writes the step's
+  // learning rates and bias corrections (sched) into state for the Adam
+  // launch after it; else point r
   const float4 *points;
-  // batch rows -> points: with perm set, row r of step s (the count in
-  // state) is point perm[(s mod per_epoch) n + r], and the launch also
-  // writes the step's learning rates and bias corrections (sched) into
-  // state for the Adam kernels after it; else through idx, if set; else
-  // rows are points
-  const uint32_t *perm;
+  const float *labels;    // exact one-atom energy of every point
   uint32_t per_epoch;
   mlp::StepState *state;
   mlp::Schedule sched;
-  const uint32_t *idx;
-  const float *labels;    // exact one-atom energy of every point
   size_t n;               // rows in this launch (a multiple of 64)
   const float *grid;      // FP32 grid features [nodes][kF]
   field::Grid g;
@@ -549,382 +541,279 @@ struct StepArgs {
 };
 
 template <int K0S>
-__global__ __launch_bounds__(64 * kStepWaves, 2) void step_kernel(const StepArgs a) {
+__global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a) {
   constexpr int K0 = 32 * K0S;
-  constexpr int NP = K0 * kH + kH * kH + 3 * kH + 1;  // a wave's partial gradients (dW2, db2: column 0)
   constexpr int NT = 64 * kStepWaves;
-  __shared__ StepRow rows[kStepWaves][64];
-  __shared__ __align__(16) float dphi[kStepWaves][64 * kF];
-  __shared__ __align__(16) bf16 tt[kStepWaves][64 * kTP + kH * kTP];  // transposed tiles; the wave partials at the end
-  static_assert(sizeof(tt) >= kStepWaves * NP * sizeof(float), "reduction buffer");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, grp = lane >> 4;
-  const size_t tile = size_t(blockIdx.x) * kStepWaves + wave;
-  const bool active = tile * 64 < a.n;
-  if (a.perm && blockIdx.x == 0 && tid == 0) mlp::schedule_hyper(a.sched, a.state->step, a.state->hyper);
-  StepRow *R = rows[wave];
-  bf16 *U = tt[wave];
-  const bf16x8 zero8 = bf16x8{};
-  float sq = 0.f;
-  // this wave's partial gradients, in MFMA output layouts
-  floatx4 gW0[K0 / 16][2], gW1[2][2], gW2[2], gB0[2], gB1[2];
-  float gB2 = 0.f;
+  // per group: X0T [K0], A0T, A1T, DZ1T, DZ0T [kH each], rows of 64 points
+  constexpr int kA0 = K0, kA1 = kA0 + kH, kZ1 = kA1 + kH, kZ0 = kZ1 + kH, kRows = kZ0 + kH;
+  __shared__ __align__(16) bf16 tt[kStepGroups][kRows * kTP];
+  __shared__ __align__(16) uint32_t phis[kStepGroups * 64][kF / 2];  // BF16 features of each point
+  __shared__ int4 cells[kStepGroups * 64];                            // lower corner node, fx, fy, fz (bits)
+  __shared__ int slots[kStepGroups * 64];
+  __shared__ float yts[kStepGroups * 64];   // standardised target
+  __shared__ float dz3s[kStepGroups * 64];  // loss gradient (BF16 value)
+  __shared__ float sqs[kStepGroups * 64];   // squared error
+  __shared__ __align__(16) float dphi[kStepGroups * 64 * kF];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave >> 2, blk = wave & 3;  // this wave's 16 points: block blk of its group
+  const size_t row0 = size_t(blockIdx.x) * (64 * kStepGroups);
+  const bool active = row0 + 64 * group < a.n;  // (uniform over the group's waves)
+  if (a.state && blockIdx.x == 0 && tid == 0) mlp::schedule_hyper(a.sched, a.state->step, a.state->hyper);
+  const int s1 = a.g.n[2], s0 = a.g.n[1] * a.g.n[2];
+  // ---- the points: four lanes each, features 2 f and 2 f + 1
+  const int pt = tid >> 2, f = tid & 3;
+  float4 p{};
+  float e = 0.f;
+  if (active) {
+    const size_t q = (a.state ? size_t(a.state->step % a.per_epoch) * a.n : size_t(0)) + row0 + size_t(pt);
+    p = a.points[q];
+    e = a.labels[q];
+  }
+  // the weights of this lane's MFMA operands, in flight with the points
+  bf16x8 fw0[2][K0S], fw1[2], fwb[2], fwp = bf16x8{};
+  float w2[2][4];
+  floatx4 bias0[2], bias1[2];
 #pragma unroll
-  for (int b = 0; b < 2; b++) {
+  for (int jn = 0; jn < 2; jn++) {
 #pragma unroll
-    for (int kb = 0; kb < K0 / 16; kb++) gW0[kb][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    gW1[0][b] = gW1[1][b] = gW2[b] = gB0[b] = gB1[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < K0S; s++)
+      fw0[jn][s] = *reinterpret_cast<const bf16x8 *>(a.w0t + size_t(16 * jn + r) * K0 + 32 * s + 8 * grp);
+    fw1[jn] = perm_row(a.w1t + size_t(16 * jn + r) * kH, grp);
+    const float4 v0 = *reinterpret_cast<const float4 *>(a.b0 + 16 * jn + 4 * grp);
+    const float4 v1 = *reinterpret_cast<const float4 *>(a.b1 + 16 * jn + 4 * grp);
+    bias0[jn] = floatx4{v0.x, v0.y, v0.z, v0.w};
+    bias1[jn] = floatx4{v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+    for (int c = 0; c < 4; c++) w2[jn][c] = lo_bf16(uint32_t(a.w2[size_t(16 * jn + 4 * grp + c) * kOut]));
+  }
+  const float b2 = a.b2[0];
+  if (a.backward) {
+#pragma unroll
+    for (int ji = 0; ji < 2; ji++) fwb[ji] = perm_row(a.w1 + size_t(16 * ji + r) * kH, grp);
+    if (r < kF) fwp = perm_row(a.w0 + size_t(r) * kH, grp);  // W0 rows 0..kF-1; rows kF..15 zero
+    // X0T's one-hot rows, cleared
+    for (int g = 0; g < kStepGroups; g++) {
+      uint4 *z = reinterpret_cast<uint4 *>(&tt[g][kF * kTP]);
+      for (int t = tid; t < (K0 - kF) * kTP / 8; t += NT) z[t] = make_uint4(0u, 0u, 0u, 0u);
+    }
   }
   if (active) {
     const float inv_h = 1.0f / a.g.h;
-    const int s1 = a.g.n[2], s0 = a.g.n[1] * a.g.n[2];
-    // ---- the point of this lane: features, target
-    {
-      const size_t row = tile * 64 + lane;
-      const uint32_t q = a.perm ? a.perm[size_t(a.state->step % a.per_epoch) * a.n + row]
-                                : (a.idx ? a.idx[row] : uint32_t(row));
-      const float4 p = a.points[q];
-      const float e = a.labels[q];
-      int ix, iy, iz;
-      float fx, fy, fz;
-      cell(p.x, a.g.lo[0], inv_h, a.g.n[0], ix, fx);
-      cell(p.y, a.g.lo[1], inv_h, a.g.n[1], iy, fy);
-      cell(p.z, a.g.lo[2], inv_h, a.g.n[2], iz, fz);
-      const int node = ix * s0 + iy * s1 + iz;
-      const float gx[2] = {1.f - fx, fx}, gy[2] = {1.f - fy, fy}, gz[2] = {1.f - fz, fz};
-      float phi[kF];
+    int ix, iy, iz;
+    float fx, fy, fz;
+    cell(p.x, a.g.lo[0], inv_h, a.g.n[0], ix, fx);
+    cell(p.y, a.g.lo[1], inv_h, a.g.n[1], iy, fy);
+    cell(p.z, a.g.lo[2], inv_h, a.g.n[2], iz, fz);
+    const int node = ix * s0 + iy * s1 + iz;
+    const float gx[2] = {1.f - fx, fx}, gy[2] = {1.f - fy, fy}, gz[2] = {1.f - fz, fz};
+    float2 u[8];
 #pragma unroll
-      for (int k = 0; k < kF; k++) phi[k] = 0.f;
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int dx = (c >> 2) & 1, dy = (c >> 1) & 1, dz = c & 1;
-        const float w = gx[dx] * gy[dy] * gz[dz];
-        const float4 *v = reinterpret_cast<const float4 *>(a.grid + size_t(node + dx * s0 + dy * s1 + dz) * kF);
-        const float4 u0 = v[0], u1 = v[1];
-        phi[0] = __builtin_fmaf(w, u0.x, phi[0]);
-        phi[1] = __builtin_fmaf(w, u0.y, phi[1]);
-        phi[2] = __builtin_fmaf(w, u0.z, phi[2]);
-        phi[3] = __builtin_fmaf(w, u0.w, phi[3]);
-        phi[4] = __builtin_fmaf(w, u1.x, phi[4]);
-        phi[5] = __builtin_fmaf(w, u1.y, phi[5]);
-        phi[6] = __builtin_fmaf(w, u1.z, phi[6]);
-        phi[7] = __builtin_fmaf(w, u1.w, phi[7]);
-      }
-      StepRow row_{};
-      row_.phi = make_uint4(pack_bf16(phi[0], phi[1]), pack_bf16(phi[2], phi[3]), pack_bf16(phi[4], phi[5]),
-                            pack_bf16(phi[6], phi[7]));
-      row_.node = node;
-      row_.fx = fx;
-      row_.fy = fy;
-      row_.fz = fz;
-      row_.slot = __float_as_int(p.w);
-      row_.yt = (fminf(e, a.norm.clip) - a.norm.mu) * a.norm.inv_sigma;
-      R[lane] = row_;
+    for (int c = 0; c < 8; c++) {
+      const int corner = node + (c >> 2) * s0 + ((c >> 1) & 1) * s1 + (c & 1);
+      u[c] = *reinterpret_cast<const float2 *>(a.grid + size_t(corner) * kF + 2 * f);
     }
-    wave_sync();
-    // ---- layer 0: [phi, one-hot] (B, from the rows) x W0^T (A, from L2)
-    floatx4 z0[2][4];
-    {
-      bf16x8 fw0[2][K0S];
+    float phi0 = 0.f, phi1 = 0.f;
 #pragma unroll
-      for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-        for (int s = 0; s < K0S; s++)
-          fw0[jn][s] = *reinterpret_cast<const bf16x8 *>(a.w0t + size_t(16 * jn + r) * K0 + 32 * s + 8 * grp);
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++) {
-        const float4 b = *reinterpret_cast<const float4 *>(a.b0 + 16 * jn + 4 * grp);
-#pragma unroll
-        for (int i = 0; i < 4; i++) z0[jn][i] = floatx4{b.x, b.y, b.z, b.w};
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const StepRow &pr = R[16 * i + r];
-        const uint4 ph = pr.phi;
-        const int slot = pr.slot;
-#pragma unroll
-        for (int s = 0; s < K0S; s++) {
-          // the one-hot column kF + slot, if it falls in this lane's 8 columns
-          const int e = kF + slot - (32 * s + 8 * grp);
-          const uint32_t one = (e >= 0 && e < 8) ? (0x3f80u << (16 * (e & 1))) : 0u;
-          const int wsel = e >> 1;
-          uint4 v = make_uint4(wsel == 0 ? one : 0u, wsel == 1 ? one : 0u, wsel == 2 ? one : 0u, wsel == 3 ? one : 0u);
-          if (s == 0 && grp == 0) v = ph;  // (columns 0..7: the features; the slot column is >= kF)
-          const bf16x8 fb = __builtin_bit_cast(bf16x8, v);
-#pragma unroll
-          for (int jn = 0; jn < 2; jn++) z0[jn][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw0[jn][s], fb, z0[jn][i], 0, 0, 0);
-        }
-      }
+    for (int c = 0; c < 8; c++) {
+      const float w = gx[c >> 2] * gy[(c >> 1) & 1] * gz[c & 1];
+      phi0 = __builtin_fmaf(w, u[c].x, phi0);
+      phi1 = __builtin_fmaf(w, u[c].y, phi1);
     }
-    // ReLU masks (bit (jn * 4 + i) * 4 + c) and the BF16 activations
-    uint32_t m0 = 0, m1 = 0;
-    floatx4 a0[2][4];
+    phis[pt][f] = pack_bf16(phi0, phi1);
+    if (f == 0) {
+      cells[pt] = make_int4(node, __float_as_int(fx), __float_as_int(fy), __float_as_int(fz));
+      slots[pt] = __float_as_int(p.w);
+      yts[pt] = (fminf(e, a.norm.clip) - a.norm.mu) * a.norm.inv_sigma;
+    }
+  }
+  __syncthreads();
+  bf16 *U = tt[group];
+  const int q16 = 64 * group + 16 * blk;  // the wave's first point in the work-group
+  const int pc = 16 * blk + r;            // this lane's column of the transposed tiles
+  if (active) {
+    // ---- layer 0: [phi, one-hot] (B) x W0^T (A)
+    const uint4 ph = *reinterpret_cast<const uint4 *>(phis[q16 + r]);
+    const int slot = slots[q16 + r];
+    floatx4 z0[2] = {bias0[0], bias0[1]};
+#pragma unroll
+    for (int s = 0; s < K0S; s++) {
+      // the one-hot column kF + slot, if it falls in this lane's 8 columns
+      const int h = kF + slot - (32 * s + 8 * grp);
+      const uint32_t one = (h >= 0 && h < 8) ? (0x3f80u << (16 * (h & 1))) : 0u;
+      const int wsel = h >> 1;
+      uint4 v = make_uint4(wsel == 0 ? one : 0u, wsel == 1 ? one : 0u, wsel == 2 ? one : 0u, wsel == 3 ? one : 0u);
+      if (s == 0 && grp == 0) v = ph;  // (columns 0..7: the features; the slot column is >= kF)
+      const bf16x8 fb = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+      for (int jn = 0; jn < 2; jn++) z0[jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw0[jn][s], fb, z0[jn], 0, 0, 0);
+    }
+    floatx4 a0[2], a1[2];  // ReLU, BF16 values
 #pragma unroll
     for (int jn = 0; jn < 2; jn++)
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const float z = z0[jn][i][c];
-          m0 |= uint32_t(z > 0.f) << ((jn * 4 + i) * 4 + c);
-          a0[jn][i][c] = bf16_round(z > 0.f ? z : 0.f);
-        }
+      for (int c = 0; c < 4; c++) a0[jn][c] = bf16_round(z0[jn][c] > 0.f ? z0[jn][c] : 0.f);
     // ---- layer 1
-    floatx4 a1[2][4];
+    floatx4 z1[2];
     {
-      bf16x8 fw1[2];
+      const bf16x8 fb = acc_operand(a0[0], a0[1]);
 #pragma unroll
-      for (int jn = 0; jn < 2; jn++) fw1[jn] = perm_row(a.w1t + size_t(16 * jn + r) * kH, grp);
-      floatx4 z1[2][4];
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++) {
-        const float4 b = *reinterpret_cast<const float4 *>(a.b1 + 16 * jn + 4 * grp);
-#pragma unroll
-        for (int i = 0; i < 4; i++) z1[jn][i] = floatx4{b.x, b.y, b.z, b.w};
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const bf16x8 fb = acc_operand(a0[0][i], a0[1][i]);
-#pragma unroll
-        for (int jn = 0; jn < 2; jn++) z1[jn][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw1[jn], fb, z1[jn][i], 0, 0, 0);
-      }
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const float z = z1[jn][i][c];
-            m1 |= uint32_t(z > 0.f) << ((jn * 4 + i) * 4 + c);
-            a1[jn][i][c] = bf16_round(z > 0.f ? z : 0.f);
-          }
+      for (int jn = 0; jn < 2; jn++) z1[jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw1[jn], fb, bias1[jn], 0, 0, 0);
     }
-    // ---- output, loss gradient
-    float w2[2][4];
 #pragma unroll
     for (int jn = 0; jn < 2; jn++)
 #pragma unroll
-      for (int c = 0; c < 4; c++) w2[jn][c] = lo_bf16(uint32_t(a.w2[size_t(16 * jn + 4 * grp + c) * kOut]));
-    const float b2 = a.b2[0];
-    float dz3[4];
+      for (int c = 0; c < 4; c++) a1[jn][c] = bf16_round(z1[jn][c] > 0.f ? z1[jn][c] : 0.f);
+    // ---- output, loss gradient
+    float y = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      float part = 0.f;
+    for (int jn = 0; jn < 2; jn++)
 #pragma unroll
-      for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) part = __builtin_fmaf(a1[jn][i][c], w2[jn][c], part);
-      part += __shfl_xor(part, 16);
-      part += __shfl_xor(part, 32);
-      const float y = part + b2;
-      const float d = y - R[16 * i + r].yt;
-      if (grp == i) {
-        sq += d * d;
-        if (a.pred) a.pred[tile * 64 + 16 * i + r] = y;
-      }
-      dz3[i] = bf16_round(a.grad_scale * d);
+      for (int c = 0; c < 4; c++) y = __builtin_fmaf(a1[jn][c], w2[jn][c], y);
+    y += __shfl_xor(y, 16);
+    y += __shfl_xor(y, 32);
+    y += b2;
+    const float d = y - yts[q16 + r];
+    const float dz3 = bf16_round(a.grad_scale * d);
+    if (grp == 0) {
+      if (a.pred) a.pred[row0 + size_t(q16 + r)] = y;
+      sqs[q16 + r] = d * d;
+      dz3s[q16 + r] = dz3;
     }
     if (a.backward) {
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        if (grp == i) R[16 * i + r].dz3 = dz3[i];
-      // transposed activations: A0T [n][p] at U, A1T at U + kH kTP
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const int n = 16 * jn + 4 * grp + c, p = 16 * i + r;
-            U[n * kTP + p] = bf16(pack_bf16(a0[jn][i][c], 0.f));
-            U[(kH + n) * kTP + p] = bf16(pack_bf16(a1[jn][i][c], 0.f));
-          }
       // dz1 = dz3 W2 * relu'(z1), exact product then BF16
-      floatx4 dz1[2][4];
+      floatx4 dz1[2], dz0[2];
 #pragma unroll
       for (int jn = 0; jn < 2; jn++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int c = 0; c < 4; c++)
-            dz1[jn][i][c] = ((m1 >> ((jn * 4 + i) * 4 + c)) & 1u) ? bf16_round(dz3[i] * w2[jn][c]) : 0.f;
-      wave_sync();
-      // dW2 = A1T . dz3 (column 0), db2
-      const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
-      const bf16x8 onesA = r == 0 ? ones : zero8;
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        uint32_t dv[4] = {0u, 0u, 0u, 0u};
-        if (r == 0)
-#pragma unroll
-          for (int h = 0; h < 4; h++)
-            dv[h] = pack_bf16(R[32 * s + 8 * grp + 2 * h].dz3, R[32 * s + 8 * grp + 2 * h + 1].dz3);
-        const bf16x8 fb = __builtin_bit_cast(bf16x8, make_uint4(dv[0], dv[1], dv[2], dv[3]));
-#pragma unroll
-        for (int jn = 0; jn < 2; jn++) {
-          const bf16x8 fa = lds8(U + (kH + 16 * jn + r) * kTP + 32 * s + 8 * grp);
-          gW2[jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, gW2[jn], 0, 0, 0);
-        }
-      }
-      {
-        float v = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) v += grp == i ? dz3[i] : 0.f;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off);
-        gB2 = v;
-      }
-      wave_sync();
-      // DZ1T [n][p] over A1T
-#pragma unroll
-      for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int c = 0; c < 4; c++)
-            U[(kH + 16 * jn + 4 * grp + c) * kTP + 16 * i + r] = bf16(pack_bf16(dz1[jn][i][c], 0.f));
-      wave_sync();
-      // dW1 = A0T . DZ1T^T, db1 = ones . DZ1T^T
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        bf16x8 fa[2], fb[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          fa[j] = lds8(U + (16 * j + r) * kTP + 32 * s + 8 * grp);
-          fb[j] = lds8(U + (kH + 16 * j + r) * kTP + 32 * s + 8 * grp);
-        }
-#pragma unroll
-        for (int jo = 0; jo < 2; jo++) {
-#pragma unroll
-          for (int ji = 0; ji < 2; ji++) gW1[ji][jo] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ji], fb[jo], gW1[ji][jo], 0, 0, 0);
-          gB1[jo] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(onesA, fb[jo], gB1[jo], 0, 0, 0);
-        }
-      }
+        for (int c = 0; c < 4; c++) dz1[jn][c] = z1[jn][c] > 0.f ? bf16_round(dz3 * w2[jn][c]) : 0.f;
       // dz0 = (dz1 W1^T) * relu'(z0): A = W1 rows (K permuted), B = dz1 from registers
-      floatx4 dz0[2][4];
       {
-        bf16x8 fw[2];
+        const bf16x8 fb = acc_operand(dz1[0], dz1[1]);
 #pragma unroll
-        for (int ji = 0; ji < 2; ji++) fw[ji] = perm_row(a.w1 + size_t(16 * ji + r) * kH, grp);
+        for (int ji = 0; ji < 2; ji++) {
+          const floatx4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwb[ji], fb, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const bf16x8 fb = acc_operand(dz1[0][i], dz1[1][i]);
-#pragma unroll
-          for (int ji = 0; ji < 2; ji++) {
-            const floatx4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[ji], fb, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < 4; c++) dz0[ji][i][c] = ((m0 >> ((ji * 4 + i) * 4 + c)) & 1u) ? bf16_round(v[c]) : 0.f;
-          }
+          for (int c = 0; c < 4; c++) dz0[ji][c] = z0[ji][c] > 0.f ? bf16_round(v[c]) : 0.f;
         }
       }
       // dL/dphi = dz0 W0[0..kF)^T: A = W0 rows 0..kF-1 (K permuted), rows kF..15 zero
-      {
-        const bf16x8 fw = r < kF ? perm_row(a.w0 + size_t(r) * kH, grp) : zero8;
+      const floatx4 dp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwp, acc_operand(dz0[0], dz0[1]),
+                                                                 floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      if (grp < 2) *reinterpret_cast<float4 *>(&dphi[(q16 + r) * kF + 4 * grp]) = make_float4(dp[0], dp[1], dp[2], dp[3]);
+      // the transposed tiles
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const floatx4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw, acc_operand(dz0[0][i], dz0[1][i]),
-                                                                    floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          if (grp < 2) *reinterpret_cast<float4 *>(&dphi[wave][(16 * i + r) * kF + 4 * grp]) = make_float4(v[0], v[1], v[2], v[3]);
+      for (int jn = 0; jn < 2; jn++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          bf16 *t = U + (16 * jn + 4 * grp + c) * kTP + pc;
+          t[kA0 * kTP] = bf16(pack_bf16(a0[jn][c], 0.f));
+          t[kA1 * kTP] = bf16(pack_bf16(a1[jn][c], 0.f));
+          t[kZ1 * kTP] = bf16(pack_bf16(dz1[jn][c], 0.f));
+          t[kZ0 * kTP] = bf16(pack_bf16(dz0[jn][c], 0.f));
         }
-      }
-      wave_sync();
-      // X0T [k][p] (k < k0) at U, DZ0T [n][p] at U + 64 kTP
-      {
-        uint4 *z = reinterpret_cast<uint4 *>(U);
-        for (int t = lane; t < K0 * kTP / 8; t += 64) z[t] = make_uint4(0u, 0u, 0u, 0u);
-        const uint4 ph = R[lane].phi;
-        const uint32_t pw[4] = {ph.x, ph.y, ph.z, ph.w};
-#pragma unroll
-        for (int k = 0; k < kF; k++) U[k * kTP + lane] = bf16((pw[k >> 1] >> (16 * (k & 1))) & 0xffffu);
-        U[(kF + R[lane].slot) * kTP + lane] = bf16(0x3f80);
-#pragma unroll
-        for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-              U[(64 + 16 * jn + 4 * grp + c) * kTP + 16 * i + r] = bf16(pack_bf16(dz0[jn][i][c], 0.f));
-      }
-      wave_sync();
-      // dW0 = X0T . DZ0T^T, db0 = ones . DZ0T^T
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        bf16x8 fb[2];
-#pragma unroll
-        for (int jn = 0; jn < 2; jn++) fb[jn] = lds8(U + (64 + 16 * jn + r) * kTP + 32 * s + 8 * grp);
-#pragma unroll
-        for (int kb = 0; kb < K0 / 16; kb++) {
-          const bf16x8 fa = lds8(U + (16 * kb + r) * kTP + 32 * s + 8 * grp);
-#pragma unroll
-          for (int jn = 0; jn < 2; jn++) gW0[kb][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb[jn], gW0[kb][jn], 0, 0, 0);
-        }
-#pragma unroll
-        for (int jn = 0; jn < 2; jn++) gB0[jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(onesA, fb[jn], gB0[jn], 0, 0, 0);
-      }
-      // grid gradient: one point per instruction, lane = (corner, feature)
-      {
-        const int cq = lane >> 3, k = lane & 7;
-        const int dx = cq >> 2, dy = (cq >> 1) & 1, dz = cq & 1;
-        const int off = dx * s0 + dy * s1 + dz;
-        for (int pt = 0; pt < 64; pt++) {
-          const StepRow &pr = R[pt];
-          const float w = (dx ? pr.fx : 1.f - pr.fx) * (dy ? pr.fy : 1.f - pr.fy) * (dz ? pr.fz : 1.f - pr.fz);
-          const long long v = llrint(double(w * dphi[wave][pt * kF + k]) * kGradScale);
-          atomicAdd(a.gacc + size_t(pr.node + off) * kF + k, static_cast<unsigned long long>(v));
-        }
-      }
+      const uint32_t pw = grp == 0 ? ph.x : (grp == 1 ? ph.y : (grp == 2 ? ph.z : ph.w));
+      U[(2 * grp) * kTP + pc] = bf16(pw & 0xffffu);
+      U[(2 * grp + 1) * kTP + pc] = bf16(pw >> 16);
+      if (grp == 0) U[(kF + slot) * kTP + pc] = bf16(0x3f80);
     }
   }
-  // squared error of the wave's points (fixed point, as the layer kernels' loss)
-  for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off);
-  if (lane == 0 && active && a.loss)
-    atomicAdd(a.loss, static_cast<unsigned long long>(fmin(double(sq) * mlp::kLossScale + 0.5, 1099511627776.0)));
-  if (!a.backward) return;  // (uniform over the launch: no barrier below is reached)
-  // ---- the work-group's gradients: each wave's partials to LDS, summed in wave order
+  if (!a.backward) return;  // (uniform over the launch)
   __syncthreads();
-  float *red = reinterpret_cast<float *>(&tt[0][0]);
-  float *P = red + wave * NP;
-  // layout: dW0 [K0][kH], dW1 [kH][kH], dW2 [kH], db0 [kH], db1 [kH], db2
-#pragma unroll
-  for (int kb = 0; kb < K0 / 16; kb++)
-#pragma unroll
-    for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-      for (int c = 0; c < 4; c++) P[(16 * kb + 4 * grp + c) * kH + 16 * jn + r] = gW0[kb][jn][c];
-#pragma unroll
-  for (int ji = 0; ji < 2; ji++)
-#pragma unroll
-    for (int jo = 0; jo < 2; jo++)
-#pragma unroll
-      for (int c = 0; c < 4; c++) P[K0 * kH + (16 * ji + 4 * grp + c) * kH + 16 * jo + r] = gW1[ji][jo][c];
-#pragma unroll
-  for (int jn = 0; jn < 2; jn++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      if (r == 0) P[K0 * kH + kH * kH + 16 * jn + 4 * grp + c] = gW2[jn][c];
-      if (grp == 0 && c == 0) {
-        P[K0 * kH + kH * kH + kH + 16 * jn + r] = gB0[jn][0];
-        P[K0 * kH + kH * kH + 2 * kH + 16 * jn + r] = gB1[jn][0];
-      }
+  // ---- grid gradient: one point per instruction, lane = (corner, feature)
+  if (active) {
+    const int cq = lane >> 3, k = lane & 7;
+    const int dx = cq >> 2, dy = (cq >> 1) & 1, dz = cq & 1;
+    unsigned long long *acc = a.gacc + size_t(dx * s0 + dy * s1 + dz) * kF + k;
+#pragma unroll 4
+    for (int i = 0; i < 16; i++) {
+      const int4 ce = cells[q16 + i];
+      const float fx = __int_as_float(ce.y), fy = __int_as_float(ce.z), fz = __int_as_float(ce.w);
+      const float w = (dx ? fx : 1.f - fx) * (dy ? fy : 1.f - fy) * (dz ? fz : 1.f - fz);
+      const long long v = llrint(double(w * dphi[(q16 + i) * kF + k]) * kGradScale);
+      atomicAdd(acc + size_t(ce.x) * kF, static_cast<unsigned long long>(v));
     }
-  if (lane == 0) P[NP - 1] = gB2;
-  __syncthreads();
+  }
+  // ---- weight and bias gradients: 16 x 16 tiles dealt to the waves, each
+  // over the groups' 64 points and added in group order
+  const bool both = row0 + 64 < a.n;  // the second group has points
+  const bf16x8 zero8 = bf16x8{};
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
   const size_t wg = blockIdx.x;
-  auto wsum = [&](int o) {  // the waves' partials of entry o, in wave order
-    float v = red[o];
+  // the product of two tile rows of the same 64 points, of both groups
+  auto product = [&](auto &&fa, auto &&fb) {
+    floatx4 sum{};
 #pragma unroll
-    for (int w = 1; w < kStepWaves; w++) v += red[w * NP + o];
-    return v;
+    for (int g = 0; g < kStepGroups; g++) {
+      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (g == 0 || both)
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa(g, 32 * s + 8 * grp), fb(g, 32 * s + 8 * grp), acc, 0, 0, 0);
+      sum = g == 0 ? acc : sum + acc;
+    }
+    return sum;
   };
-  for (int t = tid; t < K0 * kH; t += NT) a.gw[0][wg * K0 * kH + t] = wsum(t);
-  for (int t = tid; t < kH * kH; t += NT) a.gw[1][wg * kH * kH + t] = wsum(K0 * kH + t);
-  for (int t = tid; t < kH * kOut; t += NT)  // W2 [kH][kOut]: column 0
-    a.gw[2][wg * kH * kOut + t] = t % kOut ? 0.f : wsum(K0 * kH + kH * kH + t / kOut);
-  if (tid < kH) {
-    const int o0 = K0 * kH + kH * kH + kH + tid, o1 = o0 + kH;
-    a.gb[0][wg * kH + tid] = wsum(o0);
-    a.gb[1][wg * kH + tid] = wsum(o1);
+  auto tile_row = [&](int first) { return [=](int g, int col) { return lds8(&tt[g][(first + r) * kTP + col]); }; };
+  auto ones_row = [&](int, int) { return r == 0 ? ones : zero8; };
+  constexpr int kW0Tiles = K0 / 8, kTiles = kW0Tiles + 10;
+  for (int t = wave; t < kTiles; t += kStepWaves) {
+    if (t < kW0Tiles) {  // dW0 = X0T . DZ0T^T
+      const int kb = t >> 1, jn = t & 1;
+      const floatx4 v = product(tile_row(16 * kb), tile_row(kZ0 + 16 * jn));
+      float *o = a.gw[0] + wg * K0 * kH + size_t(16 * kb + 4 * grp) * kH + 16 * jn + r;
+#pragma unroll
+      for (int c = 0; c < 4; c++) o[c * kH] = v[c];
+    } else if (t < kW0Tiles + 4) {  // dW1 = A0T . DZ1T^T
+      const int ji = (t - kW0Tiles) >> 1, jo = (t - kW0Tiles) & 1;
+      const floatx4 v = product(tile_row(kA0 + 16 * ji), tile_row(kZ1 + 16 * jo));
+      float *o = a.gw[1] + wg * kH * kH + size_t(16 * ji + 4 * grp) * kH + 16 * jo + r;
+#pragma unroll
+      for (int c = 0; c < 4; c++) o[c * kH] = v[c];
+    } else if (t < kW0Tiles + 6) {  // dW2 = A1T . dz3, column 0 of [kH][kOut]
+      const int jn = t - kW0Tiles - 4;
+      const floatx4 v = product(tile_row(kA1 + 16 * jn), [&](int g, int col) {
+        if (r != 0) return zero8;
+        const float *z = &dz3s[64 * g + col];
+        return __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]),
+                                                     pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7])));
+      });
+      float *o = a.gw[2] + wg * kH * kOut + size_t(16 * jn + 4 * grp) * kOut + r;
+#pragma unroll
+      for (int c = 0; c < 4; c++) o[c * kOut] = r ? 0.f : v[c];
+    } else {  // db0 = ones . DZ0T^T, db1 = ones . DZ1T^T
+      const int i = t - kW0Tiles - 6, jn = i & 1;
+      const floatx4 v = product(ones_row, tile_row((i < 2 ? kZ0 : kZ1) + 16 * jn));
+      if (grp == 0) (i < 2 ? a.gb[0] : a.gb[1])[wg * kH + 16 * jn + r] = v[0];
+    }
   }
-  if (tid < kOut) a.gb[2][wg * kOut + tid] = tid ? 0.f : wsum(NP - 1);
+  // db2 and the loss: sums over each group's 64 points, groups in order
+  if (wave == kStepWaves - 1) {
+    float db2 = 0.f;
+    unsigned long long loss = 0;
+    for (int g = 0; g < (both ? kStepGroups : 1); g++) {
+      float v = dz3s[64 * g + lane], sq = sqs[64 * g + lane];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off);
+      for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off);
+      db2 = g == 0 ? v : db2 + v;
+      loss += static_cast<unsigned long long>(fmin(double(sq) * mlp::kLossScale + 0.5, 1099511627776.0));
+    }
+    if (lane < kOut) a.gb[2][wg * kOut + lane] = lane ? 0.f : db2;
+    if (lane == 0 && a.loss) atomicAdd(a.loss, loss);
+  }
+}
+
+// The training points and their labels in the order the batches take them:
+// a step then reads whole lines, with one dependent load less.
+__global__ void order_kernel(const float4 *__restrict__ points, const float *__restrict__ labels,
+                             const uint32_t *__restrict__ perm, size_t n, float4 *__restrict__ out_points,
+                             float *__restrict__ out_labels) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t q = perm[i];
+  out_points[i] = points[q];
+  out_labels[i] = labels[q];
 }
 
 unsigned blocks_for(size_t n, unsigned t) { return unsigned((n + t - 1) / t); }
@@ -933,28 +822,25 @@ uint64_t mix_seed(uint64_t seed, uint64_t k) { return (seed ^ (k * 0xd6e8feb8665
 
 using Acts = Workspace;
 
-// A training run's batch rows (see StepArgs::perm).
+// A training run's batch rows (see StepArgs::points).
 struct StepRows {
-  const uint32_t *perm;
   uint32_t per_epoch;
   mlp::StepState *state;
   mlp::Schedule sched;
 };
 
-// The fused step over rows [0, n) of `points` (through idx, if set):
+// The fused step over rows [0, n) of `points` (a batch of them with `rows`):
 // forward (y into pred, if set; squared error into A.loss), and with
 // `backward` the gradients -- grid into net.gacc, weights and biases as
 // one slice per work-group into A.gpart / bpart (A.splits slices).
-int launch_step(Net &net, Acts &A, const float4 *points, const uint32_t *idx, const float *labels, size_t n,
-                size_t batch, mlp::TargetNorm norm, float *pred, bool backward, hipStream_t s,
+int launch_step(Net &net, Acts &A, const float4 *points, const float *labels, size_t n, size_t batch,
+                mlp::TargetNorm norm, float *pred, bool backward, hipStream_t s,
                 const StepRows *rows = nullptr) {
   if (n == 0 || n % 64) return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet: rows must be a multiple of 64");
   StepArgs a{};
   a.points = points;
-  a.idx = idx;
   if (rows) {
     if (rows->per_epoch == 0) return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet: empty epoch");
-    a.perm = rows->perm;
     a.per_epoch = rows->per_epoch;
     a.state = rows->state;
     a.sched = rows->sched;
@@ -977,7 +863,7 @@ int launch_step(Net &net, Acts &A, const float4 *points, const uint32_t *idx, co
   a.loss = backward ? static_cast<unsigned long long *>(A.loss.ptr) : nullptr;
   a.backward = backward ? 1 : 0;
   a.gacc = static_cast<unsigned long long *>(net.gacc.ptr);
-  const unsigned blocks = blocks_for(n, 64 * kStepWaves);
+  const unsigned blocks = blocks_for(n, 64 * kStepGroups);
   if (backward) {
     if (A.slices < blocks) return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet: workspace sized for fewer rows");
     for (int l = 0; l < 3; l++) {
@@ -1026,7 +912,7 @@ int alloc_zero(DeviceBuffer &d, size_t bytes) {
 }  // namespace
 
 int reserve(const Net &net, Workspace &A, size_t B, size_t nval) {
-  const size_t slices = (B + 64 * kStepWaves - 1) / (64 * kStepWaves);
+  const size_t slices = (B + 64 * kStepGroups - 1) / (64 * kStepGroups);
   if (A.rows >= B && A.k0 == net.k0 && A.vpred.bytes >= std::max<size_t>(nval, 1) * 4) return BUDE_OK;
   A.rows = B;
   A.k0 = net.k0;
@@ -1035,7 +921,6 @@ int reserve(const Net &net, Workspace &A, size_t B, size_t nval) {
   if (!st) st = A.part.reserve(1024 * 2 * 8);
   if (!st) st = A.vpred.reserve(std::max<size_t>(nval, 1) * 4);
   if (!st) st = A.state.reserve(sizeof(mlp::StepState));
-  if (!st) st = A.idx.reserve(B * 4);
   for (int l = 0; l < 3 && !st; l++) {
     const int K = layer_k(net, l), N = layer_n(l);
     st = A.gpart[l].reserve(slices * K * N * 4);
@@ -1162,6 +1047,11 @@ int train(Net &net, Workspace &A, const float4 *points, const float *labels, con
     return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet train: the training points must be whole batches "
                                            "(a multiple of 64) and the held-out points a multiple of 64");
   if (int st = reserve(net, A, B, nval)) return st;
+  if (int st = A.opoints.reserve(ntrain * sizeof(float4))) return st;
+  if (int st = A.olabels.reserve(ntrain * sizeof(float))) return st;
+  hipLaunchKernelGGL(order_kernel, dim3(blocks_for(ntrain, 256)), dim3(256), 0, s, points, labels, perm, ntrain,
+                     static_cast<float4 *>(A.opoints.ptr), static_cast<float *>(A.olabels.ptr));
+  if (int st = hip_check(hipGetLastError(), "atomnet order")) return st;
   // target transform from the training labels
   {
     hipLaunchKernelGGL(stats_kernel, dim3(1024), dim3(256), 0, s, labels, ntrain, static_cast<double *>(A.part.ptr));
@@ -1187,13 +1077,14 @@ int train(Net &net, Workspace &A, const float4 *points, const float *labels, con
   const uint32_t step0 = uint32_t(net.step);
   auto *state = static_cast<mlp::StepState *>(A.state.ptr);
   // one training step, every per-step value taken from the device state:
-  // the fused step reads its rows through the permutation at the step count
-  // and writes the step's learning rates for the two Adam launches, the
-  // grid's Adam advances the count
-  const StepRows rows{perm, uint32_t(ntrain / B), state,
+  // the fused step reads its rows at the step count and writes the step's
+  // learning rates for the Adam launch, which advances the count
+  const StepRows rows{uint32_t(ntrain / B), state,
                       mlp::Schedule{steps, warm, step0, p.lr, p.grid_lr, 0.9f, 0.999f}};
   auto one_step = [&]() -> int {
-    if (int st = launch_step(net, A, points, nullptr, labels, B, B, norm, nullptr, true, s, &rows)) return st;
+    if (int st = launch_step(net, A, static_cast<const float4 *>(A.opoints.ptr),
+                             static_cast<const float *>(A.olabels.ptr), B, B, norm, nullptr, true, s, &rows))
+      return st;
     return adam_step_dev(net, A, state, s);
   };
   if (int st = hip_check(hipMemsetAsync(A.state.ptr, 0, sizeof(mlp::StepState), s), "hipMemsetAsync")) return st;
@@ -1224,7 +1115,7 @@ int train(Net &net, Workspace &A, const float4 *points, const float *labels, con
   double se = 0;
   if (nval) {
     DeviceBuffer &vpred = A.vpred;
-    if (int st = launch_step(net, A, points + ntrain, nullptr, labels + ntrain, nval, B, norm,
+    if (int st = launch_step(net, A, points + ntrain, labels + ntrain, nval, B, norm,
                              static_cast<float *>(vpred.ptr), false, s))
       return st;
     hipLaunchKernelGGL(sq_err_kernel, dim3(256), dim3(256), 0, s, static_cast<const float *>(vpred.ptr),
@@ -1252,8 +1143,7 @@ int forward_backward(Net &net, const float4 *points, const float *target, size_t
   if (int st = reserve(net, A, batch, 0)) return st;
   if (int st = hip_check(hipMemsetAsync(A.loss.ptr, 0, 8, s), "hipMemsetAsync")) return st;
   const mlp::TargetNorm norm{INFINITY, 0.f, 1.f, -INFINITY};
-  if (int st = launch_step(net, A, points, nullptr, target, batch, batch, norm, static_cast<float *>(A.pred.ptr), true,
-                           s))
+  if (int st = launch_step(net, A, points, target, batch, batch, norm, static_cast<float *>(A.pred.ptr), true, s))
     return st;
   // the K slices of the weight and bias gradients, summed in order into net.gw / gb
   for (int l = 0; l < 3; l++) {
