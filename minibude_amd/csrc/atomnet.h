@@ -122,31 +122,15 @@ struct Workspace {
   DeviceBuffer gpart[3], bpart[3];
   int splits[3] = {1, 1, 1};
   unsigned slices = 0;
-  // per-step state in device memory (step count, learning rates, Adam bias
-  // corrections), so that one captured step replays as every step; the
-  // training points and labels in batch order
-  DeviceBuffer state, opoints, olabels;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  Workspace() = default;
-  Workspace(const Workspace &) = delete;
-  Workspace &operator=(const Workspace &) = delete;
-  ~Workspace() { drop_graph(); }
-  void drop_graph() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    exec = nullptr;
-    graph = nullptr;
-  }
+  // the step's learning rates and Adam bias corrections; the training points
+  // and labels in batch order
+  DeviceBuffer hyper, opoints, olabels;
 };
 int reserve(const Net &net, Workspace &ws, size_t batch, size_t nval);
 
-// Training runs as one captured hipGraph of a whole step (the fused step
-// kernel, which reads its batch at the step count, then one
-// Adam launch over the weights and the grid) replayed `steps` times (every per-step value is computed on the device
-// from the step count), or, with BUDE_MI355X_TRAIN_GRAPH=0 in the
-// environment, as the same kernels launched step by step; both give the
-// same network bit for bit.
+// Training launches each step's two kernels (the fused step, which also
+// writes the step's learning rates, then one Adam launch over the weights and
+// the grid) one after the other.
 // Trains on points[0, ntrain) with labels (energy units), validates on
 // points[ntrain, ntrain + nval); sets mu / sigma / clip from the training
 // labels (target y = (min(E, clip) - mu) / sigma, clip = mu + 8 sigma).
