@@ -56,8 +56,8 @@ struct Net {
   // j + dy, l) and of node (i + dx, j + dy, l + 1) -- a cell's 8 corners
   // in one 128-byte record, one packed dot product per pair
   DeviceBuffer g, gm, gv, gacc, gzp;
-  // layers l = 0..2: W_l [K_l][N_l] (FP32 master, Adam moments, gradient,
-  // BF16 row-major and transposed copies), b_l [N_l]
+  // layers l = 0..2: W_l [K_l][N_l] (FP32 master, Adam moments, gradient
+  // [K_l][grad_n(l)], BF16 row-major and transposed copies), b_l [N_l]
   DeviceBuffer w[3], b[3], mw[3], vw[3], mb[3], vb[3], gw[3], gb[3], w16[3], w16t[3];
   // [nslots][kH] first-layer bias of each slot, b0 + W0[kF + s] (FP32):
   // inference starts the layer's MFMA accumulators from it
@@ -70,6 +70,8 @@ struct Net {
 // K and N of layer l.
 inline int layer_k(const Net &n, int l) { return l == 0 ? n.k0 : kH; }
 inline int layer_n(int l) { return l == 2 ? kOut : kH; }
+// Columns of layer l a gradient has: the output layer's one.
+inline int grad_n(int l) { return l == 2 ? 1 : kH; }
 
 // Sizes the network for `grid` and `nslots` (keeping allocations large
 // enough from an earlier call) and initialises it on stream s: grid

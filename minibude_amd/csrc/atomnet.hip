@@ -534,7 +534,7 @@ struct StepArgs {
   unsigned long long *loss;  // optional: fixed-point sum of squared errors (mlp::kLossScale)
   int backward;
   unsigned long long *gacc;  // grid gradient accumulators [nodes][kF]
-  float *gw[3], *gb[3];   // this launch's work-group slices: gw[l] [nwg][K_l][N_l], gb[l] [nwg][N_l]
+  float *gw[3], *gb[3];   // this launch's work-group slices: gw[l] [nwg][K_l][grad_n(l)], gb[l] [nwg][grad_n(l)]
 };
 
 template <int K0S>
@@ -766,7 +766,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
       float *o = a.gw[1] + wg * kH * kH + size_t(16 * ji + 4 * grp) * kH + 16 * jo + r;
 #pragma unroll
       for (int c = 0; c < 4; c++) o[c * kH] = v[c];
-    } else if (t < kW0Tiles + 6) {  // dW2 = A1T . dz3, column 0 of [kH][kOut]
+    } else if (t < kW0Tiles + 6) {  // dW2 = A1T . dz3, column 0
       const int jn = t - kW0Tiles - 4;
       const floatx4 v = product(tile_row(kA1 + 16 * jn), [&](int g, int col) {
         if (r != 0) return zero8;
@@ -774,9 +774,8 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
         return __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(z[0], z[1]), pack_bf16(z[2], z[3]),
                                                      pack_bf16(z[4], z[5]), pack_bf16(z[6], z[7])));
       });
-      float *o = a.gw[2] + wg * kH * kOut + size_t(16 * jn + 4 * grp) * kOut + r;
-#pragma unroll
-      for (int c = 0; c < 4; c++) o[c * kOut] = r ? 0.f : v[c];
+      if (r == 0)
+        *reinterpret_cast<float4 *>(a.gw[2] + wg * kH + 16 * jn + 4 * grp) = make_float4(v[0], v[1], v[2], v[3]);
     } else {  // db0 = ones . DZ0T^T, db1 = ones . DZ1T^T
       const int i = t - kW0Tiles - 6, jn = i & 1;
       const floatx4 v = product(ones_row, tile_row((i < 2 ? kZ0 : kZ1) + 16 * jn));
@@ -795,8 +794,10 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
       db2 = g == 0 ? v : db2 + v;
       loss += static_cast<unsigned long long>(fmin(double(sq) * mlp::kLossScale + 0.5, 1099511627776.0));
     }
-    if (lane < kOut) a.gb[2][wg * kOut + lane] = lane ? 0.f : db2;
-    if (lane == 0 && a.loss) atomicAdd(a.loss, loss);
+    if (lane == 0) {
+      a.gb[2][wg] = db2;
+      if (a.loss) atomicAdd(a.loss, loss);
+    }
   }
 }
 
@@ -881,11 +882,11 @@ int adam_step_dev(Net &net, const Acts &A, const float *hyper, hipStream_t s) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   mlp::AdamBatch ab{};
   for (int l = 0; l < 3; l++) {
-    const int K = layer_k(net, l), N = layer_n(l);
+    const int K = layer_k(net, l), N = grad_n(l);
     ab.t[2 * l] = {static_cast<float *>(net.w[l].ptr), static_cast<const float *>(A.gpart[l].ptr),
                    static_cast<float *>(net.mw[l].ptr), static_cast<float *>(net.vw[l].ptr),
                    static_cast<bf16 *>(net.w16[l].ptr), static_cast<bf16 *>(net.w16t[l].ptr), K, N,
-                   A.splits[l], size_t(K) * N};
+                   A.splits[l], size_t(K) * N, nullptr, nullptr, layer_n(l)};
     ab.t[2 * l + 1] = {static_cast<float *>(net.b[l].ptr), static_cast<const float *>(A.bpart[l].ptr),
                        static_cast<float *>(net.mb[l].ptr), static_cast<float *>(net.vb[l].ptr), nullptr, nullptr, 1,
                        N, A.splits[l], size_t(N)};
@@ -915,7 +916,7 @@ int reserve(const Net &net, Workspace &A, size_t B, size_t nval) {
   if (!st) st = A.vpred.reserve(std::max<size_t>(nval, 1) * 4);
   if (!st) st = A.hyper.reserve(4 * sizeof(float));
   for (int l = 0; l < 3 && !st; l++) {
-    const int K = layer_k(net, l), N = layer_n(l);
+    const int K = layer_k(net, l), N = grad_n(l);
     st = A.gpart[l].reserve(slices * K * N * 4);
     if (!st) st = A.bpart[l].reserve(slices * N * 4);
   }
@@ -1124,7 +1125,7 @@ int forward_backward(Net &net, const float4 *points, const float *target, size_t
     return st;
   // the K slices of the weight and bias gradients, summed in order into net.gw / gb
   for (int l = 0; l < 3; l++) {
-    const size_t K = size_t(layer_k(net, l)), N = size_t(layer_n(l));
+    const size_t K = size_t(layer_k(net, l)), N = size_t(grad_n(l));
     if (int st = hip_check(mlp::sum_slices(static_cast<const float *>(A.gpart[l].ptr), A.splits[l], K * N,
                                            static_cast<float *>(net.gw[l].ptr), s),
                            "atomnet dW"))

@@ -177,7 +177,7 @@ extern "C" int bude_mi355x_atomnet_forward_backward(int device, size_t batch, co
   if (!st)
     st = bude::hip_check(hipMemcpy(grad_grid, dgrid.ptr, net.nodes * kF * 4, hipMemcpyDeviceToHost), "hipMemcpy");
   for (int l = 0; l < 3 && !st; l++) {
-    const int K = layer_k(net, l), N = layer_n(l);
+    const int K = layer_k(net, l), N = grad_n(l);
     std::vector<float> gw(size_t(K) * N), gb(N);
     st = bude::hip_check(hipMemcpy(gw.data(), net.gw[l].ptr, gw.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy");
     if (!st) st = bude::hip_check(hipMemcpy(gb.data(), net.gb[l].ptr, gb.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy");
@@ -186,7 +186,7 @@ extern "C" int bude_mi355x_atomnet_forward_backward(int device, size_t batch, co
       std::copy(gw.begin(), gw.end(), grad_w[l]);
       std::copy(gb.begin(), gb.end(), grad_b[l]);
     } else {
-      for (int r = 0; r < kH; r++) grad_w[2][r] = gw[size_t(r) * kOut];
+      std::copy(gw.begin(), gw.end(), grad_w[2]);
       grad_b[2][0] = gb[0];
     }
   }

@@ -164,10 +164,11 @@ struct AdamTensor {
   const float *g;    // gradient: `splits` slices `stride` floats apart, summed in a fixed order
   float *m, *v;
   bf16 *w16, *w16t;  // optional BF16 copies (row-major and transposed)
-  int rows, cols;    // w is rows x cols row-major
+  int rows, cols;    // w is rows x cols row-major (pitch below), the gradient without gaps
   int splits;        // 0 or 1: g is the gradient itself
   size_t stride;
   bf16 *w16x = nullptr, *w16tx = nullptr;  // optional fragment-tiled BF16 copies of w and w^T (tiled_index)
+  int pitch = 0;     // entries from one row of w, m, v and w16 to the next (0: cols)
 };
 // A tensor whose gradient arrives as a fixed-point sum of integer atomics:
 // g = acc / scale, and the Adam step clears acc.  Its learning rate is

@@ -620,14 +620,15 @@ __global__ __launch_bounds__(64 * W) void adam_multi_kernel(const AdamBatch b, f
 #pragma unroll
   for (int w = 1; w < kAdamWaves; w++) gi += part[w][lane];
   const AdamTensor &T = b.t[t];
-  const float mi = b1 * T.m[i] + (1.f - b1) * gi;
-  const float vi = b2 * T.v[i] + (1.f - b2) * gi * gi;
-  T.m[i] = mi;
-  T.v[i] = vi;
-  const float wi = T.w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-  T.w[i] = wi;
+  const size_t at = T.pitch ? i / T.cols * T.pitch + i % T.cols : i;
+  const float mi = b1 * T.m[at] + (1.f - b1) * gi;
+  const float vi = b2 * T.v[at] + (1.f - b2) * gi * gi;
+  T.m[at] = mi;
+  T.v[at] = vi;
+  const float wi = T.w[at] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+  T.w[at] = wi;
   const bf16 h = to_bf16(wi);
-  if (T.w16) T.w16[i] = h;
+  if (T.w16) T.w16[at] = h;
   if (T.w16t) T.w16t[size_t(i % T.cols) * T.rows + i / T.cols] = h;
   if (T.w16x) T.w16x[tiled_index(i / T.cols, i % T.cols, size_t(T.cols))] = h;
   if (T.w16tx) T.w16tx[tiled_index(i % T.cols, i / T.cols, size_t(T.rows))] = h;
