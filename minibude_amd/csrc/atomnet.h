@@ -104,6 +104,28 @@ struct TrainParams {
   uint64_t seed = 0;
 };
 
+// Where a set of training points lies in a grid, worked out once for all
+// networks on that grid: each row's cell, in the order the batches take the
+// rows, and, where that is affordable, each batch's (node, row) terms node
+// after node, so that a step's grid gradient is gathered by the nodes instead
+// of scattered by the rows.
+struct PointIndex {
+  size_t ntrain = 0, nval = 0, batch = 0, nodes = 0;
+  bool gathered = false;
+  // per row (training rows in batch order, then the held-out points): lower
+  // corner node and fractions (int, float bits x 3); slot
+  DeviceBuffer cells, slots;
+  // gathered: per batch, 8 batch terms (row, trilinear weight bits) and
+  // first[node] .. the terms of node (nodes + 1 entries)
+  DeviceBuffer terms, first;
+};
+// The index of points[perm[i]], i < ntrain, in batches of `batch`, and of
+// points[ntrain + i], i < nval.  The terms are left out
+// (idx.gathered) when their tables would exceed `limit` bytes.
+int index_points(PointIndex &idx, const field::Grid &grid, const float4 *points, const uint32_t *perm, size_t ntrain,
+                 size_t nval, size_t batch, size_t limit, hipStream_t s);
+constexpr size_t kIndexBytes = size_t(4) << 30;
+
 struct TrainReport {
   float val_rmse = 0.f;    // one-atom energy RMSE on the held-out points (energy units)
   float final_loss = 0.f;  // mean squared error over all training steps (standardised units)
@@ -124,21 +146,22 @@ struct Workspace {
   DeviceBuffer gpart[3], bpart[3];
   int splits[3] = {1, 1, 1};
   unsigned slices = 0;
-  // the step's learning rates and Adam bias corrections; the training points
-  // and labels in batch order
-  DeviceBuffer hyper, opoints, olabels;
+  // the step's learning rates and Adam bias corrections; the training labels
+  // in batch order; dL/dphi of a batch's rows
+  DeviceBuffer hyper, olabels, dphi;
 };
 int reserve(const Net &net, Workspace &ws, size_t batch, size_t nval);
 
 // Training launches each step's two kernels (the fused step, which also
 // writes the step's learning rates, then one Adam launch over the weights and
 // the grid) one after the other.
-// Trains on points[0, ntrain) with labels (energy units), validates on
-// points[ntrain, ntrain + nval); sets mu / sigma / clip from the training
+// Trains on points[0, ntrain) with labels (energy units) as idx has them,
+// validates on points[ntrain, ntrain + nval); sets mu / sigma / clip from the training
 // labels (target y = (min(E, clip) - mu) / sigma, clip = mu + 8 sigma).
-// perm: device array of ntrain point indices, read in batches (wrapping).
-int train(Net &net, Workspace &ws, const float4 *points, const float *labels, const uint32_t *perm, size_t ntrain,
-          size_t nval, const TrainParams &p, hipStream_t s, TrainReport *rep);
+// perm: device array of ntrain point indices, read in batches (wrapping), the
+// one idx was made with.
+int train(Net &net, Workspace &ws, const PointIndex &idx, const float *labels, const uint32_t *perm,
+          const TrainParams &p, hipStream_t s, TrainReport *rep);
 
 // One forward + backward pass of the training kernels over `batch` points
 // (multiple of 64) against standardised targets: predictions, loss and the

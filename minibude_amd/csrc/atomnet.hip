@@ -10,6 +10,7 @@
 #include <random>
 #include <vector>
 
+#include "adam.h"
 #include "atomnet.h"
 #include "fasten_core.h"
 
@@ -475,7 +476,8 @@ __global__ __launch_bounds__(256, 3) void score_kernel(const ScoreArgs a, int64_
 // points is one work-group per CU).  The step is a chain of dependent stages,
 // each short: the split gives every stage all eight waves.
 //   gather    four lanes per point: two of the eight features each, phi from
-//             the FP32 grid (trilinear, corners in order)
+//             the FP32 grid (trilinear, corners in order) at the row's cell
+//             (PointIndex)
 //   per wave, 16 points (one MFMA block), registers only:
 //   forward   layer 0 on MFMA over K = k0 ([phi, one-hot slot]), ReLU, layer
 //             1 on MFMA with layer 0's accumulators as its B operand (W1^T's
@@ -487,9 +489,12 @@ __global__ __launch_bounds__(256, 3) void score_kernel(const ScoreArgs a, int64_
 //             (W1's K order permuted likewise); dL/dphi = dz0 W0[0..kF)^T on
 //             MFMA; activations and dz written transposed into LDS
 //   then, behind the only barrier of the backward:
-//   scatter   the grid gradient to the 8 corners in 2^-40 fixed point by
-//             64-bit integer atomics, one point per instruction (lane =
-//             (corner, feature)), 16 points per wave; nothing waits for them
+//   grid      dL/dphi of the row is stored for the nodes to gather
+//             (grid_nodes), or, without an index of them, scattered to the 8
+//             corners in 2^-40 fixed point by 64-bit integer atomics, one
+//             point per instruction (lane = (corner, feature)), 16 points per
+//             wave.  Both sums are exact, so the same.  The atomics cost 10 us
+//             a step: their lines move between the XCDs' L2s
 //   weights   gradients X^T dZ as MFMAs over a group's 64 points, 16 x 16
 //             tiles dealt to the waves (bias gradients against an all-ones A
 //             row); a wave adds its tile of the two groups and stores it to
@@ -514,8 +519,9 @@ __device__ __forceinline__ bf16x8 acc_operand(const floatx4 &v0, const floatx4 &
 __device__ __forceinline__ float bf16_round(float x) { return lo_bf16(pack_bf16(x, 0.f)); }
 
 struct StepArgs {
-  const float4 *points;   // row r of the launch is point r
-  const float *labels;    // exact one-atom energy of every point
+  const int4 *cells;      // PointIndex's cells and slots, from the launch's first row
+  const uint32_t *slots;
+  const float *labels;    // exact one-atom energy of every row
   size_t n;               // rows in this launch (a multiple of 64)
   // optional: the launch writes the learning rates and bias corrections of
   // step `step` of `sched` for the Adam launch after it
@@ -533,7 +539,8 @@ struct StepArgs {
   float *pred;            // optional: y of every row
   unsigned long long *loss;  // optional: fixed-point sum of squared errors (mlp::kLossScale)
   int backward;
-  unsigned long long *gacc;  // grid gradient accumulators [nodes][kF]
+  float *dphi;               // optional: dL/dphi of every row [n][kF]
+  unsigned long long *gacc;  // without dphi: grid gradient accumulators [nodes][kF]
   float *gw[3], *gb[3];   // this launch's work-group slices: gw[l] [nwg][K_l][grad_n(l)], gb[l] [nwg][grad_n(l)]
 };
 
@@ -560,10 +567,12 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
   const int s1 = a.g.n[2], s0 = a.g.n[1] * a.g.n[2];
   // ---- the points: four lanes each, features 2 f and 2 f + 1
   const int pt = tid >> 2, f = tid & 3;
-  float4 p{};
+  int4 ce{};
+  uint32_t slot_ = 0;
   float e = 0.f;
   if (active) {
-    p = a.points[row0 + size_t(pt)];
+    ce = a.cells[row0 + size_t(pt)];
+    slot_ = a.slots[row0 + size_t(pt)];
     e = a.labels[row0 + size_t(pt)];
   }
   // the weights of this lane's MFMA operands, in flight with the points
@@ -595,13 +604,8 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
     }
   }
   if (active) {
-    const float inv_h = 1.0f / a.g.h;
-    int ix, iy, iz;
-    float fx, fy, fz;
-    cell(p.x, a.g.lo[0], inv_h, a.g.n[0], ix, fx);
-    cell(p.y, a.g.lo[1], inv_h, a.g.n[1], iy, fy);
-    cell(p.z, a.g.lo[2], inv_h, a.g.n[2], iz, fz);
-    const int node = ix * s0 + iy * s1 + iz;
+    const int node = ce.x;
+    const float fx = __int_as_float(ce.y), fy = __int_as_float(ce.z), fz = __int_as_float(ce.w);
     const float gx[2] = {1.f - fx, fx}, gy[2] = {1.f - fy, fy}, gz[2] = {1.f - fz, fz};
     float2 u[8];
 #pragma unroll
@@ -618,8 +622,8 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
     }
     phis[pt][f] = pack_bf16(phi0, phi1);
     if (f == 0) {
-      cells[pt] = make_int4(node, __float_as_int(fx), __float_as_int(fy), __float_as_int(fz));
-      slots[pt] = __float_as_int(p.w);
+      cells[pt] = ce;
+      slots[pt] = int(slot_);
       yts[pt] = (fminf(e, a.norm.clip) - a.norm.mu) * a.norm.inv_sigma;
     }
   }
@@ -696,7 +700,10 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
       // dL/dphi = dz0 W0[0..kF)^T: A = W0 rows 0..kF-1 (K permuted), rows kF..15 zero
       const floatx4 dp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fwp, acc_operand(dz0[0], dz0[1]),
                                                                  floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-      if (grp < 2) *reinterpret_cast<float4 *>(&dphi[(q16 + r) * kF + 4 * grp]) = make_float4(dp[0], dp[1], dp[2], dp[3]);
+      if (grp < 2) {
+        float *o = a.dphi ? a.dphi + (row0 + size_t(q16 + r)) * kF : &dphi[(q16 + r) * kF];
+        *reinterpret_cast<float4 *>(o + 4 * grp) = make_float4(dp[0], dp[1], dp[2], dp[3]);
+      }
       // the transposed tiles
 #pragma unroll
       for (int jn = 0; jn < 2; jn++)
@@ -717,7 +724,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
   if (!a.backward) return;  // (uniform over the launch)
   __syncthreads();
   // ---- grid gradient: one point per instruction, lane = (corner, feature)
-  if (active) {
+  if (active && !a.dphi) {
     const int cq = lane >> 3, k = lane & 7;
     const int dx = cq >> 2, dy = (cq >> 1) & 1, dz = cq & 1;
     unsigned long long *acc = a.gacc + size_t(dx * s0 + dy * s1 + dz) * kF + k;
@@ -801,16 +808,194 @@ __global__ __launch_bounds__(64 * kStepWaves) void step_kernel(const StepArgs a)
   }
 }
 
-// The training points and their labels in the order the batches take them:
-// a step then reads whole lines, with one dependent load less.
-__global__ void order_kernel(const float4 *__restrict__ points, const float *__restrict__ labels,
-                             const uint32_t *__restrict__ perm, size_t n, float4 *__restrict__ out_points,
-                             float *__restrict__ out_labels) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+// A step's Adam update of the grid, a tensor of its own: the work-groups after
+// the weights'.
+struct GridAdam {
+  float *w, *m, *v;           // [nodes][kF]
+  size_t nodes;
+  unsigned long long *acc;    // without terms: the gradient in fixed point, cleared here
+  const uint2 *terms;         // the batch's (PointIndex), and its rows' dL/dphi
+  const uint32_t *first;
+  const float *dphi;
+};
+
+constexpr int kNodesPerWave = 64 / kF;
+
+__device__ __forceinline__ void adam_entry(const GridAdam &g, size_t k, float w, float m, float v, long long acc,
+                                           float b1, float b2, float eps, const float *__restrict__ hyper) {
+  mlp::adam_update(w, m, v, float(double(acc) / kGradScale), hyper[1], hyper[2], hyper[3], b1, b2, eps);
+  g.w[k] = w;
+  g.m[k] = m;
+  g.v[k] = v;
+}
+
+// A weight times dL/dphi in units of 1 / kGradScale, rounded, plus 1.5 2^52:
+// the bits of such a double are those of 1.5 2^52 plus the whole number, so
+// sums of them (less the constant) are sums of the numbers, for 4 VALU a term
+// where the conversion to 64-bit integers takes 10.  For magnitudes below
+// kNearTerm.
+constexpr double kMagic = 6755399441055744.0;
+constexpr float kNearTerm = 2048.f;
+
+// The gradient and Adam update of eight consecutive nodes per wave, lane =
+// (node, feature): the node's terms, eight in flight at a time, then Adam.
+// The waves of a work-group take nodes far from each other: the rows crowd
+// into a part of the grid, whose nodes are then spread over the device.  The
+// launch takes 10.7 us for 32,768 rows and 78,000 nodes (7.1 with the sums
+// read from memory and cleared, but those take atomics of 10 us); gathering
+// from the rows sorted by cell took 13.0 (weights formed and runs told apart
+// for every term), sums of 256-node bricks in LDS 34.7 (most rows in a few).
+__device__ __forceinline__ void grid_nodes(const GridAdam &g, int block, int nblocks, float b1, float b2, float eps,
+                                           const float *__restrict__ hyper) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const size_t q = (size_t(wave) * size_t(nblocks) + size_t(block)) * kNodesPerWave + size_t(lane >> 3);
+  const bool on = q < g.nodes;
+  const size_t at = on ? q * kF + (lane & 7) : 0;
+  const uint32_t t0 = on ? g.first[q] : 0u, t1 = on ? g.first[q + 1] : 0u;
+  const float w = g.w[at], m = g.m[at], v = g.v[at];
+  const float *dphi = g.dphi + (lane & 7);
+  constexpr int kAhead = 8;
+  long long acc = 0;
+  float most = 0.f;
+  for (uint32_t t = t0; __any(t < t1); t += kAhead) {
+    uint2 term[kAhead];
+    float dp[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) term[u] = g.terms[t + u < t1 ? t + u : 0u];  // (any term of the batch will do)
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) dp[u] = dphi[size_t(term[u].x) * kF];
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) {
+      // (past the end: a zero; a branch here would take the loads into it, one wait after another)
+      const float x = __uint_as_float(t + u < t1 ? term[u].y : 0u) * dp[u];
+      most = fmaxf(most, fabsf(x));
+      acc += __double_as_longlong(__builtin_fma(double(x), kGradScale, kMagic)) - __double_as_longlong(kMagic);
+    }
+  }
+  if (!(most < kNearTerm)) {
+    acc = 0;
+    for (uint32_t t = t0; t < t1; t++) {
+      const uint2 term = g.terms[t];
+      acc += llrint(double(__uint_as_float(term.y) * dphi[size_t(term.x) * kF]) * kGradScale);
+    }
+  }
+  if (on) adam_entry(g, at, w, m, v, acc, b1, b2, eps, hyper);
+}
+
+// P: partial sums of a gradient entry (adam_tensors).
+template <int P>
+__global__ __launch_bounds__(64 * mlp::kAdamWaves) void adam_kernel(const mlp::AdamBatch b, int tensor_blocks,
+                                                               const GridAdam g, float b1, float b2, float eps,
+                                                               const float *__restrict__ hyper) {
+  const int block = int(blockIdx.x);
+  if (block < tensor_blocks) {
+    mlp::adam_tensors<P>(b, block, b1, b2, eps, hyper);
+  } else if (g.terms) {
+    grid_nodes(g, block - tensor_blocks, int(gridDim.x) - tensor_blocks, b1, b2, eps, hyper);
+  } else {
+    const size_t k = size_t(block - tensor_blocks) * (64 * mlp::kAdamWaves) + threadIdx.x;
+    if (k >= g.nodes * kF) return;
+    const long long acc = static_cast<long long>(g.acc[k]);
+    g.acc[k] = 0ull;
+    adam_entry(g, k, g.w[k], g.m[k], g.v[k], acc, b1, b2, eps, hyper);
+  }
+}
+
+// ---- where the training points lie -------------------------------------------
+
+__device__ __forceinline__ int corner_node(const field::Grid &grid, int node, int c) {
+  return node + ((c >> 2) * grid.n[1] + ((c >> 1) & 1)) * grid.n[2] + (c & 1);
+}
+
+// Cells and slots of the rows (row i: point perm[i], i < ntrain; point i
+// behind them); with `count`, count[batch][node + 1] of a training row's eight
+// corners and the row's place among each node's terms.
+__global__ __launch_bounds__(256) void locate_kernel(const float4 *__restrict__ points,
+                                                     const uint32_t *__restrict__ perm, size_t ntrain, size_t n,
+                                                     const field::Grid grid, size_t batch, size_t nodes,
+                                                     int4 *__restrict__ cells, uint32_t *__restrict__ slots,
+                                                     uint32_t *__restrict__ count, uint4 *__restrict__ places) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n) return;
-  const uint32_t q = perm[i];
-  out_points[i] = points[q];
-  out_labels[i] = labels[q];
+  const float4 p = points[i < ntrain && perm ? perm[i] : i];
+  const float inv_h = 1.0f / grid.h;
+  int ix, iy, iz;
+  float fx, fy, fz;
+  cell(p.x, grid.lo[0], inv_h, grid.n[0], ix, fx);
+  cell(p.y, grid.lo[1], inv_h, grid.n[1], iy, fy);
+  cell(p.z, grid.lo[2], inv_h, grid.n[2], iz, fz);
+  const int node = (ix * grid.n[1] + iy) * grid.n[2] + iz;
+  cells[i] = make_int4(node, __float_as_int(fx), __float_as_int(fy), __float_as_int(fz));
+  slots[i] = uint32_t(__float_as_int(p.w));
+  if (!count || i >= ntrain) return;
+  uint32_t *mine = count + (i / batch) * (nodes + 1) + 1;
+  uint32_t at[8];
+#pragma unroll
+  for (int c = 0; c < 8; c++) at[c] = atomicAdd(&mine[corner_node(grid, node, c)], 1u);
+  places[2 * i] = make_uint4(at[0], at[1], at[2], at[3]);
+  places[2 * i + 1] = make_uint4(at[4], at[5], at[6], at[7]);
+}
+
+// first[0 .. nodes] of each batch from counts (first[0] = 0) to running sums;
+// one work-group per batch, eight entries per work-item at a time.
+__global__ __launch_bounds__(1024) void first_kernel(size_t nodes, uint32_t *__restrict__ first) {
+  __shared__ uint32_t wsum[16];
+  uint32_t *f = first + size_t(blockIdx.x) * (nodes + 1);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t base = 0;
+  for (size_t b = 0; b <= nodes; b += 8192) {
+    const size_t at = b + size_t(threadIdx.x) * 8;
+    uint32_t v[8], sum = 0;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      v[u] = at + u <= nodes ? f[at + u] : 0u;
+      sum += v[u];
+    }
+    uint32_t x = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = __shfl_up(x, d);
+      if (lane >= d) x += y;
+    }
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    uint32_t run = base + x - sum;
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) run += wsum[w];
+      base += wsum[w];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      run += v[u];
+      if (at + u <= nodes) f[at + u] = run;
+    }
+    __syncthreads();  // (wsum is rewritten)
+  }
+}
+
+__global__ __launch_bounds__(256) void terms_kernel(const int4 *__restrict__ cells, const uint4 *__restrict__ places,
+                                                    size_t ntrain, const field::Grid grid, size_t batch, size_t nodes,
+                                                    const uint32_t *__restrict__ first, uint2 *__restrict__ terms) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= ntrain) return;
+  const int4 ce = cells[i];
+  const float fx = __int_as_float(ce.y), fy = __int_as_float(ce.z), fz = __int_as_float(ce.w);
+  const size_t b = i / batch;
+  const uint32_t *f = first + b * (nodes + 1);
+  uint2 *t = terms + b * batch * 8;
+  const uint4 p0 = places[2 * i], p1 = places[2 * i + 1];
+  const uint32_t at[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const float w = (c >> 2 ? fx : 1.f - fx) * ((c >> 1) & 1 ? fy : 1.f - fy) * (c & 1 ? fz : 1.f - fz);
+    t[f[corner_node(grid, ce.x, c)] + at[c]] = make_uint2(uint32_t(i - b * batch), __float_as_uint(w));
+  }
+}
+
+// The training labels in the order the batches take them.
+__global__ void order_kernel(const float *__restrict__ labels, const uint32_t *__restrict__ perm, size_t n,
+                             float *__restrict__ out) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = labels[perm[i]];
 }
 
 unsigned blocks_for(size_t n, unsigned t) { return unsigned((n + t - 1) / t); }
@@ -826,19 +1011,23 @@ struct RunStep {
   mlp::Schedule sched;
 };
 
-// The fused step over rows [0, n) of `points`: forward (y into pred, if set; squared error into A.loss), and with
-// `backward` the gradients -- grid into net.gacc, weights and biases as
-// one slice per work-group into A.gpart / bpart (A.splits slices).
-int launch_step(Net &net, Acts &A, const float4 *points, const float *labels, size_t n, size_t batch,
+// The fused step over rows first .. first + n - 1 of idx: forward (y into
+// pred, if set; squared error into A.loss), and with `backward` the gradients
+// -- the grid's as dL/dphi into A.dphi (of a run, with idx.gathered) or
+// into net.gacc, weights and biases as one slice per work-group into A.gpart /
+// bpart (A.splits slices).
+int launch_step(Net &net, Acts &A, const PointIndex &idx, size_t first, const float *labels, size_t n, size_t batch,
                 mlp::TargetNorm norm, float *pred, bool backward, hipStream_t s,
                 const RunStep *run = nullptr) {
   if (n == 0 || n % 64) return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet: rows must be a multiple of 64");
   StepArgs a{};
-  a.points = points;
+  a.cells = static_cast<const int4 *>(idx.cells.ptr) + first;
+  a.slots = static_cast<const uint32_t *>(idx.slots.ptr) + first;
   if (run) {
     a.hyper = run->hyper;
     a.step = run->step;
     a.sched = run->sched;
+    if (idx.gathered) a.dphi = static_cast<float *>(A.dphi.ptr);
   }
   a.labels = labels;
   a.n = n;
@@ -877,8 +1066,9 @@ int launch_step(Net &net, Acts &A, const float4 *points, const float *labels, si
   return hip_check(hipGetLastError(), "atomnet step");
 }
 
-// Adam on every parameter with the step's values the step kernel wrote.
-int adam_step_dev(Net &net, const Acts &A, const float *hyper, hipStream_t s) {
+// Adam on every parameter after batch `batch` of idx, with the step's values
+// the step kernel wrote.
+int adam_step_dev(Net &net, const Acts &A, const PointIndex &idx, size_t batch, const float *hyper, hipStream_t s) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   mlp::AdamBatch ab{};
   for (int l = 0; l < 3; l++) {
@@ -892,10 +1082,27 @@ int adam_step_dev(Net &net, const Acts &A, const float *hyper, hipStream_t s) {
                        N, A.splits[l], size_t(N)};
   }
   ab.count = 6;
-  // the grid, from its fixed-point accumulators (cleared), in the same launch
-  ab.fixed = {static_cast<float *>(net.g.ptr), static_cast<unsigned long long *>(net.gacc.ptr),
-              static_cast<float *>(net.gm.ptr), static_cast<float *>(net.gv.ptr), net.nodes * kF, kGradScale};
-  return hip_check(mlp::adam_multi_dev(ab, hyper, b1, b2, eps, s), "atomnet adam");
+  // the grid in the same launch
+  GridAdam g{};
+  g.w = static_cast<float *>(net.g.ptr);
+  g.m = static_cast<float *>(net.gm.ptr);
+  g.v = static_cast<float *>(net.gv.ptr);
+  g.acc = static_cast<unsigned long long *>(net.gacc.ptr);
+  g.nodes = net.nodes;
+  const unsigned grid_blocks = blocks_for(net.nodes * kF, 64 * mlp::kAdamWaves);
+  if (idx.gathered) {
+    g.terms = static_cast<const uint2 *>(idx.terms.ptr) + batch * idx.batch * 8;
+    g.first = static_cast<const uint32_t *>(idx.first.ptr) + batch * (idx.nodes + 1);
+    g.dphi = static_cast<const float *>(A.dphi.ptr);
+  }
+  const unsigned tensor_blocks = blocks_for(mlp::adam_entries(ab), 64);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(tensor_blocks + grid_blocks), dim3(64 * mlp::kAdamWaves), 0, s, ab,
+                       int(tensor_blocks), g, b1, b2, eps, hyper);
+  };
+  if (A.splits[0] > 32) run(adam_kernel<16>);
+  else run(adam_kernel<4>);
+  return hip_check(hipGetLastError(), "atomnet adam");
 }
 
 int alloc_zero(DeviceBuffer &d, size_t bytes) {
@@ -1034,17 +1241,63 @@ hipError_t label_points(const float4 *protein, const int32_t *group_begin, const
   return hipGetLastError();
 }
 
-int train(Net &net, Workspace &A, const float4 *points, const float *labels, const uint32_t *perm, size_t ntrain,
-          size_t nval, const TrainParams &p, hipStream_t s, TrainReport *rep) {
-  const size_t B = p.batch;
+int index_points(PointIndex &idx, const field::Grid &grid, const float4 *points, const uint32_t *perm, size_t ntrain,
+                 size_t nval, size_t batch, size_t limit, hipStream_t s) {
+  const size_t n = ntrain + nval, nodes = grid.points();
+  if (n == 0 || batch == 0 || ntrain % batch || batch > (size_t(1) << 28) || nodes > 0x7fffffffu)
+    return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet index: the training points must be whole batches");
+  const size_t batches = ntrain / batch, counts = batches * (nodes + 1) * sizeof(uint32_t);
+  idx.ntrain = ntrain;
+  idx.nval = nval;
+  idx.batch = batch;
+  idx.nodes = nodes;
+  idx.gathered = ntrain > 0 && counts + ntrain * 8 * sizeof(uint2) <= limit;
+  DeviceBuffer places;  // (of a row among its nodes' terms)
+  int st = idx.cells.reserve(n * sizeof(int4));
+  if (!st) st = idx.slots.reserve(n * sizeof(uint32_t));
+  if (!st && idx.gathered) {
+    st = idx.terms.reserve(ntrain * 8 * sizeof(uint2));
+    if (!st) st = idx.first.reserve(counts);
+    if (!st) st = places.alloc(ntrain * 2 * sizeof(uint4));
+    if (st == BUDE_ERR_OUT_OF_MEMORY) {  // (training needs none of it)
+      idx.terms.reset();
+      idx.first.reset();
+      idx.gathered = false;
+      st = BUDE_OK;
+    }
+  }
+  if (st) return st;
+  auto *cells = static_cast<int4 *>(idx.cells.ptr);
+  auto *slots = static_cast<uint32_t *>(idx.slots.ptr);
+  auto *first = idx.gathered ? static_cast<uint32_t *>(idx.first.ptr) : nullptr;
+  auto *at = static_cast<uint4 *>(places.ptr);
+  if (first)
+    if (int e = hip_check(hipMemsetAsync(first, 0, counts, s), "hipMemsetAsync")) return e;
+  hipLaunchKernelGGL(locate_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, points, perm, ntrain, n, grid, batch,
+                     nodes, cells, slots, first, at);
+  if (first) {
+    hipLaunchKernelGGL(first_kernel, dim3(unsigned(batches)), dim3(1024), 0, s, nodes, first);
+    hipLaunchKernelGGL(terms_kernel, dim3(blocks_for(ntrain, 256)), dim3(256), 0, s, cells, at, ntrain, grid, batch,
+                       nodes, static_cast<const uint32_t *>(first), static_cast<uint2 *>(idx.terms.ptr));
+  }
+  if (int e = hip_check(hipGetLastError(), "atomnet index")) return e;
+  return hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");  // (places is a local)
+}
+
+int train(Net &net, Workspace &A, const PointIndex &idx, const float *labels, const uint32_t *perm,
+          const TrainParams &p, hipStream_t s, TrainReport *rep) {
+  const size_t B = p.batch, ntrain = idx.ntrain, nval = idx.nval;
   if (B == 0 || B % 64 || ntrain < B || ntrain % B || nval % 64)
     return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet train: the training points must be whole batches "
                                            "(a multiple of 64) and the held-out points a multiple of 64");
+  if (idx.batch != B || idx.nodes != net.nodes)
+    return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet train: the index is of another grid or batch size");
   if (int st = reserve(net, A, B, nval)) return st;
-  if (int st = A.opoints.reserve(ntrain * sizeof(float4))) return st;
   if (int st = A.olabels.reserve(ntrain * sizeof(float))) return st;
-  hipLaunchKernelGGL(order_kernel, dim3(blocks_for(ntrain, 256)), dim3(256), 0, s, points, labels, perm, ntrain,
-                     static_cast<float4 *>(A.opoints.ptr), static_cast<float *>(A.olabels.ptr));
+  if (idx.gathered)
+    if (int st = A.dphi.reserve(B * kF * sizeof(float))) return st;
+  hipLaunchKernelGGL(order_kernel, dim3(blocks_for(ntrain, 256)), dim3(256), 0, s, labels, perm, ntrain,
+                     static_cast<float *>(A.olabels.ptr));
   if (int st = hip_check(hipGetLastError(), "atomnet order")) return st;
   // target transform from the training labels
   {
@@ -1076,13 +1329,13 @@ int train(Net &net, Workspace &A, const float4 *points, const float *labels, con
   // steps of a screen took 109.0 ms with a captured step replayed, 96.1 with
   // 20 steps captured at once, 95.4 launched.
   for (uint32_t step = 0; step < steps; step++) {
-    const size_t row = size_t(step % per_epoch) * B;
+    const size_t batch = step % per_epoch, row = batch * B;
     const RunStep run{static_cast<float *>(A.hyper.ptr), step,
                       mlp::Schedule{steps, warm, step0, p.lr, p.grid_lr, 0.9f, 0.999f}};
-    if (int st = launch_step(net, A, static_cast<const float4 *>(A.opoints.ptr) + row,
-                             static_cast<const float *>(A.olabels.ptr) + row, B, B, norm, nullptr, true, s, &run))
+    if (int st = launch_step(net, A, idx, row, static_cast<const float *>(A.olabels.ptr) + row, B, B, norm, nullptr,
+                             true, s, &run))
       return st;
-    if (int st = adam_step_dev(net, A, run.hyper, s)) return st;
+    if (int st = adam_step_dev(net, A, idx, batch, run.hyper, s)) return st;
   }
   net.step += int(steps);
   TrainReport r{};
@@ -1093,7 +1346,7 @@ int train(Net &net, Workspace &A, const float4 *points, const float *labels, con
   double se = 0;
   if (nval) {
     DeviceBuffer &vpred = A.vpred;
-    if (int st = launch_step(net, A, points + ntrain, labels + ntrain, nval, B, norm,
+    if (int st = launch_step(net, A, idx, ntrain, labels + ntrain, nval, B, norm,
                              static_cast<float *>(vpred.ptr), false, s))
       return st;
     hipLaunchKernelGGL(sq_err_kernel, dim3(256), dim3(256), 0, s, static_cast<const float *>(vpred.ptr),
@@ -1121,7 +1374,9 @@ int forward_backward(Net &net, const float4 *points, const float *target, size_t
   if (int st = reserve(net, A, batch, 0)) return st;
   if (int st = hip_check(hipMemsetAsync(A.loss.ptr, 0, 8, s), "hipMemsetAsync")) return st;
   const mlp::TargetNorm norm{INFINITY, 0.f, 1.f, -INFINITY};
-  if (int st = launch_step(net, A, points, target, batch, batch, norm, static_cast<float *>(A.pred.ptr), true, s))
+  PointIndex idx;
+  if (int st = index_points(idx, net.grid, points, nullptr, 0, batch, batch, 0, s)) return st;
+  if (int st = launch_step(net, A, idx, 0, target, batch, batch, norm, static_cast<float *>(A.pred.ptr), true, s))
     return st;
   // the K slices of the weight and bias gradients, summed in order into net.gw / gb
   for (int l = 0; l < 3; l++) {

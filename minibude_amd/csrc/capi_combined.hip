@@ -309,6 +309,7 @@ struct bude_combined {
   bude::atomnet::Workspace aws;
   DeviceBuffer apoints, alabels, aperm, ameta;
   bude::items::Points apoint_items;  // the points sorted for their labels
+  bude::atomnet::PointIndex apoint_index;  // their places in the grid
   size_t antrain = 0, anval = 0;
   // exact energies of every pair (exhaustive) and the protein they belong to
   uint64_t exact_sum = 0;
@@ -710,10 +711,8 @@ int train_atom(bude_combined *c, uint64_t pseed) {
   tp.grid_lr = c->cfg.grid_lr;
   tp.seed = pseed;
   bude::atomnet::TrainReport rep{};
-  if (int st = bude::atomnet::train(c->anet, c->aws, static_cast<const float4 *>(c->apoints.ptr),
-                                    static_cast<const float *>(c->alabels.ptr),
-                                    static_cast<const uint32_t *>(c->aperm.ptr), c->antrain, c->anval, tp, c->stream2,
-                                    &rep))
+  if (int st = bude::atomnet::train(c->anet, c->aws, c->apoint_index, static_cast<const float *>(c->alabels.ptr),
+                                    static_cast<const uint32_t *>(c->aperm.ptr), tp, c->stream2, &rep))
     return st;
   ps.atom_val_rmse = rep.val_rmse;
   ps.res.surrogate_rmse = rep.val_rmse;
@@ -977,7 +976,13 @@ int prepare_atom_points(bude_combined *c) {
   std::iota(perm.begin(), perm.end(), 0u);
   std::mt19937_64 rng(c->cfg.seed ^ 0x9e37ull);
   std::shuffle(perm.begin(), perm.end(), rng);
-  return c->aperm.upload(perm.data(), perm.size() * 4);
+  if (int st = c->aperm.upload(perm.data(), perm.size() * 4)) return st;
+  // (BUDE_MI355X_TRAIN_INDEX_MB bounds the index's tables; training gives the same network without them)
+  const char *mb = std::getenv("BUDE_MI355X_TRAIN_INDEX_MB");
+  const size_t limit = mb ? size_t(std::max(0l, std::atol(mb))) << 20 : bude::atomnet::kIndexBytes;
+  return bude::atomnet::index_points(c->apoint_index, c->grid, static_cast<const float4 *>(c->apoints.ptr),
+                                     static_cast<const uint32_t *>(c->aperm.ptr), c->antrain, c->anval, c->cfg.batch,
+                                     limit, nullptr);
 }
 
 }  // namespace

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 
+#include "adam.h"
 #include "mlp.h"
 
 namespace bude {
@@ -548,90 +549,12 @@ __global__ void ksplit_reduce_kernel(const float *__restrict__ work, size_t n, i
   out[i] = acc;
 }
 
-// One work-group of W waves per 64 consecutive entries of the flat index
-// over the batch's tensors: wave w sums the lane's entry over slices w,
-// w + W, ... (each load a coalesced row of 64 entries), the work-group adds
-// the waves' partial sums in wave order, and the first wave applies Adam.
-// The slice sums are spread over the waves so that their loads are in
-// flight together (W = 16 for the hundreds of slices of the fused step, 4
-// for the K splits of the GEMMs); the order of every sum is fixed.
-template <int W>
-__global__ __launch_bounds__(64 * W) void adam_multi_kernel(const AdamBatch b, float lr, float b1, float b2, float eps,
-                                                            float bc1, float bc2, const float *__restrict__ hyper,
-                                                            StepState *__restrict__ advance) {
-  constexpr int kAdamWaves = W;
-  __shared__ float part[kAdamWaves][64];
-  if (hyper) {  // learning rate and bias corrections of this step from device memory
-    lr = hyper[0];
-    bc1 = hyper[2];
-    bc2 = hyper[3];
-  }
+__global__ __launch_bounds__(64 * kAdamWaves) void adam_multi_kernel(const AdamBatch b, float b1, float b2, float eps,
+                                                                     const float *__restrict__ hyper,
+                                                                     StepState *__restrict__ advance) {
   // (the step count is read only by the next step's first kernel)
   if (advance && blockIdx.x == 0 && threadIdx.x == 0) advance->step += 1;
-  if (int(blockIdx.x) >= b.tensor_blocks) {  // the fixed-point tensor: 64 W entries per work-group
-    const AdamFixed &F = b.fixed;
-    const size_t k = size_t(blockIdx.x - b.tensor_blocks) * (64 * W) + threadIdx.x;
-    if (k >= F.n) return;
-    const float gk = float(double(static_cast<long long>(F.acc[k])) / F.scale);
-    F.acc[k] = 0ull;
-    const float mk = b1 * F.m[k] + (1.f - b1) * gk;
-    const float vk = b2 * F.v[k] + (1.f - b2) * gk * gk;
-    F.m[k] = mk;
-    F.v[k] = vk;
-    F.w[k] = F.w[k] - hyper[1] * (mk / bc1) / (sqrtf(vk / bc2) + eps);
-    return;
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  size_t i = size_t(blockIdx.x) * 64 + lane;
-  int t = 0;
-  for (; t < b.count; t++) {
-    const size_t n = size_t(b.t[t].rows) * b.t[t].cols;
-    if (i < n) break;
-    i -= n;
-  }
-  const bool valid = t < b.count;
-  float gs = 0.f;
-  if (valid) {
-    const float *g = b.t[t].g + i;
-    const size_t stride = b.t[t].stride;
-    const int splits = b.t[t].splits;
-    // slices wave, wave + W, ... added in that order, eight (or four) loads in flight
-    int z = wave;
-    for (; z + 7 * kAdamWaves < splits; z += 8 * kAdamWaves) {
-      float sl[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) sl[u] = g[size_t(z + u * kAdamWaves) * stride];
-#pragma unroll
-      for (int u = 0; u < 8; u++) gs += sl[u];
-    }
-    for (; z + 3 * kAdamWaves < splits; z += 4 * kAdamWaves) {
-      float sl[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) sl[u] = g[size_t(z + u * kAdamWaves) * stride];
-#pragma unroll
-      for (int u = 0; u < 4; u++) gs += sl[u];
-    }
-    for (; z < splits; z += kAdamWaves) gs += g[size_t(z) * stride];
-  }
-  part[wave][lane] = gs;
-  __syncthreads();
-  if (wave != 0 || !valid) return;
-  float gi = part[0][lane];
-#pragma unroll
-  for (int w = 1; w < kAdamWaves; w++) gi += part[w][lane];
-  const AdamTensor &T = b.t[t];
-  const size_t at = T.pitch ? i / T.cols * T.pitch + i % T.cols : i;
-  const float mi = b1 * T.m[at] + (1.f - b1) * gi;
-  const float vi = b2 * T.v[at] + (1.f - b2) * gi * gi;
-  T.m[at] = mi;
-  T.v[at] = vi;
-  const float wi = T.w[at] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-  T.w[at] = wi;
-  const bf16 h = to_bf16(wi);
-  if (T.w16) T.w16[at] = h;
-  if (T.w16t) T.w16t[size_t(i % T.cols) * T.rows + i / T.cols] = h;
-  if (T.w16x) T.w16x[tiled_index(i / T.cols, i % T.cols, size_t(T.cols))] = h;
-  if (T.w16tx) T.w16tx[tiled_index(i % T.cols, i / T.cols, size_t(T.rows))] = h;
+  adam_tensors<4>(b, int(blockIdx.x), b1, b2, eps, hyper);
 }
 
 __global__ void tile_bf16_kernel(const float *__restrict__ w, int rows, int cols, bf16 *__restrict__ wx,
@@ -836,24 +759,10 @@ hipError_t fold_bias(const float *b, const bf16 *w0tx, const float *desc, int nl
 
 hipError_t adam_multi_dev(const AdamBatch &b, const float *hyper, float b1, float b2, float eps, hipStream_t s,
                           StepState *advance) {
-  size_t total = 0;
-  int splits = 1;
-  for (int t = 0; t < b.count; t++) {
-    total += size_t(b.t[t].rows) * b.t[t].cols;
-    splits = std::max(splits, b.t[t].splits);
-  }
-  if (total == 0 || !hyper || (b.fixed.n && (!b.fixed.w || !b.fixed.acc || !b.fixed.m || !b.fixed.v)))
-    return hipErrorInvalidValue;
-  const int W = splits > 32 ? 16 : 4;
-  AdamBatch a = b;
-  a.tensor_blocks = int(blocks_for(total, 64));
-  const unsigned blocks = unsigned(a.tensor_blocks) + blocks_for(b.fixed.n, 64u * W);
-  if (W == 16)
-    hipLaunchKernelGGL(adam_multi_kernel<16>, dim3(blocks), dim3(64 * 16), 0, s, a, 0.f, b1, b2, eps, 1.f, 1.f, hyper,
-                       advance);
-  else
-    hipLaunchKernelGGL(adam_multi_kernel<4>, dim3(blocks), dim3(64 * 4), 0, s, a, 0.f, b1, b2, eps, 1.f, 1.f, hyper,
-                       advance);
+  const size_t total = adam_entries(b);
+  if (total == 0 || !hyper) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(adam_multi_kernel, dim3(blocks_for(total, 64)), dim3(64 * kAdamWaves), 0, s, b, b1, b2, eps,
+                     hyper, advance);
   return hipGetLastError();
 }
 

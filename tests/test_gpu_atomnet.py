@@ -230,3 +230,25 @@ def test_learned_field_meets_the_prescreen_target_at_2pct(gpu_device):
           f"gate z {pair.gate_z:.2f}, fallback {pair.fallback}, train {r.train_ms:.0f} ms", flush=True)
     assert not pair.fallback and pair.keep_fraction <= 0.025
     assert rec >= 0.99
+
+
+@pytest.mark.parametrize("nposes, train_points, batch, spacing, steps", [
+    (4096, 65536, 4096, 0.75, 20),   # whole work-groups of 128 rows
+    (257, 576, 192, 0.5, 7),         # a work-group of one group of 64; many more bricks than rows
+    (64, 1048576, 1048576, 4.0, 2),  # the largest batch, crowded into a coarse grid's cells
+])
+def test_gathered_grid_gradient_equals_scattered(gpu_device, nposes, train_points, batch, spacing, steps, monkeypatch):
+    # both are exact fixed-point sums, so the networks, and the scores, are
+    # equal bit for bit whether the nodes gather the rows sorted by cell or
+    # the rows are scattered by atomics (no room for the sorted rows)
+    w = c4_like(nproteins=1, nligands=2, nposes=nposes, seed=25)
+    cfg = dict(train_points=train_points, batch=batch, steps=steps, labels_per_pair=64, gate_z=0.0,
+               grid_spacing=spacing)
+    out = {}
+    for mb in ("4096", "0"):
+        monkeypatch.setenv("BUDE_MI355X_TRAIN_INDEX_MB", mb)
+        with C.Combined(w.forcefield, w.ligands, w.poses, C.default_config("mlp", **cfg), gpu_device) as c:
+            r = c.screen(w.proteins[0])
+            out[mb] = [c.scores(l) for l in range(2)] + [np.array([r.surrogate_rmse], np.float32)]
+    for a, b in zip(out["4096"], out["0"]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
