@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <numeric>
 #include <random>
 #include <string>
@@ -494,117 +495,256 @@ extern "C" int bude_mi355x_screen_destroy(bude_screen *s) {
   return bude::ok();
 }
 
+namespace {
+
+// The device memory of a call, handed out in aligned pieces: one allocation,
+// as an allocation and its release cost the host some 10 us each (the calls
+// below took 40 and 59).
+class Arena {
+ public:
+  template <class T> size_t add(size_t n) {
+    const size_t at = bytes_;
+    bytes_ += (n * sizeof(T) + 255) & ~size_t(255);
+    return at;
+  }
+  int alloc() { return buf_.alloc(bytes_); }
+  template <class T> T *at(size_t offset) const { return reinterpret_cast<T *>(static_cast<char *>(buf_.ptr) + offset); }
+
+ private:
+  size_t bytes_ = 0;
+  DeviceBuffer buf_;
+};
+
+// A network handed in whole: its FP32 arrays and the copies the kernels read.
+struct Handed {
+  size_t w[4], b[4], wt[3], wx[3], w3;
+  explicit Handed(Arena &m, bool training) {
+    using namespace bude::mlp;
+    for (int l = 0; l < 4; l++) {
+      w[l] = m.add<float>(size_t(kRealK[l]) * kRealN[l]);
+      b[l] = m.add<float>(size_t(kRealN[l]));
+    }
+    for (int l = 0; l < 3; l++) {
+      wt[l] = m.add<bf16>(size_t(kK[l]) * kN[l]);
+      wx[l] = training && l > 0 ? m.add<bf16>(size_t(kK[l]) * kN[l]) : 0;
+    }
+    w3 = m.add<bf16>(size_t(kK[3]) * kN[3]);
+  }
+  int upload(const Arena &m, const float *const weights[4], const float *const biases[4], hipStream_t s) const {
+    using namespace bude::mlp;
+    for (int l = 0; l < 4; l++) {
+      if (int st = bude::hip_check(hipMemcpyAsync(m.at<float>(w[l]), weights[l],
+                                                  size_t(kRealK[l]) * kRealN[l] * sizeof(float),
+                                                  hipMemcpyHostToDevice, s),
+                                   "hipMemcpyAsync weights"))
+        return st;
+      if (int st = bude::hip_check(hipMemcpyAsync(m.at<float>(b[l]), biases[l], size_t(kRealN[l]) * sizeof(float),
+                                                  hipMemcpyHostToDevice, s),
+                                   "hipMemcpyAsync biases"))
+        return st;
+    }
+    return BUDE_OK;
+  }
+  bude::mlp::StageArgs stage_args(const Arena &m, bool training) const {
+    bude::mlp::StageArgs a{};
+    for (int l = 0; l < 4; l++) a.w[l] = m.at<float>(w[l]);
+    for (int l = 0; l < 3; l++) {
+      a.wt[l] = m.at<bf16>(wt[l]);
+      a.wx[l] = training && l > 0 ? m.at<bf16>(wx[l]) : nullptr;
+    }
+    a.w3 = m.at<bf16>(w3);
+    return a;
+  }
+};
+
+int check_device(int device, const char *who) {
+  int ndev = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0 || device < 0 || device >= ndev)
+    return bude::fail(BUDE_ERR_NO_DEVICE, std::string(who) + ": no such HIP device");
+  return bude::hip_check(hipSetDevice(device), "hipSetDevice");
+}
+
+// Waits for the work of a call before its memory goes, however the call ends.
+struct Drain {
+  hipStream_t s;
+  ~Drain() { (void)hipStreamSynchronize(s); }
+};
+
+}  // namespace
+
+// 8,192 rows: 1,280 us with a buffer, a clear and a copy for each array (59, 25
+// and 20 of them), 466 us; the kernels take 42.
 extern "C" int bude_mi355x_mlp_forward_backward(int device, size_t batch, const float *features, const float *target,
                                                 const float *const weights[4], const float *const biases[4],
                                                 float *pred, float *loss, float *const grad_w[4],
                                                 float *const grad_b[4]) {
+  using namespace bude::mlp;
   if (!features || !target || !weights || !biases || !pred || !loss || !grad_w || !grad_b || batch == 0 ||
       batch % 32 || batch > (1u << 16))
     return bude::fail(BUDE_ERR_INVALID_ARGUMENT,
                       "bude_mi355x_mlp_forward_backward: bad arguments (batch a multiple of 32, <= 65536)");
-  int ndev = 0;
-  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0 || device < 0 || device >= ndev)
-    return bude::fail(BUDE_ERR_NO_DEVICE, "bude_mi355x_mlp_forward_backward: no such HIP device");
-  if (int st = bude::hip_check(hipSetDevice(device), "hipSetDevice")) return st;
-  hipStream_t s = nullptr;
-  if (int st = bude::hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate")) return st;
-  struct StreamGuard {
-    hipStream_t s;
-    ~StreamGuard() { (void)hipStreamDestroy(s); }
-  } guard{s};
-  // real shapes: 21x256, 256x256, 256x256, 256x1 -> padded device layout
-  const int realK[4] = {bude::mlp::kFeat, 256, 256, 256}, realN[4] = {256, 256, 256, 1};
-  std::vector<std::vector<float>> w(4), b(4);
-  for (int l = 0; l < 4; l++) {
-    w[l].assign(size_t(kK[l]) * kN[l], 0.f);
-    b[l].assign(size_t(kN[l]), 0.f);
-    for (int r = 0; r < realK[l]; r++)
-      for (int c = 0; c < realN[l]; c++) w[l][size_t(r) * kN[l] + c] = weights[l][size_t(r) * realN[l] + c];
-    for (int c = 0; c < realN[l]; c++) b[l][c] = biases[l][c];
+  if (int st = check_device(device, "bude_mi355x_mlp_forward_backward")) return st;
+  const hipStream_t s = nullptr;
+  const size_t ld = t_ld(batch);
+  const int splits = dw_splits(batch);
+  Arena m;
+  const Handed net(m, true);
+  const size_t feat = m.add<float>(batch * kFeat), tgt = m.add<float>(batch);
+  const size_t feat16 = m.add<bf16>(batch * kIn), feat_t = m.add<bf16>(ld * kIn), dz3_t = m.add<bf16>(ld * kOut);
+  size_t a_t[3], dz_t[3], work[4], part[4];
+  for (int l = 0; l < 3; l++) {
+    a_t[l] = m.add<bf16>(ld * kHidden);
+    dz_t[l] = m.add<bf16>(ld * kHidden);
   }
-  Net net;
-  if (int st = bude::surrogate::set_weights(net, w, b, s)) return st;
-  Acts A;
-  if (int st = bude::surrogate::alloc_acts(A, batch, true)) return st;
-  std::vector<float> fpad(batch * bude::mlp::kIn, 0.f);
-  for (size_t i = 0; i < batch; i++)
-    for (int c = 0; c < bude::mlp::kFeat; c++) fpad[i * bude::mlp::kIn + c] = features[i * bude::mlp::kFeat + c];
-  DeviceBuffer f32, tgt;
-  if (int st = f32.upload(fpad.data(), fpad.size() * 4)) return st;
-  if (int st = tgt.upload(target, batch * 4)) return st;
-  if (int st = bude::hip_check(bude::mlp::to_bf16(static_cast<const float *>(f32.ptr), int(batch), bude::mlp::kIn,
-                                                  static_cast<bf16 *>(A.feat.ptr), static_cast<bf16 *>(A.feat_t.ptr),
-                                                  s, A.ld_t, true),
-                               "to_bf16"))
+  for (int l = 0; l < 4; l++) {
+    work[l] = m.add<float>(size_t(splits) * kK[l] * kN[l]);
+    part[l] = m.add<float>(size_t(splits) * kN[l]);
+  }
+  // what comes back, in one piece: the loss sum, the gradients, the predictions
+  const size_t loss_floats = sizeof(unsigned long long) / sizeof(float);
+  const size_t nout = loss_floats + kGradCount + batch, out = m.add<float>(nout);
+  if (int st = m.alloc()) return st;
+  const Drain drain{s};
+  if (int st = net.upload(m, weights, biases, s)) return st;
+  if (int st = bude::hip_check(hipMemcpyAsync(m.at<float>(feat), features, batch * kFeat * sizeof(float),
+                                              hipMemcpyHostToDevice, s),
+                               "hipMemcpyAsync features"))
     return st;
-  if (int st = bude::hip_check(hipMemsetAsync(A.loss.ptr, 0, 8, s), "hipMemsetAsync")) return st;
-  bude::mlp::RowsArgs in{};
-  in.feat = static_cast<const bf16 *>(A.feat.ptr);
-  in.energy = static_cast<const float *>(tgt.ptr);
-  in.norm = bude::mlp::TargetNorm{3.0e38f, 0.f, 1.f, -3.0e38f};
+  if (int st = bude::hip_check(hipMemcpyAsync(m.at<float>(tgt), target, batch * sizeof(float), hipMemcpyHostToDevice,
+                                              s),
+                               "hipMemcpyAsync targets"))
+    return st;
+  float *dout = m.at<float>(out);
+  StageArgs sa = net.stage_args(m, true);
+  sa.feat = m.at<float>(feat);
+  sa.rows = batch;
+  sa.ld_t = ld;
+  sa.feat16 = m.at<bf16>(feat16);
+  sa.feat_t = m.at<bf16>(feat_t);
+  sa.dz3_t = m.at<bf16>(dz3_t);
+  sa.loss = reinterpret_cast<unsigned long long *>(dout);
+  if (int st = bude::hip_check(stage(sa, s), "mlp inputs")) return st;
+  RowsArgs in{};
+  in.feat = sa.feat16;
+  in.n = batch;
+  in.ld_t = ld;
+  in.energy = m.at<float>(tgt);
+  in.norm = TargetNorm{3.0e38f, 0.f, 1.f, -3.0e38f};
   in.tail_weight = 1.f;
-  in.pred = static_cast<float *>(A.pred.ptr);
-  if (int st = bude::surrogate::rows_step(net, A, batch, in, s)) return st;
-  if (int st = bude::surrogate::weight_grads(net, A, batch, s)) return st;
-  if (int st = bude::surrogate::sum_grads(net, A, s)) return st;
-  if (int st = bude::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;
-  if (int st = bude::hip_check(hipMemcpy(pred, A.pred.ptr, batch * 4, hipMemcpyDeviceToHost), "hipMemcpy")) return st;
-  unsigned long long lsum = 0;
-  if (int st = bude::hip_check(hipMemcpy(&lsum, A.loss.ptr, 8, hipMemcpyDeviceToHost), "hipMemcpy")) return st;
-  *loss = float(double(lsum) / bude::mlp::kLossScale / double(batch));
-  for (int l = 0; l < 4; l++) {
-    std::vector<float> gw(size_t(kK[l]) * kN[l]);
-    std::vector<float> gb(static_cast<size_t>(kN[l]));
-    if (int st = bude::hip_check(hipMemcpy(gw.data(), net.gw[l].ptr, gw.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy"))
-      return st;
-    if (int st = bude::hip_check(hipMemcpy(gb.data(), net.gb[l].ptr, gb.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy"))
-      return st;
-    for (int r = 0; r < realK[l]; r++)
-      for (int c = 0; c < realN[l]; c++) grad_w[l][size_t(r) * realN[l] + c] = gw[size_t(r) * kN[l] + c];
-    for (int c = 0; c < realN[l]; c++) grad_b[l][c] = gb[c];
+  in.pred = dout + loss_floats + kGradCount;
+  in.loss = sa.loss;
+  in.feat_t = sa.feat_t;
+  in.dz3_t = sa.dz3_t;
+  for (int l = 0; l < 3; l++) {
+    in.wt[l] = sa.wt[l];
+    in.a_t[l] = m.at<bf16>(a_t[l]);
+    in.dz_t[l] = m.at<bf16>(dz_t[l]);
   }
+  for (int l = 0; l < 4; l++) {
+    in.w[l] = l == 3 ? sa.w3 : sa.wx[l];  // (w[0] unused)
+    in.bias[l] = m.at<float>(net.b[l]);
+  }
+  if (int st = bude::hip_check(rows(in, s), "mlp rows")) return st;
+  DwArgs dw{};
+  dw.count = 4;
+  dw.k = batch;
+  dw.ld = ld;
+  dw.splits = splits;
+  for (int l = 0; l < 4; l++)
+    dw.d[l] = DwProduct{l == 0 ? in.feat_t : in.a_t[l - 1], l == 3 ? in.dz3_t : in.dz_t[l], kK[l], kN[l],
+                        m.at<float>(work[l]), m.at<float>(part[l])};
+  if (int st = bude::hip_check(weight_grads(dw, s), "mlp weight gradients")) return st;
+  if (int st = bude::hip_check(grads_out(dw, dout + loss_floats, s), "mlp gradients")) return st;
+  const std::unique_ptr<float[]> host(new (std::nothrow) float[nout]);
+  if (!host) return bude::fail(BUDE_ERR_OUT_OF_MEMORY, "bude_mi355x_mlp_forward_backward: no host memory");
+  if (int st = bude::hip_check(hipMemcpyAsync(host.get(), dout, nout * sizeof(float), hipMemcpyDeviceToHost, s),
+                               "hipMemcpyAsync"))
+    return st;
+  if (int st = bude::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;
+  unsigned long long lsum = 0;
+  std::memcpy(&lsum, host.get(), sizeof lsum);
+  *loss = float(double(lsum) / kLossScale / double(batch));
+  const float *p = host.get() + loss_floats;
+  for (int l = 0; l < 4; l++) {
+    const size_t n = size_t(kRealK[l]) * kRealN[l];
+    std::copy(p, p + n, grad_w[l]);
+    p += n;
+  }
+  for (int l = 0; l < 4; l++) {
+    std::copy(p, p + kRealN[l], grad_b[l]);
+    p += kRealN[l];
+  }
+  std::copy(p, p + batch, pred);
   return bude::ok();
 }
+
+// Poses from which the next poses are copied in and the last predictions out
+// while a piece of them is scored: 2^20 poses 1,650 us in one piece, 1,340 in
+// four, 1,380 in two, 1,530 in eight.
+constexpr size_t kPredictPiece = size_t(1) << 18;
 
 extern "C" int bude_mi355x_mlp_predict(int device, const float *const poses[6], size_t n,
                                        const float *const weights[4], const float *const biases[4], float *pred) {
   if (!poses || !weights || !biases || !pred || n == 0 || n > 0xffffffffu)
     return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_mlp_predict: bad arguments");
-  int ndev = 0;
-  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0 || device < 0 || device >= ndev)
-    return bude::fail(BUDE_ERR_NO_DEVICE, "bude_mi355x_mlp_predict: no such HIP device");
-  if (int st = bude::hip_check(hipSetDevice(device), "hipSetDevice")) return st;
-  hipStream_t s = nullptr;
-  if (int st = bude::hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate")) return st;
-  struct StreamGuard {
-    hipStream_t s;
-    ~StreamGuard() { (void)hipStreamDestroy(s); }
-  } guard{s};
-  const int realK[4] = {bude::mlp::kFeat, 256, 256, 256}, realN[4] = {256, 256, 256, 1};
-  std::vector<std::vector<float>> w(4), b(4);
-  for (int l = 0; l < 4; l++) {
-    w[l].assign(size_t(kK[l]) * kN[l], 0.f);
-    b[l].assign(size_t(kN[l]), 0.f);
-    for (int r = 0; r < realK[l]; r++)
-      for (int c = 0; c < realN[l]; c++) w[l][size_t(r) * kN[l] + c] = weights[l][size_t(r) * realN[l] + c];
-    for (int c = 0; c < realN[l]; c++) b[l][c] = biases[l][c];
-  }
-  Net net;
-  if (int st = bude::surrogate::set_weights(net, w, b, s)) return st;
-  DeviceBuffer dp, out;
-  if (int st = upload_poses(dp, poses, n)) return st;
-  if (int st = out.alloc(n * 4)) return st;
-  hipDeviceProp_t props{};
-  if (int st = bude::hip_check(hipGetDeviceProperties(&props, device), "hipGetDeviceProperties")) return st;
-  const bf16 *wt[4] = {static_cast<const bf16 *>(net.w16tx[0].ptr), static_cast<const bf16 *>(net.w16tx[1].ptr),
-                       static_cast<const bf16 *>(net.w16tx[2].ptr), nullptr};
-  const float *bias[4] = {static_cast<const float *>(net.b[0].ptr), static_cast<const float *>(net.b[1].ptr),
-                          static_cast<const float *>(net.b[2].ptr), static_cast<const float *>(net.b[3].ptr)};
-  if (int st = bude::hip_check(bude::mlp::infer(static_cast<const float *>(dp.ptr), n, n, wt,
-                                                static_cast<const bf16 *>(net.w16[3].ptr), bias,
-                                                static_cast<float *>(out.ptr), 2 * props.multiProcessorCount, s),
-                               "mlp infer"))
+  if (int st = check_device(device, "bude_mi355x_mlp_predict")) return st;
+  int cus = 0;
+  if (int st = bude::hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device),
+                               "hipDeviceGetAttribute"))
     return st;
-  if (int st = bude::hip_check(hipStreamSynchronize(s), "hipStreamSynchronize")) return st;
-  return bude::hip_check(hipMemcpy(pred, out.ptr, n * 4, hipMemcpyDeviceToHost), "hipMemcpy");
+  Arena m;
+  const Handed net(m, false);
+  const size_t dposes = m.add<float>(6 * n), dout = m.add<float>(n);
+  if (int st = m.alloc()) return st;
+  // copies in on the default stream; kernels and copies out behind them, on a
+  // stream of their own where there are several pieces
+  struct Side {
+    hipStream_t s = nullptr;
+    hipEvent_t ready = nullptr;
+    ~Side() {
+      (void)hipStreamSynchronize(nullptr);
+      if (s) {
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamDestroy(s);
+      }
+      if (ready) (void)hipEventDestroy(ready);
+    }
+  } side;
+  if (n > kPredictPiece) {
+    if (int st = bude::hip_check(hipStreamCreateWithFlags(&side.s, hipStreamNonBlocking), "hipStreamCreate")) return st;
+    if (int st = bude::hip_check(hipEventCreateWithFlags(&side.ready, hipEventDisableTiming), "hipEventCreate"))
+      return st;
+  }
+  if (int st = net.upload(m, weights, biases, nullptr)) return st;
+  const bude::mlp::StageArgs sa = net.stage_args(m, false);
+  if (int st = bude::hip_check(bude::mlp::stage(sa, nullptr), "mlp inputs")) return st;
+  const bf16 *wt[4] = {sa.wt[0], sa.wt[1], sa.wt[2], nullptr};
+  const float *bias[4] = {m.at<float>(net.b[0]), m.at<float>(net.b[1]), m.at<float>(net.b[2]), m.at<float>(net.b[3])};
+  float *dp = m.at<float>(dposes), *out = m.at<float>(dout);
+  auto fetch = [&](size_t first) {
+    return bude::hip_check(hipMemcpyAsync(pred + first, out + first, std::min(kPredictPiece, n - first) * sizeof(float),
+                                          hipMemcpyDeviceToHost, side.s),
+                           "hipMemcpyAsync predictions");
+  };
+  size_t last = 0;
+  for (size_t first = 0; first < n; first += kPredictPiece) {
+    const size_t k = std::min(kPredictPiece, n - first);
+    for (int r = 0; r < 6; r++)
+      if (int st = bude::hip_check(hipMemcpyAsync(dp + size_t(r) * n + first, poses[r] + first, k * sizeof(float),
+                                                  hipMemcpyHostToDevice, nullptr),
+                                   "hipMemcpyAsync poses"))
+        return st;
+    if (side.s) {
+      if (int st = bude::hip_check(hipEventRecord(side.ready, nullptr), "hipEventRecord")) return st;
+      if (first)
+        if (int st = fetch(last)) return st;
+      if (int st = bude::hip_check(hipStreamWaitEvent(side.s, side.ready, 0), "hipStreamWaitEvent")) return st;
+    }
+    if (int st = bude::hip_check(bude::mlp::infer(dp + first, n, k, wt, sa.w3, bias, out + first, 2 * cus, side.s),
+                                 "mlp infer"))
+      return st;
+    last = first;
+  }
+  if (int st = fetch(last)) return st;
+  return bude::hip_check(hipStreamSynchronize(side.s), "hipStreamSynchronize");
 }

@@ -181,16 +181,36 @@ struct AdamBatch {
 hipError_t adam_multi_dev(const AdamBatch &b, const float *hyper, float b1, float b2, float eps, hipStream_t s,
                           StepState *advance = nullptr);
 
+// The inputs of one pass over a network that is handed in whole, from their
+// FP32 arrays in device memory to what the kernels read, in one launch: the
+// weights w[l] (kRealK[l] x kRealN[l], row-major) as fragment-tiled W_l^T (wt,
+// l < 3) and W_l (wx[l], l = 1, 2, where set) and row-major W_3 (w3, column 0);
+// with feat set the features of `rows` rows ([rows][kFeat]) as feat16 and
+// feat_t, and dz3_t and loss cleared (RowsArgs).
+constexpr int kRealK[kLayers] = {kFeat, kHidden, kHidden, kHidden};
+constexpr int kRealN[kLayers] = {kHidden, kHidden, kHidden, 1};
+struct StageArgs {
+  const float *w[4];
+  bf16 *wt[3], *wx[3], *w3;
+  const float *feat;
+  size_t rows, ld_t;
+  bf16 *feat16, *feat_t, *dz3_t;
+  unsigned long long *loss;
+};
+hipError_t stage(const StageArgs &a, hipStream_t s);
+
+// The gradients of a pass: every slice sum of DwArgs (slices in order) in the
+// layers' real shapes, W_0 .. W_3 and then b_0 .. b_3, one after the other.
+constexpr size_t kGradCount = size_t(kFeat + 2 * kHidden + 1) * kHidden + 3 * kHidden + 1;
+hipError_t grads_out(const DwArgs &a, float *out, hipStream_t s);
+
 // FP32 -> BF16 fragment-tiled copies (tiled_index) of a rows x cols matrix
 // (wx, rows a multiple of 16, cols of 32) and of its transpose (wtx, cols a
 // multiple of 16, rows of 32); either may be null.
 hipError_t tile_bf16(const float *w, int rows, int cols, bf16 *wx, bf16 *wtx, hipStream_t s);
 
-// FP32 -> BF16 of a rows x cols matrix and its transpose (cols x ldt, ldt 0:
-// rows; tiled: fragment-tiled, tiled_index, cols a multiple of 16 and ldt of
-// 32).
-hipError_t to_bf16(const float *w, int rows, int cols, bf16 *w16, bf16 *w16t, hipStream_t s, size_t ldt = 0,
-                   bool tiled = false);
+// FP32 -> BF16 of a rows x cols matrix and its transpose (cols x rows).
+hipError_t to_bf16(const float *w, int rows, int cols, bf16 *w16, bf16 *w16t, hipStream_t s);
 
 // Fused inference: predictions (standardised units) of n poses through the
 // whole network, activations kept in LDS; wt[l] = W_l^T [N_l][K_l] (BF16,

@@ -567,12 +567,74 @@ __global__ void tile_bf16_kernel(const float *__restrict__ w, int rows, int cols
 }
 
 __global__ void to_bf16_kernel(const float *__restrict__ w, int rows, int cols, bf16 *__restrict__ w16,
-                               bf16 *__restrict__ w16t, size_t ldt, int tiled) {
+                               bf16 *__restrict__ w16t) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= size_t(rows) * cols) return;
   const bf16 h = to_bf16(w[i]);
   if (w16) w16[i] = h;
-  if (w16t) w16t[tiled ? tiled_index(i % cols, i / cols, ldt) : size_t(i % cols) * ldt + i / cols] = h;
+  if (w16t) w16t[size_t(i % cols) * rows + i / cols] = h;
+}
+
+// One work-item per padded weight (the layers one after the other), then per
+// feature entry (row-major [rows][kIn]), 16 bytes of dz3_t at a time.
+constexpr size_t kPadded = size_t(kIn + 2 * kHidden) * kHidden + size_t(kHidden) * kOut;
+
+__global__ __launch_bounds__(256) void stage_kernel(const StageArgs a) {
+  size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < kPadded) {
+    int l = 0;
+    for (; l < 3; l++) {
+      const size_t n = size_t(l ? kHidden : kIn) * kHidden;
+      if (i < n) break;
+      i -= n;
+    }
+    const int cols = l < 3 ? kHidden : kOut, k = int(i) / cols, c = int(i) % cols;
+    const bf16 h = k < kRealK[l] && c < kRealN[l] ? to_bf16(a.w[l][size_t(k) * kRealN[l] + c]) : bf16(0);
+    if (l == 3) {
+      a.w3[i] = h;
+      return;
+    }
+    a.wt[l][tiled_index(c, k, size_t(l ? kHidden : kIn))] = h;
+    if (a.wx[l]) a.wx[l][tiled_index(k, c, kHidden)] = h;
+    return;
+  }
+  i -= kPadded;
+  if (a.feat && i < a.rows * kIn) {
+    const size_t row = i / kIn, c = i % kIn;
+    const bf16 h = c < kFeat ? to_bf16(a.feat[row * kFeat + c]) : bf16(0);
+    a.feat16[i] = h;
+    a.feat_t[tiled_index(c, row, a.ld_t)] = h;
+  }
+  if (a.feat && i < a.ld_t * kOut / 8) reinterpret_cast<uint4 *>(a.dz3_t)[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (a.feat && i == 0) *a.loss = 0ull;
+}
+
+__global__ __launch_bounds__(256) void grads_out_kernel(const DwArgs a, float *__restrict__ out) {
+  size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= kGradCount) return;
+  float *o = out + i;
+  const float *src = nullptr;  // the entry in slice 0
+  size_t stride = 0;
+  for (int l = 0; l < 4 && !src; l++) {
+    const size_t n = size_t(kRealK[l]) * kRealN[l];
+    if (i < n) {
+      src = a.d[l].work + i / kRealN[l] * a.d[l].N + i % kRealN[l];
+      stride = size_t(a.d[l].M) * a.d[l].N;
+    } else {
+      i -= n;
+    }
+  }
+  for (int l = 0; l < 4 && !src; l++) {
+    if (i < size_t(kRealN[l])) {
+      src = a.d[l].bias_part + i;
+      stride = size_t(a.d[l].N);
+    } else {
+      i -= size_t(kRealN[l]);
+    }
+  }
+  float acc = 0.f;
+  for (int z = 0; z < a.splits; z++) acc += src[size_t(z) * stride];
+  *o = acc;
 }
 
 // ---- fused inference ---------------------------------------------------------
@@ -774,12 +836,22 @@ hipError_t tile_bf16(const float *w, int rows, int cols, bf16 *wx, bf16 *wtx, hi
   return hipGetLastError();
 }
 
-hipError_t to_bf16(const float *w, int rows, int cols, bf16 *w16, bf16 *w16t, hipStream_t s, size_t ldt,
-                   bool tiled) {
-  if (ldt == 0) ldt = size_t(rows);
-  if (ldt < size_t(rows) || (tiled && (cols % 16 || ldt % 32))) return hipErrorInvalidValue;
+hipError_t to_bf16(const float *w, int rows, int cols, bf16 *w16, bf16 *w16t, hipStream_t s) {
   hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(size_t(rows) * cols, 256)), dim3(256), 0, s, w, rows, cols, w16,
-                     w16t, ldt, int(tiled));
+                     w16t);
+  return hipGetLastError();
+}
+
+hipError_t stage(const StageArgs &a, hipStream_t s) {
+  if (a.feat && (a.rows == 0 || a.ld_t < a.rows || a.ld_t % 32)) return hipErrorInvalidValue;
+  const size_t n = kPadded + (a.feat ? std::max(a.rows * kIn, a.ld_t * kOut / 8) : 0);
+  hipLaunchKernelGGL(stage_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t grads_out(const DwArgs &a, float *out, hipStream_t s) {
+  if (a.count != 4 || a.splits < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(grads_out_kernel, dim3(blocks_for(kGradCount, 256)), dim3(256), 0, s, a, out);
   return hipGetLastError();
 }
 

@@ -19,7 +19,7 @@ constexpr int kK[4] = {mlp::kIn, mlp::kHidden, mlp::kHidden, mlp::kHidden};
 constexpr int kN[4] = {mlp::kHidden, mlp::kHidden, mlp::kHidden, mlp::kOut};
 
 struct Net {
-  DeviceBuffer w[4], b[4], mw[4], vw[4], mb[4], vb[4], gw[4], gb[4];
+  DeviceBuffer w[4], b[4], mw[4], vw[4], mb[4], vb[4];
   // BF16 copies the kernels read, refreshed by every Adam step:
   // fragment-tiled W_l^T (l < 3: the forward products of training and
   // inference, the descriptor fold) and W_l (l = 1, 2: the backward
@@ -28,28 +28,25 @@ struct Net {
   int step = 0;
 };
 
-// The rows of one batch of `rows` poses: BF16 features, and in training the
-// transposed rows the weight-gradient products read (X^T, A_l^T, dZ_l^T,
-// dz3^T: fragment-tiled with ld_t = mlp::t_ld(rows) columns), predictions and
-// the loss sum.
+// The rows of one training batch of `rows` poses: the transposed rows the
+// weight-gradient products read (X^T, A_l^T, dZ_l^T, dz3^T: fragment-tiled
+// with ld_t = mlp::t_ld(rows) columns) and the loss sum.
 struct Acts {
   size_t rows = 0, ld_t = 0;
-  DeviceBuffer feat, feat_t, a_t[3], pred, dz3_t, dz_t[3], loss;
+  DeviceBuffer feat_t, a_t[3], dz3_t, dz_t[3], loss;
   // weight and bias gradients of layer l as splits[l] K slices (summed in a
-  // fixed order by the Adam step, in slice order by sum_grads)
+  // fixed order by the Adam step)
   DeviceBuffer gpart[4], bpart[4];
   int splits[4] = {1, 1, 1, 1};
 };
 
-int alloc_acts(Acts &A, size_t rows, bool training);
+int alloc_acts(Acts &A, size_t rows);
 // The fused rows kernel over `rows` rows (mlp::rows) with the network's
 // weights and A's buffers filled in from in's inputs and targets.
 int rows_step(const Net &net, Acts &A, size_t rows, const mlp::RowsArgs &in, hipStream_t s);
 // From the transposed rows: the weight and bias gradients as K slices in
 // A.gpart / bpart.
 int weight_grads(Net &net, Acts &A, size_t rows, hipStream_t s);
-// The slices summed in order into net.gw / gb.
-int sum_grads(Net &net, const Acts &A, hipStream_t s);
 // Uploads FP32 weights W_l [kK[l]][kN[l]] (zero padded) and biases, clears
 // the Adam state and refreshes the BF16 copies.
 int set_weights(Net &net, const std::vector<std::vector<float>> &w, const std::vector<std::vector<float>> &b,

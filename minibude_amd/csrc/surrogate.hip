@@ -12,28 +12,24 @@
 namespace bude {
 namespace surrogate {
 
-int alloc_acts(Acts &A, size_t rows, bool training) {
+int alloc_acts(Acts &A, size_t rows) {
   A.rows = rows;
   A.ld_t = mlp::t_ld(rows);
   const size_t H = mlp::kHidden, O = mlp::kOut, I = mlp::kIn, ld = A.ld_t;
-  int st = A.feat.alloc(rows * I * 2);
-  if (!st) st = A.pred.alloc(rows * 4);
-  if (training) {
-    if (!st) st = A.feat_t.alloc(ld * I * 2);
-    for (int l = 0; l < 3 && !st; l++) {
-      st = A.a_t[l].alloc(ld * H * 2);
-      if (!st) st = A.dz_t[l].alloc(ld * H * 2);
-    }
-    // dz3^T: row 0 is written every step, rows 1.. stay zero (the padded
-    // output columns of the last weight gradient)
-    if (!st) st = A.dz3_t.alloc(ld * O * 2);
-    if (!st) st = hip_check(hipMemset(A.dz3_t.ptr, 0, ld * O * 2), "hipMemset");
-    if (!st) st = A.loss.alloc(256);
-    for (int l = 0; l < 4 && !st; l++) {
-      const size_t cap = size_t(mlp::kDwSplits);
-      st = A.gpart[l].alloc(cap * kK[l] * kN[l] * 4);
-      if (!st) st = A.bpart[l].alloc(cap * kN[l] * 4);
-    }
+  int st = A.feat_t.alloc(ld * I * 2);
+  for (int l = 0; l < 3 && !st; l++) {
+    st = A.a_t[l].alloc(ld * H * 2);
+    if (!st) st = A.dz_t[l].alloc(ld * H * 2);
+  }
+  // dz3^T: row 0 is written every step, rows 1.. stay zero (the padded
+  // output columns of the last weight gradient)
+  if (!st) st = A.dz3_t.alloc(ld * O * 2);
+  if (!st) st = hip_check(hipMemset(A.dz3_t.ptr, 0, ld * O * 2), "hipMemset");
+  if (!st) st = A.loss.alloc(256);
+  for (int l = 0; l < 4 && !st; l++) {
+    const size_t cap = size_t(mlp::kDwSplits);
+    st = A.gpart[l].alloc(cap * kK[l] * kN[l] * 4);
+    if (!st) st = A.bpart[l].alloc(cap * kN[l] * 4);
   }
   return st;
 }
@@ -79,20 +75,6 @@ int weight_grads(Net &net, Acts &A, size_t rows, hipStream_t s) {
   return hip_check(mlp::weight_grads(a, s), "mlp weight gradients");
 }
 
-int sum_grads(Net &net, const Acts &A, hipStream_t s) {
-  for (int l = 0; l < 4; l++) {
-    if (int st = hip_check(mlp::sum_slices(static_cast<const float *>(A.gpart[l].ptr), A.splits[l],
-                                           size_t(kK[l]) * kN[l], static_cast<float *>(net.gw[l].ptr), s),
-                           "mlp dW"))
-      return st;
-    if (int st = hip_check(mlp::sum_slices(static_cast<const float *>(A.bpart[l].ptr), A.splits[l], size_t(kN[l]),
-                                           static_cast<float *>(net.gb[l].ptr), s),
-                           "mlp db"))
-      return st;
-  }
-  return BUDE_OK;
-}
-
 // Upload FP32 weights W_l [kK[l]][kN[l]] (zero padded) and biases; refresh BF16 copies.
 int set_weights(Net &net, const std::vector<std::vector<float>> &w, const std::vector<std::vector<float>> &b,
                 hipStream_t s) {
@@ -100,12 +82,12 @@ int set_weights(Net &net, const std::vector<std::vector<float>> &w, const std::v
     const size_t nw = size_t(kK[l]) * kN[l];
     int st = net.w[l].upload(w[l].data(), nw * 4);
     if (!st) st = net.b[l].upload(b[l].data(), size_t(kN[l]) * 4);
-    for (DeviceBuffer *d : {&net.mw[l], &net.vw[l], &net.gw[l]})
+    for (DeviceBuffer *d : {&net.mw[l], &net.vw[l]})
       if (!st) {
         st = d->alloc(nw * 4);
         if (!st) st = hip_check(hipMemset(d->ptr, 0, nw * 4), "hipMemset");
       }
-    for (DeviceBuffer *d : {&net.mb[l], &net.vb[l], &net.gb[l]})
+    for (DeviceBuffer *d : {&net.mb[l], &net.vb[l]})
       if (!st) {
         st = d->alloc(size_t(kN[l]) * 4);
         if (!st) st = hip_check(hipMemset(d->ptr, 0, size_t(kN[l]) * 4), "hipMemset");
@@ -150,7 +132,7 @@ int train(Net &net, const TrainData &d, std::vector<uint32_t> perm, const TrainP
   if (B == 0 || B % 32 || ntrain < B || !d.poses || !d.energy || (d.table && !d.lig) || (d.desc && !d.lig))
     return fail(BUDE_ERR_INVALID_ARGUMENT, "surrogate train: need at least one batch of labels");
   Acts A;
-  if (int st = alloc_acts(A, B, true)) return st;
+  if (int st = alloc_acts(A, B)) return st;
   std::mt19937_64 rng(p.seed);
   DeviceBuffer dperm, dstate;
   if (int st = dperm.alloc(ntrain * 4)) return st;

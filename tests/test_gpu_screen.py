@@ -150,3 +150,16 @@ def test_configured_12_inputs_at_2pct(gpu_device):
     assert rec > 0.5  # far above the 0.02 of a random ranking
     if rec < 0.99:
         pytest.xfail(f"the configured pose MLP keeps {rec:.3f} of the exact top 1 % at 2 % rescored, below 0.99")
+
+
+@pytest.mark.parametrize("n", [1, 129, (1 << 18) + 1, 3 * (1 << 18) - 5])
+def test_predictions_do_not_depend_on_the_pieces(gpu_device, n):
+    # large sets go through in pieces: the same bits as pose sets of 100,000
+    rng = np.random.default_rng(31)
+    shapes = ((21, 256), (256, 256), (256, 256), (256, 1))
+    W = [(rng.standard_normal(s) * 0.08).astype(np.float32) for s in shapes]
+    b = [(0.05 * rng.standard_normal(s[1])).astype(np.float32) for s in shapes]
+    poses = D.synth_poses(32, n)
+    got = S.mlp_predict(poses, W, b, gpu_device)
+    want = np.concatenate([S.mlp_predict(poses[:, i:i + 100000], W, b, gpu_device) for i in range(0, n, 100000)])
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
