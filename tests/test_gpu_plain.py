@@ -186,3 +186,17 @@ def test_every_group_size(gpu_device):
                 first = e
             else:  # the register block only changes which lane holds a pose, never the sums
                 assert np.array_equal(e.view(np.uint32), first.view(np.uint32))
+
+
+@pytest.mark.parametrize("nposes", [1, 4096, (1 << 15) + 1])
+def test_energies_of_a_call_without_passes_are_the_last_ones(gpu_device, nposes):
+    # few energies are left where the host reads them, many are copied out;
+    # either way they are there for a later call that runs no pass, and a pass
+    # that nobody reads is the one a later call returns
+    d = D.synth_deck(80, 7, nposes, seed=41)
+    with Context(d, gpu_device) as c:
+        first = c.fasten(1, 64).energies
+        assert np.array_equal(c.fasten(1, 64, 0, 0).energies, first)
+        c.fasten(1, 64, 1, 2, want_energies=False)
+        assert np.array_equal(c.fasten(1, 64, 0, 0).energies, first)
+        assert np.array_equal(c.fasten(1, 64, 1, 2).energies, first)
