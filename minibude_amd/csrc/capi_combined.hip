@@ -1306,9 +1306,10 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
       if (int st = train_atom(c, pseed)) return st;
     } else {
       if (int st = bude::hip_check(
-              bude::field::build_maps(static_cast<const float4 *>(c->s().protein.ptr),
+              bude::field::build_maps(static_cast<const float4 *>(c->s().protein.ptr), int(natpro),
                                       static_cast<const int32_t *>(c->s().group_begin.ptr),
-                                      static_cast<const bude::PairCoef *>(c->s().slot_coef.ptr), int(c->s().ngroups),
+                                      static_cast<const bude::PairCoef *>(c->s().slot_coef.ptr),
+                                      c->s().reachable ? c->s().scene.reach2 : nullptr, int(c->s().ngroups),
                                       int(nslots), c->grid, bude::plain_form(), static_cast<float *>(c->maps.ptr),
                                       c->stream2),
               "build maps"))

@@ -34,8 +34,12 @@ struct Grid {
 // pair coefficients are coef[s * ngroups + g] (g over the protein groups) at
 // point lo + h * (ix, iy, iz): 0.5 * the sum of the pair energies, groups in
 // order, exactly as the plain kernel sums one ligand atom.
-hipError_t build_maps(const float4 *protein, const int32_t *group_begin, const PairCoef *coef, int ngroups,
-                      int nslots, const Grid &g, int form, float *maps, hipStream_t s);
+// reach2: the coefficients' squared reaches (items::Scene::reach2; the natpro
+// atoms of the protein then carry their group in the w bits), or null where
+// some pair has none.
+hipError_t build_maps(const float4 *protein, int natpro, const int32_t *group_begin, const PairCoef *coef,
+                      const float4 *reach2, int ngroups, int nslots, const Grid &g, int form, float *maps,
+                      hipStream_t s);
 
 // Cells of the maps: cell (ix, iy, iz) of slot s holds its 8 corner values
 // [v000 v001 v010 v011 v100 v101 v110 v111] (index bits x y z) as FP16

@@ -137,6 +137,111 @@ __global__ __launch_bounds__(256) void map_kernel(const float4 *__restrict__ pro
   if (valid) maps[size_t(blockIdx.y) * g.points() + (size_t(ix) * size_t(g.n[1]) + size_t(iy)) * size_t(g.n[2]) + size_t(iz)] = e * 0.5f;
 }
 
+// The maps of kMapSlots slots at a time, for pairs that all have a reach
+// (items::reach_table; map_kernel is for the others): one wave per brick takes
+// the protein 64 atoms at a time (lane = atom) against its brick's box, and
+// every atom in reach of any of the slots out of its lane to all points.  A
+// pair's distance is formed once for the slots, and a hinge is added where the
+// atom is within that hinge's reach for any of them; what is left out is
+// exactly zero and the rest is summed as in map_kernel.  34 slots of 238,328
+// points against 2,046 atoms, beside the sampled-pose pass: map_kernel 955 us (it
+// takes the whole protein per slot), 360 with 6 slots, 340, 380 and 360 with 4,
+// 8 and 9; VALU issue bounds it.
+constexpr int kMapSlots = 6;
+
+template <int FORM>
+__global__ __launch_bounds__(256) void map_slots_kernel(const float4 *__restrict__ protein, int natpro,
+                                                        const PairCoef *__restrict__ coef,
+                                                        const float4 *__restrict__ reach2, int ngroups, int nslots,
+                                                        const Grid g, float *__restrict__ maps) {
+  __builtin_amdgcn_s_setprio(2);  // (as in map_kernel)
+  constexpr int S = kMapSlots;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int nb1 = (g.n[1] + 3) / 4, nb2 = (g.n[2] + 3) / 4;
+  const int64_t nbricks = int64_t((g.n[0] + 3) / 4) * nb1 * nb2;
+  const int64_t brick = int64_t(blockIdx.x) * 4 + wave;
+  if (brick >= nbricks) return;  // whole wave
+  const int b[3] = {int(brick / (int64_t(nb1) * nb2)), int((brick / nb2) % nb1), int(brick % nb2)};
+  const int i[3] = {4 * b[0] + (lane >> 4), 4 * b[1] + ((lane >> 2) & 3), 4 * b[2] + (lane & 3)};
+  const bool valid = i[0] < g.n[0] && i[1] < g.n[1] && i[2] < g.n[2];
+  float at[3], lo[3], hi[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    at[d] = g.lo[d] + float(min(i[d], g.n[d] - 1)) * g.h;
+    lo[d] = g.lo[d] + float(4 * b[d]) * g.h;
+    hi[d] = g.lo[d] + float(min(4 * b[d] + 3, g.n[d] - 1)) * g.h;
+  }
+  const int s0 = int(blockIdx.y) * S;
+  float e[S], part[S];
+#pragma unroll
+  for (int s = 0; s < S; s++) e[s] = part[s] = 0.f;
+  // the largest reaches of the slots for an atom's group
+  auto reaches = [&](int group) {
+    float4 r = make_float4(-1.f, -1.f, -1.f, -1.f);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      const float4 v = reach2[size_t(min(s0 + s, nslots - 1)) * size_t(ngroups) + size_t(group)];
+      r = make_float4(fmaxf(r.x, v.x), fmaxf(r.y, v.y), fmaxf(r.z, v.z), fmaxf(r.w, v.w));
+    }
+    return r;
+  };
+  PairCoef c[S];
+  float c0[S], e0[S];
+  int cur = -1;
+  // two steps ahead: the atoms; one step ahead: their reach
+  float4 p = protein[min(lane, natpro - 1)], p1 = protein[min(64 + lane, natpro - 1)];
+  float4 r = reaches(__float_as_int(p.w));
+  for (int k0 = 0; k0 < natpro; k0 += 64) {
+    const float4 r1 = reaches(__float_as_int(p1.w));
+    const float4 p2 = protein[min(k0 + 128 + lane, natpro - 1)];
+    const float dx = p.x - __builtin_amdgcn_fmed3f(p.x, lo[0], hi[0]);
+    const float dy = p.y - __builtin_amdgcn_fmed3f(p.y, lo[1], hi[1]);
+    const float dz = p.z - __builtin_amdgcn_fmed3f(p.z, lo[2], hi[2]);
+    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+    const bool on = k0 + lane < natpro;
+    uint64_t mask = __ballot(on && d2 < r.w);
+    const uint64_t ms = __ballot(on && d2 < r.x), mq = __ballot(on && d2 < r.y), md = __ballot(on && d2 < r.z);
+    while (mask) {
+      const int j = __builtin_ctzll(mask);
+      mask &= mask - 1;
+      const int group = __builtin_amdgcn_readlane(__float_as_int(p.w), j);
+      if (group != cur) {
+        cur = group;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+          e[s] += part[s];
+          part[s] = 0.f;
+          c[s] = coef[size_t(min(s0 + s, nslots - 1)) * size_t(ngroups) + size_t(group)];
+          c0[s] = vgpr_copy(c[s].c0);
+          e0[s] = vgpr_copy(c[s].e0);
+        }
+      }
+      const float px = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.x), j));
+      const float py = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.y), j));
+      const float pz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p.z), j));
+      const float d = pair_distance(at[0] - px, at[1] - py, at[2] - pz);
+      auto x = [&](int s) { return FORM == kFormB ? d - c[s].radij : d; };
+      if (ms >> j & 1)
+#pragma unroll
+        for (int s = 0; s < S; s++) part[s] = steric<FORM>(x(s), c[s], part[s]);
+      if (mq >> j & 1)
+#pragma unroll
+        for (int s = 0; s < S; s++) part[s] = charge<FORM>(x(s), c[s], c0[s], part[s]);
+      if (md >> j & 1)
+#pragma unroll
+        for (int s = 0; s < S; s++) part[s] = desolvation<FORM>(x(s), c[s], e0[s], part[s]);
+    }
+    p = p1;
+    p1 = p2;
+    r = r1;
+  }
+  if (!valid) return;
+  const size_t out = (size_t(i[0]) * size_t(g.n[1]) + size_t(i[1])) * size_t(g.n[2]) + size_t(i[2]);
+#pragma unroll
+  for (int s = 0; s < S; s++)
+    if (s0 + s < nslots) maps[size_t(s0 + s) * g.points() + out] = (e[s] + part[s]) * 0.5f;
+}
+
 // Cell index and fraction along one axis, clamped to the grid.
 __device__ __forceinline__ void cell(float w, float lo, float inv_h, int n, int &i0, float &f) {
   const float u = (w - lo) * inv_h;
@@ -259,13 +364,24 @@ __global__ __launch_bounds__(256) void sum_kernel(const float *__restrict__ part
 
 }  // namespace
 
-hipError_t build_maps(const float4 *protein, const int32_t *group_begin, const PairCoef *coef, int ngroups,
-                      int nslots, const Grid &g, int form, float *maps, hipStream_t s) {
+hipError_t build_maps(const float4 *protein, int natpro, const int32_t *group_begin, const PairCoef *coef,
+                      const float4 *reach2, int ngroups, int nslots, const Grid &g, int form, float *maps,
+                      hipStream_t s) {
   const size_t np = g.points();
   if (np == 0 || nslots <= 0 || nslots > 65535 || g.n[0] < 2 || g.n[1] < 2 || g.n[2] < 2 || np > 0x7fffffffu ||
       (np + 255) / 256 > 0x7fffffffu)
     return hipErrorInvalidValue;
   const size_t nbricks = size_t((g.n[0] + 3) / 4) * size_t((g.n[1] + 3) / 4) * size_t((g.n[2] + 3) / 4);
+  if (reach2) {
+    const dim3 grid(unsigned((nbricks + 3) / 4), unsigned((nslots + kMapSlots - 1) / kMapSlots));
+    if (form == kFormD)
+      hipLaunchKernelGGL(map_slots_kernel<kFormD>, grid, dim3(256), 0, s, protein, natpro, coef, reach2, ngroups,
+                         nslots, g, maps);
+    else
+      hipLaunchKernelGGL(map_slots_kernel<kFormB>, grid, dim3(256), 0, s, protein, natpro, coef, reach2, ngroups,
+                         nslots, g, maps);
+    return hipGetLastError();
+  }
   const dim3 grid(unsigned((nbricks + 3) / 4), unsigned(nslots));
   if (form == kFormD)
     hipLaunchKernelGGL(map_kernel<kFormD>, grid, dim3(256), 0, s, protein, group_begin, coef, ngroups, g, maps);

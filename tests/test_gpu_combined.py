@@ -72,6 +72,27 @@ def test_field_maps_are_single_atom_plain_energies(gpu_device):
     assert np.array_equal(m.ravel().view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("ntypes", [1, 6, 7, 13])  # whole batches of slots and remainders
+def test_every_map_is_its_types_plain_energies(gpu_device, ntypes):
+    ff = D.synth_forcefield(33, ntypes)
+    lig = D.synth_ligand(34, 40, ntypes)
+    lig["type"] = np.arange(40) % ntypes
+    pro = D.synth_protein(35, 130, ntypes)
+    cfg = C.default_config("field", grid_spacing=1.0, max_val_rmse=1e9, gate_z=0.0)
+    with C.Combined(ff, [lig], [D.synth_poses(36, 512)], cfg, gpu_device) as c:
+        c.screen(pro)
+        lo, h, n = c.grid()
+        maps = {int(t): c.map(int(t)) for t in np.unique(lig["type"])}
+    g = [lo[k] + h * np.arange(n[k], dtype=np.float32) for k in range(3)]
+    X, Y, Z = np.meshgrid(*g, indexing="ij")
+    poses = np.zeros((6, X.size), np.float32)
+    poses[3], poses[4], poses[5] = X.ravel(), Y.ravel(), Z.ravel()
+    for t, m in maps.items():
+        atom = np.array([(0.0, 0.0, 0.0, t)], dtype=lig.dtype)
+        want = plain_energies(pro, atom, ff, poses, gpu_device)
+        assert np.array_equal(m.ravel().view(np.uint32), want.view(np.uint32)), t
+
+
 @pytest.mark.parametrize("groups,chunks,launch_tiles", [("8", 0, 0), ("8", 3, 0), ("8", 2, 5), ("1", 0, 0)])
 def test_field_score_is_trilinear_sum_over_atoms(gpu_device, monkeypatch, groups, chunks, launch_tiles):
     # groups: the scorer's atoms split by map slot over the 8 XCDs (partial
