@@ -1274,14 +1274,14 @@ hipError_t label_points(const float4 *protein, const int32_t *group_begin, const
 int index_points(PointIndex &idx, const field::Grid &grid, const float4 *points, const uint32_t *perm, size_t ntrain,
                  size_t nval, size_t batch, size_t limit, hipStream_t s) {
   const size_t n = ntrain + nval, nodes = grid.points();
-  if (n == 0 || batch == 0 || ntrain % batch || batch > (size_t(1) << 28) || nodes > 0x7fffffffu)
+  if (n == 0 || batch == 0 || ntrain % batch || nodes > 0x7fffffffu)
     return fail(BUDE_ERR_INVALID_ARGUMENT, "atomnet index: the training points must be whole batches");
   const size_t batches = ntrain / batch, counts = batches * (nodes + 1) * sizeof(uint32_t);
   idx.ntrain = ntrain;
   idx.nval = nval;
   idx.batch = batch;
   idx.nodes = nodes;
-  idx.gathered = ntrain > 0 && counts + ntrain * 8 * sizeof(uint2) <= limit;
+  idx.gathered = ntrain > 0 && batch <= (size_t(1) << 28) && counts + ntrain * 8 * sizeof(uint2) <= limit;
   DeviceBuffer places;  // (of a row among its nodes' terms)
   int st = idx.cells.reserve(n * sizeof(int4));
   if (!st) st = idx.slots.reserve(n * sizeof(uint32_t));

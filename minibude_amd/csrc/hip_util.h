@@ -35,6 +35,7 @@ struct DeviceBuffer {
     reset();
     if (n == 0) n = 4;
     if (int st = hip_check(hipMalloc(&ptr, n), "hipMalloc")) {
+      (void)hipGetLastError();  // (reported here: a caller that goes on without the memory is not to find it after its next launch)
       ptr = nullptr;
       return st;
     }
@@ -73,6 +74,7 @@ struct PinnedBuffer {
     if (ptr) (void)hipHostFree(ptr);
     ptr = nullptr;
     if (int st = hip_check(hipHostMalloc(&ptr, n ? n : 4, hipHostMallocDefault), "hipHostMalloc")) {
+      (void)hipGetLastError();  // (as above)
       ptr = nullptr;
       return st;
     }
