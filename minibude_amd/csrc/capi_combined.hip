@@ -269,12 +269,12 @@ struct bude_combined {
   // ceil(keep n) selected rows of each pair (sorted_rows; the tiled kernel
   // scores rows past them: ties, and what widening adds), every pose of every
   // pair (planned when first wanted) and of a protein's fallback pairs, on
-  // the first stream; the sampled poses on the third.  sorted_ok: their memory could be had.
+  // the first stream; the sampled poses on the third.
   std::vector<std::unique_ptr<bude::items::Plan>> chunk_sorted;
   bude::items::Plan whole_sorted, all_sorted, fb_sorted, label_sorted;
   bude::items::Workspace work, label_work;
   DeviceBuffer sorted_rows;
-  bool sorted_ok = false, label_sorted_ok = false, all_planned = false;
+  bool all_planned = false;
   bool plan_ok = false;               // the selection tables above are complete
   bude::field::Grid grid{};
   // the screen's proteins: the one screened last is slots[cur]; a batch
@@ -392,17 +392,21 @@ int plan_sorted(const bude_combined *c, bude::items::Plan &plan, const std::vect
   return plan.build(atoms, off, int(c->slot_type.size()), segs);
 }
 
-// Room for a planned pass; *ok is false when the device has none (the tiled
-// kernels then score instead).
-int reserve_sorted(const bude::items::Plan &plan, bude::items::Workspace &w, bool *ok) {
+// Room for a planned pass, where the device has it (the tiled kernels score
+// instead where it has none).
+int reserve_sorted(const bude::items::Plan &plan, bude::items::Workspace &w) {
   const int st = plan.reserve(w);
-  *ok = st == BUDE_OK;
   return st == BUDE_ERR_OUT_OF_MEMORY ? BUDE_OK : st;
 }
 
-// Whether protein slot ps is scored by this sorted pass.
-bool use_sorted(const ProteinSlot &ps, const bude::items::Plan &plan, bool ok) {
-  return ok && ps.reachable && plan.worth(size_t(ps.scene.natpro));
+// Whether a sorted pass of protein slot ps pays.
+bool sorted_pays(const ProteinSlot &ps, const bude::items::Plan &plan) {
+  return ps.reachable && plan.worth(size_t(ps.scene.natpro));
+}
+
+// Whether protein slot ps is scored by this sorted pass, with scratch w.
+bool use_sorted(const ProteinSlot &ps, const bude::items::Plan &plan, const bude::items::Workspace &w) {
+  return sorted_pays(ps, plan) && plan.fits(w);
 }
 
 // Work tables of one persistent batched launch scoring spans[i].n poses of
@@ -470,7 +474,7 @@ int launch_exact(bude_combined *c, const float *poses, size_t stride, float *ene
 // screen returns comes from the sorted or the tiled kernels.
 int launch_sampled(bude_combined *c, const float *poses, size_t stride, float *energies, const DeviceBuffer &meta,
                    const DeviceBuffer &tiles, int ntiles, hipStream_t stream) {
-  if (use_sorted(c->s(), c->label_sorted, c->label_sorted_ok))
+  if (use_sorted(c->s(), c->label_sorted, c->label_work))
     return bude::hip_check(c->label_sorted.launch(c->s().scene, c->label_work, poses, stride, nullptr, energies, stream),
                            "combined sampled-pose pass");
   if (ntiles == 0) return BUDE_OK;
@@ -495,12 +499,11 @@ int launch_sampled(bude_combined *c, const float *poses, size_t stride, float *e
 int exact_ragged(bude_combined *c, const std::vector<Span> &spans, const float *poses, size_t stride,
                  float *energies, DeviceBuffer &meta, DeviceBuffer &tiles, const bude::items::Plan *plan = nullptr) {
   if (plan && !spans.empty()) {
-    bool ok = plan->fits(c->work);
-    if (!ok && use_sorted(c->s(), *plan, true)) {  // (growing the scratch frees what queued passes use)
+    if (sorted_pays(c->s(), *plan) && !plan->fits(c->work)) {  // (growing the scratch frees what queued passes use)
       if (int st = bude::hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return st;
-      if (int st = reserve_sorted(*plan, c->work, &ok)) return st;
+      if (int st = reserve_sorted(*plan, c->work)) return st;
     }
-    if (use_sorted(c->s(), *plan, ok))
+    if (use_sorted(c->s(), *plan, c->work))
       return bude::hip_check(plan->launch(c->s().scene, c->work, poses, stride, nullptr, energies, c->stream),
                              "combined sorted pass");
   }
@@ -843,13 +846,12 @@ int plan_selection(bude_combined *c, float keep) {
   }
   if (int st = c->sorted_rows.assign(sorted_rows.data(), L * 4)) return st;
   c->chunk_sorted.clear();
-  c->sorted_ok = true;
-  for (size_t k = 0; k <= K && c->sorted_ok; k++) {  // (the last: the whole set)
+  for (size_t k = 0; k <= K; k++) {  // (the last: the whole set)
     bude::items::Plan *plan = &c->whole_sorted;
     if (k < K) plan = (c->chunk_sorted.push_back(std::make_unique<bude::items::Plan>()), c->chunk_sorted.back().get());
     const long a = k < K ? long(c->chunk_lig[k]) : 0, b = k < K ? long(c->chunk_lig[k + 1]) : long(L);
     if (int st = plan_sorted(c, *plan, std::vector<bude::items::Segment>(rows.begin() + a, rows.begin() + b))) return st;
-    if (int st = reserve_sorted(*plan, c->work, &c->sorted_ok)) return st;
+    if (int st = reserve_sorted(*plan, c->work)) return st;
   }
   c->plan_ok = true;
   return BUDE_OK;
@@ -1098,7 +1100,7 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     st = c->lab_off_dev.upload(bounds.data(), bounds.size() * sizeof(uint32_t));
     if (!st) st = c->lab_stats.alloc(nligands * sizeof(bude::gate::Stats));
     if (!st) st = plan_sorted(c.get(), c->label_sorted, segs);
-    if (!st) st = reserve_sorted(c->label_sorted, c->label_work, &c->label_sorted_ok);
+    if (!st) st = reserve_sorted(c->label_sorted, c->label_work);
   }
   if (!st) st = c->win_dev.alloc(kWindowRows * 8);
   if (!st) st = c->win_host.alloc(kWindowRows * 8);
@@ -1256,7 +1258,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   int nt_label = 0;
   int64_t ft_all = 0, ft_label = 0;
   const std::vector<int64_t> &tb_all = c->tb_all_host;
-  if (!use_sorted(c->s(), c->label_sorted, c->label_sorted_ok))
+  if (!use_sorted(c->s(), c->label_sorted, c->label_work))
     if (int st = prepare_exact(c, lab_spans, c->meta_label, c->tiles_label, &nt_label, bude::kSplitTile, c->stream3))
       return st;
   if (!mlp) {
@@ -1280,9 +1282,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     }
   }
   const size_t K = c->chunk_lig.size() - 1;
-  auto chunk_sorted = [&](size_t k) {
-    return c->sorted_ok && use_sorted(c->s(), *c->chunk_sorted[k], true);
-  };
+  auto chunk_sorted = [&](size_t k) { return use_sorted(c->s(), *c->chunk_sorted[k], c->work); };
   int2 *rs_tiles = static_cast<int2 *>(c->s().tiles_rs.ptr);
   int32_t *rs_ntiles = static_cast<int32_t *>(c->s().rs_ntiles.ptr);
 
@@ -1575,7 +1575,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
                                   chunk_sorted(k) ? c->chunk_sorted[k].get() : nullptr)) return st;
     }
   } else {
-    const bool sorted = nrs > 0 && use_sorted(c->s(), c->whole_sorted, c->sorted_ok);
+    const bool sorted = nrs > 0 && use_sorted(c->s(), c->whole_sorted, c->work);
     if (int st = select_and_tables(c, widened ? c->s().wplan : c->plan, 0,
                                    static_cast<const int32_t *>(c->s().rs_sel.ptr), nrs, rs_tiles, rs_ntiles + K,
                                    sorted, c->stream))

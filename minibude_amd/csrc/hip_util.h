@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdlib>
 #include <string>
 
 #include "bude_internal.h"
@@ -15,6 +16,14 @@ inline int hip_fail(hipError_t e, const char *what) {
 }
 
 inline int hip_check(hipError_t e, const char *what) { return e == hipSuccess ? BUDE_OK : hip_fail(e, what); }
+
+// Whether BUDE_MI355X_MAX_ALLOC_MB (not set: any size) lets one allocation be n
+// bytes; a larger one is taken as out of memory.  What the library does without
+// it can be tested with this.
+inline bool alloc_allowed(size_t n) {
+  const char *mb = std::getenv("BUDE_MI355X_MAX_ALLOC_MB");
+  return !mb || n <= size_t(std::strtoull(mb, nullptr, 10)) << 20;
+}
 
 // Owning device allocation (hipMalloc / hipFree).
 struct DeviceBuffer {
@@ -34,7 +43,7 @@ struct DeviceBuffer {
   int alloc(size_t n) {
     reset();
     if (n == 0) n = 4;
-    if (int st = hip_check(hipMalloc(&ptr, n), "hipMalloc")) {
+    if (int st = hip_check(alloc_allowed(n) ? hipMalloc(&ptr, n) : hipErrorOutOfMemory, "hipMalloc")) {
       (void)hipGetLastError();  // (reported here: a caller that goes on without the memory is not to find it after its next launch)
       ptr = nullptr;
       return st;
@@ -43,11 +52,13 @@ struct DeviceBuffer {
     return BUDE_OK;
   }
   // Keeps the current allocation when it already holds n bytes; a growing
-  // buffer gets a quarter of headroom, so sizes that vary a little from call
-  // to call settle on one allocation.
+  // buffer gets a quarter of headroom where there is memory for it, so sizes
+  // that vary a little from call to call settle on one allocation.  The old
+  // allocation goes before the new one is made.
   int reserve(size_t n) {
     if (ptr && bytes >= n) return BUDE_OK;
-    return alloc(ptr ? n + n / 4 : n);
+    const int st = alloc(ptr ? n + n / 4 : n);
+    return st == BUDE_ERR_OUT_OF_MEMORY ? alloc(n) : st;
   }
   // Copies n bytes in, reusing the allocation when it is large enough.
   int assign(const void *src, size_t n) {

@@ -55,10 +55,7 @@ bool worth_sorting(size_t natpro, double items, size_t nsegs);
 
 // Device scratch of a pass; one stream at a time may use it.
 struct Workspace {
-  DeviceBuffer items, partial, xform, hist, base, bounds;
-  void release() {
-    for (DeviceBuffer *b : {&items, &partial, &xform, &hist, &base, &bounds}) b->reset();
-  }
+  DeviceBuffer buf;
 };
 
 // The work of one pass, split into chunks of at most kChunkItems items.
@@ -66,12 +63,14 @@ class Plan {
  public:
   // atoms: every ligand's atoms (w bits: slot), ligand l's at lig_off[l] ..
   // lig_off[l + 1] - 1.  The tables are uploaded synchronously; no pass over
-  // an earlier plan may be in flight.  A ligand too large for a chunk leaves
-  // the plan empty.
+  // an earlier plan may be in flight.  A ligand too large for a chunk, or no
+  // memory for the tables, leaves the plan empty (worth() is then false).
   int build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
             const std::vector<Segment> &segs);
+  // Grows w to what a pass needs.  Without the memory for it w is what it was
+  // (or empty), and the status says so: ask fits() before every pass.
   int reserve(Workspace &w) const;
-  bool fits(const Workspace &w) const;
+  bool fits(const Workspace &w) const { return w.buf.bytes >= layout()[6]; }
   // Queues the pass: energies[row] of every row of every segment.  index:
   // the pose row of row i of a segment is pose_off + index[pose_off + i].
   hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
@@ -85,8 +84,8 @@ class Plan {
     uint32_t nitems, npartial, nxform, nrows;
     int nunits;
   };
-  // bytes of items, partial, xform, hist and base
-  std::array<size_t, 5> need() const;
+  // offsets of items, partial, xform, hist, base and bounds in the workspace, and its size
+  std::array<size_t, 7> layout() const;
   std::vector<Chunk> chunks_;
   DeviceBuffer tables_, atoms_;
   int nslots_ = 0;

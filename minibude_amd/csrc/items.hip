@@ -969,12 +969,17 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
     ch.slot_units = put(slot_units.data(), slot_units.size() * 4);
     chunks_.push_back(ch);
   }
-  if (int st = atoms_.assign(grouped.data(), grouped.size() * sizeof(float4))) return st;
-  return tables_.assign(bytes.data(), bytes.size());
+  int st = atoms_.assign(grouped.data(), grouped.size() * sizeof(float4));
+  if (!st) st = tables_.assign(bytes.data(), bytes.size());
+  if (st == BUDE_ERR_OUT_OF_MEMORY) {
+    chunks_.clear();
+    st = BUDE_OK;
+  }
+  return st;
 }
 
-std::array<size_t, 5> Plan::need() const {
-  std::array<size_t, 5> n{};
+std::array<size_t, 7> Plan::layout() const {
+  std::array<size_t, 6> n{};
   for (const Chunk &c : chunks_) {
     n[0] = std::max(n[0], size_t(c.nitems) * sizeof(float4));
     n[1] = std::max(n[1], size_t(c.npartial) * sizeof(float));
@@ -982,29 +987,22 @@ std::array<size_t, 5> Plan::need() const {
     n[3] = std::max(n[3], (size_t(c.nrows) << c.cell_bits) * sizeof(uint32_t));
     n[4] = std::max(n[4], (size_t(nslots_) << c.cell_bits) * sizeof(uint32_t));
   }
-  return n;
+  n[5] = kMaxBounds * 6 * sizeof(float);
+  std::array<size_t, 7> at{};
+  for (size_t i = 0; i < 6; i++) at[i + 1] = at[i] + ((n[i] + 255) & ~size_t(255));
+  return at;
 }
 
 int Plan::reserve(Workspace &w) const {
-  const std::array<size_t, 5> n = need();
-  int st = w.items.reserve(n[0]);
-  if (!st) st = w.partial.reserve(n[1]);
-  if (!st) st = w.xform.reserve(n[2]);
-  if (!st) st = w.hist.reserve(n[3]);
-  if (!st) st = w.base.reserve(n[4]);
-  if (!st) st = w.bounds.reserve(kMaxBounds * 6 * sizeof(float));
+  const size_t old = w.buf.bytes;
+  const int st = w.buf.reserve(layout()[6]);
+  if (st == BUDE_ERR_OUT_OF_MEMORY && old) (void)w.buf.alloc(old);  // (other plans' passes go on with it)
   return st;
-}
-
-bool Plan::fits(const Workspace &w) const {
-  const std::array<size_t, 5> n = need();
-  return n[0] <= w.items.bytes && n[1] <= w.partial.bytes && n[2] <= w.xform.bytes && n[3] <= w.hist.bytes &&
-         n[4] <= w.base.bytes && w.bounds.bytes >= kMaxBounds * 6 * sizeof(float);
 }
 
 hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                         float *energies, hipStream_t s) const {
-  if (!fits(w)) return hipErrorInvalidValue;
+  if (chunks_.empty() || !fits(w)) return hipErrorInvalidValue;
   Space sp{};
   for (int k = 0; k < 3; k++) {
     sp.lo[k] = sc.lo[k];
@@ -1013,12 +1011,14 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
   sp.radius = radius_;
   const auto *tables = static_cast<const char *>(tables_.ptr);
   const auto *atoms = static_cast<const float4 *>(atoms_.ptr);
-  auto *items = static_cast<float4 *>(w.items.ptr);
-  auto *partial = static_cast<float *>(w.partial.ptr);
-  auto *xf = static_cast<float4 *>(w.xform.ptr);
-  auto *hist = static_cast<uint32_t *>(w.hist.ptr);
-  auto *base = static_cast<uint32_t *>(w.base.ptr);
-  auto *bounds = static_cast<float *>(w.bounds.ptr);
+  const std::array<size_t, 7> at = layout();
+  auto *scratch = static_cast<char *>(w.buf.ptr);
+  auto *items = reinterpret_cast<float4 *>(scratch + at[0]);
+  auto *partial = reinterpret_cast<float *>(scratch + at[1]);
+  auto *xf = reinterpret_cast<float4 *>(scratch + at[2]);
+  auto *hist = reinterpret_cast<uint32_t *>(scratch + at[3]);
+  auto *base = reinterpret_cast<uint32_t *>(scratch + at[4]);
+  auto *bounds = reinterpret_cast<float *>(scratch + at[5]);
   for (const Chunk &c : chunks_) {
     const auto *blocks = reinterpret_cast<const Block *>(tables + c.blocks);
     const auto *tasks = reinterpret_cast<const Task *>(tables + c.tasks);
@@ -1165,10 +1165,7 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   scene_.form = plain_form();
   protein_box(groups.xyzw, largest, scene_.lo, scene_.hi);
   const int st = plan_.reserve(work_);
-  if (st == BUDE_ERR_OUT_OF_MEMORY) {  // (the tiled kernels need none of it)
-    work_.release();
-    return BUDE_OK;
-  }
+  if (st == BUDE_ERR_OUT_OF_MEMORY) return BUDE_OK;  // (the tiled kernels need none of it)
   usable_ = st == BUDE_OK;
   return st;
 }
