@@ -34,7 +34,7 @@ struct bude_ctx {
   size_t natpro = 0, natlig = 0, ntypes = 0, nposes = 0, ngroups = 0;
   bude::DeviceBuffer protein, group_begin, coef, ligand, poses, energies;
   bude::items::Deck sorted;
-  float *direct = nullptr;  // scratch of the direct pass, behind the energies (null: not used)
+  bude::DeviceBuffer direct;  // scratch of the direct pass (empty: not used)
   // where the last pass of a call leaves its energies for the host to read
   // (not allocated: they are copied out)
   bude::PinnedBuffer result;
@@ -148,25 +148,28 @@ extern "C" int bude_mi355x_create(int device, const BudeAtom *protein, size_t na
     st = bude::hip_check(hipMemcpy(static_cast<float *>(c->poses.ptr) + k * nposes, poses[k], nposes * sizeof(float),
                                    hipMemcpyHostToDevice),
                          "hipMemcpy poses");
+  if (!st) st = c->energies.alloc(nposes * sizeof(float));
+  if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
+  if (!st) st = bude::hip_check(hipEventCreate(&c->ev0), "hipEventCreate");
+  if (!st) st = bude::hip_check(hipEventCreate(&c->ev1), "hipEventCreate");
+  // what a pass can do without comes last: the sorted pass's scratch, then the direct pass's
   if (!st)
     st = c->sorted.prepare(groups, forcefield, std::vector<BudeAtom>(ligand, ligand + natlig), {0, int32_t(natlig)},
                            {bude::items::Segment{0, 0, int64_t(nposes)}});
-  const size_t direct = bude::items::direct_bytes(nposes, natlig), padded = (nposes + 63) / 64 * 64;
-  const bool use_direct = !c->sorted.usable() && direct <= bude::items::kDirectBytes;
-  if (!st) st = c->energies.alloc(padded * sizeof(float) + (use_direct ? direct : 0));
+  const size_t direct = bude::items::direct_bytes(nposes, natlig);
+  if (!st && !c->sorted.usable() && direct <= bude::items::kDirectBytes) {
+    st = c->direct.alloc(direct);
+    if (st == BUDE_ERR_OUT_OF_MEMORY) st = BUDE_OK;  // (the tiled kernel, then)
+  }
   // A copy of few energies costs 12 us and more a call whatever their number;
   // the last pass stores them over the bus instead (a call of 64 poses 39 and
   // 27 us, 4,097 61 and 48, 16,384 97 and 91).  With more of them the memory
   // for it, pinned, costs more than calls gain soon (65,536: 150 and 140 us a
   // call, but 300 us here).  Only a pass that writes an energy once goes there.
-  if (!st && nposes <= kHostResult && (c->sorted.usable() || use_direct)) {
+  if (!st && nposes <= kHostResult && (c->sorted.usable() || c->direct.ptr)) {
     st = c->result.alloc(nposes * sizeof(float));
     if (st == BUDE_ERR_OUT_OF_MEMORY) st = BUDE_OK;  // (copied out, then)
   }
-  if (!st && use_direct) c->direct = static_cast<float *>(c->energies.ptr) + padded;
-  if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
-  if (!st) st = bude::hip_check(hipEventCreate(&c->ev0), "hipEventCreate");
-  if (!st) st = bude::hip_check(hipEventCreate(&c->ev1), "hipEventCreate");
   if (!st) st = bude::hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
   if (st) {
     delete c;
@@ -204,7 +207,7 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   a.form = bude::plain_form();
   bude::items::DirectArgs direct{a.protein, a.group_begin, a.coef,   a.ligand, a.poses, a.energies, a.stride,
                                  a.nposes,  a.natlig,      a.ngroups, a.form,   nullptr,
-                                 ctx->direct};
+                                 static_cast<float *>(ctx->direct.ptr)};
   const size_t passes = warmup + iterations;
 
   for (size_t i = 0; i < passes; i++) {
@@ -214,7 +217,7 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
     const hipError_t le = ctx->sorted.usable()
                               ? ctx->sorted.launch(a.protein, a.poses, a.stride, nullptr, a.energies, ctx->stream)
-                          : ctx->direct ? bude::items::launch_direct(direct, ctx->stream)
+                          : ctx->direct.ptr ? bude::items::launch_direct(direct, ctx->stream)
                                             : bude::launch_plain(a, int(wgsize), ctx->stream);
     if (int st = bude::hip_check(le, "fasten_plain launch")) return st;
     if (int st = bude::hip_check(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord")) return st;

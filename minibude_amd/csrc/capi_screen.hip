@@ -336,6 +336,8 @@ extern "C" int bude_mi355x_screen_load(bude_screen *s, const float *const poses[
   s->nsel = 0;
   s->plan_n = 0;  // (the next run plans for these poses)
   s->all_planned = false;
+  s->sel_deck.release();
+  s->all_deck.release();
   int st = upload_poses(s->cand, poses, n);
   if (!st) st = s->pred.alloc(n * 4);
   if (!st) st = s->sel_idx.alloc(n * 4);
@@ -364,10 +366,11 @@ extern "C" int bude_mi355x_screen_run(bude_screen *s, BudeScreenResult *res) {
   hipStream_t st_ = s->stream;
   const auto t0 = std::chrono::steady_clock::now();
   if (s->plan_n != n || s->plan_k != k) {  // (uploads before any launch of this run)
+    s->plan_n = 0;
     if (int st = s->plan.prepare({bude::sel::Segment{0, uint32_t(n), uint32_t(k)}})) return st;
-    if (int st = plan_deck(s, k, s->sel_deck)) return st;
     const uint32_t done = uint32_t(k);
     if (int st = s->rs_done.assign(&done, sizeof(done))) return st;
+    if (int st = plan_deck(s, k, s->sel_deck)) return st;
     s->plan_n = n;
     s->plan_k = k;
   }

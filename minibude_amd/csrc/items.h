@@ -76,6 +76,11 @@ class Plan {
   hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                     float *energies, hipStream_t s) const;
   bool worth(size_t natpro) const { return !chunks_.empty() && worth_sorting(natpro, items_, nsegs_); }
+  void clear() {
+    chunks_.clear();
+    tables_.reset();
+    atoms_.reset();
+  }
 
  private:
   struct Chunk {
@@ -144,10 +149,15 @@ class Deck {
   int prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
               const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
   bool usable() const { return usable_; }
+  // Not usable() any more, and holding no memory.
+  void release();
   hipError_t launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index, float *energies,
                     hipStream_t s) const;
 
  private:
+  // prepare() up to *ok, whether there is a pass to run
+  int plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
+           const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs, bool *ok);
   bool usable_ = false;
   Scene scene_;
   Plan plan_;

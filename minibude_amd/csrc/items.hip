@@ -1131,6 +1131,21 @@ hipError_t launch_direct(const DirectArgs &a, hipStream_t s) {
 int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
                   const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs) {
   usable_ = false;
+  bool ok = false;
+  const int st = plan(groups, ff, atoms, lig_off, segs, &ok);
+  if (st || !ok) release();
+  usable_ = st == BUDE_OK && ok;
+  return st == BUDE_ERR_OUT_OF_MEMORY ? BUDE_OK : st;  // (the tiled kernels need none of it)
+}
+
+void Deck::release() {
+  usable_ = false;
+  plan_.clear();
+  for (DeviceBuffer *b : {&work_.buf, &coef_, &reach2_}) b->reset();
+}
+
+int Deck::plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
+               const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs, bool *ok) {
   const size_t natpro = size_t(groups.begin.back());
   double items = 0;
   for (const Segment &s : segs)
@@ -1164,10 +1179,9 @@ int Deck::prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std
   scene_.ngroups = int(groups.ngroups());
   scene_.form = plain_form();
   protein_box(groups.xyzw, largest, scene_.lo, scene_.hi);
-  const int st = plan_.reserve(work_);
-  if (st == BUDE_ERR_OUT_OF_MEMORY) return BUDE_OK;  // (the tiled kernels need none of it)
-  usable_ = st == BUDE_OK;
-  return st;
+  if (int st = plan_.reserve(work_)) return st;
+  *ok = true;
+  return BUDE_OK;
 }
 
 hipError_t Deck::launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index,

@@ -6,6 +6,9 @@ import numpy as np
 import pytest
 
 from minibude_amd import combined as C
+from minibude_amd import deck as D
+from minibude_amd import screen as S
+from minibude_amd.model import Context
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +49,31 @@ def test_a_pass_without_room_leaves_later_screens_as_they_are(gpu_device, monkey
             out[mb] = got
             monkeypatch.delenv(LIMIT, raising=False)
     assert all(same_bits(a, b) for a, b in zip(out[None], out["24"]))
+
+
+@pytest.mark.parametrize("mb", ["16", "4"])  # no room to sort; none for the direct pass's sums (6.8 MB) either
+def test_a_deck_without_room_for_scratch_is_scored(gpu_device, monkeypatch, mb):
+    d = D.synth_deck(938, 26, 65536, seed=52)
+    with Context(d, gpu_device) as c:
+        want = c.fasten(1, 64).energies
+    monkeypatch.setenv(LIMIT, mb)
+    with Context(d, gpu_device) as c:
+        assert same_bits(c.fasten(1, 64).energies, want)
+
+
+def test_a_prescreen_without_room_for_scratch_is_scored(gpu_device, monkeypatch):
+    w = S.screen_workload(ntrain=16384, nscreen=60000, natlig=20, natpro=900)
+    cfg = S.default_config(epochs=1, batch=1024, keep_fraction=0.1)
+    out = {}
+    for mb in (None, "8"):
+        with S.Screen(w.protein, w.ligand, w.forcefield, cfg, gpu_device) as s:
+            if mb:
+                monkeypatch.setenv(LIMIT, mb)
+            got = []
+            s.train(w.train_poses)
+            for poses in (w.screen_poses[:, :50000], w.screen_poses):
+                s.load(np.ascontiguousarray(poses))
+                s.run()
+                got += [*s.selected(), s.exhaustive()[0]]
+            out[mb] = got
+    assert all(same_bits(a, b) for a, b in zip(out[None], out["8"]))
