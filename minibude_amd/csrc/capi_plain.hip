@@ -211,8 +211,8 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   const size_t passes = warmup + iterations;
 
   for (size_t i = 0; i < passes; i++) {
-    ctx->in_result = energies_out && ctx->result.ptr && i + 1 == passes;
-    if (ctx->in_result) direct.energies = a.energies = static_cast<float *>(ctx->result.ptr);
+    const bool to_host = energies_out && ctx->result.ptr && i + 1 == passes;
+    if (to_host) direct.energies = a.energies = static_cast<float *>(ctx->result.ptr);
     const auto t0 = std::chrono::steady_clock::now();
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
     const hipError_t le = ctx->sorted.usable()
@@ -222,6 +222,7 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
     if (int st = bude::hip_check(le, "fasten_plain launch")) return st;
     if (int st = bude::hip_check(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord")) return st;
     if (int st = bude::hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return st;
+    ctx->in_result = to_host;
     if (host_ms) host_ms[i] = ms_since(t0);
     if (device_ms) {
       float ms = 0.f;
