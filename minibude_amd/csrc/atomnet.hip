@@ -1145,8 +1145,7 @@ int alloc_zero(DeviceBuffer &d, size_t bytes) {
 int reserve(const Net &net, Workspace &A, size_t B, size_t nval) {
   const size_t slices = (B + 64 * kStepGroups - 1) / (64 * kStepGroups);
   if (A.rows >= B && A.k0 == net.k0 && A.vpred.bytes >= std::max<size_t>(nval, 1) * 4) return BUDE_OK;
-  A.rows = B;
-  A.k0 = net.k0;
+  A.rows = 0;  // (complete only when everything is there)
   int st = A.pred.reserve(B * 4);
   if (!st) st = A.loss.reserve(slices * 8);
   if (!st) st = A.part.reserve(1024 * 2 * 8);
@@ -1157,8 +1156,11 @@ int reserve(const Net &net, Workspace &A, size_t B, size_t nval) {
     st = A.gpart[l].reserve(slices * K * N * 4);
     if (!st) st = A.bpart[l].reserve(slices * N * 4);
   }
-  if (!st) A.slices = unsigned(slices);
-  return st;
+  if (st) return st;
+  A.slices = unsigned(slices);
+  A.rows = B;
+  A.k0 = net.k0;
+  return BUDE_OK;
 }
 
 int set_params(Net &net, const float *grid, const float *const w[3], const float *const b[3], hipStream_t s) {
