@@ -271,6 +271,7 @@ struct bude_combined {
   // pair (planned when first wanted) and of a protein's fallback pairs, on
   // the first stream; the sampled poses on the third.
   std::vector<std::unique_ptr<bude::items::Plan>> chunk_sorted;
+  std::vector<bude::items::Segment> rescored;  // the rows that are always selected
   bude::items::Plan whole_sorted, all_sorted, fb_sorted, label_sorted;
   bude::items::Workspace work, label_work;
   DeviceBuffer sorted_rows;
@@ -837,24 +838,52 @@ int plan_selection(bude_combined *c, float keep) {
       ps.chunk_ev.push_back(e);
     }
   }
-  // the sorted rescoring passes, over the rows that are always selected
   std::vector<uint32_t> sorted_rows(L);
-  std::vector<bude::items::Segment> rows(L);
+  c->rescored.resize(L);
   for (size_t i = 0; i < L; i++) {
     sorted_rows[i] = segs[i].k;
-    rows[i] = bude::items::Segment{int32_t(i), int64_t(c->pose_off[i]), int64_t(segs[i].k)};
+    c->rescored[i] = bude::items::Segment{int32_t(i), int64_t(c->pose_off[i]), int64_t(segs[i].k)};
   }
   if (int st = c->sorted_rows.assign(sorted_rows.data(), L * 4)) return st;
   c->chunk_sorted.clear();
-  for (size_t k = 0; k <= K; k++) {  // (the last: the whole set)
-    bude::items::Plan *plan = &c->whole_sorted;
-    if (k < K) plan = (c->chunk_sorted.push_back(std::make_unique<bude::items::Plan>()), c->chunk_sorted.back().get());
-    const long a = k < K ? long(c->chunk_lig[k]) : 0, b = k < K ? long(c->chunk_lig[k + 1]) : long(L);
-    if (int st = plan_sorted(c, *plan, std::vector<bude::items::Segment>(rows.begin() + a, rows.begin() + b))) return st;
-    if (int st = reserve_sorted(*plan, c->work)) return st;
-  }
+  for (size_t k = 0; k < K; k++) c->chunk_sorted.push_back(std::make_unique<bude::items::Plan>());
+  c->whole_sorted.clear();
   c->plan_ok = true;
   return BUDE_OK;
+}
+
+// The sorted rescoring passes of every chunk and of the whole set, with their
+// scratch where there is memory for it.
+int plan_rescoring(bude_combined *c) {
+  const size_t K = c->chunk_sorted.size();
+  for (size_t k = 0; k <= K; k++) {  // (the last: the whole set)
+    bude::items::Plan &plan = k < K ? *c->chunk_sorted[k] : c->whole_sorted;
+    const long a = k < K ? long(c->chunk_lig[k]) : 0, b = k < K ? long(c->chunk_lig[k + 1]) : long(c->nlig);
+    const std::vector<bude::items::Segment> rows(c->rescored.begin() + a, c->rescored.begin() + b);
+    if (int st = plan_sorted(c, plan, rows)) return st;
+    if (int st = reserve_sorted(plan, c->work)) return st;
+  }
+  return BUDE_OK;
+}
+
+// Gives back the device memory the object can do without (the sorted passes'
+// scratch, the training index's tables) once nothing is in flight; false when
+// it holds none.
+bool give_back(bude_combined *c) {
+  if (!c->work.buf.ptr && !c->label_work.buf.ptr && !c->apoint_index.gathered) return false;
+  for (hipStream_t s : {c->stream, c->stream2, c->stream3}) (void)hipStreamSynchronize(s);
+  c->work.buf.reset();
+  c->label_work.buf.reset();
+  c->apoint_index.gathered = false;
+  c->apoint_index.terms.reset();
+  c->apoint_index.first.reset();
+  return true;
+}
+
+// f(), again where it finds no memory and there is some to give back.
+template <class F> int with_room(bude_combined *c, F &&f) {
+  const int st = f();
+  return st == BUDE_ERR_OUT_OF_MEMORY && give_back(c) ? f() : st;
 }
 
 int sync(bude_combined *c) { return bude::hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize"); }
@@ -978,7 +1007,10 @@ int prepare_atom_points(bude_combined *c) {
   std::iota(perm.begin(), perm.end(), 0u);
   std::mt19937_64 rng(c->cfg.seed ^ 0x9e37ull);
   std::shuffle(perm.begin(), perm.end(), rng);
-  if (int st = c->aperm.upload(perm.data(), perm.size() * 4)) return st;
+  return c->aperm.upload(perm.data(), perm.size() * 4);
+}
+
+int index_atom_points(bude_combined *c) {
   // (BUDE_MI355X_TRAIN_INDEX_MB bounds the index's tables; training gives the same network without them)
   const char *mb = std::getenv("BUDE_MI355X_TRAIN_INDEX_MB");
   const size_t limit = mb ? size_t(std::max(0l, std::atol(mb))) << 20 : bude::atomnet::kIndexBytes;
@@ -1086,8 +1118,8 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     if (!st) st = ps.coef.reserve(natoms * ntypes_ * sizeof(bude::PairCoef));
     if (!st) st = stage_reserve(ps, stage_bound(c.get(), pro_max));
   }
+  std::vector<bude::items::Segment> segs(nligands);
   if (!st) {  // the sampled poses: as many of every pair for every protein, gathered pair after pair
-    std::vector<bude::items::Segment> segs(nligands);
     int64_t at = 0;
     for (size_t i = 0; i < nligands; i++) {
       const int64_t n = int64_t(std::min<size_t>(cfg->labels_per_pair, nposes[i]));
@@ -1099,8 +1131,6 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
     bounds.push_back(uint32_t(at));
     st = c->lab_off_dev.upload(bounds.data(), bounds.size() * sizeof(uint32_t));
     if (!st) st = c->lab_stats.alloc(nligands * sizeof(bude::gate::Stats));
-    if (!st) st = plan_sorted(c.get(), c->label_sorted, segs);
-    if (!st) st = reserve_sorted(c->label_sorted, c->label_work);
   }
   if (!st) st = c->win_dev.alloc(kWindowRows * 8);
   if (!st) st = c->win_host.alloc(kWindowRows * 8);
@@ -1109,6 +1139,11 @@ extern "C" int bude_mi355x_combined_create(int device, const BudeFFParams *force
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream3, hipStreamNonBlocking), "hipStreamCreate");
+  // what the screens can do without comes last (give_back)
+  if (!st && cfg->surrogate == BUDE_SURROGATE_ATOM_MLP) st = index_atom_points(c.get());
+  if (!st) st = plan_rescoring(c.get());
+  if (!st) st = plan_sorted(c.get(), c->label_sorted, segs);
+  if (!st) st = reserve_sorted(c->label_sorted, c->label_work);
   if (!st) st = bude::hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
   if (st) return st;
   *out = c.release();
@@ -1636,7 +1671,7 @@ extern "C" int bude_mi355x_combined_screen(bude_combined *c, const BudeAtom *pro
     return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_combined_screen: a batch is running");
   if (int st = bude::hip_check(hipSetDevice(c->device), "hipSetDevice")) return st;
   *res = BudeCombinedResult{};
-  int st = screen_begin(c, protein, natpro);
+  int st = with_room(c, [&] { return screen_begin(c, protein, natpro); });
   if (!st) st = screen_end(c);
   if (st) {  // leave nothing in flight behind an error
     (void)hipStreamSynchronize(c->stream);
@@ -1679,7 +1714,7 @@ extern "C" int bude_mi355x_combined_screen_batch(bude_combined *c, size_t nprote
     }
     const int slot = prev >= 0 ? prev ^ 1 : c->cur;
     c->cur = slot;
-    st = screen_begin(c, proteins[i], natpro[i]);
+    st = with_room(c, [&] { return screen_begin(c, proteins[i], natpro[i]); });
     if (st) break;
     if (prev >= 0) st = finish(prev, i - 1);
     c->cur = slot;
@@ -1711,11 +1746,12 @@ extern "C" int bude_mi355x_combined_set_keep(bude_combined *c, float keep_fracti
   if (int st = bude::hip_check(hipSetDevice(c->device), "hipSetDevice")) return st;
   if (int st = bude::hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return st;
   if (int st = bude::hip_check(hipStreamSynchronize(c->stream2), "hipStreamSynchronize")) return st;
-  if (int st = plan_selection(c, keep_fraction)) {
+  if (int st = with_room(c, [&] { return plan_selection(c, keep_fraction); })) {
     c->s().valid = false;
     return st;
   }
   c->cfg.keep_fraction = keep_fraction;
+  if (int st = plan_rescoring(c)) return st;
   return bude::ok();
 }
 
@@ -1758,7 +1794,7 @@ int fetch_window(bude_combined *c, size_t ligand) {
   c->win_slot = -1;
   if (rows > c->win_rows) {
     c->win_rows = 0;
-    if (int st = c->win_dev.alloc(rows * 8)) return st;
+    if (int st = with_room(c, [&] { return c->win_dev.alloc(rows * 8); })) return st;
     if (int st = c->win_host.alloc(rows * 8)) return st;
     c->win_rows = rows;
   }
@@ -1837,7 +1873,7 @@ extern "C" int bude_mi355x_combined_exhaustive(bude_combined *c, double *device_
   if (!c->s().valid)
     return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_combined_exhaustive: no protein screened yet");
   if (int st = bude::hip_check(hipSetDevice(c->device), "hipSetDevice")) return st;
-  if (int st = c->exact_all.reserve(c->total * 4)) return st;
+  if (int st = with_room(c, [&] { return c->exact_all.reserve(c->total * 4); })) return st;
   std::vector<Span> all(c->nlig);
   for (size_t l = 0; l < c->nlig; l++) all[l] = Span{l, c->pose_off[l], c->nposes[l]};
   if (!c->all_planned) {
@@ -1886,9 +1922,11 @@ extern "C" int bude_mi355x_combined_recall(bude_combined *c, float top_fraction,
   }
   bude::sel::Plan plan;
   DeviceBuffer tidx, tn;
-  int st = plan.prepare(segs);
-  if (!st) st = tidx.alloc(c->total * 4);
-  if (!st) st = tn.alloc(c->nlig * 4);
+  int st = with_room(c, [&] {
+    int e = plan.prepare(segs);
+    if (!e) e = tidx.alloc(c->total * 4);
+    return e ? e : tn.alloc(c->nlig * 4);
+  });
   if (!st)
     st = bude::hip_check(bude::sel::select_lowest_segments(plan, static_cast<const float *>(c->exact_all.ptr),
                                                            static_cast<uint32_t *>(tidx.ptr),

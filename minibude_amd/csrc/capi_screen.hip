@@ -78,6 +78,14 @@ struct bude_screen {
     if (stream) (void)hipStreamDestroy(stream);
   }
 
+  // The sorted passes' memory given back; the next run plans anew.
+  void release_plans() {
+    plan_n = 0;
+    all_planned = false;
+    sel_deck.release();
+    all_deck.release();
+  }
+
   bude::PlainArgs plain(const float *poses, size_t stride, size_t n, float *energies) const {
     bude::PlainArgs a{};
     a.protein = static_cast<const float4 *>(protein.ptr);
@@ -241,6 +249,7 @@ extern "C" int bude_mi355x_screen_train(bude_screen *s, const float *const poses
   hipStream_t st_ = s->stream;
 
   // 1. exact labels from the plain kernel
+  s->release_plans();  // (training needs the memory more)
   DeviceBuffer tp, te;
   if (int st = upload_poses(tp, poses, n)) return st;
   if (int st = te.alloc(n * 4)) return st;
@@ -334,10 +343,7 @@ extern "C" int bude_mi355x_screen_load(bude_screen *s, const float *const poses[
   if (int st = bude::hip_check(hipSetDevice(s->device), "hipSetDevice")) return st;
   s->ncand = n;
   s->nsel = 0;
-  s->plan_n = 0;  // (the next run plans for these poses)
-  s->all_planned = false;
-  s->sel_deck.release();
-  s->all_deck.release();
+  s->release_plans();
   int st = upload_poses(s->cand, poses, n);
   if (!st) st = s->pred.alloc(n * 4);
   if (!st) st = s->sel_idx.alloc(n * 4);
@@ -473,7 +479,12 @@ extern "C" int bude_mi355x_screen_exhaustive(bude_screen *s, float *energies, do
   if (!s || s->ncand == 0) return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "bude_mi355x_screen_exhaustive: no poses");
   if (int st = bude::hip_check(hipSetDevice(s->device), "hipSetDevice")) return st;
   DeviceBuffer out;
-  if (int st = out.alloc(s->ncand * 4)) return st;
+  int ast = out.alloc(s->ncand * 4);
+  if (ast == BUDE_ERR_OUT_OF_MEMORY) {
+    s->release_plans();
+    ast = out.alloc(s->ncand * 4);
+  }
+  if (ast) return ast;
   bude::items::Deck d;
   if (int st = plan_deck(s, s->ncand, d)) return st;
   if (int st = bude::hip_check(hipEventRecord(s->ev[0], s->stream), "hipEventRecord")) return st;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <string>
 
@@ -17,12 +18,15 @@ inline int hip_fail(hipError_t e, const char *what) {
 
 inline int hip_check(hipError_t e, const char *what) { return e == hipSuccess ? BUDE_OK : hip_fail(e, what); }
 
-// Whether BUDE_MI355X_MAX_ALLOC_MB (not set: any size) lets one allocation be n
-// bytes; a larger one is taken as out of memory.  What the library does without
-// it can be tested with this.
-inline bool alloc_allowed(size_t n) {
-  const char *mb = std::getenv("BUDE_MI355X_MAX_ALLOC_MB");
-  return !mb || n <= size_t(std::strtoull(mb, nullptr, 10)) << 20;
+// Bytes all DeviceBuffers hold, and whether BUDE_MI355X_MAX_MEMORY_MB (not set:
+// no bound) lets them be n more; an allocation beyond it is out of memory.
+inline std::atomic<size_t> device_bytes{0};
+inline bool take_device_bytes(size_t n) {
+  const size_t held = device_bytes.fetch_add(n) + n;
+  const char *mb = std::getenv("BUDE_MI355X_MAX_MEMORY_MB");
+  if (!mb || held <= size_t(std::strtoull(mb, nullptr, 10)) << 20) return true;
+  device_bytes.fetch_sub(n);
+  return false;
 }
 
 // Owning device allocation (hipMalloc / hipFree).
@@ -37,13 +41,16 @@ struct DeviceBuffer {
 
   void reset() {
     if (ptr) (void)hipFree(ptr);
+    device_bytes.fetch_sub(bytes);
     ptr = nullptr;
     bytes = 0;
   }
   int alloc(size_t n) {
     reset();
     if (n == 0) n = 4;
-    if (int st = hip_check(alloc_allowed(n) ? hipMalloc(&ptr, n) : hipErrorOutOfMemory, "hipMalloc")) {
+    const bool room = take_device_bytes(n);
+    if (int st = hip_check(room ? hipMalloc(&ptr, n) : hipErrorOutOfMemory, "hipMalloc")) {
+      if (room) device_bytes.fetch_sub(n);
       (void)hipGetLastError();  // (reported here: a caller that goes on without the memory is not to find it after its next launch)
       ptr = nullptr;
       return st;
