@@ -134,7 +134,7 @@ struct CellGrid {
 };
 
 __device__ __forceinline__ CellGrid cell_grid(const float *__restrict__ bounds, int nbounds, const Space &sp,
-                                              float *red /* LDS, 96 */) {
+                                              float *red /* LDS, 6 */) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // waves 0-2 the minima, 3-5 the maxima
   if (wave < 6) {
@@ -273,6 +273,7 @@ __global__ __launch_bounds__(256) void column_kernel(const int32_t *__restrict__
                                                      uint32_t *__restrict__ hist, uint32_t *__restrict__ base) {
   const int slot = blockIdx.y, ncells = 1 << bits;
   const int c = int(blockIdx.x) * 256 + int(threadIdx.x);
+  if (c >= ncells) return;
   const int r1 = slot_rows[slot + 1];
   uint32_t run = 0;
   int r = slot_rows[slot];
@@ -736,7 +737,8 @@ void score_items(const Scene &sc, int rb, const float4 *items, const int32_t *sl
   else score([](auto... args) { launch_score_rb<kFormB>(args...); });
 }
 
-// Items of one chunk: 20 bytes each in the workspace.
+// Items of one chunk.  Each takes 20 bytes of scratch, its counts up to 16 more
+// (Plan::build), and a pose's transform 48.
 constexpr int64_t kChunkItems = int64_t(1) << 26;
 
 // The device hands work-group i to XCD i mod 8, each with an L2 of its own.
@@ -931,6 +933,12 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
     const int64_t mean = nitems / std::max<int64_t>(1, used);
     ch.rb = items_per_lane(mean);
     ch.cell_bits = mean >= 16384 ? 12 : 9;
+    // Short segments have many rows of few items: no more than four counts an
+    // item, so that the counts stay a part of the scratch (2,048 ligands of 64
+    // atoms x 64 poses against 300 atoms: 1,244 MB and 1,480 us a pass with 12
+    // bits, 432 and 590 with 9; 256 of 52 x 256 against 4,096: 198 MB and 502
+    // us, 100 and 504; one count an item costs 730 there, the cells too coarse).
+    while (ch.cell_bits > 0 && nrows << ch.cell_bits > 4 * nitems) ch.cell_bits -= 3;
     std::vector<Row> rows;
     std::vector<std::vector<int32_t>> refs_of(blocks.size());
     for (int t = 0; t < nslots; t++) {
@@ -1033,7 +1041,7 @@ hipError_t Plan::launch(const Scene &sc, const Workspace &w, const float *poses,
     launch_bin_ppt<0>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),
                       size_t(c.nxform), static_cast<const float *>(bounds), nb, sp, c.cell_bits, hist,
                       static_cast<const uint32_t *>(base), items);
-    hipLaunchKernelGGL(column_kernel, dim3((1u << c.cell_bits) / 256u, unsigned(nslots_)), dim3(256), 0, s, slot_rows,
+    hipLaunchKernelGGL(column_kernel, dim3(((1u << c.cell_bits) + 255u) / 256u, unsigned(nslots_)), dim3(256), 0, s, slot_rows,
                        c.cell_bits, hist, base);
     hipLaunchKernelGGL(scan_kernel, dim3(unsigned(nslots_)), dim3(kThreads), 0, s, slot_items, c.cell_bits, base);
     launch_bin_ppt<1>(c.ppt, c.ntasks, s, tasks, blocks, refs, rows, atoms, static_cast<const float4 *>(xf),

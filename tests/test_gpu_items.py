@@ -137,3 +137,43 @@ def test_forcefields_without_a_reach(gpu_device, field, value):
     d = D.synth_deck(600, 20, 65536, seed=73)
     d.forcefield[field][3] = value
     same(d, gpu_device, f"{field}={value}")
+
+
+@pytest.mark.parametrize("nlig, natlig, nposes, ntypes", [
+    (40, 64, 64, 34),      # rows of few items: 9 bits of cells
+    (60, 600, 8, 200),     # 6
+    (30, 4096, 1, 1000),   # 3
+    (20, 5000, 1, 5000),   # a row for every atom: one cell a type
+])
+def test_short_segments_equal_direct(gpu_device, nlig, natlig, nposes, ntypes):
+    ff = D.synth_forcefield(90, ntypes)
+    pro = D.synth_protein(90, 5000, min(ntypes, 12))
+    ligs = [D.synth_ligand(100 + i, natlig, ntypes) for i in range(nlig)]
+    if ntypes >= natlig:
+        for l in ligs:
+            l["type"] = np.arange(natlig)
+    poses = [D.synth_poses(200 + i, nposes) for i in range(nlig)]
+    want = []
+    for l, q in zip(ligs, poses):  # (the direct pass: too few items each to sort)
+        with Context(D.Deck(pro, l, ff, q), gpu_device) as c:
+            want.append(c.fasten(1, 64).energies)
+    with Batch(LigandSet(pro, ff, ligs, poses), gpu_device) as b:
+        b.clear()
+        b.run(BatchConfig(1, 64, 4, 0, 1), warmup=1, iterations=2)
+        for i in range(nlig):
+            assert np.array_equal(b.energies(i).view(np.uint32), want[i].view(np.uint32)), i
+
+
+def test_scratch_of_short_segments_is_bounded(gpu_device):
+    # 4.2 M items in 1,024 segments: 20 bytes an item, up to 16 of counts, 48 a
+    # pose, and the batch itself (a row of 4,096 counts per type and segment
+    # would be 490 MB alone)
+    nlig, natlig, nposes = 1024, 64, 64
+    ls = LigandSet(D.synth_protein(91, 300, 34), D.synth_forcefield(91, 34),
+                   [D.synth_ligand(300 + i, natlig, 34) for i in range(nlig)],
+                   [D.synth_poses(400 + i, nposes) for i in range(nlig)])
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    with Batch(ls, gpu_device):
+        held = before - torch.cuda.mem_get_info()[0]
+    assert held < nlig * natlig * nposes * 36 + nlig * natlig * 34 * 32 + nlig * nposes * 100 + (64 << 20)
