@@ -107,7 +107,7 @@ bool few_tiles(const bude_batch *b) {
 // work-groups per tile where the tiles are few (the configuration shapes
 // the persistent kernel only), else the persistent kernel.
 int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
-  if (b->sorted.usable())
+  if (b->sorted.worth(cfg->ppwi, cfg->ppwi))
     return bude::hip_check(b->sorted.launch(static_cast<const float4 *>(b->protein.ptr),
                                             static_cast<const float *>(b->poses.ptr), b->total_poses, nullptr,
                                             static_cast<float *>(b->energies.ptr), b->stream),
@@ -137,14 +137,15 @@ int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
 }
 
 int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
-  const auto key = b->sorted.usable() ? std::make_tuple(0, 0, 0, 0)
-                                      : std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
+  const bool sorted = b->sorted.worth(cfg->ppwi, cfg->ppwi);
+  const auto key = sorted ? std::make_tuple(0, 0, 0, 0)
+                          : std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
   auto it = b->graphs.find(key);
   if (it == b->graphs.end()) {
     // build tiles before capture (the upload is not capturable)
     const bude::DeviceBuffer *tb = nullptr;
     int nt = 0;
-    if (!b->sorted.usable())
+    if (!sorted)
       if (int st = tiles_for(b, few_tiles(b) ? 1 : cfg->ppwi, cfg->order, &tb, &nt)) return st;
     auto g = std::make_unique<GraphExec>();
     if (int st = bude::hip_check(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),

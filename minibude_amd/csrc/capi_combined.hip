@@ -402,7 +402,7 @@ int reserve_sorted(const bude::items::Plan &plan, bude::items::Workspace &w) {
 
 // Whether a sorted pass of protein slot ps pays.
 bool sorted_pays(const ProteinSlot &ps, const bude::items::Plan &plan) {
-  return ps.reachable && plan.worth(size_t(ps.scene.natpro));
+  return ps.reachable && plan.worth(size_t(ps.scene.natpro), size_t(ps.scene.ngroups), kBatchPpwi);
 }
 
 // Whether protein slot ps is scored by this sorted pass, with scratch w.

@@ -209,16 +209,23 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
                                  a.nposes,  a.natlig,      a.ngroups, a.form,   nullptr,
                                  static_cast<float *>(ctx->direct.ptr)};
   const size_t passes = warmup + iterations;
+  // Few energies: the tiled kernel never pays, as they would be copied out.
+  const bude::items::Work work{ctx->natpro, ctx->ngroups, 1, double(ctx->natlig) * double(ctx->nposes),
+                               double(ctx->nposes)};
+  const bool few = ctx->nposes <= kHostResult;
+  const int rb = bude::plain_register_block(int(ppwi), int(wgsize));
+  const bool sorted = few ? ctx->sorted.usable() : ctx->sorted.worth(int(ppwi), rb);
+  const bool use_direct = !sorted && ctx->direct.ptr && (few || bude::items::worth_direct(work, int(ppwi), rb));
 
   for (size_t i = 0; i < passes; i++) {
-    const bool to_host = energies_out && ctx->result.ptr && i + 1 == passes;
+    const bool to_host = energies_out && ctx->result.ptr && (sorted || use_direct) && i + 1 == passes;
     if (to_host) direct.energies = a.energies = static_cast<float *>(ctx->result.ptr);
     const auto t0 = std::chrono::steady_clock::now();
     if (int st = bude::hip_check(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord")) return st;
-    const hipError_t le = ctx->sorted.usable()
-                              ? ctx->sorted.launch(a.protein, a.poses, a.stride, nullptr, a.energies, ctx->stream)
-                          : ctx->direct.ptr ? bude::items::launch_direct(direct, ctx->stream)
-                                            : bude::launch_plain(a, int(wgsize), ctx->stream);
+    const hipError_t le =
+        sorted       ? ctx->sorted.launch(a.protein, a.poses, a.stride, nullptr, a.energies, ctx->stream)
+        : use_direct ? bude::items::launch_direct(direct, ctx->stream)
+                     : bude::launch_plain(a, int(wgsize), ctx->stream);
     if (int st = bude::hip_check(le, "fasten_plain launch")) return st;
     if (int st = bude::hip_check(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord")) return st;
     if (int st = bude::hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return st;

@@ -115,7 +115,7 @@ int plan_deck(const bude_screen *s, size_t n, bude::items::Deck &d) {
 // Exact energies of n poses on the library's stream, through the planned
 // pass where it applies.
 hipError_t score_all(const bude_screen *s, const bude::items::Deck &d, const float *poses, size_t n, float *energies) {
-  if (d.usable())
+  if (d.worth(1, 1))
     return d.launch(static_cast<const float4 *>(s->protein.ptr), poses, n, nullptr, energies, s->stream);
   return bude::launch_plain(s->plain(poses, n, n, energies), 256, s->stream);
 }
@@ -136,7 +136,7 @@ int upload_poses(DeviceBuffer &d, const float *const poses[6], size_t n) {
 // (bit-identical) over the rest.  The tables come from the selection's count
 // on the device; the host does not wait for it.
 int rescore(bude_screen *s) {
-  const bool sorted = s->sel_deck.usable();
+  const bool sorted = s->sel_deck.worth(1, 1);
   if (sorted)
     if (int st = bude::hip_check(s->sel_deck.launch(static_cast<const float4 *>(s->protein.ptr),
                                                     static_cast<const float *>(s->cand.ptr), s->ncand,

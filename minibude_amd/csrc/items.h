@@ -50,8 +50,16 @@ bool reach_table(const std::vector<PairCoef> &coef, size_t ngroups, std::vector<
 // The box of the grouped protein's finite atoms widened by `reach`.
 void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float hi[3]);
 
-// Whether sorting pays for `items` items of `nsegs` segments against natpro atoms.
-bool worth_sorting(size_t natpro, double items, size_t nsegs);
+// The work of a pass: `items` items of `poses` poses in nsegs segments.
+struct Work {
+  size_t natpro = 0, ngroups = 0, nsegs = 0;
+  double items = 0, poses = 0;
+};
+
+// Whether sorting pays, and whether the direct pass does, where the other
+// choice is a tiled kernel with ppwi poses per work-item in register blocks of rb.
+bool worth_sorting(const Work &w, int ppwi, int rb);
+bool worth_direct(const Work &w, int ppwi, int rb);
 
 // Device scratch of a pass; one stream at a time may use it.
 struct Workspace {
@@ -64,7 +72,7 @@ class Plan {
   // atoms: every ligand's atoms (w bits: slot), ligand l's at lig_off[l] ..
   // lig_off[l + 1] - 1.  The tables are uploaded synchronously; no pass over
   // an earlier plan may be in flight.  A ligand too large for a chunk, or no
-  // memory for the tables, leaves the plan empty (worth() is then false).
+  // memory for the tables, leaves the plan empty().
   int build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
             const std::vector<Segment> &segs);
   // Grows w to what a pass needs.  Without the memory for it w is what it was
@@ -75,7 +83,10 @@ class Plan {
   // the pose row of row i of a segment is pose_off + index[pose_off + i].
   hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                     float *energies, hipStream_t s) const;
-  bool worth(size_t natpro) const { return !chunks_.empty() && worth_sorting(natpro, items_, nsegs_); }
+  bool worth(size_t natpro, size_t ngroups, int ppwi) const {
+    return !chunks_.empty() && worth_sorting(Work{natpro, ngroups, nsegs_, items_, poses_}, ppwi, ppwi);
+  }
+  bool empty() const { return chunks_.empty(); }
   void clear() {
     chunks_.clear();
     tables_.reset();
@@ -96,7 +107,7 @@ class Plan {
   int nslots_ = 0;
   size_t nsegs_ = 0;
   float radius_ = 0.f;  // of the ligand atoms about their frame's origin
-  double items_ = 0;
+  double items_ = 0, poses_ = 0;
 };
 
 // Single atoms at given points, sorted once and scored against any number of
@@ -142,13 +153,14 @@ hipError_t launch_direct(const DirectArgs &a, hipStream_t s);
 
 // Everything one deck's passes need on the sorted path, from the host deck:
 // scene, plan and workspace.  usable() is false where the path does not
-// apply (see worth_sorting, pair_reach) or its memory cannot be had; the
-// caller then scores with the tiled kernels.
+// apply (see worth_sorting, pair_reach) or its memory cannot be had, worth()
+// where a tiled kernel is the faster; the caller then scores with that.
 class Deck {
  public:
   int prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
               const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
   bool usable() const { return usable_; }
+  bool worth(int ppwi, int rb) const { return usable_ && worth_sorting(shape_, ppwi, rb); }
   // Not usable() any more, and holding no memory.
   void release();
   hipError_t launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index, float *energies,
@@ -159,6 +171,7 @@ class Deck {
   int plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
            const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs, bool *ok);
   bool usable_ = false;
+  Work shape_;
   Scene scene_;
   Plan plan_;
   Workspace work_;

@@ -817,15 +817,61 @@ void protein_box(const std::vector<float> &xyzw, float reach, float lo[3], float
   }
 }
 
-bool worth_sorting(size_t natpro, double items, size_t nsegs) {
-  // The direct pass scores some 1.8e9 pairs a millisecond; the sort's seven
+namespace {
+
+// Estimates of a pass in microseconds beyond a launch and its wait, for the
+// choice between the forms; ps per item and pose.  Measured over proteins of
+// 1 to 4,096 atoms (1 to 34 groups), ligands of 1 to 500, 65,536 to 4 M poses.
+//
+// Tiled: 64 x 64 atoms x 1,048,576 poses 34, 25, 25 and 28 ps an item with 1,
+// 2, 4 and 8 poses a register block, 16 x 64 13, 8.2, 7.4 and 7.7, 1 x 64 1.7
+// to 1.1, 4,096 x 26 1,207; a group costs the more the fewer atoms it has and
+// poses share it.  With w waves per SIMD it takes 1 + 2.3 / (sqrt(rb) w^1.5)
+// times as long (64 x 64 with rb 1: 3.9 at w = 1, 1.31 at 4).
+double tiled_us(const Work &w, int ppwi, int rb) {
+  const double natpro = double(w.natpro), groups = double(w.ngroups) * std::min(1.0, 64.0 / natpro);
+  const double full = w.items * (0.29 * natpro + groups * (0.1 + 0.4 / rb)) + 8.0 * w.poses;
+  return full * 1e-6 * (1.0 + 2.3 / std::sqrt(double(rb)) * std::pow(65536.0 * ppwi / w.poses, 1.5));
+}
+
+// Sorted, small proteins: 30 ps an item however few the atoms (1 x 64 x
+// 1,048,576 26, 64 x 64 and 128 x 64 29.9), 58 where a pose has one.
+double sorted_us(const Work &w) {
+  return 30.0 + (w.items * (29.5 + 0.008 * double(w.natpro)) + 29.0 * w.poses) * 1e-6;
+}
+
+// Direct: 5 ps an item (1 x 64 x 262,144), 15.7 (16 x 8), 42 (64 x 8), and a
+// second launch.
+double direct_us(const Work &w) {
+  const double natpro = double(w.natpro);
+  const double item = 0.305 * natpro + (4.0 + 0.55 * double(w.ngroups)) * std::min(1.0, 64.0 / natpro);
+  return 6.0 + (w.items * item + 12.0 * w.poses) * 1e-6;
+}
+
+}  // namespace
+
+bool worth_sorting(const Work &w, int ppwi, int rb) {
+  // Against the direct pass: that scores some 1.8e9 pairs a millisecond; the sort's seven
   // launches cost 40-50 us whatever the size, and with few items (large
   // boxes) scoring them grows with the protein.  Both measured, direct and
   // sorted, over 64 .. 131,072 poses: 300 x 8 atoms cross at 1.5e8 pairs
   // (67 and 65 us), 700 x 19 at 1e8, 938 x 26 at 1.4e8, 938 x 64 at 2e8,
   // 4,096 x 26 at 4.4e8 (189 and 192 us), 4,096 x 96 at 6e8.  A segment is to
   // fill the work-groups that sort it.
-  return items * double(natpro) >= 6e7 + 8e4 * double(natpro) && items >= 4096.0 * double(nsegs);
+  // Against a tiled kernel: sorting moves some 30 bytes an item, which costs
+  // more than the few pairs of a small protein (64 x 64 x 1,048,576: 2,000 us,
+  // 1,690 tiled with two poses per work-item; 4 x 64 x 262,144: 504 and 91).
+  const double natpro = double(w.natpro);
+  return w.items * natpro >= 6e7 + 8e4 * natpro && w.items >= 4096.0 * double(w.nsegs) &&
+         sorted_us(w) <= tiled_us(w, ppwi, rb);
+}
+
+bool worth_direct(const Work &w, int ppwi, int rb) {
+  // (1 x 64 x 262,144: 102 us, 44 tiled with two poses per work-item; 64 x 8 x
+  // 262,144: 107 and 105; larger proteins: nothing between them where the
+  // tiled kernel has the poses to fill the device, else the direct pass.  A
+  // tenth is within the estimates)
+  return w.natpro >= 128 || direct_us(w) <= 1.15 * tiled_us(w, ppwi, rb);
 }
 
 int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
@@ -833,7 +879,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
   chunks_.clear();
   nslots_ = nslots;
   nsegs_ = segs.size();
-  items_ = 0;
+  items_ = poses_ = 0;
   radius_ = 0.f;
   // every ligand's atoms grouped by type (stable), w bits: place in the ligand
   const size_t nlig = lig_off.size() - 1;
@@ -870,6 +916,7 @@ int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &li
     const int64_t L = lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)];
     if (L <= 0 || L > kChunkItems / 64) return BUDE_OK;
     items_ += double(L) * double(s.n);
+    poses_ += double(s.n);
     for (int64_t j = 0; j < s.n;) {
       int64_t take = std::min(s.n - j, room / L);
       if (take < s.n - j) take = take / 64 * 64;
@@ -1155,10 +1202,12 @@ void Deck::release() {
 int Deck::plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
                const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs, bool *ok) {
   const size_t natpro = size_t(groups.begin.back());
-  double items = 0;
-  for (const Segment &s : segs)
-    items += double(lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)]) * double(s.n);
-  if (!worth_sorting(natpro, items, segs.size())) return BUDE_OK;
+  shape_ = Work{natpro, groups.ngroups(), segs.size()};
+  for (const Segment &s : segs) {
+    shape_.items += double(lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)]) * double(s.n);
+    shape_.poses += double(s.n);
+  }
+  if (!worth_sorting(shape_, 1, 1) && !worth_sorting(shape_, 8, 8)) return BUDE_OK;
   // slots: the forcefield types the ligands use, ascending
   std::vector<int32_t> types;
   for (const BudeAtom &a : atoms) types.push_back(a.type);
@@ -1180,7 +1229,7 @@ int Deck::plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::v
   if (int st = coef_.upload(coef.data(), coef.size() * sizeof(PairCoef))) return st;
   if (int st = reach2_.upload(reach2.data(), reach2.size() * sizeof(float4))) return st;
   if (int st = plan_.build(slotted, lig_off, int(types.size()), segs)) return st;
-  if (!plan_.worth(natpro)) return BUDE_OK;
+  if (plan_.empty()) return BUDE_OK;
   scene_.coef = static_cast<const PairCoef *>(coef_.ptr);
   scene_.reach2 = static_cast<const float4 *>(reach2_.ptr);
   scene_.natpro = int(natpro);

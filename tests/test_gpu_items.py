@@ -177,3 +177,36 @@ def test_scratch_of_short_segments_is_bounded(gpu_device):
     with Batch(ls, gpu_device):
         held = before - torch.cuda.mem_get_info()[0]
     assert held < nlig * natlig * nposes * 36 + nlig * natlig * 34 * 32 + nlig * nposes * 100 + (64 << 20)
+
+
+@pytest.mark.parametrize("natpro, natlig, nposes", [(1, 64, 262145), (4, 64, 262144), (16, 8, 1048576),
+                                                    (64, 64, 1048576), (64, 1, 1048577)])
+def test_small_proteins_equal_tiled_and_are_no_slower(gpu_device, natpro, natlig, nposes):
+    # sorting an item costs more than the few pairs of a small protein (the
+    # sorted pass takes 2.5 to 20 times the tiled kernel's time in these but
+    # the fourth); half again is far above what a repeated pass varies by
+    d = D.synth_deck(natpro, natlig, nposes, seed=92)
+    with Context(d, gpu_device) as c, Batch(LigandSet(d.protein, d.forcefield, [d.ligand], [d.poses]), gpu_device) as b:
+        for ppwi in (1, 4):
+            b.clear()
+            t = min(b.run_separate(ppwi, 64, 1, 6)[1:])
+            got = c.fasten(ppwi, 64, 1, 6)
+            assert np.array_equal(got.energies.view(np.uint32), b.energies(0).view(np.uint32)), ppwi
+            assert min(got.device_ms[1:]) <= 1.5 * t + 0.02, ppwi
+
+
+def test_a_batch_against_a_small_protein_equals_tiled(gpu_device):
+    # sorted with one pose per work-item, the persistent kernel with more
+    n = 6
+    ls = LigandSet(D.synth_protein(93, 60, 34), D.synth_forcefield(93, 34),
+                   [D.synth_ligand(94 + i, 40 + i, 34) for i in range(n)],
+                   [D.synth_poses(104 + i, 180000 + 11 * i) for i in range(n)])
+    with Batch(ls, gpu_device) as b:
+        b.run_separate(1, 64)
+        want = [b.energies(i) for i in range(n)]
+        for graph in (0, 1):
+            for ppwi in (1, 2, 4, 8):
+                b.clear()
+                b.run(BatchConfig(ppwi, 64, 4, 0, graph), warmup=0, iterations=2)
+                for i in range(n):
+                    assert np.array_equal(b.energies(i).view(np.uint32), want[i].view(np.uint32)), (graph, ppwi, i)
