@@ -213,7 +213,7 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   const bude::items::Work work{ctx->natpro, ctx->ngroups, 1, double(ctx->natlig) * double(ctx->nposes),
                                double(ctx->nposes)};
   const bool few = ctx->nposes <= kHostResult;
-  const int rb = bude::plain_register_block(int(ppwi), int(wgsize));
+  const int rb = bude::plain_register_block(int(ppwi), int(wgsize), ctx->nposes);
   const bool sorted = few ? ctx->sorted.usable() : ctx->sorted.worth(int(ppwi), rb);
   const bool use_direct = !sorted && ctx->direct.ptr && (few || bude::items::worth_direct(work, int(ppwi), rb));
 

@@ -23,8 +23,8 @@ struct PlainArgs {
   int form;                  // 0: hinges in b = d - radij, 1: hinges in d
 };
 
-// Poses per register block actually held in VGPRs for (ppwi, wgsize).
-int plain_register_block(int ppwi, int wgsize);
+// Poses per register block actually held in VGPRs.
+int plain_register_block(int ppwi, int wgsize, size_t nposes);
 
 // One launch over all poses; wgsize in {64, 128, 256, 512, 1024}; ppwi a
 // power of two in [1, 128].

@@ -103,17 +103,20 @@ hipError_t launch_rb(const PlainArgs &a, int wg, size_t blocks, hipStream_t s) {
 
 }  // namespace
 
-int plain_register_block(int ppwi, int wgsize) {
+int plain_register_block(int ppwi, int wgsize, size_t nposes) {
   // VGPR budget per work-item shrinks with the work-group size (1024
-  // work-items = 4 waves per SIMD = 128 VGPRs each).
-  const int cap = wgsize >= 1024 ? 4 : 8;
+  // work-items = 4 waves per SIMD = 128 VGPRs each).  With four waves or more
+  // per SIMD (256 CUs of 4) blocks of eight, of which two fit on a SIMD, lose
+  // to blocks of four: 16 x 16 atoms x 4 M poses at ppwi 8 517 and 464 us, 938
+  // x 8 10,459 and 10,116; with two waves they win (64 x 64 x 1 M 1,755, 2,087).
+  const int cap = wgsize >= 1024 || nposes >= size_t(262144) * size_t(ppwi) ? 4 : 8;
   return ppwi < cap ? ppwi : cap;
 }
 
 hipError_t launch_plain(const PlainArgs &a, int wgsize, hipStream_t s) {
   const size_t items = (a.nposes + size_t(a.ppwi) - 1) / size_t(a.ppwi);
   const size_t blocks = (items + size_t(wgsize) - 1) / size_t(wgsize);
-  switch (plain_register_block(a.ppwi, wgsize)) {
+  switch (plain_register_block(a.ppwi, wgsize, a.nposes)) {
     case 1: return launch_rb<1>(a, wgsize, blocks, s);
     case 2: return launch_rb<2>(a, wgsize, blocks, s);
     case 4: return launch_rb<4>(a, wgsize, blocks, s);
