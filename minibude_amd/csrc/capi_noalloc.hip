@@ -277,7 +277,10 @@ extern "C" int bude_mi355x_fasten_noalloc(int device, const BudeAtom *protein, s
   // poses at a time: all of them, or the whole tiles whose atom sums fit
   const size_t fit = room / (natlig * sizeof(float)) / 64 * 64;
   const size_t at_once = std::min(fit, nposes);
-  if (at_once) {
+  // (the tiled kernel waits for the deck check first: some 12 us)
+  const bude::items::Work work{natpro, ntypes, 1, double(natlig) * double(nposes), double(nposes)};
+  const int rb = bude::plain_register_block(int(ppwi), int(wgsize), nposes);
+  if (at_once && bude::items::worth_direct(work, int(ppwi), rb, (nposes + at_once - 1) / at_once, 12.0)) {
     for (size_t j = 0; j < nposes; j += at_once) {
       const bude::items::DirectArgs a{grouped,       group_begin, coef,        lig4,        poses + j,
                                       energies + j,  pose_stride, std::min(at_once, nposes - j), int(natlig),
@@ -288,7 +291,7 @@ extern "C" int bude_mi355x_fasten_noalloc(int device, const BudeAtom *protein, s
     return read_status();
   }
 
-  // a ligand whose sums do not fit for 64 poses: the tiled kernel, after the check
+  // many poses, or a ligand whose sums do not fit for 64: the tiled kernel, after the check
   if (int st = read_status()) return st;
   bude::PlainArgs a{};
   a.protein = grouped;

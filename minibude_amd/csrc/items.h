@@ -59,7 +59,8 @@ struct Work {
 // Whether sorting pays, and whether the direct pass does, where the other
 // choice is a tiled kernel with ppwi poses per work-item in register blocks of rb.
 bool worth_sorting(const Work &w, int ppwi, int rb);
-bool worth_direct(const Work &w, int ppwi, int rb);
+// passes: launches the direct pass is split into; wait_us: what the tiled kernel costs more than its launch.
+bool worth_direct(const Work &w, int ppwi, int rb, size_t passes = 1, double wait_us = 0.0);
 
 // Device scratch of a pass; one stream at a time may use it.
 struct Workspace {

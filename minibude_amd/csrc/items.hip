@@ -866,12 +866,16 @@ bool worth_sorting(const Work &w, int ppwi, int rb) {
          sorted_us(w) <= tiled_us(w, ppwi, rb);
 }
 
-bool worth_direct(const Work &w, int ppwi, int rb) {
-  // (1 x 64 x 262,144: 102 us, 44 tiled with two poses per work-item; 64 x 8 x
+bool worth_direct(const Work &w, int ppwi, int rb, size_t passes, double wait_us) {
+  // 1 x 64 x 262,144: 102 us, 44 tiled with two poses per work-item; 64 x 8 x
   // 262,144: 107 and 105; larger proteins: nothing between them where the
   // tiled kernel has the poses to fill the device, else the direct pass.  A
-  // tenth is within the estimates)
-  return w.natpro >= 128 || direct_us(w) <= 1.15 * tiled_us(w, ppwi, rb);
+  // tenth is within the estimates.  Split into many launches (3 us each) the
+  // direct pass loses to a full tiled kernel: 64 x 64 x 1,048,576 in 65
+  // launches 3,090 us, 1,810 tiled; 300 x 64 7,110 and 6,480.
+  const bool large = w.natpro >= 128;
+  if (large && passes == 1) return true;
+  return direct_us(w) + 3.0 * double(passes - 1) <= (large ? 1.0 : 1.15) * tiled_us(w, ppwi, rb) + wait_us;
 }
 
 int Plan::build(const std::vector<float4> &atoms, const std::vector<int32_t> &lig_off, int nslots,
