@@ -41,6 +41,7 @@ struct bude_batch {
   std::vector<bude::LigandMeta> meta_host;
   bude::DeviceBuffer protein, group_begin, coef, ligands, meta, poses, energies, counter;
   bude::items::Deck sorted;
+  bude::TileWork work;
   // tile lists per (ppwi, order)
   std::map<std::pair<int, int>, std::unique_ptr<bude::DeviceBuffer>> tiles;
   std::map<std::pair<int, int>, int> ntiles;
@@ -94,28 +95,24 @@ int tiles_for(bude_batch *b, int ppwi, int order, const bude::DeviceBuffer **buf
   return BUDE_OK;
 }
 
-// Whether a batch that is not sorted is so small that a wave of the
-// persistent kernel would score one tile or a few nearly alone on its SIMD:
-// fewer than four 64-pose tiles per SIMD of 256 CUs.
-bool few_tiles(const bude_batch *b) {
-  size_t t = 0;
-  for (size_t n : b->nposes) t += (n + 63) / 64;
-  return t <= 4096;
-}
+// Tiles of 64 poses whatever the configuration where a batch that is not
+// sorted has so few that a wave of the persistent kernel would score one of
+// them or a few nearly alone on its SIMD: fewer than four per SIMD of 256 CUs.
+int tile_ppwi(const bude_batch *b, const BudeBatchConfig *cfg) { return b->work.tiles <= 4096 ? 1 : cfg->ppwi; }
 
 // One pass over the batch: the sorted-item pass where it applies, else
-// work-groups per tile where the tiles are few (the configuration shapes
-// the persistent kernel only), else the persistent kernel.
+// work-groups per tile where the tiles are few (worth_tiles), else the
+// persistent kernel (which alone takes its shape from the configuration).
 int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
-  if (b->sorted.worth(cfg->ppwi, cfg->ppwi))
+  if (b->sorted.worth(cfg->ppwi, cfg->ppwi, bude::items::persistent_pose(cfg->ppwi)))
     return bude::hip_check(b->sorted.launch(static_cast<const float4 *>(b->protein.ptr),
                                             static_cast<const float *>(b->poses.ptr), b->total_poses, nullptr,
                                             static_cast<float *>(b->energies.ptr), b->stream),
                            "sorted batch launch");
   const bude::DeviceBuffer *tb = nullptr;
   int nt = 0;
-  const bool few = few_tiles(b);
-  if (int st = tiles_for(b, few ? 1 : cfg->ppwi, cfg->order, &tb, &nt)) return st;
+  const int ppwi = tile_ppwi(b, cfg);
+  if (int st = tiles_for(b, ppwi, cfg->order, &tb, &nt)) return st;
   bude::BatchArgs a{};
   a.protein = static_cast<const float4 *>(b->protein.ptr);
   a.group_begin = static_cast<const int32_t *>(b->group_begin.ptr);
@@ -130,14 +127,15 @@ int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
   a.ngroups = int(b->ngroups);
   a.ntiles = nt;
   a.form = bude::plain_form();
-  if (few) return bude::hip_check(bude::launch_tiles(a, std::min(nt, 2 * b->cus), b->stream), "fasten_tile launch");
+  if (bude::worth_tiles(b->work, b->natpro, b->ngroups))
+    return bude::hip_check(bude::launch_tiles(a, std::min(nt, 2 * b->cus), b->stream), "fasten_tile launch");
   const int waves = b->cus * 4 * cfg->waves_per_simd;
   const int blocks = std::max(1, waves / (cfg->wgsize / 64));
-  return bude::hip_check(bude::launch_batch(a, cfg->ppwi, cfg->wgsize, blocks, b->stream), "fasten_batch launch");
+  return bude::hip_check(bude::launch_batch(a, ppwi, cfg->wgsize, blocks, b->stream), "fasten_batch launch");
 }
 
 int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
-  const bool sorted = b->sorted.worth(cfg->ppwi, cfg->ppwi);
+  const bool sorted = b->sorted.worth(cfg->ppwi, cfg->ppwi, bude::items::persistent_pose(cfg->ppwi));
   const auto key = sorted ? std::make_tuple(0, 0, 0, 0)
                           : std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
   auto it = b->graphs.find(key);
@@ -146,7 +144,7 @@ int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
     const bude::DeviceBuffer *tb = nullptr;
     int nt = 0;
     if (!sorted)
-      if (int st = tiles_for(b, few_tiles(b) ? 1 : cfg->ppwi, cfg->order, &tb, &nt)) return st;
+      if (int st = tiles_for(b, tile_ppwi(b, cfg), cfg->order, &tb, &nt)) return st;
     auto g = std::make_unique<GraphExec>();
     if (int st = bude::hip_check(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
                                  "hipStreamBeginCapture"))
@@ -235,6 +233,7 @@ extern "C" int bude_mi355x_batch_create(int device, const BudeAtom *protein, siz
     atoms.insert(atoms.end(), ligands[i], ligands[i] + natlig[i]);
     lig_off.push_back(int32_t(atoms.size()));
     segs.push_back(bude::items::Segment{int32_t(i), int64_t(total), int64_t(nposes[i])});
+    b->work.add(natlig[i], nposes[i]);
     b->meta_host.push_back(m);
     b->natlig.push_back(int32_t(natlig[i]));
     b->nposes.push_back(nposes[i]);

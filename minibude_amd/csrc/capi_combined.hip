@@ -173,7 +173,7 @@ Norm norm_of(std::vector<float> e, float clip_q, float tail_q) {
 // One protein's screen: its tables, selection, exact energies of the
 // selection, per-pair results, sampled poses and events.
 struct ProteinSlot {
-  size_t ngroups = 0;
+  size_t natpro = 0, ngroups = 0;
   std::vector<int32_t> coef_off;
   DeviceBuffer protein, group_begin, coef, slot_coef, reach2;
   // what the sorted passes score against (its tables are slot_coef and
@@ -400,9 +400,12 @@ int reserve_sorted(const bude::items::Plan &plan, bude::items::Workspace &w) {
   return st == BUDE_ERR_OUT_OF_MEMORY ? BUDE_OK : st;
 }
 
-// Whether a sorted pass of protein slot ps pays.
+// Whether a sorted pass of protein slot ps pays.  Rows through an index, on a
+// device that scores the next ones, cost the persistent kernel more than twice
+// a pose of a batch: 16 x 262,144 poses against 40 atoms, a tenth rescored,
+// 725 us sorted and 1,160.
 bool sorted_pays(const ProteinSlot &ps, const bude::items::Plan &plan) {
-  return ps.reachable && plan.worth(size_t(ps.scene.natpro), size_t(ps.scene.ngroups), kBatchPpwi);
+  return ps.reachable && plan.worth(ps.natpro, ps.ngroups, kBatchPpwi, 2.0 * bude::items::persistent_pose(kBatchPpwi));
 }
 
 // Whether protein slot ps is scored by this sorted pass, with scratch w.
@@ -743,8 +746,10 @@ int select_and_tables(bude_combined *c, const bude::sel::Plan &plan, size_t firs
 
 // Exact energies of the selected poses into exact_sel, on the first stream:
 // with `plan`, its rows by the sorted pass; those listed by tiles / *ntiles
-// (written on the device by select_and_tables) by work-groups per tile.
-int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, const bude::items::Plan *plan) {
+// (written on the device by select_and_tables) by work-groups per tile (few
+// behind a sorted pass) or the persistent kernel.  The pairs are [first, last).
+int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, size_t first, size_t last,
+                   const bude::items::Plan *plan) {
   if (plan)
     if (int st = bude::hip_check(plan->launch(c->s().scene, c->work, static_cast<const float *>(c->poses.ptr), c->total,
                                               static_cast<const uint32_t *>(c->s().sel_idx.ptr),
@@ -765,7 +770,18 @@ int launch_rescore(bude_combined *c, const int2 *tiles, const int32_t *ntiles, c
   a.form = bude::plain_form();
   a.pose_index = static_cast<const uint32_t *>(c->s().sel_idx.ptr);
   a.ntiles_dev = ntiles;
-  return bude::hip_check(bude::launch_tiles(a, 2 * c->cus, c->stream), "combined rescoring launch");
+  bude::TileWork work;  // what is expected: the tiles are counted on the device
+  if (!plan)
+    for (size_t l = first; l < last; l++)
+      if (!c->s().fallback[l])
+        work.add(c->lig[l].size(), size_t(std::ceil(double(c->s().keep[l]) * double(c->nposes[l]))));
+  if (bude::worth_tiles(work, c->s().natpro, c->s().ngroups))
+    return bude::hip_check(bude::launch_tiles(a, 2 * c->cus, c->stream), "combined rescoring launch");
+  a.counter = static_cast<unsigned int *>(c->counter.ptr);
+  const bude::PinnedGrid g =
+      bude::pinned_grid(c->cus, c->lds_per_cu, batch_waves_per_simd(int64_t(work.tiles), c->cus));
+  a.lds_bytes = g.lds_bytes;
+  return bude::hip_check(bude::launch_batch_indexed(a, g.blocks, c->stream), "combined rescoring launch");
 }
 
 // The ligands [a, b) heaviest first (ties in index order).
@@ -1188,6 +1204,7 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
   //    pair l's at coef_off[l] = lig_off[l] * ngroups) is expanded from it
   //    on the device
   const bude::ProteinGroups groups = bude::group_protein(protein, natpro);
+  c->s().natpro = natpro;
   c->s().ngroups = groups.ngroups();
   const size_t natoms = size_t(c->lig_off.back()) + c->lig.back().size(), ncoef = natoms * c->s().ngroups;
   if (ncoef > 0x7fffffffu) return bude::fail(BUDE_ERR_INVALID_ARGUMENT, "combined: pair tables too large");
@@ -1606,8 +1623,9 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
         return st;
       if (k == 0)
         if (int st = record(c, 7)) return st;
-      if (int st = launch_rescore(c, rs_tiles + c->chunk_tile[k], rs_ntiles + k,
-                                  chunk_sorted(k) ? c->chunk_sorted[k].get() : nullptr)) return st;
+      if (int st = launch_rescore(c, rs_tiles + c->chunk_tile[k], rs_ntiles + k, c->chunk_lig[k], c->chunk_lig[k + 1],
+                                  chunk_sorted(k) ? c->chunk_sorted[k].get() : nullptr))
+        return st;
     }
   } else {
     const bool sorted = nrs > 0 && use_sorted(c->s(), c->whole_sorted, c->work);
@@ -1618,7 +1636,8 @@ int screen_begin(bude_combined *c, const BudeAtom *protein, size_t natpro) {
     if (int st = record(c, 10)) return st;  // the scores are read
     if (int st = record(c, 7)) return st;
     if (nrs)
-      if (int st = launch_rescore(c, rs_tiles, rs_ntiles + K, sorted ? &c->whole_sorted : nullptr)) return st;
+      if (int st = launch_rescore(c, rs_tiles, rs_ntiles + K, 0, L, sorted ? &c->whole_sorted : nullptr))
+        return st;
   }
   // the counts land in pinned memory: the host does not wait here
   if (int st = bude::hip_check(hipMemcpyAsync(c->s().nsel_host, c->s().sel_n.ptr, L * 4, hipMemcpyDeviceToHost,

@@ -44,6 +44,7 @@ double ms_since(std::chrono::steady_clock::time_point t0) {
 struct bude_screen {
   int device = 0;
   int cus = 0;
+  size_t lds_per_cu = 0;
   BudeScreenConfig cfg{};
   // plain-kernel deck (labels, rescoring, fallback)
   size_t natlig = 0, ngroups = 0;
@@ -60,7 +61,7 @@ struct bude_screen {
   DeviceBuffer cand, pred, sel_idx, sel_n, exact;
   // rescoring: rows through sel_idx, one ligand whose pose count and tiles
   // (first pose of 64) the device writes from the selection's size
-  DeviceBuffer rs_tiles, rs_meta, rs_order, rs_ntiles;
+  DeviceBuffer rs_tiles, rs_meta, rs_counter, rs_order, rs_ntiles;
   bude::sel::Plan plan;  // one segment: the loaded poses, k = ceil(keep_fraction * n)
   size_t plan_n = 0, plan_k = 0;
   // the sorted passes over the selection's first plan_k rows (the tiled
@@ -132,8 +133,8 @@ int upload_poses(DeviceBuffer &d, const float *const poses[6], size_t n) {
 
 // Exact energies of the selected poses (rows sel_idx[0, nsel) of the
 // candidates) into exact[0, nsel): the sorted pass over the plan_k rows that
-// are always there, where it applies, and work-groups per 64 poses
-// (bit-identical) over the rest.  The tables come from the selection's count
+// are always there, where it applies, and work-groups per 64 poses or the
+// persistent kernel (bit-identical) over the rest.  The tables come from the selection's count
 // on the device; the host does not wait for it.
 int rescore(bude_screen *s) {
   const bool sorted = s->sel_deck.worth(1, 1);
@@ -167,7 +168,14 @@ int rescore(bude_screen *s) {
   a.form = bude::plain_form();
   a.pose_index = static_cast<const uint32_t *>(s->sel_idx.ptr);
   a.ntiles_dev = static_cast<const int32_t *>(s->rs_ntiles.ptr);
-  return bude::hip_check(bude::launch_tiles(a, 2 * s->cus, s->stream), "rescore launch");
+  bude::TileWork work;  // what is expected: the tiles are counted on the device
+  if (!sorted) work.add(s->natlig, s->plan_k);
+  if (bude::worth_tiles(work, s->groups.xyzw.size() / 4, s->ngroups))
+    return bude::hip_check(bude::launch_tiles(a, 2 * s->cus, s->stream), "rescore launch");
+  a.counter = static_cast<unsigned int *>(s->rs_counter.ptr);
+  const bude::PinnedGrid g = bude::pinned_grid(s->cus, s->lds_per_cu, 3);
+  a.lds_bytes = g.lds_bytes;
+  return bude::hip_check(bude::launch_batch_indexed(a, g.blocks, s->stream), "rescore launch");
 }
 
 // Surrogate predictions (normalised target units) for n poses whose 6 rows
@@ -205,6 +213,7 @@ extern "C" int bude_mi355x_screen_create(int device, const BudeAtom *protein, si
   hipDeviceProp_t props{};
   if (int st = bude::hip_check(hipGetDeviceProperties(&props, device), "hipGetDeviceProperties")) return st;
   s->cus = props.multiProcessorCount;
+  s->lds_per_cu = props.maxSharedMemoryPerMultiProcessor;
   s->natlig = natlig;
   s->atoms.assign(ligand, ligand + natlig);
   s->ff.assign(forcefield, forcefield + ntypes);
@@ -349,6 +358,7 @@ extern "C" int bude_mi355x_screen_load(bude_screen *s, const float *const poses[
   if (!st) st = s->sel_idx.alloc(n * 4);
   if (!st) st = s->exact.alloc(n * 4);
   if (!st) st = s->rs_tiles.alloc((n + 63) / 64 * sizeof(int2));
+  if (!st) st = s->rs_counter.alloc(sizeof(unsigned int));
   if (!st) st = s->rs_ntiles.alloc(sizeof(int32_t));
   if (!st) {  // the one ligand's row of the rescoring meta (its pose count comes from the selection)
     const bude::LigandMeta m{0, int32_t(s->natlig), 0, 0, 0, 0};

@@ -34,7 +34,7 @@ struct BatchArgs {
   int form;                     // hinge form (plain_form())
   unsigned lds_bytes;           // dynamic LDS per work-group, unused by the kernel: sized so that exactly
                                 // n work-groups fit on a CU, it pins the waves per SIMD (0: no pinning)
-  // launch_tiles only (null: not used): row j of ligand l is pose meta[l].pose_off + pose_index[meta[l].pose_off + j]
+  // launch_tiles and launch_batch_indexed only (null: not used): row j of ligand l is pose meta[l].pose_off + pose_index[meta[l].pose_off + j]
   // (energies still at meta[l].pose_off + j), and the tile count is read from device memory
   const uint32_t *pose_index;
   const int32_t *ntiles_dev;
@@ -68,6 +68,20 @@ hipError_t launch_batch(const BatchArgs &a, int rb, int wgsize, int blocks, hipS
 // done[l], the rows another pass scores (0 when done is null).
 hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel_n, const uint32_t *done,
                                 LigandMeta *meta, int2 *tiles, int32_t *ntiles, hipStream_t s);
+
+// launch_batch over rows that are a per-segment selection (pose_index) with
+// tiles and tile count written by an earlier kernel (ntiles_dev): one pose
+// per work-item (rb 1), work-groups of 256.  Energies are bit-equal to
+// launch_batch's for the same poses.
+hipError_t launch_batch_indexed(const BatchArgs &a, int blocks, hipStream_t s);
+
+// The work of a pass over tiles of 64 poses, and whether launch_tiles is the
+// faster form for it (else launch_batch with rb 1).
+struct TileWork {
+  double tiles = 0, items = 0, rounds = 0;
+  void add(size_t natlig, size_t poses);
+};
+bool worth_tiles(const TileWork &w, size_t natpro, size_t ngroups);
 
 // The pass over few tiles of 64 poses: `blocks` work-groups of 16 waves, each
 // sharing a tile at a time.  Rows may be a per-segment selection

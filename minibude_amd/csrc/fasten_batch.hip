@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "bude_internal.h"
 #include "fasten_batch.h"
@@ -30,13 +31,16 @@ __global__ void reset_counter_kernel(unsigned int *__restrict__ counter) {
   if (threadIdx.x == 0) counter[0] = 0u;
 }
 
-template <int RB, int WG, int FORM>
+// INDEXED: pose rows through pose_index, tile count from ntiles_dev (both
+// written by earlier kernels on the device).
+template <int RB, int WG, int FORM, bool INDEXED = false>
 __global__ __launch_bounds__(WG) void fasten_batch_kernel(
     const float4 *__restrict__ protein, const int32_t *__restrict__ group_begin, const PairCoef *__restrict__ coef,
     const float4 *__restrict__ ligands, const LigandMeta *__restrict__ meta, const int2 *__restrict__ tiles,
     const float *__restrict__ poses, float *__restrict__ energies, unsigned int *__restrict__ counter, size_t stride,
-    int ngroups, int ntiles) {
+    int ngroups, int ntiles, const uint32_t *__restrict__ pose_index, const int32_t *__restrict__ ntiles_dev) {
   const int lane = threadIdx.x & 63;
+  if constexpr (INDEXED) ntiles = *ntiles_dev;
   for (;;) {
     // One atomic per wave; every wave leaves once the list is exhausted.
     unsigned int t = 0;
@@ -51,7 +55,9 @@ __global__ __launch_bounds__(WG) void fasten_batch_kernel(
 #pragma unroll
     for (int k = 0; k < RB; ++k) {
       const int j = tile.y + lane + k * 64;
-      tr[k] = make_xform(poses, stride, size_t(m.pose_off) + size_t(j < m.nposes ? j : m.nposes - 1));
+      size_t q = size_t(m.pose_off) + size_t(j < m.nposes ? j : m.nposes - 1);
+      if constexpr (INDEXED) q = size_t(m.pose_off) + pose_index[q];
+      tr[k] = make_xform(poses, stride, q);
       e[k] = 0.f;
     }
     for (int il = 0; il < m.natlig; ++il) {
@@ -79,7 +85,7 @@ __global__ __launch_bounds__(WG) void fasten_batch_kernel(
   }
 }
 
-// The form for few tiles: one work-group of 16 waves per tile of 64 poses,
+// The form for few tiles (worth_tiles): one work-group of 16 waves per tile of 64 poses,
 // its waves sharing the ligand's atoms, whose energies meet in LDS and are
 // added in order by wave 0.  A wave that scores a tile alone is a chain over
 // every pair (56 x 2,046 atoms: 4-6 ms, however few the tiles; the rows that
@@ -244,11 +250,11 @@ hipError_t launch_rb_wg(const BatchArgs &a, int blocks, hipStream_t s) {
   if (a.form == kFormD)
     hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<RB, WG, kFormD>), dim3(unsigned(blocks)), dim3(WG),
                        a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles);
+                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles, nullptr, nullptr);
   else
     hipLaunchKernelGGL(HIP_KERNEL_NAME(fasten_batch_kernel<RB, WG, kFormB>), dim3(unsigned(blocks)), dim3(WG),
                        a.lds_bytes, s, a.protein, a.group_begin, a.coef, a.ligands, a.meta, a.tiles, a.poses,
-                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles);
+                       a.energies, a.counter, a.stride, a.ngroups, a.ntiles, nullptr, nullptr);
   return hipGetLastError();
 }
 
@@ -302,6 +308,46 @@ hipError_t build_rescore_tables(const int32_t *order, int n, const uint32_t *sel
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(rescore_tables_kernel, dim3(1), dim3(256), 0, s, order, n, sel_n, done, meta, tiles, ntiles);
   return hipGetLastError();
+}
+
+hipError_t launch_batch_indexed(const BatchArgs &a, int blocks, hipStream_t s) {
+  if (!a.pose_index || !a.ntiles_dev || blocks < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, s, a.counter);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(256), a.lds_bytes, s, a.protein, a.group_begin, a.coef,
+                       a.ligands, a.meta, a.tiles, a.poses, a.energies, a.counter, a.stride, a.ngroups, 0,
+                       a.pose_index, a.ntiles_dev);
+  };
+  if (a.form == kFormD) run(fasten_batch_kernel<1, 256, kFormD, true>);
+  else run(fasten_batch_kernel<1, 256, kFormB, true>);
+  return hipGetLastError();
+}
+
+// Both forms in microseconds.  A round of a shared tile scores up to 16 of its
+// atoms, one per wave: 4 times what a wave alone takes for an atom with 16, 2.2
+// with two (two work-groups share a CU, and 512 tiles are in flight), rounds
+// wait for each other.  The persistent kernel scores all pairs at the
+// device's rate with four waves per SIMD (4,096 tiles) and more, and lets
+// waves stand alone below that; its queue and reset cost some 60 us.  4,096
+// tiles of 2, 8, 17, 33 and 40 atoms against 4,096: shared 2,295, 3,188,
+// 7,743, 13,230 and 14,170 us, persistent 843, 3,010, 6,170, 11,730 and
+// 14,190; 1,024 tiles of 17 2,036 and 3,500, 256 of them 527 and 2,558; 4,096
+// tiles of 1 and 17 against 16 atoms 78 and 173, 122 and 182.
+void TileWork::add(size_t natlig, size_t poses) {
+  const double n = double((poses + 63) / 64), rest = double(natlig % 16);
+  tiles += n;
+  items += double(natlig) * double(poses);
+  rounds += n * (4.0 * double(natlig / 16) + (rest > 0 ? 1.9 + 0.13 * rest : 0.0));
+}
+
+bool worth_tiles(const TileWork &w, size_t natpro, size_t ngroups) {
+  if (w.tiles > 4096 || w.tiles <= 0) return w.tiles <= 0;
+  const double p = double(natpro), g = double(ngroups);
+  const double alone = 0.033 * p + 0.2 * g;  // one wave, one atom
+  const double shared = 1.12 * alone * w.rounds / std::min(512.0, w.tiles);
+  const double full = w.items * (0.29 * p + 0.5 * g * std::min(1.0, 64.0 / p)) * 1e-6;
+  return shared <= 60.0 + full * (1.0 + (p < 400 ? 2.3 : 1.2) * std::pow(1024.0 / w.tiles, 1.5));
 }
 
 hipError_t launch_tiles(const BatchArgs &a, int blocks, hipStream_t s) {

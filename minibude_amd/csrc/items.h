@@ -58,7 +58,11 @@ struct Work {
 
 // Whether sorting pays, and whether the direct pass does, where the other
 // choice is a tiled kernel with ppwi poses per work-item in register blocks of rb.
-bool worth_sorting(const Work &w, int ppwi, int rb);
+// pose_ps: the tiled kernel's cost of a pose besides its items' (kPlainPose,
+// or the persistent kernel's), in ps of the whole device.
+constexpr double kPlainPose = 8.0;
+inline double persistent_pose(int rb) { return 40.0 + 160.0 / rb; }
+bool worth_sorting(const Work &w, int ppwi, int rb, double pose_ps = kPlainPose);
 // passes: launches the direct pass is split into; wait_us: what the tiled kernel costs more than its launch.
 bool worth_direct(const Work &w, int ppwi, int rb, size_t passes = 1, double wait_us = 0.0);
 
@@ -84,8 +88,8 @@ class Plan {
   // the pose row of row i of a segment is pose_off + index[pose_off + i].
   hipError_t launch(const Scene &sc, const Workspace &w, const float *poses, size_t stride, const uint32_t *index,
                     float *energies, hipStream_t s) const;
-  bool worth(size_t natpro, size_t ngroups, int ppwi) const {
-    return !chunks_.empty() && worth_sorting(Work{natpro, ngroups, nsegs_, items_, poses_}, ppwi, ppwi);
+  bool worth(size_t natpro, size_t ngroups, int ppwi, double pose_ps) const {
+    return !chunks_.empty() && worth_sorting(Work{natpro, ngroups, nsegs_, items_, poses_}, ppwi, ppwi, pose_ps);
   }
   bool empty() const { return chunks_.empty(); }
   void clear() {
@@ -161,7 +165,9 @@ class Deck {
   int prepare(const ProteinGroups &groups, const BudeFFParams *ff, const std::vector<BudeAtom> &atoms,
               const std::vector<int32_t> &lig_off, const std::vector<Segment> &segs);
   bool usable() const { return usable_; }
-  bool worth(int ppwi, int rb) const { return usable_ && worth_sorting(shape_, ppwi, rb); }
+  bool worth(int ppwi, int rb, double pose_ps = kPlainPose) const {
+    return usable_ && worth_sorting(shape_, ppwi, rb, pose_ps);
+  }
   // Not usable() any more, and holding no memory.
   void release();
   hipError_t launch(const float4 *protein, const float *poses, size_t stride, const uint32_t *index, float *energies,

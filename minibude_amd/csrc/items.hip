@@ -827,10 +827,12 @@ namespace {
 // 2, 4 and 8 poses a register block, 16 x 64 13, 8.2, 7.4 and 7.7, 1 x 64 1.7
 // to 1.1, 4,096 x 26 1,207; a group costs the more the fewer atoms it has and
 // poses share it.  With w waves per SIMD it takes 1 + 2.3 / (sqrt(rb) w^1.5)
-// times as long (64 x 64 with rb 1: 3.9 at w = 1, 1.31 at 4).
-double tiled_us(const Work &w, int ppwi, int rb) {
+// times as long (64 x 64 with rb 1: 3.9 at w = 1, 1.31 at 4).  The persistent
+// kernel takes a pose's transform and its place in the queue worse: 256 x 20 x
+// 4,096 poses against one atom 265 us with rb 1, 131 with 4.
+double tiled_us(const Work &w, int ppwi, int rb, double pose_ps = kPlainPose) {
   const double natpro = double(w.natpro), groups = double(w.ngroups) * std::min(1.0, 64.0 / natpro);
-  const double full = w.items * (0.29 * natpro + groups * (0.1 + 0.4 / rb)) + 8.0 * w.poses;
+  const double full = w.items * (0.29 * natpro + groups * (0.1 + 0.4 / rb)) + pose_ps * w.poses;
   return full * 1e-6 * (1.0 + 2.3 / std::sqrt(double(rb)) * std::pow(65536.0 * ppwi / w.poses, 1.5));
 }
 
@@ -850,7 +852,7 @@ double direct_us(const Work &w) {
 
 }  // namespace
 
-bool worth_sorting(const Work &w, int ppwi, int rb) {
+bool worth_sorting(const Work &w, int ppwi, int rb, double pose_ps) {
   // Against the direct pass: that scores some 1.8e9 pairs a millisecond; the sort's seven
   // launches cost 40-50 us whatever the size, and with few items (large
   // boxes) scoring them grows with the protein.  Both measured, direct and
@@ -863,7 +865,7 @@ bool worth_sorting(const Work &w, int ppwi, int rb) {
   // 1,690 tiled with two poses per work-item; 4 x 64 x 262,144: 504 and 91).
   const double natpro = double(w.natpro);
   return w.items * natpro >= 6e7 + 8e4 * natpro && w.items >= 4096.0 * double(w.nsegs) &&
-         sorted_us(w) <= tiled_us(w, ppwi, rb);
+         sorted_us(w) <= tiled_us(w, ppwi, rb, pose_ps);
 }
 
 bool worth_direct(const Work &w, int ppwi, int rb, size_t passes, double wait_us) {
@@ -1211,7 +1213,7 @@ int Deck::plan(const ProteinGroups &groups, const BudeFFParams *ff, const std::v
     shape_.items += double(lig_off[size_t(s.lig) + 1] - lig_off[size_t(s.lig)]) * double(s.n);
     shape_.poses += double(s.n);
   }
-  if (!worth_sorting(shape_, 1, 1) && !worth_sorting(shape_, 8, 8)) return BUDE_OK;
+  if (!worth_sorting(shape_, 1, 1, persistent_pose(1)) && !worth_sorting(shape_, 8, 8)) return BUDE_OK;
   // slots: the forcefield types the ligands use, ascending
   std::vector<int32_t> types;
   for (const BudeAtom &a : atoms) types.push_back(a.type);

@@ -6,10 +6,11 @@ holds a pose, never the sums."""
 import numpy as np
 import pytest
 
-import oracle_lib as O
+from minibude_amd import combined as C
 from minibude_amd import deck as D
+from minibude_amd import screen as S
 from minibude_amd.batch import Batch, LigandSet
-from minibude_amd.model import Context
+from minibude_amd.capi import BatchConfig
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +32,53 @@ def test_blocks_over_a_full_device_equal_single_poses(gpu_device, ppwi):
             b.clear()
             b.run_separate(ppwi, wgsize)
             assert np.array_equal(bits(b.energies(0)), bits(want)), wgsize
+
+
+def unreachable(natpro, natlig, nposes, seed, ntypes=34):
+    """Ligands of natlig[i] atoms with nposes[i] poses that have a pair without a reach."""
+    ff = D.synth_forcefield(seed, ntypes)
+    ff["radius"][3] = 0.0
+    pro = D.synth_protein(seed, natpro, ntypes)
+    pro["type"][0] = 3
+    ligs = [D.synth_ligand(seed + 1 + i, n, ntypes) for i, n in enumerate(natlig)]
+    for l in ligs:
+        l["type"][0] = 3
+    return LigandSet(pro, ff, ligs, [D.synth_poses(seed + 1 + i, n) for i, n in enumerate(nposes)])
+
+
+def test_few_tiles_of_small_ligands(gpu_device):
+    # a tile's 16 waves have nothing to share in a ligand of two atoms: the
+    # persistent kernel takes them, in a quarter of the time that eight atoms
+    # take (shared tiles took three quarters)
+    times = []
+    for natlig in (2, 8):
+        ls = unreachable(4096, [natlig] * 64, [4096] * 64, 44)
+        with Batch(ls, gpu_device) as b:
+            b.run_separate(1, 64)
+            want = [b.energies(i) for i in range(64)]
+            for cfg in (BatchConfig(1, 64, 4, 0, 1), BatchConfig(4, 256, 8, 1, 0)):
+                b.clear()
+                t = min(b.run(cfg, 1, 4)[1:])
+                assert all(np.array_equal(bits(b.energies(i)), bits(want[i])) for i in range(64)), (natlig, cfg.ppwi)
+            times.append(t)
+    assert times[0] < 0.5 * times[1]
+
+
+def test_selections_of_many_rows_without_a_reach(gpu_device):
+    # some 9,400 and 4,700 tiles of selected rows, through the index
+    ls = unreachable(300, [5, 17], [400000, 200000], 46)
+    cfg = C.default_config("field", keep_fraction=0.5, widen_max=0.5, gate_z=0.0, grid_spacing=1.5)
+    with C.Combined(ls.forcefield, ls.ligands, ls.poses, cfg, gpu_device) as c:
+        c.screen(ls.protein)
+        c.exhaustive()
+        for l in range(2):
+            idx, e = c.selected(l)
+            assert len(idx) >= len(c.exact(l)) // 2 and np.array_equal(bits(e), bits(c.exact(l)[idx])), l
+    cfg = S.default_config(epochs=1, batch=1024, keep_fraction=0.75)
+    with S.Screen(ls.protein, ls.ligands[0], ls.forcefield, cfg, gpu_device) as s:
+        s.train(D.synth_poses(48, 16384))
+        s.load(ls.poses[0])
+        s.run()
+        idx, e = s.selected()
+        exact = s.exhaustive()[0]
+        assert len(idx) >= 300000 and np.array_equal(bits(e), bits(exact[idx]))
