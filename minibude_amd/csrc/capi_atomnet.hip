@@ -77,12 +77,19 @@ extern "C" int bude_mi355x_atom_energies(int device, const BudeAtom *protein, si
   std::vector<BudeAtom> probe(ntypes);
   for (size_t t = 0; t < ntypes; t++) probe[t] = BudeAtom{0.f, 0.f, 0.f, int32_t(t)};
   const std::vector<bude::PairCoef> coef = bude::coef_table(probe.data(), ntypes, groups, forcefield);
-  bude::DeviceBuffer dprot, dbegin, dcoef, dpts, dout;
-  int st = dprot.upload(groups.xyzw.data(), groups.xyzw.size() * 4);
-  if (!st) st = dcoef.upload(coef.data(), coef.size() * sizeof(bude::PairCoef));
+  // Sorted by type and place on the device, or, a few points against a small
+  // protein, grouped on the host: the sort's launches cost 40 us, the grouping
+  // 7 ns a point and the unsorted pass 0.1 us a protein atom (8 atoms x 1,000
+  // points 99 us grouped, 137 sorted; 300 x 1,000 133 and 153; 300 x 10,000 202
+  // and 183; 1,000 x 1,000 191 and 173; 4,096 x 64 555 and 389).
   std::vector<float4> reach2;
   float largest = 0.f;
-  if (!st && bude::items::reach_table(coef, ng, reach2, &largest)) {  // sorted by type and place on the device
+  const bool sort = n + 6 * natpro >= 7000 && bude::items::reach_table(coef, ng, reach2, &largest);
+  bude::DeviceBuffer dprot, dbegin, dcoef, dpts, dout;
+  int st = dprot.upload(groups.xyzw.data(), groups.xyzw.size() * 4);
+  if (!st && !sort) st = dbegin.upload(groups.begin.data(), groups.begin.size() * 4);
+  if (!st) st = dcoef.upload(coef.data(), coef.size() * sizeof(bude::PairCoef));
+  if (!st && sort) {
     bude::DeviceBuffer dtypes, dreach;
     st = dreach.upload(reach2.data(), reach2.size() * sizeof(float4));
     if (!st) st = dpts.upload(points, n * 3 * sizeof(float));
@@ -104,8 +111,8 @@ extern "C" int bude_mi355x_atom_energies(int device, const BudeAtom *protein, si
     if (!st) st = bude::hip_check(hipMemcpy(out, dout.ptr, n * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
     return st ? st : bude::ok();
   }
-  // no reach (a radius sum that is not positive, a weight that is not
-  // finite): points grouped by type into whole 64-point blocks (a block's
+  // (also without a reach: a radius sum that is not positive, a weight that is
+  // not finite) points grouped by type into whole 64-point blocks (a block's
   // padding repeats its last point)
   std::vector<std::vector<size_t>> by(ntypes);
   for (size_t i = 0; i < n; i++) by[size_t(types[i])].push_back(i);
@@ -124,7 +131,6 @@ extern "C" int bude_mi355x_atom_energies(int device, const BudeAtom *protein, si
     }
   }
   const size_t np = where.size();
-  if (!st) st = dbegin.upload(groups.begin.data(), groups.begin.size() * 4);
   if (!st) st = dpts.upload(pts.data(), pts.size() * 4);
   if (!st) st = dout.alloc(np * 4);
   if (!st)

@@ -242,3 +242,17 @@ def test_a_batch_against_a_small_protein_equals_tiled(gpu_device):
                 b.run(BatchConfig(ppwi, 64, 4, 0, graph), warmup=0, iterations=2)
                 for i in range(n):
                     assert np.array_equal(b.energies(i).view(np.uint32), want[i].view(np.uint32)), (graph, ppwi, i)
+
+
+@pytest.mark.parametrize("natpro, npoints", [(1000, 999), (1000, 1000), (300, 5199), (300, 5200)])
+def test_atom_energies_either_side_of_sorting(gpu_device, natpro, npoints):
+    rng = np.random.default_rng(95)
+    pro, ff = D.synth_protein(96, natpro, 34), D.synth_forcefield(96, 34)
+    pts = rng.uniform(-20, 20, (npoints + 500, 3)).astype(np.float32)
+    types = rng.integers(0, 34, npoints + 500).astype(np.int32)
+    got = atomnet.atom_energies(pro, ff, pts[:npoints], types[:npoints], gpu_device)
+    more = atomnet.atom_energies(pro, ff, np.repeat(pts, 2, 0), np.repeat(types, 2), gpu_device)[::2]  # (sorted)
+    few = np.concatenate([atomnet.atom_energies(pro, ff, pts[i:i + 50], types[i:i + 50], gpu_device)
+                          for i in range(0, npoints, 50)])[:npoints]  # (grouped on the host)
+    assert np.array_equal(got.view(np.uint32), more[:npoints].view(np.uint32))
+    assert np.array_equal(got.view(np.uint32), few.view(np.uint32))
