@@ -29,11 +29,12 @@ in HBM.  Prints ONE JSON line:
                 resolves (|E| >= 0.002 * M, M = 0.5 * sum |term| from the
                 committed FP64 fixture), and |E - E_fp64| / M within 16 FP32
                 epsilons on every pose (the reference's own FP32: 8.8)
-  sweep         the 40-point ppwi x wgsize sweep of the plain kernel
+  sweep         the 40-point ppwi x wgsize sweep (the workload's deck is
+                scored by sorted items, whatever the point)
   batched       the ragged screen (256 ligands of 8-96 atoms, 4,096-65,536
-                poses each, one 4,096-atom protein) in one persistent
-                hipGraph-replayed launch at the launch shape the batched
-                autotuner picks on it, vs 256 separate plain launches
+                poses each, one 4,096-atom protein) in one
+                hipGraph-replayed pass, at the configuration the batched
+                autotuner returns for it, vs 256 separate plain launches
   screen        the learned prescreen (4,096-atom protein, 26-atom ligand,
                 16.8M fresh poses, lowest 2 % rescored exactly): the pose MLP
                 with the 12 configured inputs and with 21, each trained on
@@ -235,7 +236,7 @@ def batched() -> dict:
     ls = ragged_workload()
     log(f"batched: {len(ls.ligands)} ligands, {ls.total_poses} poses, {ls.interactions:.3e} interactions")
     with Batch(ls, 0) as b:
-        # the launch shape is the project's autotuner's choice on this batch
+        # the configuration is the autotuner's choice on this batch
         t0 = time.time()
         cfg, tune_ms = b.autotune()
         tune_s = time.time() - t0
@@ -253,9 +254,10 @@ def batched() -> dict:
         "speedup_vs_separate": round(ts / t, 2),
         "config": cfg.as_dict(),
         "autotune": {"seconds": round(tune_s, 2), "best_ms": round(tune_ms, 3),
-                     "search": ("bude_mi355x_batch_autotune on this batch: 24 candidates (tile width 64/128/256 "
+                     "search": ("bude_mi355x_batch_autotune on this batch: of 24 candidates (tile width 64/128/256 "
                                 "poses, work-group 64/256, 4/8 waves per SIMD, heaviest-first or ligand order; "
-                                "hipGraph replays), each timed once, the 4 fastest by the median of 3")},
+                                "hipGraph replays) each that gives another pass (a sorted batch has one) timed "
+                                "once, the 4 fastest by the median of 3")},
     }
     log(f"batched: {out}")
     return out

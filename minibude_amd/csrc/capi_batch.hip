@@ -9,6 +9,7 @@
 #include <map>
 #include <memory>
 #include <numeric>
+#include <set>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -100,11 +101,23 @@ int tiles_for(bude_batch *b, int ppwi, int order, const bude::DeviceBuffer **buf
 // them or a few nearly alone on its SIMD: fewer than four per SIMD of 256 CUs.
 int tile_ppwi(const bude_batch *b, const BudeBatchConfig *cfg) { return b->work.tiles <= 4096 ? 1 : cfg->ppwi; }
 
+// What of a configuration a pass over this batch depends on: nothing (sorted),
+// the tiles' order (work-groups per tile), or its shape and order.
+using Shape = std::tuple<int, int, int, int>;
+bool sorted_pass(const bude_batch *b, const BudeBatchConfig *cfg) {
+  return b->sorted.worth(cfg->ppwi, cfg->ppwi, bude::items::persistent_pose(cfg->ppwi));
+}
+Shape shape_of(const bude_batch *b, const BudeBatchConfig *cfg) {
+  if (sorted_pass(b, cfg)) return {0, 0, 0, 0};
+  if (bude::worth_tiles(b->work, b->natpro, b->ngroups)) return {1, 0, 0, cfg->order};
+  return {tile_ppwi(b, cfg), cfg->wgsize, cfg->waves_per_simd, cfg->order};
+}
+
 // One pass over the batch: the sorted-item pass where it applies, else
 // work-groups per tile where the tiles are few (worth_tiles), else the
 // persistent kernel (which alone takes its shape from the configuration).
 int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
-  if (b->sorted.worth(cfg->ppwi, cfg->ppwi, bude::items::persistent_pose(cfg->ppwi)))
+  if (sorted_pass(b, cfg))
     return bude::hip_check(b->sorted.launch(static_cast<const float4 *>(b->protein.ptr),
                                             static_cast<const float *>(b->poses.ptr), b->total_poses, nullptr,
                                             static_cast<float *>(b->energies.ptr), b->stream),
@@ -135,15 +148,13 @@ int launch_once(bude_batch *b, const BudeBatchConfig *cfg) {
 }
 
 int graph_for(bude_batch *b, const BudeBatchConfig *cfg, hipGraphExec_t *exec) {
-  const bool sorted = b->sorted.worth(cfg->ppwi, cfg->ppwi, bude::items::persistent_pose(cfg->ppwi));
-  const auto key = sorted ? std::make_tuple(0, 0, 0, 0)
-                          : std::make_tuple(cfg->ppwi, cfg->wgsize, cfg->waves_per_simd, cfg->order);
+  const Shape key = shape_of(b, cfg);
   auto it = b->graphs.find(key);
   if (it == b->graphs.end()) {
     // build tiles before capture (the upload is not capturable)
     const bude::DeviceBuffer *tb = nullptr;
     int nt = 0;
-    if (!sorted)
+    if (!sorted_pass(b, cfg))
       if (int st = tiles_for(b, tile_ppwi(b, cfg), cfg->order, &tb, &nt)) return st;
     auto g = std::make_unique<GraphExec>();
     if (int st = bude::hip_check(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal),
@@ -315,13 +326,16 @@ extern "C" int bude_mi355x_batch_autotune(bude_batch *b, BudeBatchConfig *best, 
   // Candidate tile widths, work-group sizes, persistent-grid depths and tile
   // orders, by successive halving: every candidate's graph is built and
   // replayed twice (the second replay timed), then the four fastest are
-  // timed as the median of three more replays each.
+  // timed as the median of three more replays each.  Of candidates that give
+  // the same pass only the first is timed (all of them where it is sorted).
   std::vector<std::pair<double, BudeBatchConfig>> round1;
+  std::set<Shape> timed_shapes;
   for (int ppwi : {1, 2, 4})
     for (int wg : {64, 256})
       for (int wps : {4, 8})
         for (int order : {0, 1}) {
           BudeBatchConfig c{ppwi, wg, wps, order, 1};
+          if (!timed_shapes.insert(shape_of(b, &c)).second) continue;
           double ms[2] = {0, 0};
           if (int st = bude_mi355x_batch_run(b, &c, 1, 1, ms)) return st;
           round1.emplace_back(ms[1], c);

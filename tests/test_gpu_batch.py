@@ -2,6 +2,8 @@
 same per-pose operation sequence) and the oracle, on ragged shapes the
 reference driver never runs (pose counts that divide nothing, 1-pose
 ligands, ligands larger than a wavefront)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -67,3 +69,16 @@ def test_separate_baseline_and_autotune(gpu_device):
         b.run(cfg)
         for i in range(16):
             assert np.array_equal(b.energies(i).view(np.uint32), sep[i].view(np.uint32))
+
+
+def test_autotune_times_a_pass_once(gpu_device):
+    # every candidate of a sorted batch gives the same pass: the first is
+    # returned, after one warm-up, one timed and three more passes (not 60)
+    ls = ragged_workload(nligands=16, natpro=3000, seed=7, natlig_range=(60, 96), nposes_range=(30000, 40000))
+    with Batch(ls, gpu_device) as b:
+        b.run(BatchConfig(1, 64, 4, 0, 0))
+        t = time.perf_counter()
+        cfg, ms = b.autotune()
+        wall = (time.perf_counter() - t) * 1e3
+    assert (cfg.ppwi, cfg.wgsize, cfg.waves_per_simd, cfg.order, cfg.use_graph) == (1, 64, 4, 0, 1)
+    assert wall <= 20 * ms + 20
