@@ -69,7 +69,8 @@ int bude_mi355x_compatible(int device, size_t ppwi, size_t wgsize, int *ok);
 /* ---- plain fasten_main: HipBude::fasten, src/hip/fasten.hpp:212-267 ---- */
 typedef struct bude_ctx bude_ctx;
 
-/* Allocates device buffers on `device` and copies the deck in
+/* Allocates device buffers on `device` (with up to some 5 GB of scratch for
+ * sorting, where it pays and there is memory for it) and copies the deck in
  * (src/hip/fasten.hpp:214-232, the reference's contextTime).  poses[k]
  * points at row k of the deck's SoA pose table, nposes floats each
  * (src/main.cpp:294-311): rows 0-2 are the tilt/roll/pan angles in radians,
@@ -78,16 +79,19 @@ int bude_mi355x_create(int device, const BudeAtom *protein, size_t natpro, const
                        const BudeFFParams *forcefield, size_t ntypes, const float *const poses[6], size_t nposes,
                        bude_ctx **out);
 
-/* Runs warmup + iterations launches of the kernel with `ppwi` poses per
- * work-item and `wgsize` work-items per work-group over all poses
- * (src/hip/fasten.hpp:234-248), then copies the energies out
- * (src/hip/fasten.hpp:250-251; energies_out may be NULL to skip the copy).
- * Per launch, in order (warmup first), writes:
- *   host_ms[i]   host wall time of launch + hipStreamSynchronize, the
+/* Runs warmup + iterations passes over all poses (src/hip/fasten.hpp:234-248),
+ * then hands the energies out (src/hip/fasten.hpp:250-251; energies_out may
+ * be NULL to skip that).  A pass is the form that suits the deck: sorted
+ * items, a work-group per (64 poses, ligand atom), or the kernel with `ppwi`
+ * poses per work-item and `wgsize` work-items per work-group, the only one
+ * these two shape; every form gives the same bits.
+ * Per pass, in order (warmup first), writes:
+ *   host_ms[i]   host wall time of its launches + hipStreamSynchronize, the
  *                reference's Sample::kernelTimes (may be NULL)
- *   device_ms[i] hipEvent time of the launch on the library's stream
+ *   device_ms[i] hipEvent time of its launches on the library's stream
  *                (may be NULL)
- * Both arrays hold warmup + iterations entries. */
+ * Both arrays hold warmup + iterations entries.  Up to 32,768 energies the
+ * last pass writes where the host reads them, inside its times. */
 int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, size_t warmup, size_t iterations,
                        float *energies_out, double *host_ms, double *device_ms);
 
@@ -101,8 +105,9 @@ int bude_mi355x_destroy(bude_ctx *ctx);
  *      reference (whose model allocates and frees in every fasten call); it
  *      is for callers that cannot allocate device memory: code under stream
  *      capture, tight serving loops, harnesses that forbid hipMalloc. ----
- * One pass of the plain kernel over caller device memory, with the
- * energies bude_mi355x_create + bude_mi355x_fasten give for the same deck,
+ * One pass over caller device memory (split into as many launches as the
+ * scratch below needs, or shaped by ppwi and wgsize where that is the faster),
+ * with the energies bude_mi355x_create + bude_mi355x_fasten give for the same deck,
  * bit for bit.  Every pointer is a device pointer: protein[natpro],
  * ligand[natlig] and forcefield[ntypes] deck records, `poses` six rows of
  * pose_stride floats (row k at poses + k * pose_stride, the first nposes of
@@ -126,7 +131,11 @@ int bude_mi355x_fasten_noalloc(int device, const BudeAtom *protein, size_t natpr
                                void *stream);
 
 /* ---- batched ragged fasten_main: one protein, many ligands with their own
- *      atom and pose counts, in ONE persistent launch.  No counterpart in the
+ *      atom and pose counts, in one pass: sorted items where that pays, else
+ *      one persistent launch or, of few poses, a work-group per tile of 64.
+ *      The configuration shapes the persistent launch only (its tiles are of
+ *      64 poses where those are few), the order the tiles of both; every form
+ *      gives the same bits.  No counterpart in the
  *      reference, whose driver runs one (ligand, pose set) per
  *      Bude<PPWI>::fasten call (src/main.cpp:517-541) and skips pose counts
  *      that do not divide ppwi*wgsize (src/main.cpp:525-530); every pose of
@@ -139,7 +148,7 @@ typedef struct BudeBatchConfig {
   int32_t wgsize;         /* work-items per work-group: 64, 128, 256, 512 */
   int32_t waves_per_simd; /* persistent grid depth: CUs * 4 * waves_per_simd waves, 1..16 */
   int32_t order;          /* 0: tiles of the heaviest ligands first, 1: ligand order */
-  int32_t use_graph;      /* 1: replay a captured hipGraph (counter reset + kernel) */
+  int32_t use_graph;      /* 1: replay a captured hipGraph of the pass */
 } BudeBatchConfig;
 
 /* ligands[i] has natlig[i] atoms; poses[i] holds 6 rows of nposes[i] floats
@@ -147,8 +156,8 @@ typedef struct BudeBatchConfig {
 int bude_mi355x_batch_create(int device, const BudeAtom *protein, size_t natpro, const BudeFFParams *forcefield,
                              size_t ntypes, size_t nligands, const BudeAtom *const *ligands, const size_t *natlig,
                              const float *const *poses, const size_t *nposes, bude_batch **out);
-/* warmup + iterations persistent launches; device_ms[i] = hipEvent time of
- * launch i (counter reset included), may be NULL. */
+/* warmup + iterations passes; device_ms[i] = hipEvent time of pass i, may be
+ * NULL. */
 int bude_mi355x_batch_run(bude_batch *b, const BudeBatchConfig *cfg, size_t warmup, size_t iterations,
                           double *device_ms);
 /* The baseline the batch replaces: one plain launch per ligand, in ligand
@@ -156,7 +165,8 @@ int bude_mi355x_batch_run(bude_batch *b, const BudeBatchConfig *cfg, size_t warm
 int bude_mi355x_batch_run_separate(bude_batch *b, size_t ppwi, size_t wgsize, size_t warmup, size_t iterations,
                                    double *device_ms);
 /* Times candidate configurations (tile width, work-group size, grid depth,
- * tile order; graph replay) on this batch and returns the fastest. */
+ * tile order; graph replay) on this batch, one of those that give the same
+ * pass, and returns the fastest (the first where all are the same). */
 int bude_mi355x_batch_autotune(bude_batch *b, BudeBatchConfig *best, double *best_ms);
 /* Energies of ligand `ligand` (nposes[ligand] floats) from the last run. */
 int bude_mi355x_batch_energies(bude_batch *b, size_t ligand, float *out);
@@ -361,8 +371,9 @@ int bude_mi355x_combined_selected(bude_combined *c, size_t ligand, uint32_t *idx
                                   size_t *n);
 /* The last screen's sampled poses of one pair (what the MLP trained on, or
  * the field was validated on): pose indices within the ligand's pose set,
- * in sampling order, and their exact energies, which come from a split
- * kernel (four lanes per pose) and match the tiled kernel's to rounding.
+ * in sampling order, and their exact energies (a rescored pose's, bit for
+ * bit, where the samples are sorted; else from a split kernel, four lanes per
+ * pose, equal to rounding).
  * idx and energies may both be NULL to query *n. */
 int bude_mi355x_combined_labels(const bude_combined *c, size_t ligand, uint32_t *idx, float *energies, size_t cap,
                                 size_t *n);

@@ -1,5 +1,5 @@
 """Batched ragged screening: many ligands (own atom and pose counts) against
-one protein in one persistent launch (bude_mi355x_batch_* in the C ABI).
+one protein in one pass (bude_mi355x_batch_* in the C ABI).
 """
 from __future__ import annotations
 
