@@ -569,3 +569,29 @@ def test_batch_edges_and_errors(gpu_device):
         for l in range(3):
             idx, e = c.selected(l)
             assert np.array_equal(idx, one[l][0]) and np.array_equal(e.view(np.uint32), one[l][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("chunks", [1, 3])
+def test_sorted_rescoring_in_a_batch_of_proteins(gpu_device, chunks):
+    # selections large enough to sort (120,000 items of a chunk and more),
+    # every pose there four times, so that the ties at the threshold are rows
+    # past the sorted ones; one by one, overlapped, and against every pose
+    w = C.combined_workload(nproteins=3, nligands=6, nposes=5000, seed=61, natpro_range=(2000, 2600),
+                            natlig_range=(30, 70))
+    poses = [np.ascontiguousarray(np.tile(p, 4)) for p in w.poses]
+    cfg = C.default_config("field", keep_fraction=0.1003, gate_z=0.0, grid_spacing=1.0, pipeline_chunks=chunks)
+    with C.Combined(w.forcefield, w.ligands, poses, cfg, gpu_device) as c:
+        want = []
+        for p in w.proteins:
+            c.screen(p)
+            sel = [c.selected(l) for l in range(6)]
+            c.exhaustive()
+            for l, (idx, e) in enumerate(sel):
+                assert len(idx) >= kept(0.1003, 20000) and len(idx) % 4 == 0
+                assert np.array_equal(e.view(np.uint32), c.exact(l)[idx].view(np.uint32))
+            want.append(sel)
+        got = []
+        c.screen_batch(w.proteins, lambda i: got.append([c.selected(l) for l in range(6)]))
+    for a, b in zip(want, got):
+        for (i0, e0), (i1, e1) in zip(a, b):
+            assert np.array_equal(i0, i1) and np.array_equal(e0.view(np.uint32), e1.view(np.uint32))

@@ -6,6 +6,7 @@ holds a pose, never the sums."""
 import numpy as np
 import pytest
 
+import oracle_lib as O
 from minibude_amd import combined as C
 from minibude_amd import deck as D
 from minibude_amd import screen as S
@@ -82,3 +83,41 @@ def test_selections_of_many_rows_without_a_reach(gpu_device):
         idx, e = s.selected()
         exact = s.exhaustive()[0]
         assert len(idx) >= 300000 and np.array_equal(bits(e), bits(exact[idx]))
+
+
+def test_every_block_and_group_size(gpu_device):
+    # groups of 0 to 23 atoms and some larger, so that every exit of the
+    # pipelined pair loop is taken, by every register block and work-group
+    # size, against the FP64 oracle (16 FP32 epsilons of the sum of the terms'
+    # magnitudes, as for the deck's own call)
+    ntypes = 34
+    sizes = [t if t < 24 else 24 + 3 * (t - 24) for t in range(ntypes)]
+    pro = D.synth_protein(51, sum(sizes), ntypes)
+    pro["type"] = np.repeat(np.arange(ntypes, dtype=np.int32), sizes)
+    d = D.Deck(pro[np.random.default_rng(6).permutation(len(pro))], D.synth_ligand(52, 12, ntypes),
+               D.synth_forcefield(51, ntypes), D.synth_poses(53, 2000))
+    e64, mag = O.fasten_f64_mag(d, 0, d.nposes)
+    with Batch(LigandSet(d.protein, d.forcefield, [d.ligand], [d.poses]), gpu_device) as b:
+        b.run_separate(1, 64)
+        want = b.energies(0)
+        ok = mag > 0
+        assert np.all(want[~ok] == 0.0)
+        assert np.max(np.abs(want.astype(np.float64) - e64)[ok] / mag[ok]) < 16.0 * 2.0 ** -24
+        for ppwi in (1, 2, 4, 8, 16, 128):
+            for wgsize in (64, 128, 256, 512, 1024):
+                b.clear()
+                b.run_separate(ppwi, wgsize)
+                assert np.array_equal(bits(b.energies(0)), bits(want)), (ppwi, wgsize)
+
+
+@pytest.mark.parametrize("cfg", [BatchConfig(1, 64, 4, 0, 0), BatchConfig(2, 256, 8, 1, 1), BatchConfig(4, 128, 2, 0, 1),
+                                 BatchConfig(8, 512, 1, 1, 0)], ids=lambda c: f"p{c.ppwi}w{c.wgsize}")
+def test_persistent_kernel_equals_tiled(gpu_device, cfg):
+    ls = unreachable(120, [1, 7, 20, 33], [150001, 64, 90000, 60063], 54)  # 4,690 tiles of 64
+    with Batch(ls, gpu_device) as b:
+        b.run_separate(1, 64)
+        want = [b.energies(i) for i in range(4)]
+        b.clear()
+        b.run(cfg, warmup=1, iterations=2)
+        for i in range(4):
+            assert np.array_equal(bits(b.energies(i)), bits(want[i])), i
