@@ -34,7 +34,9 @@ struct bude_ctx {
   size_t natpro = 0, natlig = 0, ntypes = 0, nposes = 0, ngroups = 0;
   bude::DeviceBuffer protein, group_begin, coef, ligand, poses, energies;
   bude::items::Deck sorted;
-  bude::DeviceBuffer direct;  // scratch of the direct pass (empty: not used)
+  // scratch of the direct pass (null: not used): behind the energies, or by itself
+  float *direct = nullptr;
+  bude::DeviceBuffer direct_buf;
   // where the last pass of a call leaves its energies for the host to read
   // (not allocated: they are copied out)
   bude::PinnedBuffer result;
@@ -42,6 +44,10 @@ struct bude_ctx {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double context_ms = 0.0;
+
+  bude::items::Work work() const {
+    return {natpro, ngroups, 1, double(natlig) * double(nposes), double(nposes)};
+  }
 
   ~bude_ctx() {
     if (ev0) (void)hipEventDestroy(ev0);
@@ -148,7 +154,18 @@ extern "C" int bude_mi355x_create(int device, const BudeAtom *protein, size_t na
     st = bude::hip_check(hipMemcpy(static_cast<float *>(c->poses.ptr) + k * nposes, poses[k], nposes * sizeof(float),
                                    hipMemcpyHostToDevice),
                          "hipMemcpy poses");
-  if (!st) st = c->energies.alloc(nposes * sizeof(float));
+  // A deck of a size that is not sorted has the direct pass's sums behind its
+  // energies, where there is memory for both: a call's first pass over an
+  // allocation of their own takes 5 us longer (64 poses 50 us, 45).
+  const bude::items::Work work = c->work();
+  const size_t direct = bude::items::direct_bytes(nposes, natlig), padded = (nposes + 63) / 64 * 64;
+  const bool behind = direct <= bude::items::kDirectBytes && !bude::items::worth_sorting(work, 1, 1) &&
+                      !bude::items::worth_sorting(work, 8, 8);
+  if (!st) {
+    st = c->energies.alloc(padded * sizeof(float) + (behind ? direct : 0));
+    if (!st && behind) c->direct = static_cast<float *>(c->energies.ptr) + padded;
+    if (st == BUDE_ERR_OUT_OF_MEMORY && behind) st = c->energies.alloc(nposes * sizeof(float));
+  }
   if (!st) st = bude::hip_check(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev0), "hipEventCreate");
   if (!st) st = bude::hip_check(hipEventCreate(&c->ev1), "hipEventCreate");
@@ -156,17 +173,17 @@ extern "C" int bude_mi355x_create(int device, const BudeAtom *protein, size_t na
   if (!st)
     st = c->sorted.prepare(groups, forcefield, std::vector<BudeAtom>(ligand, ligand + natlig), {0, int32_t(natlig)},
                            {bude::items::Segment{0, 0, int64_t(nposes)}});
-  const size_t direct = bude::items::direct_bytes(nposes, natlig);
-  if (!st && !c->sorted.usable() && direct <= bude::items::kDirectBytes) {
-    st = c->direct.alloc(direct);
+  if (!st && !c->sorted.usable() && !behind && direct <= bude::items::kDirectBytes) {
+    st = c->direct_buf.alloc(direct);
     if (st == BUDE_ERR_OUT_OF_MEMORY) st = BUDE_OK;  // (the tiled kernel, then)
+    c->direct = static_cast<float *>(c->direct_buf.ptr);
   }
   // A copy of few energies costs 12 us and more a call whatever their number;
   // the last pass stores them over the bus instead (a call of 64 poses 39 and
   // 27 us, 4,097 61 and 48, 16,384 97 and 91).  With more of them the memory
   // for it, pinned, costs more than calls gain soon (65,536: 150 and 140 us a
   // call, but 300 us here).  Only a pass that writes an energy once goes there.
-  if (!st && nposes <= kHostResult && (c->sorted.usable() || c->direct.ptr)) {
+  if (!st && nposes <= kHostResult && (c->sorted.usable() || c->direct)) {
     st = c->result.alloc(nposes * sizeof(float));
     if (st == BUDE_ERR_OUT_OF_MEMORY) st = BUDE_OK;  // (copied out, then)
   }
@@ -207,15 +224,13 @@ extern "C" int bude_mi355x_fasten(bude_ctx *ctx, size_t ppwi, size_t wgsize, siz
   a.form = bude::plain_form();
   bude::items::DirectArgs direct{a.protein, a.group_begin, a.coef,   a.ligand, a.poses, a.energies, a.stride,
                                  a.nposes,  a.natlig,      a.ngroups, a.form,   nullptr,
-                                 static_cast<float *>(ctx->direct.ptr)};
+                                 ctx->direct};
   const size_t passes = warmup + iterations;
   // Few energies: the tiled kernel never pays, as they would be copied out.
-  const bude::items::Work work{ctx->natpro, ctx->ngroups, 1, double(ctx->natlig) * double(ctx->nposes),
-                               double(ctx->nposes)};
   const bool few = ctx->nposes <= kHostResult;
   const int rb = bude::plain_register_block(int(ppwi), int(wgsize), ctx->nposes);
   const bool sorted = few ? ctx->sorted.usable() : ctx->sorted.worth(int(ppwi), rb);
-  const bool use_direct = !sorted && ctx->direct.ptr && (few || bude::items::worth_direct(work, int(ppwi), rb));
+  const bool use_direct = !sorted && ctx->direct && (few || bude::items::worth_direct(ctx->work(), int(ppwi), rb));
 
   for (size_t i = 0; i < passes; i++) {
     const bool to_host = energies_out && ctx->result.ptr && (sorted || use_direct) && i + 1 == passes;

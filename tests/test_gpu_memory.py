@@ -84,9 +84,13 @@ def test_a_pass_without_room_leaves_later_screens_as_they_are(gpu_device, bound,
     assert all(same_bits(a, b) for a, b in zip(*out))
 
 
-@pytest.mark.parametrize("mb", [16, 4])  # no room to sort; none for the direct pass's sums (6.8 MB) either
-def test_a_deck_without_room_for_scratch_is_scored(gpu_device, bound, mb):
-    d = D.synth_deck(938, 26, 65536, seed=52)
+@pytest.mark.parametrize("natpro, natlig, nposes, mb", [
+    (938, 26, 65536, 16),   # no room to sort
+    (938, 26, 65536, 4),    # nor for the direct pass's sums (6.8 MB)
+    (30, 400, 32768, 16),   # not sorted: no room for the sums (52 MB)
+])
+def test_a_deck_without_room_for_scratch_is_scored(gpu_device, bound, natpro, natlig, nposes, mb):
+    d = D.synth_deck(natpro, natlig, nposes, seed=52)
     with Context(d, gpu_device) as c:
         want = c.fasten(1, 64).energies
     bound.here().more(mb)
