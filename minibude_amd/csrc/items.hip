@@ -164,9 +164,8 @@ __device__ __forceinline__ uint32_t axis_cell(float x, float lo, float inv) {
 
 // Cells are numbered along a Hilbert curve: consecutive cells share a face,
 // so items that straddle cells keep a small box (in Morton order a step can
-// cross the whole grid; scoring 4,096 x 64 atoms x 1,048,576 poses tested 165
-// atoms per item instead of 182, and 201 instead of 240 with a sixteenth of
-// the poses).  Steps of Skilling's transform ("Programming the Hilbert
+// cross the whole grid; 9 % fewer atoms per item over 4,096 x 64 atoms x
+// 1,048,576 poses, 16 % with a sixteenth of the poses).  Steps of Skilling's transform ("Programming the Hilbert
 // curve", AIP Conf. Proc. 707, 2004) for a 16^3 grid.
 constexpr uint16_t hilbert_place(uint32_t x, uint32_t y, uint32_t z) {
   uint32_t v[3] = {x, y, z};
@@ -409,9 +408,10 @@ __device__ __forceinline__ void mask_pairs(uint64_t mask, float x, float y, floa
 }
 
 // The same, each atom with the hinges whose reach it is in only (bits of ms,
-// mq, md); the others are exactly zero for all the items (of 165 atoms per
-// item of the 4,096 x 64 deck, 31 are within steric reach, 101 within the
-// charge's, 132 within the desolvation's: 9.2 VALU per pair instead of 11.1).
+// mq, md); the others are exactly zero for all the items (of the 150 atoms per
+// item of the 4,096 x 64 deck a fifth are within steric reach, three fifths
+// within the charge's, four fifths within the desolvation's: 9.2 VALU of
+// arithmetic per pair instead of 11.1).
 // The tests are scalar branches between a pair's 6 distance VALU and the 2 of
 // each hinge: they pay with four items per lane or more (4,096 x 64 x
 // 1,048,576: 5.00 -> 4.46 ms; with one or two the branches cost as much).
@@ -455,7 +455,8 @@ constexpr int kShare = 4096;
 // (lane = atom) against its own items' box, and every atom in reach out of its lane (three
 // readlanes) to all lanes' RB items.  RB > 1 shares the steps and the
 // readlanes between items at the price of a larger box; VALU issue bounds it
-// (about 12 VALU per pair in reach of the box and 3 / RB for its atom).
+// (11 VALU per pair in reach of the box with eight items per lane, its atom's
+// lane reads and the box tests among them).
 template <int RB, int FORM, bool LIST>
 __global__ __launch_bounds__(256) void score_kernel(const float4 *__restrict__ protein, int natpro,
                                                     const PairCoef *__restrict__ coef,
